@@ -14,11 +14,13 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/sjf.h"
@@ -82,6 +84,8 @@ struct sjf_engine {
     std::vector<uint32_t> matw_h;
     std::vector<sjf_material> lut_h;
     uint32_t* matw = nullptr;
+    uint32_t* seg = nullptr;  // material segment codes (k_segments)
+    double pole_bytes = 0;    // pole state the step moves
     void* lut = nullptr;
     int nmat = 1;
     int maxp = 0;
@@ -253,39 +257,65 @@ double inv_eps_at(const sjf_engine* e, long q, int c) {
 // Row-of-threads form: (rows + 1) thread rows of nz threads per workgroup, 32-bit offsets.
 bool thread_rows_fit(const sjf_engine* e, int rows) { return rows >= 1 && (long)(rows + 1) * e->g.nz <= 1024; }
 
-// Field bytes one step of these engines moves (E and H read and written) above which the one-row
-// step kernels store with the non-temporal hint.  Measured on MI355X (FP32): 1024x768x512 7.17 ->
-// 6.86 ms per step, 512x512x256 1.230 -> 1.205 ms, the 256x256x128 reverse step 0.282 -> 0.267
-// ms, one 192x192x96 design variant (170 MB of fields) 12.46 -> 12.75 G cell-updates/s per
-// gradient; the 96^3 FP64 box (85 MB, which the 256 MB Infinity Cache holds from one step to the
-// next) 0.046 -> 0.059 ms with the hint, so it keeps plain stores.
-constexpr double kStreamBytes = 128e6;
 double field_bytes(const sjf_engine* e) { return 12.0 * e->prec * (double)e->N; }
 
-// z cells per pass of a register-rows workgroup with `rows` rows per thread: the set value, else
-// 128-cell passes for one row per thread on a non-periodic z line that is a multiple of 256
-// cells above 256 or longer than 1024, else the whole line.  Measured on MI355X, 1024x768x512
-// FP32: one pass of 512 threads leaves two 8-wave workgroups per CU (4 waves per SIMD of the 5
-// the registers allow) and runs 8.07 ms per step; two passes of 256 threads (5 workgroups per
-// CU) run 7.31 ms.  With the non-temporal stores, two boxes: 256-cell passes 6.45 and 6.87 ms,
-// 128-cell passes (ten 2-wave workgroups per CU) 6.20 and 6.69 ms, 64-cell passes 6.80 ms.
-// On 512x512x256 one pass wins: 128-cell passes 1.295 against 1.183 ms.
-int zseg_of(const sjf_engine* e, int rows) {
+// Field bytes above which the one-row reverse step stores with the non-temporal hint (measured on
+// MI355X: 256x256x128 FP32 0.282 -> 0.267 ms).
+constexpr double kAdjStreamBytes = 128e6;
+
+// Bytes one step touches above which its stores take the non-temporal hint: below, the 256 MB Infinity
+// Cache holds what a step wrote until the next one reads it.  Pole state counts in whole 64-cell
+// segments, so the line lies above that size.  Measured on MI355X, us per step without and with the
+// hint: FP64 96x96x96 (184 MB) 39.8, 48.9; FP32 150x150x96 (234 MB) 47.2, 50.2; FP32 150x150x160
+// periodic (282 MB) 65.9, 63.4; FP32 151x133x117 (285 MB) 53.8, 57.0; FP64 120x120x96 (291 MB) 67.8,
+// 70.4; FP64 128x128x100 (350 MB) 87.5, 78.4; FP32 192x192x96 (386 MB) 80.0, 74.6; FP32 200x200x125
+// (592 MB) 125.2, 113.9.
+constexpr double kStreamBytes = 300e6;
+// What one step touches: two field sets, pole state, PML auxiliaries, material words
+double step_set_bytes(const sjf_engine* e) {
+    double b = field_bytes(e) + e->pole_bytes + (e->uniform ? 0.0 : 4.0 * (double)e->N);
+    for (int d = 0; d < 3; ++d) b += 6.0 * e->prec * (double)e->slab[d];
+    return b;
+}
+
+// Whether a tile's exchange planes (values) and the coefficients of nmat materials fit 64 KiB.  The
+// padded table and a second copy of the planes then stay within the CU's 160 KiB.
+template <typename T>
+bool lds_fits(size_t values, int nmat) {
+    return sizeof(T) * values + (14 * sizeof(T) + 8) * (size_t)nmat <= 65536;
+}
+
+// z cells per pass of a register-rows workgroup with `rows` rows per thread: the set value, else the
+// whole line, but 128-cell passes for one row per thread on a non-periodic z line longer than the
+// 1024 threads of a workgroup.  The tile that the library chooses also takes 256-cell passes in FP64
+// above 512 cells (a 1024-thread FP64 workgroup spills) and otherwise spans the line (448x224x512
+// FP32: one pass 0.731 ms per step, 128-cell passes 0.846 ms: their tile takes 161 registers, 3 waves
+// per SIMD, the one-pass tile 109 and 4); a tile set by the caller (given) keeps its documented
+// 128-cell passes on lines above 256 cells that are a multiple of 256.
+int zseg_of(const sjf_engine* e, int rows, bool given) {
     const int nz = e->g.nz;
     if (e->zseg > 0) return std::min(e->zseg, nz);
-    if (rows == 1 && !e->g.periodic[2] && nz > 256 && (nz % 256 == 0 || nz > 1024)) return 128;
+    if (rows == 1 && !e->g.periodic[2]) {
+        if (nz > 1024 || (given && nz > 256 && nz % 256 == 0)) return 128;
+        if (!given && e->prec == 8 && nz > 512) return 256;
+    }
     return nz;
 }
 
-// FP64 tiles stop at 512 threads: at 1024 the register budget of 128 per thread spills
-int default_thread_rows(const sjf_engine* e) { return std::max(1, (e->prec == 8 ? 512 : 1024) / e->g.nz - 1); }
+// Thread rows a row-of-threads tile owns by default: as many as 1024 threads hold (FP64 512: at 1024
+// the register budget of 128 per thread spills) with the halo row, spread evenly over the grid's rows.
+int default_thread_rows(const sjf_engine* e) {
+    const int most = std::max(1, (e->prec == 8 ? 512 : 1024) / e->g.nz - 1);
+    const int tiles = (e->g.ny + most - 1) / most;
+    return (e->g.ny + tiles - 1) / tiles;
+}
 
-int block_threads_for(const sjf_engine* e, int form, int ty) {
-    const int t = form == SJF_TILE_THREAD_ROWS ? (ty + 1) * e->g.nz : zseg_of(e, ty);
+int block_threads_for(const sjf_engine* e, int form, int ty, bool given) {
+    const int t = form == SJF_TILE_THREAD_ROWS ? (ty + 1) * e->g.nz : zseg_of(e, ty, given);
     return ((t + 63) / 64) * 64;
 }
 
-int block_threads(const sjf_engine* e) { return block_threads_for(e, e->form, e->ty); }
+int block_threads(const sjf_engine* e) { return block_threads_for(e, e->form, e->ty, e->tile_set); }
 
 int tiles_of(const sjf_engine* e, int ty, int xc) {
     const int nty = (e->g.ny + ty - 1) / ty;
@@ -303,11 +333,11 @@ int np_variant_of(int maxp, bool uniform) {
 }
 
 template <typename T>
-sjf::StepArgs<T> step_args(const sjf_engine* e, int ty, int xc) {
+sjf::StepArgs<T> step_args(const sjf_engine* e, int ty, int xc, bool given = false) {
     sjf::StepArgs<T> a;
     std::memset(&a, 0, sizeof(a));
     a.rt = ty + 1;
-    a.zseg = zseg_of(e, ty);
+    a.zseg = zseg_of(e, ty, given);
     a.nx = e->g.nx;
     a.ny = e->g.ny;
     a.nz = e->g.nz;
@@ -324,6 +354,7 @@ sjf::StepArgs<T> step_args(const sjf_engine* e, int ty, int xc) {
     a.uniform = e->uniform ? 1 : 0;
     a.nmat = e->nmat;
     a.matw = e->matw;
+    a.seg = e->seg;
     a.lut = (const sjf::MatLut<T>*)e->lut;
     a.Q = (T*)e->Qbuf;
     a.P = (T*)e->Pbuf;
@@ -353,8 +384,9 @@ struct LaunchSet {
     int prec = 4, ty = 1, npv = 0, block = 64;
     int form = SJF_TILE_REGISTER_ROWS;
     int xc = 0;  // x-chunk of every instance of a batch (0: each engine's own)
+    bool tile_set = false;  // form and xc of a batch were set by the caller
     bool zpass = false;  // register form with some z line stepped in passes (k_step_z)
-    bool nts = false;    // one-row tiles store with the non-temporal hint (field_bytes > kStreamBytes)
+    bool nts = false;    // stores with the non-temporal hint (step_set_bytes > kStreamBytes)
     size_t lds = 0;
     std::vector<long> versions;
     bool built = false;
@@ -453,22 +485,23 @@ int build_set_t(LaunchSet* s) {
         const int rows = (s == e->own) ? e->ty
                                        : (s->form == SJF_TILE_THREAD_ROWS ? default_thread_rows(e) : s->ty);
         const int xc = (s == e->own || s->xc <= 0) ? e->xc : std::min(s->xc, e->g.nx);
-        args.push_back(step_args<T>(e, rows, xc));
+        const bool given = s == e->own ? e->tile_set : s->tile_set;
+        args.push_back(step_args<T>(e, rows, xc, given));
         first.push_back(t);
         t += tiles_of(e, rows, xc);
         maxp = std::max(maxp, e->maxp);
         all_uniform = all_uniform && e->uniform;
-        block = std::max(block, block_threads_for(e, s->form, rows));
-        if (s->form == SJF_TILE_REGISTER_ROWS && zseg_of(e, rows) < e->g.nz) {
+        block = std::max(block, block_threads_for(e, s->form, rows, given));
+        if (s->form == SJF_TILE_REGISTER_ROWS && zseg_of(e, rows, given) < e->g.nz) {
             if (rows != 1) return fail(e0, SJF_E_UNSUPPORTED, "z passes run one row per thread");
             zh = std::max<size_t>(zh, 4 * (size_t)xc);
         }
-        if (block_threads_for(e, s->form, rows) > 1024)
+        if (block_threads_for(e, s->form, rows, given) > 1024)
             return fail(e0, SJF_E_UNSUPPORTED, "a z line longer than 1024 cells needs one row per thread (z passes)");
     }
     s->zpass = zh > 0;
     double fb = 0;
-    for (sjf_engine* e : s->eng) fb += field_bytes(e);
+    for (sjf_engine* e : s->eng) fb += step_set_bytes(e);
     s->nts = fb > kStreamBytes;
     first.push_back(t);
     s->ntiles = t;
@@ -476,9 +509,10 @@ int build_set_t(LaunchSet* s) {
     s->npv = np_variant_of(maxp, all_uniform);
     int nmat = 1;
     for (sjf_engine* e : s->eng) nmat = std::max(nmat, e->nmat);
-    s->lds = (s->form == SJF_TILE_THREAD_ROWS ? sizeof(T) * 6 * block : sizeof(T) * 4 * s->ty * block) +
-             sizeof(sjf::MatLut<T>) * nmat + sizeof(T) * zh;
-    if (s->lds > 65536)
+    s->lds = (s->form == SJF_TILE_THREAD_ROWS ? sizeof(T) * 12 * block : sizeof(T) * 4 * s->ty * (block + 1)) +
+             sjf::lut_lds_bytes<T>(nmat) + sizeof(T) * zh;
+    // (the row-of-threads tile holds its exchange planes twice: 64 KiB bound one copy)
+    if (!lds_fits<T>((s->form == SJF_TILE_THREAD_ROWS ? 6 : 4 * s->ty) * (size_t)block + zh, nmat))
         return fail(e0, SJF_E_UNSUPPORTED, "tile needs more than 64 KiB of LDS; use fewer rows");
     int rc = upload_vec(e0, s->stream, &s->d_args, args);
     if (!rc) rc = upload_vec(e0, s->stream, (void**)&s->d_tile_first, first);
@@ -644,54 +678,54 @@ bool set_stale(const LaunchSet* s) {
         }                                                                                \
     } while (0)
 
-template <typename T, int NP, int MAXT>
+// The fused step of a launch set, by its form and workgroup size.  Kernels whose registers leave room
+// for a 1024-thread workgroup (128 per lane: the FP32 one-row tile) are compiled for it alone.
+template <typename T, int NP>
 int launch_step_np(LaunchSet* s) {
     const dim3 grid(s->ntiles), block(s->block);
     const auto* args = (const sjf::StepArgs<T>*)s->d_args;
     const int n = (int)s->eng.size();
+#define SJF_LAUNCH(...) hipLaunchKernelGGL((__VA_ARGS__), grid, block, s->lds, s->stream, args, s->d_tile_first, n)
     if (s->form == SJF_TILE_THREAD_ROWS) {
-        hipLaunchKernelGGL((sjf::k_step_rows<T, NP, MAXT>), grid, block, s->lds, s->stream, args, s->d_tile_first, n);
-        SETCHK(s, hipGetLastError());
-        return SJF_OK;
+        if (s->block <= 512) {
+            if (s->nts) SJF_LAUNCH(sjf::k_step_rows<T, NP, 512, true>);
+            else SJF_LAUNCH(sjf::k_step_rows<T, NP, 512>);
+        } else if (s->nts) {
+            SJF_LAUNCH(sjf::k_step_rows<T, NP, 1024, true>);
+        } else {
+            SJF_LAUNCH(sjf::k_step_rows<T, NP, 1024>);
+        }
+    } else if (s->zpass) {
+        if (s->block > 256) SJF_LAUNCH(sjf::k_step_z<T, NP, 1024>);
+        else if (s->nts) SJF_LAUNCH(sjf::k_step_z<T, NP, 256, true>);
+        else SJF_LAUNCH(sjf::k_step_z<T, NP, 256>);
+    } else if (s->ty == 1) {
+        constexpr int M = sizeof(T) == 4 ? 1024 : 512;
+        if (s->block > M) SJF_LAUNCH(sjf::k_step<T, 1, NP, 1024>);
+        else if (s->nts) SJF_LAUNCH(sjf::k_step<T, 1, NP, M, true>);
+        else SJF_LAUNCH(sjf::k_step<T, 1, NP, M>);
+    } else if (s->ty == 2) {
+        if (s->block <= 512) SJF_LAUNCH(sjf::k_step<T, 2, NP, 512>);
+        else SJF_LAUNCH(sjf::k_step<T, 2, NP, 1024>);
+    } else if (s->ty == 4) {
+        if (s->block <= 512) SJF_LAUNCH(sjf::k_step<T, 4, NP, 512>);
+        else SJF_LAUNCH(sjf::k_step<T, 4, NP, 1024>);
+    } else {
+        return fail(s->eng[0], SJF_E_ARG, "tile rows must be 1, 2 or 4");
     }
-    if (s->zpass) {
-        if (s->nts)
-            hipLaunchKernelGGL((sjf::k_step_z<T, NP, MAXT, true>), grid, block, s->lds, s->stream, args, s->d_tile_first, n);
-        else
-            hipLaunchKernelGGL((sjf::k_step_z<T, NP, MAXT>), grid, block, s->lds, s->stream, args, s->d_tile_first, n);
-        SETCHK(s, hipGetLastError());
-        return SJF_OK;
-    }
-    switch (s->ty) {
-        case 1:
-            if (s->nts)
-                hipLaunchKernelGGL((sjf::k_step<T, 1, NP, MAXT, true>), grid, block, s->lds, s->stream, args, s->d_tile_first, n);
-            else
-                hipLaunchKernelGGL((sjf::k_step<T, 1, NP, MAXT>), grid, block, s->lds, s->stream, args, s->d_tile_first, n);
-            break;
-        case 2: hipLaunchKernelGGL((sjf::k_step<T, 2, NP, MAXT>), grid, block, s->lds, s->stream, args, s->d_tile_first, n); break;
-        case 4: hipLaunchKernelGGL((sjf::k_step<T, 4, NP, MAXT>), grid, block, s->lds, s->stream, args, s->d_tile_first, n); break;
-        default: return fail(s->eng[0], SJF_E_ARG, "tile rows must be 1, 2 or 4");
-    }
+#undef SJF_LAUNCH
     SETCHK(s, hipGetLastError());
     return SJF_OK;
 }
 
-template <typename T, int MAXT>
-int launch_step_b(LaunchSet* s) {
-    switch (s->npv) {
-        case 0: return launch_step_np<T, 0, MAXT>(s);
-        case 1: return launch_step_np<T, 1, MAXT>(s);
-        case 3: return launch_step_np<T, 3, MAXT>(s);
-        default: return launch_step_np<T, 4, MAXT>(s);
-    }
-}
-
 template <typename T>
 int launch_step_t(LaunchSet* s) {
-    if (s->block <= 256) return launch_step_b<T, 256>(s);
-    if (s->block <= 512) return launch_step_b<T, 512>(s);
-    return launch_step_b<T, 1024>(s);
+    switch (s->npv) {
+        case 0: return launch_step_np<T, 0>(s);
+        case 1: return launch_step_np<T, 1>(s);
+        case 3: return launch_step_np<T, 3>(s);
+        default: return launch_step_np<T, 4>(s);
+    }
 }
 
 // One time step of every engine in the set.  `sample` launches the monitor gather first.
@@ -933,26 +967,56 @@ int timed_set(LaunchSet* s, long n, double* ms_total, double* ms_kernel_mean) {
 
 // ======================================================================== engine helpers ==
 
+// Waves per SIMD that the step kernel of an engine's tile runs (its registers; see the kernels).
+template <typename T>
+int tile_waves(const sjf_engine* e) {
+    auto of = [&](auto np) {
+        constexpr int NP = decltype(np)::value;
+        if (e->form == SJF_TILE_THREAD_ROWS) return sjf::rows_waves<T, NP>();
+        return zseg_of(e, 1, false) < e->g.nz ? sjf::step_waves<T, 1, NP, true>() : sjf::step_waves<T, 1, NP>();
+    };
+    switch (np_variant_of(e->maxp, e->uniform)) {
+        case 0: return of(std::integral_constant<int, 0>{});
+        case 1: return of(std::integral_constant<int, 1>{});
+        case 3: return of(std::integral_constant<int, 3>{});
+        default: return of(std::integral_constant<int, 4>{});
+    }
+}
+
+// Default tile, after a change of the materials (their pole slots set the kernel's registers).
+//
+// Form: thread rows where a workgroup holds three owned rows or more, which share one halo row and
+// leave few lanes idle on a z line of any length (FP32 below 256 cells, FP64 below 128).  Measured on
+// MI355X, us per step of the best x-chunk, thread rows and one register row per workgroup: FP64 41^3
+// 13.0, 15.3; 72x64x56 20.4, 21.0; 96^3 36.1, 42.0; 101^3 39.7, 54.0; 128^3 105.7, 105.3; FP32
+// 192x192x96 80.4, 93.9; 151x133x117 54.4, 70.2; 256x256x128 191.7, 201.7; 150x150x200 90.0, 112.7;
+// 120x160x250 95.9, 120.6; 512x512x256 1061, 1039.
+//
+// x-chunk: a workgroup's time is its chunk and about two planes of start-up, and the chip runs
+// `slots` workgroups at once; a launch that needs a little more than a whole number of such rounds
+// waits for a last one that is nearly empty (192x192x96 FP32, 9 thread rows, 256 slots: 242
+// workgroups of 18 planes 80.6 us, 264 of 16 planes 112 us, 484 of 9 planes 83.9 us).  So: the
+// rounds for which rounds * (chunk + 2) is least, with chunks of at most 64 planes (a longer march
+// drifts apart) and at most 16 rounds.
 void choose_tile(sjf_engine* e) {
     if (e->tile_set) return;
-    // Defaults measured on MI355X: for short z lines (nz < 96) the row-of-threads form wins
-    // (up to ~1024 threads per workgroup, few halo rows); from 96 cells on one row per thread
-    // keeps more waves resident (192x192x96 FP32: 0.120 ms against 0.126 ms for 4 thread rows;
-    // 96^3 FP64: 0.0467 against 0.0485 ms).  The autotuner refines per workload.
-    long target_groups = 16384;
-    e->form = SJF_TILE_REGISTER_ROWS;
-    e->ty = 1;
-    const int rows = e->g.nz > 96 ? default_thread_rows(e) : std::min(3, default_thread_rows(e));
-    if (e->g.nz < 96 && thread_rows_fit(e, rows)) {
-        e->form = SJF_TILE_THREAD_ROWS;
-        e->ty = rows;
-        target_groups = 2048;
+    const int rows = default_thread_rows(e), full = e->prec == 8 ? 128 : 256;
+    const bool thread_rows = e->g.nz < full && zseg_of(e, 1, false) == e->g.nz && thread_rows_fit(e, rows);
+    e->form = thread_rows ? SJF_TILE_THREAD_ROWS : SJF_TILE_REGISTER_ROWS;
+    e->ty = thread_rows ? rows : 1;
+    const int waves = e->prec == 4 ? tile_waves<float>(e) : tile_waves<double>(e);
+    const long slots = 256L * std::max(1, 4 * waves / (block_threads(e) / 64));
+    const int nx = e->g.nx, nty = (e->g.ny + e->ty - 1) / e->ty;
+    long best = LONG_MAX;
+    int xc = std::min(nx, 64);
+    for (int m = 1; m <= 16; ++m) {
+        const long nxc = std::min<long>(nx, m * slots / nty);
+        if (nxc < 1) continue;
+        const int c = (int)((nx + nxc - 1) / nxc);
+        if (c > 64) continue;
+        if (m * (c + 2L) < best) best = m * (c + 2L), xc = c;
     }
-    const int nty = (e->g.ny + e->ty - 1) / e->ty;
-    long nxc = std::max(1L, (target_groups + nty - 1) / nty);
-    nxc = std::min<long>(nxc, e->g.nx);
-    const int xc = (int)((e->g.nx + nxc - 1) / nxc);
-    e->xc = std::max(std::min(4, e->g.nx), std::min(xc, e->g.nx));
+    e->xc = xc;
 }
 
 int free_all(sjf_engine* e) {
@@ -961,6 +1025,7 @@ int free_all(sjf_engine* e) {
     for (int b = 0; b < 2; ++b) dev_free(e->Fbuf[b]);
     dev_free(e->d_step);
     dev_free(e->matw);
+    dev_free(e->seg);
     dev_free(e->lut);
     dev_free(e->dinv);
     dev_free(e->emap);
@@ -1029,12 +1094,12 @@ int read_component_box(sjf_engine* e, int comp, const int* lo, const int* hi, do
 
 template <typename T>
 int upload_lut_t(sjf_engine* e) {
-    std::vector<sjf::MatLut<T>> l(e->nmat);
+    std::vector<sjf::MatLut<T>> l(e->nmat + 1);  // the last: zeros, for design voxels
+    std::memset((void*)l.data(), 0, sizeof(sjf::MatLut<T>) * l.size());
     const double dt = e->dt;
     for (int m = 0; m < e->nmat; ++m) {
         const sjf_material& M = e->lut_h[m];
         sjf::MatLut<T>& L = l[m];
-        std::memset(&L, 0, sizeof(L));
         L.inv_eps = (T)(1.0 / M.eps_inf);
         L.eps_inf = (T)M.eps_inf;
         L.np = M.npoles;
@@ -1044,19 +1109,42 @@ int upload_lut_t(sjf_engine* e) {
             const double gm = 2 * M_PI * M.gamma[s];
             const double g = gm * dt / 2;
             const double Lf = M.is_drude[s] ? 0.0 : 1.0;
-            L.alpha[s] = (T)((1 - g) / (1 + g));
-            L.beta[s] = (T)(-Lf * w0 * w0 * dt * dt / (1 + g));
-            L.c3[s] = (T)(M.sigma[s] * (w0 * w0) * dt * dt / (1 + g));
+            L.pole[s].alpha = (T)((1 - g) / (1 + g));
+            L.pole[s].beta = (T)(-Lf * w0 * w0 * dt * dt / (1 + g));
+            L.pole[s].c3 = (T)(M.sigma[s] * (w0 * w0) * dt * dt / (1 + g));
+            L.pole[s].lor = (T)Lf;
             if (!M.is_drude[s]) L.lorentz_mask |= 1 << s;
         }
     }
     dev_free(e->lut);
-    int rc = dev_alloc(e, &e->lut, sizeof(sjf::MatLut<T>) * e->nmat);
+    int rc = dev_alloc(e, &e->lut, sizeof(sjf::MatLut<T>) * l.size());
     if (rc) return rc;
-    return h2d(e, e->lut, l.data(), sizeof(sjf::MatLut<T>) * e->nmat);
+    return h2d(e, e->lut, l.data(), sizeof(sjf::MatLut<T>) * l.size());
 }
 
 int upload_lut(sjf_engine* e) { return e->prec == 4 ? upload_lut_t<float>(e) : upload_lut_t<double>(e); }
+
+// Segment codes of the material words and the LUT on the device (after a change of either), and the
+// bytes of pole state the step moves (whole segments).
+int update_segments(sjf_engine* e) {
+    const long rows = (long)e->g.nx * e->g.ny, n = rows * ((e->g.nz + 63) / 64);
+    if (int rc = dev_alloc(e, (void**)&e->seg, sizeof(uint32_t) * (n + 3))) return rc;
+    auto* slots = (unsigned long long*)(e->seg + n + (n & 1));
+    unsigned long long count = 0;
+    HIPCHK(e, hipMemcpyAsync(slots, &count, sizeof(count), hipMemcpyHostToDevice, e->stream));
+    const dim3 grid((unsigned)((n + 3) / 4)), block(256);
+    if (e->prec == 4)
+        hipLaunchKernelGGL((sjf::k_segments<float>), grid, block, 0, e->stream, e->matw, (const sjf::MatLut<float>*)e->lut,
+                           e->seg, rows, e->g.nz, e->nmat, slots);
+    else
+        hipLaunchKernelGGL((sjf::k_segments<double>), grid, block, 0, e->stream, e->matw,
+                           (const sjf::MatLut<double>*)e->lut, e->seg, rows, e->g.nz, e->nmat, slots);
+    HIPCHK(e, hipGetLastError());
+    HIPCHK(e, hipMemcpyAsync(&count, slots, sizeof(count), hipMemcpyDeviceToHost, e->stream));
+    HIPCHK(e, hipStreamSynchronize(e->stream));
+    e->pole_bytes = 64.0 * 3 * (e->Pbuf ? 2 : 1) * e->prec * (double)count;
+    return SJF_OK;
+}
 
 // 1/eps_inf of the effective map on the device in the plane layout [x][Ex Ey Ez][y][z]
 template <typename T>
@@ -1174,11 +1262,14 @@ int apply_materials(sjf_engine* e) {
     dev_free(e->Pbuf);
     if (maxp > 0) {
         rc = dev_alloc(e, &e->Qbuf, (size_t)e->prec * 3 * maxp * e->N);
-        if (!rc && anylor) rc = dev_alloc(e, &e->Pbuf, (size_t)e->prec * 3 * maxp * e->N);
+        // FP32 slots alternate between the two arrays, Drude ones included
+        if (!rc && (anylor || e->prec == 4)) rc = dev_alloc(e, &e->Pbuf, (size_t)e->prec * 3 * maxp * e->N);
         if (rc) return rc;
     }
     rc = upload_lut(e);
+    if (!rc) rc = update_segments(e);
     if (rc) return rc;
+    choose_tile(e);
     e->version++;
     return SJF_OK;
 }
@@ -1332,7 +1423,7 @@ void launch_adj_one_row(sjf_engine* e, const sjf::AdjArgs<T>& g, int block, unsi
 template <typename T, int NP>
 void launch_adj_np(sjf_engine* e, const sjf::AdjArgs<T>& g, int block, unsigned tiles, size_t lds) {
     // the reverse step streams the adjoint fields as the forward step streams E and H
-    if (field_bytes(e) > kStreamBytes) launch_adj_one_row<T, NP, true>(e, g, block, tiles, lds);
+    if (field_bytes(e) > kAdjStreamBytes) launch_adj_one_row<T, NP, true>(e, g, block, tiles, lds);
     else launch_adj_one_row<T, NP, false>(e, g, block, tiles, lds);
 }
 
@@ -1359,8 +1450,8 @@ int launch_adj_step(sjf_engine* e, const sjf::AdjArgs<T>& g, int npv, int block,
 // LDS of the reverse step: E-term and H-term exchange planes and the material table
 template <typename T>
 size_t adj_lds_bytes(const sjf_engine* e, bool rows, int block) {
-    const size_t lut = sizeof(sjf::MatLut<T>) * e->nmat;
-    return rows ? sizeof(T) * (8 * (size_t)block + 2 * (size_t)e->g.nz) + lut : sizeof(T) * 12 * (size_t)block + lut;
+    const size_t lut = sjf::lut_lds_bytes<T>(e->nmat);
+    return rows ? sizeof(T) * (8 * (size_t)block + 2 * (((size_t)e->g.nz + 1) & ~(size_t)1)) + lut : sizeof(T) * 12 * (size_t)block + lut;
 }
 
 template <typename T>
@@ -1473,7 +1564,8 @@ int adjoint_run_t(sjf_engine* e, long nsteps, long K, long gap, double* J_out, d
     const int block = (((rows ? arows + 1 : 1) * e->g.nz + 63) / 64) * 64;
     const unsigned tiles = (unsigned)((long)g.f.nty * ((e->g.nx + g.f.xc - 1) / g.f.xc));
     const size_t lds = adj_lds_bytes<T>(e, rows, block);
-    if (lds > 65536) return bail(fail(e, SJF_E_UNSUPPORTED, "adjoint tile needs more than 64 KiB of LDS"));
+    if (!lds_fits<T>(rows ? 8 * (size_t)block + 2 * (size_t)e->g.nz : 12 * (size_t)block, e->nmat))
+        return bail(fail(e, SJF_E_UNSUPPORTED, "adjoint tile needs more than 64 KiB of LDS"));
     const int npv = np_variant_of(e->maxp, e->uniform);
     auto ebar = [&]() { return g.A[g.rd]; };
     const double ie[3] = {inv_eps_at(e, gap, 0), inv_eps_at(e, gap, 1), inv_eps_at(e, gap, 2)};
@@ -1740,9 +1832,10 @@ int batch_adjoint_run_t(LaunchSet* s, long nsteps, long K, const long* gaps, con
     const auto* tabp = (const sjf::AdjBatchDev<T>*)d_tab;
     const sjf::AdjArgs<T>* argd[2] = {(const sjf::AdjArgs<T>*)d_args0, (const sjf::AdjArgs<T>*)d_args1};
     const int block = brows ? bblock : ((e0->g.nz + 63) / 64) * 64;
-    const size_t lds = (brows ? sizeof(T) * (8 * (size_t)block + 2 * (size_t)e0->g.nz) : sizeof(T) * 12 * (size_t)block) +
-                       sizeof(sjf::MatLut<T>) * nmat;
-    if (lds > 65536) return bail(fail(e0, SJF_E_UNSUPPORTED, "adjoint tile needs more than 64 KiB of LDS"));
+    const size_t lds = (brows ? sizeof(T) * (8 * (size_t)block + 2 * (((size_t)e0->g.nz + 1) & ~(size_t)1)) : sizeof(T) * 12 * (size_t)block) +
+                       sjf::lut_lds_bytes<T>(nmat);
+    if (!lds_fits<T>(brows ? 8 * (size_t)block + 2 * (size_t)e0->g.nz : 12 * (size_t)block, nmat))
+        return bail(fail(e0, SJF_E_UNSUPPORTED, "adjoint tile needs more than 64 KiB of LDS"));
     const int npv = np_variant_of(e0->maxp, e0->uniform);
     const dim3 grid_v((unsigned)((maxv + 255) / 256), (unsigned)n);
     auto record = [&](long sl, int objective) -> int {
@@ -2226,8 +2319,10 @@ int sjf_set_design_eps(sjf_engine* e, const int lo[3], const int hi[3], const do
                 e->matw_h[q] = e->given_w[q] = 0x00ffffffu;
             }
     rc = h2d(e, e->matw, e->matw_h.data(), sizeof(uint32_t) * e->N);
+    if (!rc) rc = update_segments(e);
     if (rc) return rc;
     e->uniform = false;
+    choose_tile(e);
     e->version++;
     return SJF_OK;
 }
@@ -2591,6 +2686,7 @@ int sjf_set_zsegment(sjf_engine* e, int cells) {
     if (cells > 0 && cells < e->g.nz && e->g.periodic[2])
         return fail(e, SJF_E_ARG, "z passes need a non-periodic z axis");
     e->zseg = cells;
+    choose_tile(e);
     e->version++;
     return SJF_OK;
 }
@@ -2664,20 +2760,17 @@ int sjf_batch_create(sjf_engine* const* engines, int n, sjf_batch** out) {
     s->own_stream = true;
     s->prec = e0->prec;
     s->ty = 1;
-    // measured on MI355X: with some z line shorter than 96 cells (the sweep of 64 instances,
-    // 64^3 to 192x192x128) the row-of-threads form with 6-plane x-chunks (2.78 ms per step)
-    // beats one row per thread (2.89-2.96 ms at 6-32 planes); with every line of 96 cells or more
-    // (the 16 design variants, 192x192x96) one row per thread with 16-plane chunks wins (3.38
-    // against 3.54 ms per gradient step)
-    bool short_z = false;
-    for (int i = 0; i < n; ++i) short_z = short_z || engines[i]->g.nz < 96;
-    s->form = short_z ? SJF_TILE_THREAD_ROWS : SJF_TILE_REGISTER_ROWS;
-    s->xc = short_z ? 6 : 16;
+    // Thread rows where some instance would take them alone (choose_tile) and all fit.  Measured on
+    // MI355X, us per step, thread rows and one register row: 24 grids of 64^3 to 192x192x128 (FP32)
+    // 915, 1074; six of 192x192x96 467, 487; two 170, 191.  The chunk matters little with many rounds
+    // of workgroups (24 grids: 4 planes 919, 6 915, 8 918, 12 941, 18 955; four grids: 4 planes 139,
+    // 6 132, 8 132, 12 130, 18 159).
+    s->form = SJF_TILE_REGISTER_ROWS;
     for (int i = 0; i < n; ++i)
-        if (!thread_rows_fit(engines[i], default_thread_rows(engines[i]))) {
-            s->form = SJF_TILE_REGISTER_ROWS;
-            s->xc = 16;
-        }
+        if (engines[i]->g.nz < (engines[i]->prec == 8 ? 128 : 256)) s->form = SJF_TILE_THREAD_ROWS;
+    for (int i = 0; i < n; ++i)
+        if (!thread_rows_fit(engines[i], default_thread_rows(engines[i]))) s->form = SJF_TILE_REGISTER_ROWS;
+    s->xc = s->form == SJF_TILE_THREAD_ROWS ? 8 : 16;
     for (int i = 0; i < n; ++i) {
         s->eng.push_back(engines[i]);
         engines[i]->batch = b;
@@ -2703,6 +2796,7 @@ int sjf_batch_set_tile(sjf_batch* b, int form, int xchunk) {
     s->form = form;
     s->ty = 1;
     s->xc = xchunk;
+    s->tile_set = true;
     s->built = false;
     return SJF_OK;
 }

@@ -42,16 +42,25 @@ constexpr bool kPolePair = sizeof(T) == 4;
 constexpr int kDesignMat = 255;
 constexpr int kMaxDftFreqs = 64;
 
+// recurrence coefficients of one pole; lor: 1 for a Lorentz pole, 0 for a Drude one (and unused slots)
 template <typename T>
-struct MatLut {
+struct __align__(16) PoleCoef {
+    T alpha, beta, c3, lor;
+};
+
+// One entry per material and, last, one of zeros that design voxels index.
+template <typename T>
+struct __align__(16) MatLut {
     T inv_eps;
     T eps_inf;
     int np;
     int lorentz_mask;
-    T alpha[kMaxPoles];
-    T beta[kMaxPoles];
-    T c3[kMaxPoles];
+    PoleCoef<T> pole[kMaxPoles];
 };
+
+// bytes the material table takes in LDS
+template <typename T>
+__host__ __device__ constexpr size_t lut_lds_bytes(int nmat) { return sizeof(MatLut<T>) * (nmat + 1); }
 
 // Kernel arguments of the fused step.  Few base pointers on purpose: the component, pole-slot
 // and PML-segment arrays are addressed as offsets from them, so the whole argument block stays
@@ -69,8 +78,9 @@ struct StepArgs {
     T* F[2];              // field sets [x][Ex Ey Ez Hx Hy Hz][y][z]; step n reads F[n&1], writes F[~n&1]
     const long* d_step;   // the engine's step counter
     int uniform;  // 1: single non-dispersive material, no material word read
-    int nmat;
+    int nmat;     // materials; the id of design voxels in the words
     const uint32_t* matw;
+    const uint32_t* seg;  // one code per 64 cells of a z line (k_segments), [x][y][(nz + 63) / 64]
     const MatLut<T>* lut;
     T* Q;     // [x][slot * 3 + comp][y][z]
     T* P;     // [x][slot * 3 + comp][y][z] (Lorentz slots)
@@ -87,6 +97,8 @@ struct StepArgs {
 };
 
 #define GLOBAL __attribute__((address_space(1)))
+// memory no kernel writes while it is read: uniform reads go through the scalar cache
+#define CONST __attribute__((address_space(4)))
 
 __device__ __forceinline__ int wrap_or_ghost(int c, int n, int periodic) {
     if (c >= 0 && c < n) return c;
@@ -97,17 +109,32 @@ __device__ __forceinline__ int wrap_or_ghost(int c, int n, int periodic) {
     return m < 0 ? m + n : m;
 }
 
+// the same for c in [-1, n]
+__device__ __forceinline__ int wrap_one(int c, int n, int periodic) {
+    return c < 0 ? (periodic ? n - 1 : -1) : c < n ? c : periodic ? 0 : -1;
+}
+// c in [0, ...): past the end of a periodic axis of any length back into it, else unchanged
+__device__ __forceinline__ int wrap_up(int c, int n, int periodic) { return periodic && c >= n ? 0 : c; }
+
 template <typename T>
 __device__ __forceinline__ bool in_pml(const StepArgs<T>& a, int d, int c, int n) {
     return a.pml_on[d] && (c < a.plo[d] || c >= n - a.phi[d]);
 }
 
-// CPML update of one auxiliary: psi <- b psi + a d; returns d + psi.
+// The sums of the update, with the fused products spelled out: every kernel form and every place of
+// a plane's H (its own, the halo's, a chunk's first plane) then rounds alike, whatever else the
+// compiler fuses.
+__device__ __forceinline__ float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double fma_(double a, double b, double c) { return __builtin_fma(a, b, c); }
+// the updated CPML auxiliary b psi + c d of a term d, which adds it
 template <typename T>
-__device__ __forceinline__ T cpml(T d, T b, T c, T& psi) {
-    psi = b * psi + c * d;
-    return d + psi;
-}
+__device__ __forceinline__ T aux_next(T d, T b, T c, T psi) { return fma_(b, psi, c * d); }
+// H - cdt (x - y)
+template <typename T>
+__device__ __forceinline__ T h_next(T h, T cdt, T x, T y) { return fma_(-cdt, x - y, h); }
+// E + inv (cdt curl - sum of Q^{n+1})
+template <typename T>
+__device__ __forceinline__ T e_next(T e, T inv, T cdt, T curl, T sq) { return fma_(inv, fma_(cdt, curl, -sq), e); }
 
 // LDS-scoped workgroup barrier: orders only the LDS exchange, so global loads issued before it
 // (next-plane prefetch) and global stores stay in flight across it.
@@ -130,6 +157,10 @@ typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 constexpr uint32_t kOOB = 0x80000000u;
 __device__ __forceinline__ Rsrc rsrc(const void* p) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)0x80000000u, 0x00020000);
+}
+// the same over nothing unless `need` (uniform): loads return 0 without a memory access
+__device__ __forceinline__ Rsrc rsrc(const void* p, bool need) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, need ? (int)0x80000000u : 0, 0x00020000);
 }
 template <typename T>
 __device__ __forceinline__ T bld(Rsrc r, uint32_t v, uint32_t s);
@@ -157,52 +188,172 @@ template <bool NT = false>
 __device__ __forceinline__ void bst(Rsrc r, uint32_t v, uint32_t s, double x) {
     __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, x), r, (int)v, (int)s, NT ? 2 : 0);
 }
+// two consecutive values
+template <typename T>
+using Pair2 = T __attribute__((ext_vector_type(2)));
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+template <typename T>
+__device__ __forceinline__ Pair2<T> bld2(Rsrc r, uint32_t v, uint32_t s) {
+    if constexpr (sizeof(T) == 4) return __builtin_bit_cast(Pair2<T>, __builtin_amdgcn_raw_buffer_load_b64(r, (int)v, (int)s, 0));
+    else return __builtin_bit_cast(Pair2<T>, __builtin_amdgcn_raw_buffer_load_b128(r, (int)v, (int)s, 0));
+}
+template <bool NT = false, typename P>
+__device__ __forceinline__ void bst2(Rsrc r, uint32_t v, uint32_t s, P x) {
+    if constexpr (sizeof(P) == 8) __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, x), r, (int)v, (int)s, NT ? 2 : 0);
+    else __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x), r, (int)v, (int)s, NT ? 2 : 0);
+}
+// the lane offset of a pair from that of a value (kOOB stays out of range)
+__device__ __forceinline__ uint32_t two(uint32_t o) { return o == kOOB ? kOOB : 2u * o; }
 // true in every lane of the wavefront when p holds in at least one active lane (wave-uniform)
 __device__ __forceinline__ bool wave_any(bool p) { return __builtin_amdgcn_ballot_w64(p) != 0; }
+
+// A register copy the compiler does not look through.  Where a value moves on to a register that an
+// earlier one leaves (plane i + 1 becoming plane i), it would otherwise rename instead and copy the
+// next plane's loads at the end of the loop, waiting for them.
+__device__ __forceinline__ float reg_copy(float x) {
+    float y;
+    asm("v_mov_b32 %0, %1" : "=v"(y) : "v"(x));
+    return y;
+}
+__device__ __forceinline__ uint32_t reg_copy(uint32_t x) {
+    uint32_t y;
+    asm("v_mov_b32 %0, %1" : "=v"(y) : "v"(x));
+    return y;
+}
+__device__ __forceinline__ double reg_copy(double x) {
+    double y;
+    asm("v_mov_b64 %0, %1" : "=v"(y) : "v"(x));
+    return y;
+}
+
+// Computes x here: keeps the compiler from sinking what x is made of past the loads that follow, into
+// the registers it still occupies.
+__device__ __forceinline__ void pin(float& x) { asm volatile("" : "+v"(x)); }
+__device__ __forceinline__ void pin(double& x) { asm volatile("" : "+v"(x)); }
 
 // Field and polarisation layout: x planes of components, [x][comp][y][z] for a field set (six
 // components) and [x][slot * 3 + comp][y][z] for Q and P.  One x plane of a set is contiguous,
 // so a kernel addresses a plane through one descriptor and a component by a 32-bit offset.
 __host__ __device__ __forceinline__ long field_index(long q, int c, long nyz) { return q + (5 * (q / nyz) + c) * nyz; }
 
+// the material table (with its last entry of zeros) into LDS
+template <typename T>
+__device__ __forceinline__ void copy_lut(const StepArgs<T>& a, MatLut<T>* lds) {
+    GLOBAL const u32x4* src = (GLOBAL const u32x4*)a.lut;
+    u32x4* dst = reinterpret_cast<u32x4*>(lds);
+    const int n = (int)(sizeof(MatLut<T>) / 16) * (a.nmat + 1);
+    for (int q = threadIdx.x; q < n; q += blockDim.x) dst[q] = src[q];
+}
+
+// ---- material segments ----------------------------------------------------------------------
+// What the 64 cells of one z segment run.  Segments of one material for all three E components
+// carry its id (bits 0-7) and pole count (8-10); other segments the flag kSegMixed, the largest pole
+// count of a cell, and kSegDesign when a design voxel is among them.  kSegSpecial: mixed or with
+// poles, so that the material table is needed.
+constexpr uint32_t kSegMixed = 0x80000000u, kSegDesign = 0x40000000u, kSegSpecial = 0x20000000u;
+// In the words themselves, above the three ids: the largest pole count of the cell's materials, and
+// whether a component is a design voxel.
+constexpr uint32_t kWordDesign = 0x08000000u;
+__device__ __forceinline__ int word_poles(uint32_t w) { return (int)((w >> 24) & 7); }
+__device__ __forceinline__ int seg_material(uint32_t code) { return (int)(code & 0xff); }
+__device__ __forceinline__ int seg_poles(uint32_t code) { return (int)((code >> 8) & 7); }
+
+// Segment codes of the material words, one wavefront per segment; in the words the design ids
+// (kDesignMat) become nmat, the index of the table's entry of zeros, and the marks above are set.
+// slots: pole slots of all segments.
+template <typename T>
+__global__ void __launch_bounds__(256) k_segments(uint32_t* __restrict__ matw, const MatLut<T>* __restrict__ lut,
+                                                  uint32_t* __restrict__ seg, long rows, int nz, int nmat,
+                                                  unsigned long long* __restrict__ slots) {
+    const int nseg = (nz + 63) >> 6, lane = threadIdx.x & 63;
+    const long q = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (q >= rows * nseg) return;
+    const long row = q / nseg;
+    const int k = (int)(q - row * nseg) * 64 + lane;
+    const bool in = k < nz;
+    uint32_t w = in ? matw[row * nz + k] : 0u;
+    bool des = false;
+    int np = 0;
+    uint32_t out = 0u;  // the three ids
+    for (int c = 0; c < 3; ++c) {
+        int m = (w >> (8 * c)) & 0xff;
+        const bool d = in && (m == kDesignMat || m == nmat);
+        m = d ? nmat : m;
+        des = des || d;
+        if (in) np = max(np, lut[m].np);
+        out |= (uint32_t)m << (8 * c);
+    }
+    if (in) matw[row * nz + k] = out | (uint32_t)np << 24 | (des ? kWordDesign : 0u);
+    const uint32_t first = (uint32_t)__builtin_amdgcn_readfirstlane((int)out);
+    const uint32_t id = first & 0xff;
+    const bool mixed = first != id * 0x010101u || wave_any(des) || wave_any(in && out != first);
+    uint32_t code = mixed ? kSegMixed | kSegSpecial | (wave_any(des) ? kSegDesign : 0u) : id;
+    for (int n = kMaxPoles; n > 0; --n)
+        if (wave_any(np >= n)) {
+            code |= kSegSpecial | (uint32_t)n << 8;
+            break;
+        }
+    if (lane == 0) seg[q] = code;
+    if (lane == 0 && seg_poles(code) > 0) atomicAdd(slots, (unsigned long long)seg_poles(code));
+}
+
 // Fused H / polarisation / E update of one time step.  TY: y rows per thread; NP: pole slots
 // compiled in (>= the largest pole count of any material).
 // A workgroup covers one z line (thread k = cell k) of TY consecutive y rows and marches along
-// x.  Each plane iteration issues every global load it needs first (fields, PML auxiliaries,
-// polarisation state, and E and material words of the planes ahead), then computes H, exchanges
-// the z neighbours of H through LDS, and computes E.
-// Addressing: a thread's byte offset within a component plane depends only on its row and z cell,
-// so it is fixed for the whole march; each access is a per-plane descriptor, that lane offset and
-// a uniform component offset.  Ghost rows, lanes past the end of the z line and lanes outside a
-// z PML layer, a pole slot or the design region carry the out-of-range offset instead of
-// branching; whole-wavefront conditions (row, plane, x/y PML, any lane in a z layer / using a
-// slot / in the design region) are uniform branches.
+// x.  On grids that the caches hold the step is bound by the instructions a plane takes and by the
+// latency of what it waits for, on large ones by memory; so:
+//   * Every register that a plane's update has read is loaded again for the plane that needs it
+//     next as soon as it has been read -- H, the PML auxiliaries, the pole state and the material
+//     words for plane i + 1, E for plane i + 2.  No load is waited for in the iteration that issues
+//     it, and none is copied from register to register while it is in flight (such a copy waits for
+//     the load and, both counting in vmcnt, for the iteration's stores).  The loop starts with the
+//     E phase, the first H phase standing before it, and the last H phase runs past the chunk: all
+//     ways into the loop then have the same loads and stores in flight in the same order, and the
+//     wait counts need not assume the worse of two.  The loads and stores of a plane that is not
+//     needed (past the chunk, past a metallic edge) go through a descriptor of length zero: they
+//     return 0 or are dropped without a memory access.
+//   * One word per 64 cells of a z line (k_segments) says whether a wavefront's cells all run one
+//     material without poles; then its constant is a scalar and neither the per-cell words nor the
+//     material table are read.
+//   * A thread's byte offset within a component plane depends only on its row and z cell, so it is
+//     fixed for the whole march; each access is a per-plane descriptor, that lane offset and a
+//     uniform component offset.  Ghost rows, lanes past the end of the z line and lanes outside a
+//     z PML layer, a pole slot or the design region carry the out-of-range offset instead of
+//     branching; what holds for a whole wavefront (row, plane, x/y PML, any lane in a z layer,
+//     material segment) is a bit of a scalar and a branch.  Registers that a branch alone loads and
+//     uses are left unset otherwise.
+// Measured on MI355X, us per step before (every register loaded in the iteration that uses it, rotated
+// by copies) and now: FP32 512x512x256 1183, 1047 (5.0 TB/s of fields, what a plain copy that marches
+// alike reaches); 448x224x512 922, 732; 192x192x96 118, 94; FP64 96^3 51, 42.
 template <typename T, int TY, int NP, bool ZP, bool NTS>
 __device__ __forceinline__ void step_tile(const StepArgs<T>& a, const int t) {
     constexpr uint32_t TS = sizeof(T);
+    constexpr int NS = NP > 0 ? NP : 1;
+    typedef T Pair __attribute__((ext_vector_type(2)));
+    typedef T Erows[TY + 2][3];  // E of rows -1..TY (Ey of row TY unused)
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const int B = blockDim.x;
-    T* sh = reinterpret_cast<T*>(smem_raw);  // [2 parity][2 comp][TY][B]
-    MatLut<T>* slut = reinterpret_cast<MatLut<T>*>(sh + 4 * TY * B);
-    {
-        GLOBAL const uint32_t* src = (GLOBAL const uint32_t*)a.lut;
-        uint32_t* dst = reinterpret_cast<uint32_t*>(slut);
-        const int words = (int)(sizeof(MatLut<T>) / 4) * a.nmat;
-        for (int q = threadIdx.x; q < words; q += B) dst[q] = src[q];
-    }
+    Pair* sh = reinterpret_cast<Pair*>(smem_raw);  // [2 parity][TY][B + 1] (Hx, Hy); slot B: zero
+    MatLut<T>* slut = reinterpret_cast<MatLut<T>*>(sh + 2 * TY * (B + 1));
+    copy_lut(a, slut);
+    if (threadIdx.x < 2 * TY) sh[threadIdx.x * (B + 1) + B] = Pair{T(0), T(0)};
 
-    const long step = *(GLOBAL const long*)a.d_step;
-    const char* F0 = (const char*)a.F[step & 1];
-    const char* F1 = (const char*)a.F[(step + 1) & 1];
-    const char* matw = (const char*)a.matw;
-    GLOBAL const T* coef = (GLOBAL const T*)a.coef;
-    const uint32_t hr = (step & 1) ? 4 : 2;  // H auxiliary pair read this step
-    const uint32_t hw = (step & 1) ? 2 : 4;  // and written
-    // FP32 Lorentz pole slots hold P^n and P^{n-1}: P^n in the Q array on even steps and in
-    // the P array on odd ones, P^{n+1} overwrites P^{n-1}.  Drude slots hold Q^n in the Q array.
-    const bool podd = (step & 1) != 0;
+    const long step = *(CONST const long*)a.d_step;
+    const bool odd = (step & 1) != 0;
+    const char* F0 = (const char*)a.F[odd ? 1 : 0];
+    const long F01 = (const char*)a.F[odd ? 0 : 1] - F0;  // from the set read to the set written
+    const int hr = odd ? 2 : 1;  // H auxiliary pair read this step
+    const int hw = odd ? 1 : 2;  // and written
+    // FP32 pole slots alternate between two arrays: step n reads P^n (Lorentz) or Q^n (Drude) from
+    // Q when n is even, from P when it is odd, and writes the new value to the other, where a
+    // Lorentz pole has read P^{n-1}.  FP64 slots hold Q^n and P^n.
+    const char* Pcur = (const char*)(kPolePair<T> && odd ? a.P : a.Q);
+    const char* Pold = (const char*)(kPolePair<T> && odd ? a.Q : a.P);
+    CONST const uint32_t* seg = (CONST const uint32_t*)a.seg;
+    CONST const T* coef = (CONST const T*)a.coef;
+    CONST const MatLut<T>* clut = (CONST const MatLut<T>*)a.lut;
     const int nx = a.nx, ny = a.ny, nz = a.nz;
-    const int tyi = t % a.nty, xci = t / a.nty;
+    const int xci = t / a.nty, tyi = t - xci * a.nty;
     const int j0 = tyi * TY;
     const int x0 = xci * a.xc;
     const int x1 = min(x0 + a.xc, nx);
@@ -211,398 +362,459 @@ __device__ __forceinline__ void step_tile(const StepArgs<T>& a, const int t) {
     // its z neighbour; passes alternate between two halves of zh.
     const int Z = ZP ? a.zseg : nz;  // ZP: compiled for z passes
     const int npass = ZP ? (nz + Z - 1) / Z : 1;
-    T* zh = reinterpret_cast<T*>(slut + a.nmat);  // [2 pass parity][xc][TY][Hx, Hy]
+    Pair* zh = reinterpret_cast<Pair*>((unsigned char*)slut + lut_lds_bytes<T>(a.nmat));  // [2 pass parity][xc][TY]
     const int kl = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nseg = (nz + 63) >> 6;
+    const bool uniform = a.uniform != 0;
+    const bool emap = a.emap != nullptr;
+    const T cdt = a.cdt;
+    const uint32_t PB = (uint32_t)ny * (uint32_t)nz * TS;  // bytes of one component plane
+    const long FPB = 6L * PB;                             // bytes of one x plane of a field set
+    const long QPB = (long)a.nqp * PB;                    // and of the polarisation
+    const int Ly = a.plo[1] + a.phi[1], Lz = a.plo[2] + a.phi[2];
+    const uint32_t SP0 = (uint32_t)(2 * a.S[0] * TS), SP1 = (uint32_t)(2 * a.S[1] * TS), SP2 = (uint32_t)(2 * a.S[2] * TS);
+    const Rsrc rpx = rsrc(a.psi[0]), rpy = rsrc(a.psi[1]), rpz = rsrc(a.psi[2]);
+    CONST const T* cx = coef + a.coff[0];
+    CONST const T* cy = coef + a.coff[1];
+    // planes outside [xlo, xlo + xin) lie in an x layer
+    const int xlo = a.pml_on[0] ? a.plo[0] : 0;
+    const unsigned xin = a.pml_on[0] ? (unsigned)(nx - a.phi[0] - a.plo[0]) : 0xffffffffu;
+    auto in_x = [&](int p) { return (unsigned)(p - xlo) >= xin; };
+
+    int gj[TY + 2];  // global row of local row r-1 (r = 0 is the halo row below the tile), -1 outside
+    int sy[TY + 1];  // its row within the y layers
+    uint32_t fl = 0; // bits r: row r lies in a y layer; 8 + r: row r is inside the grid; 16 + r: owned row r - 1
+#pragma unroll
+    for (int r = 0; r < TY + 2; ++r) gj[r] = TY > 1 ? wrap_or_ghost(j0 + r - 1, ny, a.py) : wrap_one(j0 + r - 1, ny, a.py);
+#pragma unroll
+    for (int r = 0; r < TY + 1; ++r) {
+        const bool y = gj[r] >= 0 && in_pml(a, 1, gj[r], ny);
+        sy[r] = y ? (gj[r] < a.plo[1] ? gj[r] : gj[r] - (ny - a.phi[1]) + a.plo[1]) : 0;
+        fl |= (y ? 1u << r : 0u) | (gj[r] >= 0 ? 0x100u << r : 0u) | (r > 0 && j0 + r - 1 < ny ? 0x10000u << r : 0u);
+    }
+    fl = __builtin_amdgcn_readfirstlane(fl);
+    auto in_y = [&](int r) { return ((fl >> r) & 1) != 0; };
+    auto valid = [&](int r) { return ((fl >> (8 + r)) & 1) != 0; };
+    auto own = [&](int r) { return TY == 1 || ((fl >> (17 + r)) & 1) != 0; };
+    const bool yany = (fl & 0xff) != 0;
+    auto xslab = [&](int p) -> uint32_t { return (uint32_t)(p < a.plo[0] ? p : p - (nx - a.phi[0]) + a.plo[0]) * 2u * PB; };
+    auto yslab = [&](int p, int r) -> uint32_t { return (uint32_t)((p * Ly + sy[r]) * nz) * 2u * TS; };
+
     for (int pass = 0; pass < npass; ++pass) {
         const int k = pass * Z + kl;
         const bool kin = kl < Z && k < nz;
-        const int kp1 = wrap_or_ghost(k + 1, nz, a.pz);
-        const uint32_t PB = (uint32_t)ny * (uint32_t)nz * TS;  // bytes of one component plane
-        const long FPB = 6L * PB;                             // bytes of one x plane of a field set
-        const long QPB = (long)a.nqp * PB;                    // and of the polarisation
-        const long PW = (long)ny * nz * 4;                    // and of the material words
-        const T cdt = a.cdt;
-        const bool uniform = a.uniform != 0;
-        const int Ly = a.plo[1] + a.phi[1], Lz = a.plo[2] + a.phi[2];
-        const uint32_t SB0 = (uint32_t)(a.S[0] * TS), SB1 = (uint32_t)(a.S[1] * TS), SB2 = (uint32_t)(a.S[2] * TS);
-        const Rsrc rpx = rsrc(a.psi[0]), rpy = rsrc(a.psi[1]), rpz = rsrc(a.psi[2]);
-
-        int gj[TY + 2];        // global row of local row r-1 (r = 0 is the halo row below the tile)
-        bool rv[TY + 2];       // row inside the grid (uniform)
+        const int kp1 = k + 1 < nz ? k + 1 : a.pz ? 0 : -1;
         uint32_t oR[TY + 2];   // byte offset of (row, k) within a component plane, or kOOB
-        uint32_t oW[TY + 2];   // the same for the 4-byte material words
-#pragma unroll
-        for (int r = 0; r < TY + 2; ++r) {
-            gj[r] = wrap_or_ghost(j0 + r - 1, ny, a.py);
-            rv[r] = gj[r] >= 0;
-            const bool ok = rv[r] && kin;
-            oR[r] = ok ? (uint32_t)(gj[r] * nz + k) * TS : kOOB;
-            oW[r] = ok ? (uint32_t)(gj[r] * nz + k) * 4u : kOOB;
-        }
         uint32_t oK1[TY + 1];  // byte offset of (row, k + 1), or kOOB
 #pragma unroll
+        for (int r = 0; r < TY + 2; ++r) oR[r] = gj[r] >= 0 && kin ? (uint32_t)(gj[r] * nz + k) * TS : kOOB;
+#pragma unroll
         for (int r = 0; r < TY + 1; ++r)
-            oK1[r] = (rv[r] && kin && kp1 >= 0) ? (uint32_t)(gj[r] * nz + kp1) * TS : kOOB;
-        bool own_row[TY];
-#pragma unroll
-        for (int r = 0; r < TY; ++r) own_row[r] = (j0 + r) < ny;
-        bool ypml[TY + 1];
-        int sy[TY + 1];
-#pragma unroll
-        for (int r = 0; r < TY + 1; ++r) {
-            ypml[r] = rv[r] && in_pml(a, 1, gj[r], ny);
-            sy[r] = ypml[r] ? (gj[r] < a.plo[1] ? gj[r] : gj[r] - (ny - a.phi[1]) + a.plo[1]) : 0;
-        }
+            oK1[r] = (gj[r] >= 0 && kin && kp1 >= 0) ? (uint32_t)(gj[r] * nz + kp1) * TS : kOOB;
 
         const bool zpml = kin && in_pml(a, 2, k, nz);
         const bool zany = wave_any(zpml);  // some lane of this wavefront lies in a z PML layer
-        const uint32_t oK = kin ? (uint32_t)k * TS : kOOB;
-        const uint32_t oZ = zpml ? (uint32_t)(k < a.plo[2] ? k : k - (nz - a.phi[2]) + a.plo[2]) * TS : kOOB;
-        GLOBAL const T* cz = coef + a.coff[2];
-        const T bEz = zpml ? cz[k] : T(0), aEz = zpml ? cz[nz + k] : T(0);
-        const T bHz = zpml ? cz[2 * nz + k] : T(0), aHz = zpml ? cz[3 * nz + k] : T(0);
+        const uint32_t oK = kin ? (uint32_t)k * 2u * TS : kOOB;  // in a y slab
+        const uint32_t oZ = zpml ? (uint32_t)(k < a.plo[2] ? k : k - (nz - a.phi[2]) + a.plo[2]) * 2u * TS : kOOB;
+        T bEz = T(0), aEz = T(0), bHz = T(0), aHz = T(0);
+        if (zpml) {
+            GLOBAL const T* cz = (GLOBAL const T*)a.coef + a.coff[2];
+            bEz = cz[k], aEz = cz[nz + k], bHz = cz[2 * nz + k], aHz = cz[3 * nz + k];
+        }
+        // segment of this wavefront (one past the line, in a batch of longer lines, has no cell)
+        const int sg = min((ZP ? pass * (Z >> 6) : 0) + wave, nseg - 1);
+        // the z neighbour below: the lane below in this pass, else the periodic image (one pass),
+        // else the zero slot; the first lane of a later pass reads zh
+        const int kb = kl > 0 ? kl - 1 : (a.pz ? nz - 1 : B);
+        lds_barrier();  // the material table; the exchange slots of the previous pass
 
-        lds_barrier();
+        // the registers each plane loads anew
+        Erows ec, en;                                      // E^n of planes i and i + 1
+        T h0[TY + 1][3], ek[TY + 1][2];                    // H^{n-1/2} of plane i; E^n at k + 1
+        Pair pHx[TY + 1], pHy[TY + 1], pHz[TY + 1];        // H auxiliaries
+        Pair pEx[TY], pEy[TY], pEz[TY];                    // E auxiliaries
+        T em[TY][3];                                       // 1/eps of the maps
+        T Qv[TY][3][NS], Pv[TY][3][NS];                    // pole state
+        uint32_t mw[TY], mwn[TY];                          // material words of planes i, i + 1
+        T hp[TY][2];                                       // H^{n+1/2} (Hy, Hz) of plane i - 1
+        T h[TY + 1][3], e0[TY][3];                         // H^{n+1/2} and E^n (owned rows) of plane i
+        T iv[TY], inv[TY][3], sq[TY][3];                   // 1/eps (of a one-material segment, of each E) and sum of Q^{n+1}
+        T dv[TY][3];                                       // 1/eps and material words of design voxels
+        uint32_t dw[TY];
+        uint32_t cc[TY], cn[TY], cnn[TY];                  // segment codes of planes i, i + 1, i + 2
 
-        T ec[TY + 2][3];  // E^n on plane i, rows -1..TY
-        T en[TY + 2][3];  // E^n on plane i+1
-        T hp[TY][2];      // H^{n+1/2} (Hy, Hz) on plane i-1, rows 0..TY-1
-        uint32_t mw[TY];  // material words of plane i, owned rows
-
-        const int istart = (x0 > 0 || a.px) ? x0 - 1 : x0;
-        {
-            const int p0 = wrap_or_ghost(istart, nx, a.px);
-            const int p1 = wrap_or_ghost(istart + 1, nx, a.px);
-            const Rsrc r0 = rsrc(F0 + (long)(p0 >= 0 ? p0 : 0) * FPB);
-            const Rsrc r1 = rsrc(F0 + (long)(p1 >= 0 ? p1 : 0) * FPB);
+        auto code_of = [&](int p, int r) -> uint32_t { return seg[(uint32_t)((p * ny + gj[r + 1]) * nseg + sg)]; };
+        auto load_e = [&](const char* f, bool need, Erows& e) {
+            const Rsrc rn = rsrc(f, need);
 #pragma unroll
-            for (int r = 0; r < TY + 2; ++r) {
-                const uint32_t o0 = p0 >= 0 ? oR[r] : kOOB, o1 = p1 >= 0 ? oR[r] : kOOB;
+            for (int r = 0; r < TY + 2; ++r)
+#pragma unroll
+                for (int c = 0; c < 3; ++c)
+                    if (c != 1 || r < TY + 1) e[r][c] = bld<T>(rn, oR[r], c * PB);
+        };
+        auto load_h = [&](const char* f, bool need) {
+            const Rsrc rn = rsrc(f, need);
+#pragma unroll
+            for (int r = 0; r < TY + 1; ++r) {
+#pragma unroll
+                for (int c = 0; c < 3; ++c) h0[r][c] = bld<T>(rn, oR[r], (3 + c) * PB);
+#pragma unroll
+                for (int c = 0; c < 2; ++c) ek[r][c] = bld<T>(rn, oK1[r], c * PB);
+            }
+        };
+        auto zrow = [&](int p, int r) -> uint32_t { return (uint32_t)((p * ny + gj[r]) * Lz) * 2u * TS; };
+        auto load_psi_h = [&](int p) {
+            if (zany) {
+#pragma unroll
+                for (int r = 0; r < TY + 1; ++r)
+                    if (valid(r)) pHz[r] = bld2<T>(rpz, oZ, hr * SP2 + zrow(p, r));
+            }
+            if (__builtin_expect(yany, 0)) {
+#pragma unroll
+                for (int r = 0; r < TY + 1; ++r)
+                    if (in_y(r)) pHy[r] = bld2<T>(rpy, oK, hr * SP1 + yslab(p, r));
+            }
+            if (__builtin_expect(in_x(p), 0)) {
+                const uint32_t so = hr * SP0 + xslab(p);
+#pragma unroll
+                for (int r = 0; r < TY + 1; ++r) pHx[r] = bld2<T>(rpx, two(oR[r]), so);
+            }
+        };
+        auto load_psi_e = [&](int p, int r) {
+            if (zany) pEz[r] = bld2<T>(rpz, oZ, zrow(p, r + 1));
+            if (__builtin_expect(yany, 0)) {
+                if (in_y(r + 1)) pEy[r] = bld2<T>(rpy, oK, yslab(p, r + 1));
+            }
+            if (__builtin_expect(in_x(p), 0)) pEx[r] = bld2<T>(rpx, two(oR[r + 1]), xslab(p));
+            if (__builtin_expect(emap, 0)) {
+                const Rsrc re = rsrc((const char*)a.emap + (long)p * 3 * PB);
+#pragma unroll
+                for (int c = 0; c < 3; ++c) em[r][c] = bld<T>(re, oR[r + 1], c * PB);
+            }
+        };
+        auto load_word = [&](int p, int r, uint32_t code, uint32_t& w) {  // where a segment is mixed
+            if (code & kSegMixed) {
+                const uint32_t o = oR[r + 1];
+                w = bld<uint32_t>(rsrc((const char*)a.matw + (long)p * ny * nz * 4), TS == 4 || o == kOOB ? o : o / 2, 0);
+            }
+        };
+        // material words of a segment of one material are its id three times
+        auto words = [&](uint32_t code, uint32_t w) { return code & kSegMixed ? w : (uint32_t)seg_material(code) * 0x010101u; };
+        // pole state of plane p, whose segment code is `code` and material words are w
+        auto load_poles = [&](int p, int r, uint32_t code, uint32_t w) {
+            const int npx = seg_poles(code);
+            const Rsrc rc = rsrc(Pcur + (long)p * QPB), ro = rsrc(Pold + (long)p * QPB);
+            int np[3], lm[3];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                const MatLut<T>& L = slut[(w >> (8 * c)) & 0xff];
+                np[c] = L.np;
+                lm[c] = L.lorentz_mask;
+            }
+#pragma unroll
+            for (int s = 0; s < NP; ++s) {
+                if (s >= npx) break;
 #pragma unroll
                 for (int c = 0; c < 3; ++c) {
-                    ec[r][c] = bld<T>(r0, o0, c * PB);
-                    en[r][c] = bld<T>(r1, o1, c * PB);
+                    // (a Drude slot reads one value; the second array may be absent without Lorentz poles)
+                    Qv[r][c][s] = bld<T>(rc, s < np[c] ? oR[r + 1] : kOOB, (s * 3 + c) * PB);
+                    Pv[r][c][s] = bld<T>(ro, (lm[c] >> s) & 1 ? oR[r + 1] : kOOB, (s * 3 + c) * PB);
                 }
             }
-            const bool mw0 = !uniform && istart >= x0;
-            const Rsrc rm = rsrc(matw + (long)(p0 >= 0 ? p0 : 0) * PW);
+        };
+
+        // ---- the chunk's first planes; H (y and z components) of the plane before it
+        int pi = x0, pn = wrap_up(x0 + 1, nx, a.px), pnn = wrap_up(pn + 1, nx, a.px);  // nx or more: past the edge
+        const char* fW = F0 + (long)pi * FPB;  // plane i, then i + 1 and i + 2, of the set read
+        const char* fN = F0 + (long)min(pn, nx - 1) * FPB;
+        const char* fNN = F0 + (long)min(pnn, nx - 1) * FPB;
+#pragma unroll
+        for (int r = 0; r < TY; ++r) {
+            cc[r] = uniform || !own(r) ? 0u : code_of(pi, r);
+            cn[r] = uniform || !own(r) || x0 + 1 >= x1 ? 0u : code_of(pn, r);
+            hp[r][0] = hp[r][1] = T(0);
+        }
+        load_e(fW, true, ec);
+        if (x0 > 0 || a.px) {
+            const int p = x0 > 0 ? x0 - 1 : nx - 1;
+            const bool xp = in_x(p);
+            const Rsrc rn = rsrc(F0 + (long)p * FPB);
+            T eh[TY + 1][3], hh[TY][2], ekx[TY];
+            Pair qx[TY], qy[TY], qz[TY];
+#pragma unroll
+            for (int r = 0; r < TY + 1; ++r)  // rows 0..TY; row TY: Ex alone
+#pragma unroll
+                for (int c = 0; c < 3; ++c)
+                    if (c == 0 || r < TY) eh[r][c] = bld<T>(rn, oR[r + 1], c * PB);
 #pragma unroll
             for (int r = 0; r < TY; ++r) {
-                hp[r][0] = hp[r][1] = T(0);
-                mw[r] = 0u;
-                if (mw0 && own_row[r]) mw[r] = bld<uint32_t>(rm, oW[r + 1], 0);
+                hh[r][0] = bld<T>(rn, oR[r + 1], 4 * PB);
+                hh[r][1] = bld<T>(rn, oR[r + 1], 5 * PB);
+                ekx[r] = bld<T>(rn, oK1[r + 1], 0);
+                if (!own(r)) continue;
+                if (xp) qx[r] = bld2<T>(rpx, two(oR[r + 1]), hr * SP0 + xslab(p));
+                if (in_y(r + 1)) qy[r] = bld2<T>(rpy, oK, hr * SP1 + yslab(p, r + 1));
+                if (zany) qz[r] = bld2<T>(rpz, oZ, hr * SP2 + zrow(p, r + 1));
+            }
+#pragma unroll
+            for (int r = 0; r < TY; ++r) {
+                if (!own(r)) continue;
+                T dEx_y = eh[r + 1][0] - eh[r][0];
+                T dEx_z = ekx[r] - eh[r][0];
+                T dEz_x = ec[r + 1][2] - eh[r][2];
+                T dEy_x = ec[r + 1][1] - eh[r][1];
+                if (in_y(r + 1)) dEx_y += aux_next(dEx_y, cy[2 * ny + gj[r + 1]], cy[3 * ny + gj[r + 1]], qy[r].y);
+                if (zany) dEx_z += aux_next(dEx_z, bHz, aHz, qz[r].y);
+                if (xp) {
+                    const T b = cx[2 * nx + p], c = cx[3 * nx + p];
+                    dEz_x += aux_next(dEz_x, b, c, qx[r].x);
+                    dEy_x += aux_next(dEy_x, b, c, qx[r].y);
+                }
+                hp[r][0] = h_next(hh[r][0], cdt, dEx_z, dEz_x);
+                hp[r][1] = h_next(hh[r][1], cdt, dEy_x, dEx_y);
+            }
+        }
+        load_e(fN, pn < nx, en);
+        load_h(fW, true);
+        load_psi_h(pi);
+#pragma unroll
+        for (int r = 0; r < TY; ++r) {
+            if (!own(r)) continue;
+            load_psi_e(pi, r);
+            load_word(pi, r, cc[r], mw[r]);
+            load_word(pn, r, cn[r], mwn[r]);
+            if (cc[r] & kSegSpecial) {
+                mw[r] = words(cc[r], mw[r]);
+                if (NP > 0 && seg_poles(cc[r]) > 0) load_poles(pi, r, cc[r], mw[r]);
             }
         }
 
-        for (int i = istart; i < x1; ++i) {
-            const bool own_plane = i >= x0;
-            const bool has_next = i + 1 < x1;
-            const int pi = wrap_or_ghost(i, nx, a.px);
-            const int pn = wrap_or_ghost(i + 1, nx, a.px);
-            const int pnn = wrap_or_ghost(i + 2, nx, a.px);
-            const bool xpml = in_pml(a, 0, pi, nx);
-            const uint32_t sxo = xpml ? (uint32_t)(pi < a.plo[0] ? pi : pi - (nx - a.phi[0]) + a.plo[0]) * PB : 0u;
-            GLOBAL const T* cx = coef + a.coff[0];
-            const T bEx = xpml ? cx[pi] : T(0), aEx = xpml ? cx[nx + pi] : T(0);
-            const T bHx = xpml ? cx[2 * nx + pi] : T(0), aHx = xpml ? cx[3 * nx + pi] : T(0);
-            const Rsrc rF = rsrc(F0 + (long)pi * FPB);
-            const Rsrc rW = rsrc(F1 + (long)pi * FPB);
-
-            // ---------------------------------------------------------------- loads ----------
-            T enn[TY + 2][3];
-            uint32_t mwn[TY];
-            {
-                // plane i + 2 (a ghost plane reads as zero; after the last plane nothing is read)
-                const bool nn_ok = has_next && pnn >= 0;
-                const Rsrc rn = rsrc(F0 + (long)(nn_ok ? pnn : pi) * FPB);
+        auto h_phase = [&](const int i) __attribute__((always_inline)) {
+            const bool live = i < x1, next = i + 1 < x1;
+            const bool xpml = live && in_x(pi);
+            const Rsrc rW = rsrc(fW + F01, live);
 #pragma unroll
-                for (int r = 0; r < TY + 2; ++r) {
-                    const uint32_t o = nn_ok ? oR[r] : kOOB;
-                    enn[r][0] = bld<T>(rn, o, 0);
-                    enn[r][1] = (r < TY + 1) ? bld<T>(rn, o, PB) : T(0);
-                    enn[r][2] = bld<T>(rn, o, 2 * PB);
-                }
-                const bool mwn_ok = !uniform && has_next && pn >= 0;
-                const Rsrc rm = rsrc(matw + (long)(mwn_ok ? pn : pi) * PW);
-#pragma unroll
-                for (int r = 0; r < TY; ++r) {
-                    mwn[r] = 0u;
-                    if (mwn_ok && own_row[r]) mwn[r] = bld<uint32_t>(rm, oW[r + 1], 0);
-                }
+            for (int r = 0; r < TY; ++r) {
+                cnn[r] = uniform || !own(r) || i + 2 >= x1 ? 0u : code_of(pnn, r);
+                iv[r] = clut[seg_material(cc[r])].inv_eps;
             }
-            T h0[TY + 1][3], ek1[TY + 1][2], pH[TY + 1][3][2];
+            T d[TY + 1][6];  // dEz_y, dEx_y, dEy_z, dEx_z, dEz_x, dEy_x
 #pragma unroll
             for (int r = 0; r < TY + 1; ++r) {
+                d[r][0] = ec[r + 1][2] - ec[r][2];
+                d[r][1] = ec[r + 1][0] - ec[r][0];
+                d[r][2] = ek[r][1] - ec[r][1];
+                d[r][3] = ek[r][0] - ec[r][0];
+                d[r][4] = en[r][2] - ec[r][2];
+                d[r][5] = en[r][1] - ec[r][1];
+            }
+            if (zany) {  // lanes outside the layers: b = a = 0 leaves the term unchanged
 #pragma unroll
-                for (int c = 0; c < 3; ++c) h0[r][c] = bld<T>(rF, oR[r], (3 + c) * PB);
-#pragma unroll
-                for (int c = 0; c < 2; ++c) ek1[r][c] = bld<T>(rF, oK1[r], c * PB);
-#pragma unroll
-                for (int d = 0; d < 3; ++d) pH[r][d][0] = pH[r][d][1] = T(0);
-                if (rv[r] && xpml) {
-                    pH[r][0][0] = bld<T>(rpx, oR[r], hr * SB0 + sxo);
-                    pH[r][0][1] = bld<T>(rpx, oR[r], (hr + 1) * SB0 + sxo);
-                }
-                if (ypml[r]) {
-                    const uint32_t so = (uint32_t)((pi * Ly + sy[r]) * nz) * TS;
-                    pH[r][1][0] = bld<T>(rpy, oK, hr * SB1 + so);
-                    pH[r][1][1] = bld<T>(rpy, oK, (hr + 1) * SB1 + so);
-                }
-                if (rv[r] && zany) {
-                    const uint32_t so = (uint32_t)((pi * ny + gj[r]) * Lz) * TS;
-                    pH[r][2][0] = bld<T>(rpz, oZ, hr * SB2 + so);
-                    pH[r][2][1] = bld<T>(rpz, oZ, (hr + 1) * SB2 + so);
+                for (int r = 0; r < TY + 1; ++r) {
+                    if (!valid(r)) continue;
+                    const T q0 = aux_next(d[r][2], bHz, aHz, pHz[r].x), q1 = aux_next(d[r][3], bHz, aHz, pHz[r].y);
+                    d[r][2] += q0;
+                    d[r][3] += q1;
+                    if (r > 0 && own(r - 1) && live) bst2<NTS>(rpz, oZ, hw * SP2 + zrow(pi, r), Pair{q0, q1});
                 }
             }
-            T pE[TY][3][2];
-            T Qv[TY][3][NP > 0 ? NP : 1], Pv[TY][3][NP > 0 ? NP : 1];
-            const Rsrc rQ = rsrc((const char*)a.Q + (long)pi * QPB);
-            const Rsrc rP = rsrc((const char*)a.P + (long)pi * QPB);
+            if (__builtin_expect(yany, 0)) {
+#pragma unroll
+                for (int r = 0; r < TY + 1; ++r) {
+                    if (!in_y(r)) continue;
+                    const T b = cy[2 * ny + gj[r]], c = cy[3 * ny + gj[r]];
+                    const T q0 = aux_next(d[r][0], b, c, pHy[r].x), q1 = aux_next(d[r][1], b, c, pHy[r].y);
+                    d[r][0] += q0;
+                    d[r][1] += q1;
+                    if (r > 0 && own(r - 1) && live) bst2<NTS>(rpy, oK, hw * SP1 + yslab(pi, r), Pair{q0, q1});
+                }
+            }
+            if (__builtin_expect(xpml, 0)) {
+                const T b = cx[2 * nx + pi], c = cx[3 * nx + pi];
+                const uint32_t so = hw * SP0 + xslab(pi);
+#pragma unroll
+                for (int r = 0; r < TY + 1; ++r) {
+                    const T q0 = aux_next(d[r][4], b, c, pHx[r].x), q1 = aux_next(d[r][5], b, c, pHx[r].y);
+                    d[r][4] += q0;
+                    d[r][5] += q1;
+                    if (r > 0 && own(r - 1)) bst2<NTS>(rpx, two(oR[r]), so, Pair{q0, q1});
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < TY + 1; ++r) {
+                h[r][0] = h_next(h0[r][0], cdt, d[r][0], d[r][2]);
+                h[r][1] = h_next(h0[r][1], cdt, d[r][3], d[r][4]);
+                h[r][2] = h_next(h0[r][2], cdt, d[r][5], d[r][1]);
+                // outside a metallic edge H is identically zero (ghost row of the halo)
+                if (!valid(r)) h[r][0] = h[r][1] = h[r][2] = T(0);
+#pragma unroll
+                for (int c = 0; c < 3; ++c) pin(h[r][c]);
+                if (r > 0 && own(r - 1)) {
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) bst<NTS>(rW, oR[r], (3 + c) * PB, h[r][c]);
+                }
+            }
+            Pair* buf = sh + (i & 1) * TY * (B + 1);
+#pragma unroll
+            for (int r = 0; r < TY; ++r) {
+                buf[r * (B + 1) + kl] = Pair{h[r + 1][0], h[r + 1][1]};
+#pragma unroll
+                for (int c = 0; c < 3; ++c) e0[r][c] = reg_copy(ec[r + 1][c]);
+            }
+            if (ZP && live && pass + 1 < npass && kl == Z - 1) {
+                Pair* zo = zh + ((pass & 1) * a.xc + (i - x0)) * TY;
+#pragma unroll
+                for (int r = 0; r < TY; ++r) zo[r] = Pair{h[r + 1][0], h[r + 1][1]};
+            }
+            // ------------------------------- polarisation: sum of Q^{n+1} over the poles; 1/eps
 #pragma unroll
             for (int r = 0; r < TY; ++r) {
 #pragma unroll
-                for (int d = 0; d < 3; ++d) pE[r][d][0] = pE[r][d][1] = T(0);
-#pragma unroll
-                for (int c = 0; c < 3; ++c)
-#pragma unroll
-                    for (int s = 0; s < (NP > 0 ? NP : 1); ++s) Qv[r][c][s] = Pv[r][c][s] = T(0);
-                if (!(own_plane && own_row[r])) continue;
-                const uint32_t o = oR[r + 1];
-                if (xpml) {
-                    pE[r][0][0] = bld<T>(rpx, o, sxo);
-                    pE[r][0][1] = bld<T>(rpx, o, SB0 + sxo);
-                }
-                if (ypml[r + 1]) {
-                    const uint32_t so = (uint32_t)((pi * Ly + sy[r + 1]) * nz) * TS;
-                    pE[r][1][0] = bld<T>(rpy, oK, so);
-                    pE[r][1][1] = bld<T>(rpy, oK, SB1 + so);
-                }
-                if (zany) {
-                    const uint32_t so = (uint32_t)((pi * ny + gj[r + 1]) * Lz) * TS;
-                    pE[r][2][0] = bld<T>(rpz, oZ, so);
-                    pE[r][2][1] = bld<T>(rpz, oZ, SB2 + so);
-                }
-                if (NP > 0 && !uniform) {
-                    int np[3], lm[3];
+                for (int c = 0; c < 3; ++c) inv[r][c] = iv[r], sq[r][c] = T(0);
+                if (!own(r)) continue;
+                const uint32_t code = cc[r];
+                if (code & kSegSpecial) {
+                    const MatLut<T>* L[3];
 #pragma unroll
                     for (int c = 0; c < 3; ++c) {
-                        const int m = (mw[r] >> (8 * c)) & 0xff;
-                        const int mc = m == kDesignMat ? 0 : m;  // LUT index (design voxels have no poles)
-                        np[c] = m == kDesignMat ? 0 : slut[mc].np;
-                        lm[c] = slut[mc].lorentz_mask;
+                        L[c] = slut + ((mw[r] >> (8 * c)) & 0xff);
+                        inv[r][c] = L[c]->inv_eps;
                     }
+                    const int npx = seg_poles(code);
+                    if (NP > 0 && npx > 0) {
+                        const Rsrc rc = rsrc(Pcur + (long)pi * QPB), ro = rsrc(Pold + (long)pi * QPB);
+                        int np[3];
 #pragma unroll
-                    for (int s = 0; s < NP; ++s) {
-                        if (!wave_any(s < np[0] || s < np[1] || s < np[2])) continue;
-#pragma unroll
-                        for (int c = 0; c < 3; ++c) {
-                            Qv[r][c][s] = bld<T>(rQ, s < np[c] ? o : kOOB, (s * 3 + c) * PB);
-                            Pv[r][c][s] = bld<T>(rP, (s < np[c] && ((lm[c] >> s) & 1)) ? o : kOOB, (s * 3 + c) * PB);
-                        }
-                    }
-                }
-            }
-
-            // ---------------------------------------------------------------- H^{n+1/2} -------
-            T h[TY + 1][3];
-#pragma unroll
-            for (int r = 0; r < TY + 1; ++r) {
-                const bool ok = rv[r];
-                const int j = gj[r];
-                const bool wr = own_plane && r >= 1 && own_row[r > 0 ? r - 1 : 0] && ok;
-                T dEz_y = ec[r + 1][2] - ec[r][2];
-                T dEx_y = ec[r + 1][0] - ec[r][0];
-                T dEy_z = ek1[r][1] - ec[r][1];
-                T dEx_z = ek1[r][0] - ec[r][0];
-                T dEz_x = en[r][2] - ec[r][2];
-                T dEy_x = en[r][1] - ec[r][1];
-                if (ypml[r]) {
-                    GLOBAL const T* cy = coef + a.coff[1];
-                    const T b = cy[2 * ny + j], c = cy[3 * ny + j];
-                    dEz_y = cpml(dEz_y, b, c, pH[r][1][0]);
-                    dEx_y = cpml(dEx_y, b, c, pH[r][1][1]);
-                    if (wr) {
-                        const uint32_t so = (uint32_t)((pi * Ly + sy[r]) * nz) * TS;
-                        bst<NTS>(rpy, oK, hw * SB1 + so, pH[r][1][0]);
-                        bst<NTS>(rpy, oK, (hw + 1) * SB1 + so, pH[r][1][1]);
-                    }
-                }
-                if (ok && zany) {  // lanes outside the layers: b = a = 0 leaves the term unchanged
-                    dEy_z = cpml(dEy_z, bHz, aHz, pH[r][2][0]);
-                    dEx_z = cpml(dEx_z, bHz, aHz, pH[r][2][1]);
-                    if (wr) {
-                        const uint32_t so = (uint32_t)((pi * ny + j) * Lz) * TS;
-                        bst<NTS>(rpz, oZ, hw * SB2 + so, pH[r][2][0]);
-                        bst<NTS>(rpz, oZ, (hw + 1) * SB2 + so, pH[r][2][1]);
-                    }
-                }
-                if (ok && xpml) {
-                    dEz_x = cpml(dEz_x, bHx, aHx, pH[r][0][0]);
-                    dEy_x = cpml(dEy_x, bHx, aHx, pH[r][0][1]);
-                    if (wr) {
-                        bst<NTS>(rpx, oR[r], hw * SB0 + sxo, pH[r][0][0]);
-                        bst<NTS>(rpx, oR[r], (hw + 1) * SB0 + sxo, pH[r][0][1]);
-                    }
-                }
-                // outside a metallic edge H is identically zero (ghost row of the halo)
-                h[r][0] = ok ? h0[r][0] - cdt * (dEz_y - dEy_z) : T(0);
-                h[r][1] = ok ? h0[r][1] - cdt * (dEx_z - dEz_x) : T(0);
-                h[r][2] = ok ? h0[r][2] - cdt * (dEy_x - dEx_y) : T(0);
-                if (wr) {
-                    bst<NTS>(rW, oR[r], 3 * PB, h[r][0]);
-                    bst<NTS>(rW, oR[r], 4 * PB, h[r][1]);
-                    bst<NTS>(rW, oR[r], 5 * PB, h[r][2]);
-                }
-            }
-
-            if (own_plane) {
-                T* buf = sh + (i & 1) * 2 * TY * B;
-#pragma unroll
-                for (int r = 0; r < TY; ++r) {
-                    buf[r * B + kl] = h[r + 1][0];
-                    buf[(TY + r) * B + kl] = h[r + 1][1];
-                }
-                if (ZP && pass + 1 < npass && kl == Z - 1) {
-                    T* zo = zh + ((pass & 1) * a.xc + (i - x0)) * 2 * TY;
-#pragma unroll
-                    for (int r = 0; r < TY; ++r) {
-                        zo[2 * r] = h[r + 1][0];
-                        zo[2 * r + 1] = h[r + 1][1];
-                    }
-                }
-                lds_barrier();
-
-                // ------------------------------------------------------------ E^{n+1} ---------
-#pragma unroll
-                for (int r = 0; r < TY; ++r) {
-                    if (!own_row[r]) continue;
-                    const int j = gj[r + 1];
-                    const uint32_t o = oR[r + 1];
-                    // z neighbour below: the lane below in this pass, else the previous
-                    // pass's last lane (zh), else the periodic image (one pass), else a ghost
-                    T hxkm = T(0), hykm = T(0);
-                    if (kl > 0) {
-                        hxkm = buf[r * B + kl - 1];
-                        hykm = buf[(TY + r) * B + kl - 1];
-                    } else if (ZP && pass > 0) {
-                        const T* zi = zh + (((pass - 1) & 1) * a.xc + (i - x0)) * 2 * TY;
-                        hxkm = zi[2 * r];
-                        hykm = zi[2 * r + 1];
-                    } else if (a.pz) {  // periodic z runs one pass: the image of k = 0 is nz - 1
-                        hxkm = buf[r * B + nz - 1];
-                        hykm = buf[(TY + r) * B + nz - 1];
-                    }
-                    T dHz_y = h[r + 1][2] - h[r][2];
-                    T dHx_y = h[r + 1][0] - h[r][0];
-                    T dHy_z = h[r + 1][1] - hykm;
-                    T dHx_z = h[r + 1][0] - hxkm;
-                    T dHz_x = h[r + 1][2] - hp[r][1];
-                    T dHy_x = h[r + 1][1] - hp[r][0];
-                    if (ypml[r + 1]) {
-                        GLOBAL const T* cy = coef + a.coff[1];
-                        const T b = cy[j], c = cy[ny + j];
-                        dHz_y = cpml(dHz_y, b, c, pE[r][1][0]);
-                        dHx_y = cpml(dHx_y, b, c, pE[r][1][1]);
-                        const uint32_t so = (uint32_t)((pi * Ly + sy[r + 1]) * nz) * TS;
-                        bst<NTS>(rpy, oK, so, pE[r][1][0]);
-                        bst<NTS>(rpy, oK, SB1 + so, pE[r][1][1]);
-                    }
-                    if (zany) {
-                        dHy_z = cpml(dHy_z, bEz, aEz, pE[r][2][0]);
-                        dHx_z = cpml(dHx_z, bEz, aEz, pE[r][2][1]);
-                        const uint32_t so = (uint32_t)((pi * ny + j) * Lz) * TS;
-                        bst<NTS>(rpz, oZ, so, pE[r][2][0]);
-                        bst<NTS>(rpz, oZ, SB2 + so, pE[r][2][1]);
-                    }
-                    if (xpml) {
-                        dHz_x = cpml(dHz_x, bEx, aEx, pE[r][0][0]);
-                        dHy_x = cpml(dHy_x, bEx, aEx, pE[r][0][1]);
-                        bst<NTS>(rpx, o, sxo, pE[r][0][0]);
-                        bst<NTS>(rpx, o, SB0 + sxo, pE[r][0][1]);
-                    }
-                    const T curl[3] = {dHz_y - dHy_z, dHx_z - dHz_x, dHy_x - dHx_y};
-                    if (uniform) {
-                        const T inv = slut[0].inv_eps;
-#pragma unroll
-                        for (int c = 0; c < 3; ++c) bst<NTS>(rW, o, c * PB, ec[r + 1][c] + inv * (cdt * curl[c]));
-                    } else {
-                        int mm[3];
-                        bool des[3];
-                        T inv[3];
-#pragma unroll
-                        for (int c = 0; c < 3; ++c) {
-                            const int m = (mw[r] >> (8 * c)) & 0xff;
-                            des[c] = m == kDesignMat;
-                            mm[c] = des[c] ? 0 : m;
-                            inv[c] = slut[mm[c]].inv_eps;
-                        }
-                        if (a.emap) {  // per-cell eps_inf (smoothed maps)
-                            const Rsrc re = rsrc((const char*)a.emap + (long)pi * 3 * PB);
-#pragma unroll
-                            for (int c = 0; c < 3; ++c) inv[c] = bld<T>(re, o, c * PB);
-                        }
-                        if (wave_any(des[0] || des[1] || des[2])) {
-                            // design voxels: 1/eps from the design array [dx][dy][dz]
-                            const Rsrc rd = rsrc(a.dinv);
-                            const uint32_t dq = (uint32_t)(((pi - a.dlo[0]) * (a.dhi[1] - a.dlo[1]) + (j - a.dlo[1])) *
-                                                               (a.dhi[2] - a.dlo[2]) + (kl + pass * Z - a.dlo[2])) * TS;
-#pragma unroll
-                            for (int c = 0; c < 3; ++c) {
-                                const T v = bld<T>(rd, des[c] ? dq : kOOB, 0);
-                                inv[c] = des[c] ? v : inv[c];
-                            }
-                        }
-                        T sq[3] = {T(0), T(0), T(0)};
+                        for (int c = 0; c < 3; ++c) np[c] = L[c]->np;
 #pragma unroll
                         for (int s = 0; s < NP; ++s) {
-                            int npl[3];
+                            if (s >= npx) break;
+                            PoleCoef<T> p[3];
 #pragma unroll
-                            for (int c = 0; c < 3; ++c) npl[c] = des[c] ? 0 : slut[mm[c]].np;
-                            if (!wave_any(s < npl[0] || s < npl[1] || s < npl[2])) continue;
+                            for (int c = 0; c < 3; ++c) p[c] = L[c]->pole[s];
 #pragma unroll
                             for (int c = 0; c < 3; ++c) {
-                                const MatLut<T>& L = slut[mm[c]];
-                                const bool vq = s < npl[c];
-                                const bool vp = vq && ((L.lorentz_mask >> s) & 1);
+                                const uint32_t so = (s * 3 + c) * PB;
+                                const bool vq = s < np[c];
+                                const T cur = Qv[r][c][s], old = Pv[r][c][s];
                                 T qn;
-                                if constexpr (kPolePair<T>) {
-                                    const T cur = podd ? Pv[r][c][s] : Qv[r][c][s];  // Lorentz: P^n
-                                    const T old = podd ? Qv[r][c][s] : Pv[r][c][s];  // and P^{n-1}
-                                    qn = vp ? L.alpha[s] * (cur - old) + L.beta[s] * cur + L.c3[s] * ec[r + 1][c]
-                                            : L.alpha[s] * Qv[r][c][s] + L.c3[s] * ec[r + 1][c];
-                                    qn = vq ? qn : T(0);
-                                    bst<NTS>(rP, (vp && !podd) ? o : kOOB, (s * 3 + c) * PB, cur + qn);
-                                    bst<NTS>(rQ, (vq && !(vp && !podd)) ? o : kOOB, (s * 3 + c) * PB, vp ? cur + qn : qn);
-                                } else {
-                                    // Pv is zero unless vp (out-of-range load), so beta * Pv adds nothing then
-                                    qn = L.alpha[s] * Qv[r][c][s] + L.c3[s] * ec[r + 1][c] + L.beta[s] * Pv[r][c][s];
-                                    qn = vq ? qn : T(0);
-                                    bst<NTS>(rP, vp ? o : kOOB, (s * 3 + c) * PB, Pv[r][c][s] + qn);
-                                    bst<NTS>(rQ, vq ? o : kOOB, (s * 3 + c) * PB, qn);
+                                if constexpr (kPolePair<T>) {  // Lorentz: P^n, P^{n-1}; Drude (lor = beta = 0): Q^n
+                                    qn = fma_(p[c].c3, e0[r][c], fma_(p[c].alpha, fma_(-p[c].lor, old, cur), p[c].beta * cur));
+                                    bst<NTS>(ro, vq ? oR[r + 1] : kOOB, so, fma_(p[c].lor, cur, qn));
+                                } else {  // Q^n, P^n (zero for a Drude pole)
+                                    qn = fma_(p[c].beta, old, fma_(p[c].c3, e0[r][c], p[c].alpha * cur));
+                                    bst<NTS>(ro, vq && p[c].lor != T(0) ? oR[r + 1] : kOOB, so, old + qn);
+                                    bst<NTS>(rc, vq ? oR[r + 1] : kOOB, so, qn);
                                 }
-                                sq[c] += qn;
+                                sq[r][c] += vq ? qn : T(0);
                             }
                         }
+                    }
+                    if (code & kSegDesign) {
+                        // design voxels: 1/eps from the design array [dx][dy][dz]
+                        const Rsrc rd = rsrc(a.dinv);
+                        const uint32_t dq = (uint32_t)(((pi - a.dlo[0]) * (a.dhi[1] - a.dlo[1]) + (gj[r + 1] - a.dlo[1])) *
+                                                           (a.dhi[2] - a.dlo[2]) + (k - a.dlo[2])) * TS;
 #pragma unroll
-                        for (int c = 0; c < 3; ++c) bst<NTS>(rW, o, c * PB, ec[r + 1][c] + inv[c] * (cdt * curl[c] - sq[c]));
+                        for (int c = 0; c < 3; ++c) dv[r][c] = bld<T>(rd, (int)((mw[r] >> (8 * c)) & 0xff) == a.nmat ? dq : kOOB, 0);
+                        dw[r] = mw[r];
                     }
                 }
+                if (cn[r] & kSegSpecial) {
+                    const uint32_t w = words(cn[r], mwn[r]);
+                    if (NP > 0 && seg_poles(cn[r]) > 0) load_poles(pn, r, cn[r], w);
+                    mw[r] = reg_copy(w);
+                }
+                load_word(pnn, r, cnn[r], mwn[r]);
             }
+            // ------------------------------- loads for the planes ahead
+#pragma unroll
+            for (int r = 0; r < TY + 2; ++r)
+#pragma unroll
+                for (int c = 0; c < 3; ++c)
+                    if (c != 1 || r < TY + 1) ec[r][c] = reg_copy(en[r][c]);
+            load_h(fN, next);
+            load_e(fNN, next && pnn < nx, en);
+            if (next) load_psi_h(pn);
+        };
 
+        auto e_phase = [&](const int i) __attribute__((always_inline)) {
+            const bool next = i + 1 < x1;
+            const bool xpml = in_x(pi);
+            const Rsrc rW = rsrc(fW + F01);
+            const Pair* buf = sh + (i & 1) * TY * (B + 1);
+            // ------------------------------- E^{n+1}
+            lds_barrier();
 #pragma unroll
             for (int r = 0; r < TY; ++r) {
-                hp[r][0] = h[r + 1][1];
-                hp[r][1] = h[r + 1][2];
-                mw[r] = mwn[r];
-            }
-#pragma unroll
-            for (int r = 0; r < TY + 2; ++r) {
-#pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                    ec[r][c] = en[r][c];
-                    en[r][c] = enn[r][c];
+                if (!own(r)) continue;
+                const uint32_t o = oR[r + 1];
+                const Pair* below = buf + r * (B + 1) + kb;
+                if (ZP && pass > 0 && kl == 0) below = zh + (((pass - 1) & 1) * a.xc + (i - x0)) * TY + r;
+                const Pair hk = *below;
+                T dHz_y = h[r + 1][2] - h[r][2];
+                T dHx_y = h[r + 1][0] - h[r][0];
+                T dHy_z = h[r + 1][1] - hk.y;
+                T dHx_z = h[r + 1][0] - hk.x;
+                T dHz_x = h[r + 1][2] - hp[r][1];
+                T dHy_x = h[r + 1][1] - hp[r][0];
+                if (zany) {
+                    const T q0 = aux_next(dHy_z, bEz, aEz, pEz[r].x), q1 = aux_next(dHx_z, bEz, aEz, pEz[r].y);
+                    dHy_z += q0;
+                    dHx_z += q1;
+                    bst2<NTS>(rpz, oZ, zrow(pi, r + 1), Pair{q0, q1});
                 }
+                if (__builtin_expect(yany, 0)) {
+                    if (in_y(r + 1)) {
+                        const T b = cy[gj[r + 1]], c = cy[ny + gj[r + 1]];
+                        const T q0 = aux_next(dHz_y, b, c, pEy[r].x), q1 = aux_next(dHx_y, b, c, pEy[r].y);
+                        dHz_y += q0;
+                        dHx_y += q1;
+                        bst2<NTS>(rpy, oK, yslab(pi, r + 1), Pair{q0, q1});
+                    }
+                }
+                if (__builtin_expect(xpml, 0)) {
+                    const T b = cx[pi], c = cx[nx + pi];
+                    const T q0 = aux_next(dHz_x, b, c, pEx[r].x), q1 = aux_next(dHy_x, b, c, pEx[r].y);
+                    dHz_x += q0;
+                    dHy_x += q1;
+                    bst2<NTS>(rpx, two(o), xslab(pi), Pair{q0, q1});
+                }
+                const T curl[3] = {dHz_y - dHy_z, dHx_z - dHz_x, dHy_x - dHx_y};
+                if (__builtin_expect(emap, 0)) {
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) inv[r][c] = em[r][c];
+                }
+                if (cc[r] & kSegDesign) {
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) inv[r][c] = (int)((dw[r] >> (8 * c)) & 0xff) == a.nmat ? dv[r][c] : inv[r][c];
+                }
+#pragma unroll
+                for (int c = 0; c < 3; ++c) bst<NTS>(rW, o, c * PB, e_next(e0[r][c], inv[r][c], cdt, curl[c], sq[r][c]));
+                hp[r][0] = reg_copy(h[r + 1][1]);
+                hp[r][1] = reg_copy(h[r + 1][2]);
+                if (next) load_psi_e(pn, r);
+                cc[r] = cn[r];
+                cn[r] = cnn[r];
             }
+            // the next plane
+            fW = fN;
+            fN = fNN;
+            pi = pn;
+            pn = pnn;
+            ++pnn;
+            fNN += FPB;
+            if (__builtin_expect(pnn >= nx, 0)) {
+                if (a.px) pnn = 0;
+                fNN = F0;  // of plane 0, or not read
+            }
+        };
+
+        h_phase(x0);
+        for (int i = x0; i < x1; ++i) {
+            e_phase(i);
+            h_phase(i + 1);
         }
     }  // pass
 }
@@ -611,386 +823,428 @@ __device__ __forceinline__ void step_tile(const StepArgs<T>& a, const int t) {
 // y row per thread); thread row 0 recomputes H on the row below the tile (the y halo) and rows
 // 1..rt-1 own rows j0..j0+rt-2.  The y and z neighbours of E (for H) and of H (for E) are
 // exchanged through LDS, so each field value is loaded from global memory once per tile and
-// the y halo costs one extra row per rt-1 owned rows instead of one per row.  The tile
-// marches along x; E of the next two planes and H of the next plane are prefetched into
-// registers one iteration ahead.  The top thread row loads E of the row above the tile
-// (Ex, Ez) itself.  Addressing as in step_tile: per-plane descriptors and 32-bit offsets.
-template <typename T, int NP>
+// the y halo costs one extra row per rt-1 owned rows instead of one per row.  The top thread
+// row loads E of the row above the tile (Ex, Ez) itself.  The tile marches along x; loads,
+// register copies, loop shape and addressing as in step_tile.  One barrier per plane: E of plane
+// i + 1, which H^{n+1/2} of plane i needs anyway, goes to LDS together with that H (both in two
+// halves used in turn), so a plane's H phase starts from what the barrier before it published.
+// A wavefront can span rows, so row conditions are per lane and the wavefront's material is found
+// from its words (k_segments marks in them the cells with poles and the design voxels).
+// Bound by the latency of a plane's serial part (exchange, barrier, pole recursion) at 4 waves per
+// SIMD on grids of up to about 3 M cells, by memory above.  Measured on MI355X, us per step before
+// (two barriers, loads waited for in the iteration that issued them) and now: 24 FP32 grids of 64^3
+// to 192x192x128 in one launch 1126, 915; FP32 141x129x95 76.6, 40.2; FP32 151x133x117 77.4 (one
+// row), 53.6; FP64 101x101x101 58.6 (one row), 41.4; FP64 41x41x41 22.3, 13.0.
+template <typename T, int NP, bool NTS>
 __device__ __forceinline__ void step_rows(const StepArgs<T>& a, const int t) {
+    constexpr uint32_t W = sizeof(T);
+    constexpr int NS = NP > 0 ? NP : 1;
+    typedef Pair2<T> Pair;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const int B = blockDim.x;
-    T* sE = reinterpret_cast<T*>(smem_raw);  // [3][B] E^n of the current plane
-    T* sH = sE + 3 * B;                       // [3][B] H^{n+1/2} of the current plane
-    MatLut<T>* slut = reinterpret_cast<MatLut<T>*>(sH + 3 * B);
-    {
-        GLOBAL const uint32_t* src = (GLOBAL const uint32_t*)a.lut;
-        uint32_t* dst = reinterpret_cast<uint32_t*>(slut);
-        const int words = (int)(sizeof(MatLut<T>) / 4) * a.nmat;
-        for (int q = threadIdx.x; q < words; q += B) dst[q] = src[q];
-    }
+    Pair* sExz = reinterpret_cast<Pair*>(smem_raw);       // [2][B] (Ex, Ez) of E^n
+    Pair* sHxz = sExz + 2 * B;                            // [2][B] (Hx, Hz) of H^{n+1/2}
+    T* sEy = reinterpret_cast<T*>(sHxz + 2 * B);          // [2][B] Ey
+    T* sHy = sEy + 2 * B;                                 // [2][B] Hy
+    MatLut<T>* slut = reinterpret_cast<MatLut<T>*>(sHy + 2 * B);
+    copy_lut(a, slut);
 
-    const long step = *(GLOBAL const long*)a.d_step;
-    const char* F0 = (const char*)a.F[step & 1];
-    const char* F1 = (const char*)a.F[(step + 1) & 1];
-    const char* matw = (const char*)a.matw;
-    GLOBAL const T* coef = (GLOBAL const T*)a.coef;
-    const uint32_t hr = (step & 1) ? 4 : 2;  // H auxiliary pair read this step
-    const uint32_t hw = (step & 1) ? 2 : 4;  // and written
-    // FP32 Lorentz pole slots hold P^n and P^{n-1}: P^n in the Q array on even steps and in
-    // the P array on odd ones, P^{n+1} overwrites P^{n-1}.  Drude slots hold Q^n in the Q array.
-    const bool podd = (step & 1) != 0;
+    const long step = *(CONST const long*)a.d_step;
+    const bool odd = (step & 1) != 0;
+    const char* F0 = (const char*)a.F[odd ? 1 : 0];
+    const long F01 = (const char*)a.F[odd ? 0 : 1] - F0;  // from the set read to the set written
+    const uint32_t hr = odd ? 2 : 1;  // H auxiliary pair read this step
+    const uint32_t hw = odd ? 1 : 2;  // and written
+    const char* Pcur = (const char*)(kPolePair<T> && odd ? a.P : a.Q);  // pole slots as in step_tile
+    const char* Pold = (const char*)(kPolePair<T> && odd ? a.Q : a.P);
+    CONST const T* coef = (CONST const T*)a.coef;
+    CONST const MatLut<T>* clut = (CONST const MatLut<T>*)a.lut;
     const int nx = a.nx, ny = a.ny, nz = a.nz;
     const int RT = a.rt, R = RT - 1;
     const int tid = threadIdx.x;
     const bool act = tid < RT * nz;
     const int r = act ? tid / nz : 0;
     const int k = act ? tid - r * nz : 0;
-    const int tyi = t % a.nty, xci = t / a.nty;
+    const int xci = t / a.nty, tyi = t - xci * a.nty;
     const int jr = tyi * R + r - 1;  // unwrapped global row of this thread row
     const int j = act ? wrap_or_ghost(jr, ny, a.py) : -1;
     const bool valid = j >= 0;
     const bool owned = act && r >= 1 && jr < ny;  // implies valid
     const bool top = act && r == RT - 1;
-    const int jt = top ? wrap_or_ghost(jr + 1, ny, a.py) : -1;
-    const int kp1 = wrap_or_ghost(k + 1, nz, a.pz);
-    const int km1 = wrap_or_ghost(k - 1, nz, a.pz);
+    const int ju = act ? wrap_or_ghost(jr + 1, ny, a.py) : -1;  // the row above
+    const int kp1 = k + 1 < nz ? k + 1 : a.pz ? 0 : -1;
+    const int km1 = k > 0 ? k - 1 : a.pz ? nz - 1 : -1;
     const T cdt = a.cdt;
     const bool uniform = a.uniform != 0;
-    constexpr uint32_t W = sizeof(T);
+    const bool emap = a.emap != nullptr;
     const uint32_t PB = (uint32_t)ny * (uint32_t)nz * W;  // bytes of one component plane
     const long FPB = 6L * PB;                            // bytes of one x plane of a field set
     const long QPB = (long)a.nqp * PB;                   // and of the polarisation
     const long PW = (long)ny * nz * 4;                   // and of the material words
-    // lane offsets within a component plane; kOOB for lanes that neither read nor write
-    const uint32_t oc = valid ? ((uint32_t)j * nz + k) * W : kOOB;
-    const uint32_t ot = jt >= 0 ? ((uint32_t)jt * nz + k) * W : kOOB;
-    const uint32_t ow = owned ? ((uint32_t)j * nz + k) * 4u : kOOB;
-    const uint32_t oo = owned ? oc : kOOB;
-    const uint32_t SB0 = (uint32_t)(a.S[0] * W), SB1 = (uint32_t)(a.S[1] * W), SB2 = (uint32_t)(a.S[2] * W);
-    const Rsrc rpx = rsrc(a.psi[0]), rpy = rsrc(a.psi[1]), rpz = rsrc(a.psi[2]);
     const int Ly = a.plo[1] + a.phi[1], Lz = a.plo[2] + a.phi[2];
+    const uint32_t YP = (uint32_t)(Ly * nz) * 2u * W, ZP = (uint32_t)(ny * Lz) * 2u * W;  // bytes of a slab per plane
+    const uint32_t SP0 = (uint32_t)(2 * a.S[0] * W), SP1 = (uint32_t)(2 * a.S[1] * W), SP2 = (uint32_t)(2 * a.S[2] * W);
+    const Rsrc rpx = rsrc(a.psi[0]), rpy = rsrc(a.psi[1]), rpz = rsrc(a.psi[2]);
+    // planes outside [xlo, xlo + xin) lie in an x layer
+    const int xlo = a.pml_on[0] ? a.plo[0] : 0;
+    const unsigned xin = a.pml_on[0] ? (unsigned)(nx - a.phi[0] - a.plo[0]) : 0xffffffffu;
+    auto in_x = [&](int p) { return (unsigned)(p - xlo) >= xin; };
+    auto xslab = [&](int p) -> uint32_t { return (uint32_t)(p < a.plo[0] ? p : p - (nx - a.phi[0]) + a.plo[0]) * 2u * PB; };
+    CONST const T* cx = coef + a.coff[0];
 
+    // lane offsets; kOOB for lanes that neither read nor write
+    const uint32_t oc = valid ? ((uint32_t)j * nz + k) * W : kOOB;          // the cell
+    const uint32_t oo = owned ? oc : kOOB;                                  // owned cells
+    const uint32_t ot = top && ju >= 0 ? ((uint32_t)ju * nz + k) * W : kOOB;  // the row above the tile
+    const uint32_t ow = owned ? ((uint32_t)j * nz + k) * 4u : kOOB;         // material words
     const bool ypml = valid && in_pml(a, 1, j, ny);
     const bool zpml = valid && in_pml(a, 2, k, nz);
+    const uint32_t oy = ypml ? (uint32_t)((j < a.plo[1] ? j : j - (ny - a.phi[1]) + a.plo[1]) * nz + k) * 2u * W : kOOB;
+    const uint32_t oz = zpml ? (uint32_t)(j * Lz + (k < a.plo[2] ? k : k - (nz - a.phi[2]) + a.plo[2])) * 2u * W : kOOB;
+    const uint32_t oyw = owned ? oy : kOOB, ozw = owned ? oz : kOOB;
     // wavefront-uniform summaries of the per-lane conditions
-    const bool yany = wave_any(ypml), zany = wave_any(zpml), tany = wave_any(jt >= 0), oany = wave_any(owned);
+    const bool yany = wave_any(ypml), zany = wave_any(zpml), tany = wave_any(ot != kOOB);
     T bEy = T(0), aEy = T(0), bHy = T(0), aHy = T(0);
     if (ypml) {
-        GLOBAL const T* cy = coef + a.coff[1];
-        bEy = cy[j];
-        aEy = cy[ny + j];
-        bHy = cy[2 * ny + j];
-        aHy = cy[3 * ny + j];
+        GLOBAL const T* cy = (GLOBAL const T*)a.coef + a.coff[1];
+        bEy = cy[j], aEy = cy[ny + j], bHy = cy[2 * ny + j], aHy = cy[3 * ny + j];
     }
     T bEz = T(0), aEz = T(0), bHz = T(0), aHz = T(0);
     if (zpml) {
-        GLOBAL const T* cz = coef + a.coff[2];
-        bEz = cz[k];
-        aEz = cz[nz + k];
-        bHz = cz[2 * nz + k];
-        aHz = cz[3 * nz + k];
+        GLOBAL const T* cz = (GLOBAL const T*)a.coef + a.coff[2];
+        bEz = cz[k], aEz = cz[nz + k], bHz = cz[2 * nz + k], aHz = cz[3 * nz + k];
     }
-    const int syl = ypml ? (j < a.plo[1] ? j : j - (ny - a.phi[1]) + a.plo[1]) : 0;
-    const int szl = zpml ? (k < a.plo[2] ? k : k - (nz - a.phi[2]) + a.plo[2]) : 0;
-    lds_barrier();  // LUT in LDS: the first plane's pole loads read it before the plane's barriers
+    // exchange slots of the row above (top row: te), the row below and the z neighbours
+    const int up = (top || !act) ? tid : tid + nz, dn = owned ? tid - nz : tid;
+    const int kup = kp1 >= 0 ? r * nz + kp1 : tid, kdn = km1 >= 0 ? r * nz + km1 : tid;
 
     const int x0 = xci * a.xc;
     const int x1 = min(x0 + a.xc, nx);
-    const int istart = (x0 > 0 || a.px) ? x0 - 1 : x0;
 
-    T ec[3], en[3], te[2] = {T(0), T(0)}, ten[2] = {T(0), T(0)}, hc[3], hp[2] = {T(0), T(0)};
-    uint32_t mw = 0;
-    {
-        const int p0 = wrap_or_ghost(istart, nx, a.px);
-        const int p1 = wrap_or_ghost(istart + 1, nx, a.px);
-        const Rsrc r0 = rsrc(F0 + (long)p0 * FPB);
-        const Rsrc r1 = rsrc(F0 + (long)(p1 < 0 ? 0 : p1) * FPB);
-        const uint32_t o1 = p1 >= 0 ? oc : kOOB;
+    // the registers each plane loads anew
+    T ec[3], en[3];                    // E^n of planes i and i + 1
+    T te[2] = {T(0), T(0)}, ten[2] = {T(0), T(0)};  // (Ex, Ez) of the row above the tile: zero past the edge
+    T h0[3];                           // H^{n-1/2} of plane i
+    Pair pHx, pHy, pHz, pEx, pEy, pEz; // PML auxiliaries
+    T em[3];                           // 1/eps of the maps
+    T Qv[3][NS], Pv[3][NS];            // pole state
+    uint32_t mw = 0, mwn = 0;          // material words of planes i, i + 1
+    T hp[2] = {T(0), T(0)};            // H^{n+1/2} (Hy, Hz) of plane i - 1
+    T h[3], e0[3], inv[3], sq[3], dv[3];
+    uint32_t dw = 0;
+    uint32_t cls = 0;                  // material of the wavefront on plane i (classify)
+
+    auto load_e = [&](const char* f, bool need) {
+        const Rsrc rn = rsrc(f, need);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) en[c] = bld<T>(rn, oc, c * PB);
+        if (tany) {
+            ten[0] = bld<T>(rn, ot, 0);
+            ten[1] = bld<T>(rn, ot, 2 * PB);
+        }
+    };
+    auto load_h = [&](const char* f, bool need) {
+        const Rsrc rn = rsrc(f, need);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) h0[c] = bld<T>(rn, oc, (3 + c) * PB);
+    };
+    auto load_psi_h = [&](int p) {
+        if (zany) pHz = bld2<T>(rpz, oz, hr * SP2 + p * ZP);
+        if (yany) pHy = bld2<T>(rpy, oy, hr * SP1 + p * YP);
+        if (__builtin_expect(in_x(p), 0)) pHx = bld2<T>(rpx, two(oc), hr * SP0 + xslab(p));
+    };
+    auto load_psi_e = [&](int p) {
+        if (zany) pEz = bld2<T>(rpz, ozw, p * ZP);
+        if (yany) pEy = bld2<T>(rpy, oyw, p * YP);
+        if (__builtin_expect(in_x(p), 0)) pEx = bld2<T>(rpx, two(oo), xslab(p));
+        if (__builtin_expect(emap, 0)) {
+            const Rsrc re = rsrc((const char*)a.emap + (long)p * 3 * PB);
+#pragma unroll
+            for (int c = 0; c < 3; ++c) em[c] = bld<T>(re, oo, c * PB);
+        }
+    };
+    // kSegSpecial with the most pole slots of a lane (bits 8-10), or the id of the one material, without
+    // poles, of the wavefront's cells
+    auto classify = [&](uint32_t w) -> uint32_t {
+        const uint32_t first = (uint32_t)__builtin_amdgcn_readfirstlane((int)w), id = first & 0xff;
+        if (first == id * 0x010101u && !wave_any(w != first)) return id;
+        uint32_t code = kSegSpecial;
+        if (wave_any((w & kWordDesign) != 0)) code |= kSegDesign;
+        const int np = word_poles(w);
+#pragma unroll
+        for (int s = NP; s > 0; --s)
+            if (wave_any(np >= s)) {
+                code |= (uint32_t)s << 8;
+                break;
+            }
+        return code;
+    };
+    auto load_poles = [&](int p, uint32_t code, uint32_t w) {
+        const int npx = seg_poles(code);
+        const Rsrc rc = rsrc(Pcur + (long)p * QPB), ro = rsrc(Pold + (long)p * QPB);
+        int np[3], lm[3];
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
-            ec[c] = bld<T>(r0, oc, c * PB);
-            en[c] = bld<T>(r1, o1, c * PB);
-            hc[c] = bld<T>(r0, oc, (3 + c) * PB);
+            const MatLut<T>& L = slut[(w >> (8 * c)) & 0xff];
+            np[c] = L.np;
+            lm[c] = L.lorentz_mask;
         }
-        // the row above the tile: only lanes of the top thread row load it
-        if (tany) {
-            const uint32_t t1 = p1 >= 0 ? ot : kOOB;
-            te[0] = bld<T>(r0, ot, 0);
-            te[1] = bld<T>(r0, ot, 2 * PB);
-            ten[0] = bld<T>(r1, t1, 0);
-            ten[1] = bld<T>(r1, t1, 2 * PB);
-        }
-        if (!uniform && istart >= x0 && oany) mw = bld<uint32_t>(rsrc(matw + (long)p0 * PW), ow, 0);
-    }
-
-    for (int i = istart; i < x1; ++i) {
-        const bool own_plane = i >= x0;
-        const bool has_next = i + 1 < x1;
-        const int pi = wrap_or_ghost(i, nx, a.px);
-        const Rsrc rW = rsrc(F1 + (long)pi * FPB);
-        const uint32_t wo = own_plane ? oo : kOOB;  // lanes that write this plane
-        const bool wany = own_plane && oany;
-
-        // ------------------------------------------------------------ loads -----------------
-        T enn[3] = {T(0), T(0), T(0)}, tenn[2] = {T(0), T(0)}, hn[3] = {T(0), T(0), T(0)};
-        uint32_t mwn = 0;
-        if (has_next) {
-            const int pn = wrap_or_ghost(i + 1, nx, a.px);
-            const int pnn = wrap_or_ghost(i + 2, nx, a.px);
-            const Rsrc rn = rsrc(F0 + (long)pn * FPB);
-            const Rsrc rnn = rsrc(F0 + (long)(pnn < 0 ? 0 : pnn) * FPB);
-            const uint32_t onn = pnn >= 0 ? oc : kOOB;
 #pragma unroll
-            for (int c = 0; c < 3; ++c) enn[c] = bld<T>(rnn, onn, c * PB);
-            if (tany) {
-                const uint32_t tn = pnn >= 0 ? ot : kOOB;
-                tenn[0] = bld<T>(rnn, tn, 0);
-                tenn[1] = bld<T>(rnn, tn, 2 * PB);
-            }
-#pragma unroll
-            for (int c = 0; c < 3; ++c) hn[c] = bld<T>(rn, oc, (3 + c) * PB);
-            if (!uniform && oany) mwn = bld<uint32_t>(rsrc(matw + (long)pn * PW), ow, 0);
-        }
-        const bool xpml = in_pml(a, 0, pi, nx);
-        T bEx = T(0), aEx = T(0), bHx = T(0), aHx = T(0);
-        uint32_t sxo = 0;
-        if (xpml) {
-            GLOBAL const T* cx = coef + a.coff[0];
-            bEx = cx[pi];
-            aEx = cx[nx + pi];
-            bHx = cx[2 * nx + pi];
-            aHx = cx[3 * nx + pi];
-            sxo = (uint32_t)(pi < a.plo[0] ? pi : pi - (nx - a.phi[0]) + a.plo[0]) * PB;
-        }
-        // slab lane offsets of this plane (kOOB outside the layer)
-        const uint32_t oy = ypml ? (uint32_t)((pi * Ly + syl) * nz + k) * W : kOOB;
-        const uint32_t oz = zpml ? (uint32_t)((pi * ny + j) * Lz + szl) * W : kOOB;
-        const uint32_t oyw = own_plane && owned ? oy : kOOB, ozw = own_plane && owned ? oz : kOOB;
-        T pH[3][2], pE[3][2];
-#pragma unroll
-        for (int d = 0; d < 3; ++d) pH[d][0] = pH[d][1] = pE[d][0] = pE[d][1] = T(0);
-        if (xpml) {
-            pH[0][0] = bld<T>(rpx, oc, hr * SB0 + sxo);
-            pH[0][1] = bld<T>(rpx, oc, (hr + 1) * SB0 + sxo);
-            if (wany) {
-                pE[0][0] = bld<T>(rpx, wo, sxo);
-                pE[0][1] = bld<T>(rpx, wo, SB0 + sxo);
-            }
-        }
-        if (yany) {
-            pH[1][0] = bld<T>(rpy, oy, hr * SB1);
-            pH[1][1] = bld<T>(rpy, oy, (hr + 1) * SB1);
-            if (wany) {
-                pE[1][0] = bld<T>(rpy, oyw, 0);
-                pE[1][1] = bld<T>(rpy, oyw, SB1);
-            }
-        }
-        if (zany) {
-            pH[2][0] = bld<T>(rpz, oz, hr * SB2);
-            pH[2][1] = bld<T>(rpz, oz, (hr + 1) * SB2);
-            if (wany) {
-                pE[2][0] = bld<T>(rpz, ozw, 0);
-                pE[2][1] = bld<T>(rpz, ozw, SB2);
-            }
-        }
-        T Qv[3][NP > 0 ? NP : 1], Pv[3][NP > 0 ? NP : 1];
-#pragma unroll
-        for (int c = 0; c < 3; ++c)
-#pragma unroll
-            for (int s = 0; s < (NP > 0 ? NP : 1); ++s) Qv[c][s] = Pv[c][s] = T(0);
-        const Rsrc rQ = rsrc((const char*)a.Q + (long)pi * QPB);
-        const Rsrc rP = rsrc((const char*)a.P + (long)pi * QPB);
-        int mm[3] = {0, 0, 0}, npl[3] = {0, 0, 0};
-        bool des[3] = {false, false, false};
-        if (NP > 0 && !uniform && wany) {
+        for (int s = 0; s < NP; ++s) {
+            if (s >= npx) break;
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
-                const int m = (mw >> (8 * c)) & 0xff;
-                des[c] = m == kDesignMat;
-                mm[c] = des[c] ? 0 : m;
-                npl[c] = des[c] ? 0 : slut[mm[c]].np;
-            }
-#pragma unroll
-            for (int s = 0; s < NP; ++s) {
-                if (!wave_any(s < npl[0] || s < npl[1] || s < npl[2])) continue;
-#pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                    const bool vq = s < npl[c];
-                    const bool vp = vq && ((slut[mm[c]].lorentz_mask >> s) & 1);
-                    Qv[c][s] = bld<T>(rQ, vq ? wo : kOOB, (s * 3 + c) * PB);
-                    Pv[c][s] = bld<T>(rP, vp ? wo : kOOB, (s * 3 + c) * PB);
-                }
+                // (a Drude slot reads one value; the second array may be absent without Lorentz poles)
+                Qv[c][s] = bld<T>(rc, s < np[c] ? oo : kOOB, (s * 3 + c) * PB);
+                Pv[c][s] = bld<T>(ro, (lm[c] >> s) & 1 ? oo : kOOB, (s * 3 + c) * PB);
             }
         }
+    };
 
-        // ------------------------------------------------------------ H^{n+1/2} on plane i --
-        sE[tid] = ec[0];
-        sE[B + tid] = ec[1];
-        sE[2 * B + tid] = ec[2];
-        lds_barrier();
-        T h[3];
+    // ---- the chunk's first planes; H (y and z components) of the plane before it
+    int pi = x0, pn = wrap_up(x0 + 1, nx, a.px), pnn = wrap_up(pn + 1, nx, a.px);  // nx or more: past the edge
+    const char* fW = F0 + (long)pi * FPB;  // plane i, then i + 1 and i + 2, of the set read
+    const char* fN = F0 + (long)min(pn, nx - 1) * FPB;
+    const char* fNN = F0 + (long)min(pnn, nx - 1) * FPB;
+    load_e(fW, true);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) ec[c] = en[c];
+    te[0] = ten[0];
+    te[1] = ten[1];
+    load_h(fW, true);
+    if (!uniform) {
+        mw = bld<uint32_t>(rsrc((const char*)a.matw + (long)pi * PW), ow, 0);
+        mwn = bld<uint32_t>(rsrc((const char*)a.matw + (long)min(pn, nx - 1) * PW, x0 + 1 < x1), ow, 0);
+    }
+    if (x0 > 0 || a.px) {
+        const int p = x0 > 0 ? x0 - 1 : nx - 1;
+        const bool xp = in_x(p);
+        const Rsrc rn = rsrc(F0 + (long)p * FPB);
+        const uint32_t ou = owned && ju >= 0 ? ((uint32_t)ju * nz + k) * W : kOOB;
+        const uint32_t ok = owned && kp1 >= 0 ? ((uint32_t)j * nz + kp1) * W : kOOB;
+        T eh[3], eu, ekx, hh[2];
+        Pair qx, qy, qz;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) eh[c] = bld<T>(rn, oo, c * PB);
+        eu = bld<T>(rn, ou, 0);
+        ekx = bld<T>(rn, ok, 0);
+        hh[0] = bld<T>(rn, oo, 4 * PB);
+        hh[1] = bld<T>(rn, oo, 5 * PB);
+        if (xp) qx = bld2<T>(rpx, two(oo), hr * SP0 + xslab(p));
+        if (yany) qy = bld2<T>(rpy, oyw, hr * SP1 + p * YP);
+        if (zany) qz = bld2<T>(rpz, ozw, hr * SP2 + p * ZP);
+        T dEx_y = eu - eh[0], dEx_z = ekx - eh[0], dEz_x = ec[2] - eh[2], dEy_x = ec[1] - eh[1];
+        if (yany) dEx_y += aux_next(dEx_y, bHy, aHy, qy.y);
+        if (zany) dEx_z += aux_next(dEx_z, bHz, aHz, qz.y);
+        if (xp) {
+            const T b = cx[2 * nx + p], c = cx[3 * nx + p];
+            dEz_x += aux_next(dEz_x, b, c, qx.x);
+            dEy_x += aux_next(dEy_x, b, c, qx.y);
+        }
+        hp[0] = h_next(hh[0], cdt, dEx_z, dEz_x);
+        hp[1] = h_next(hh[1], cdt, dEy_x, dEx_y);
+    }
+    sExz[(x0 & 1) * B + tid] = Pair{ec[0], ec[2]};
+    sEy[(x0 & 1) * B + tid] = ec[1];
+    lds_barrier();  // also the material table
+    load_e(fN, pn < nx);
+    load_psi_h(pi);
+    load_psi_e(pi);
+    if (!uniform) {
+        cls = classify(mw);
+        if (NP > 0 && seg_poles(cls) > 0) load_poles(pi, cls, mw);
+    }
+
+    auto h_phase = [&](const int i) __attribute__((always_inline)) {
+        const bool live = i < x1, next = i + 1 < x1;
+        const bool xpml = live && in_x(pi);
+        const Rsrc rW = rsrc(fW + F01, live);
+        const int half = (i & 1) * B, other = B - half;
+        const T iv = clut[cls & 0xff].inv_eps;
+        // ------------------------------- H^{n+1/2}
         {
-            const int up = (top || !act) ? tid : tid + nz;  // the row above within the tile (top row: te)
-            const T exj = top ? te[0] : sE[up];
-            const T ezj = top ? te[1] : sE[2 * B + up];
-            const T exk = kp1 >= 0 ? sE[r * nz + kp1] : T(0);
-            const T eyk = kp1 >= 0 ? sE[B + r * nz + kp1] : T(0);
-            T dEz_y = ezj - ec[2];
-            T dEx_y = exj - ec[0];
-            T dEy_z = eyk - ec[1];
-            T dEx_z = exk - ec[0];
+            const Pair eu = sExz[half + up];
+            const T exk = sExz[half + kup].x, eyk = sEy[half + kup];
+            T dEz_y = (top ? te[1] : eu.y) - ec[2];
+            T dEx_y = (top ? te[0] : eu.x) - ec[0];
+            T dEy_z = (kp1 >= 0 ? eyk : T(0)) - ec[1];
+            T dEx_z = (kp1 >= 0 ? exk : T(0)) - ec[0];
             T dEz_x = en[2] - ec[2];
             T dEy_x = en[1] - ec[1];
-            // lanes outside a PML layer carry zero coefficients and auxiliaries: no change
-            if (yany) {
-                dEz_y = cpml(dEz_y, bHy, aHy, pH[1][0]);
-                dEx_y = cpml(dEx_y, bHy, aHy, pH[1][1]);
-            }
+            // lanes outside a PML layer carry zero coefficients: no change
             if (zany) {
-                dEy_z = cpml(dEy_z, bHz, aHz, pH[2][0]);
-                dEx_z = cpml(dEx_z, bHz, aHz, pH[2][1]);
+                const T q0 = aux_next(dEy_z, bHz, aHz, pHz.x), q1 = aux_next(dEx_z, bHz, aHz, pHz.y);
+                dEy_z += q0;
+                dEx_z += q1;
+                if (live) bst2<NTS>(rpz, ozw, hw * SP2 + pi * ZP, Pair{q0, q1});
             }
-            if (xpml) {
-                dEz_x = cpml(dEz_x, bHx, aHx, pH[0][0]);
-                dEy_x = cpml(dEy_x, bHx, aHx, pH[0][1]);
+            if (yany) {
+                const T q0 = aux_next(dEz_y, bHy, aHy, pHy.x), q1 = aux_next(dEx_y, bHy, aHy, pHy.y);
+                dEz_y += q0;
+                dEx_y += q1;
+                if (live) bst2<NTS>(rpy, oyw, hw * SP1 + pi * YP, Pair{q0, q1});
+            }
+            if (__builtin_expect(xpml, 0)) {
+                const T b = cx[2 * nx + pi], c = cx[3 * nx + pi];
+                const T q0 = aux_next(dEz_x, b, c, pHx.x), q1 = aux_next(dEy_x, b, c, pHx.y);
+                dEz_x += q0;
+                dEy_x += q1;
+                bst2<NTS>(rpx, two(oo), hw * SP0 + xslab(pi), Pair{q0, q1});
             }
             // outside a metallic edge H is identically zero (ghost rows)
-            h[0] = valid ? hc[0] - cdt * (dEz_y - dEy_z) : T(0);
-            h[1] = valid ? hc[1] - cdt * (dEx_z - dEz_x) : T(0);
-            h[2] = valid ? hc[2] - cdt * (dEy_x - dEx_y) : T(0);
-            if (wany) {
-                bst(rW, wo, 3 * PB, h[0]);
-                bst(rW, wo, 4 * PB, h[1]);
-                bst(rW, wo, 5 * PB, h[2]);
-                if (xpml) {
-                    bst(rpx, wo, hw * SB0 + sxo, pH[0][0]);
-                    bst(rpx, wo, (hw + 1) * SB0 + sxo, pH[0][1]);
-                }
-                if (yany) {
-                    bst(rpy, oyw, hw * SB1, pH[1][0]);
-                    bst(rpy, oyw, (hw + 1) * SB1, pH[1][1]);
-                }
-                if (zany) {
-                    bst(rpz, ozw, hw * SB2, pH[2][0]);
-                    bst(rpz, ozw, (hw + 1) * SB2, pH[2][1]);
-                }
-            }
+            h[0] = valid ? h_next(h0[0], cdt, dEz_y, dEy_z) : T(0);
+            h[1] = valid ? h_next(h0[1], cdt, dEx_z, dEz_x) : T(0);
+            h[2] = valid ? h_next(h0[2], cdt, dEy_x, dEx_y) : T(0);
         }
-        sH[tid] = h[0];
-        sH[B + tid] = h[1];
-        sH[2 * B + tid] = h[2];
-        lds_barrier();
-
-        // ------------------------------------------------------------ E^{n+1} on plane i ----
-        if (wany) {
-            const int dn = owned ? tid - nz : tid;  // the row below within the tile
-            const T hxj = sH[dn];
-            const T hzj = sH[2 * B + dn];
-            const T hxk = km1 >= 0 ? sH[r * nz + km1] : T(0);
-            const T hyk = km1 >= 0 ? sH[B + r * nz + km1] : T(0);
-            T dHz_y = h[2] - hzj;
-            T dHx_y = h[0] - hxj;
-            T dHy_z = h[1] - hyk;
-            T dHx_z = h[0] - hxk;
-            T dHz_x = h[2] - hp[1];
-            T dHy_x = h[1] - hp[0];
-            if (yany) {
-                dHz_y = cpml(dHz_y, bEy, aEy, pE[1][0]);
-                dHx_y = cpml(dHx_y, bEy, aEy, pE[1][1]);
-                bst(rpy, oyw, 0, pE[1][0]);
-                bst(rpy, oyw, SB1, pE[1][1]);
-            }
-            if (zany) {
-                dHy_z = cpml(dHy_z, bEz, aEz, pE[2][0]);
-                dHx_z = cpml(dHx_z, bEz, aEz, pE[2][1]);
-                bst(rpz, ozw, 0, pE[2][0]);
-                bst(rpz, ozw, SB2, pE[2][1]);
-            }
-            if (xpml) {
-                dHz_x = cpml(dHz_x, bEx, aEx, pE[0][0]);
-                dHy_x = cpml(dHy_x, bEx, aEx, pE[0][1]);
-                bst(rpx, wo, sxo, pE[0][0]);
-                bst(rpx, wo, SB0 + sxo, pE[0][1]);
-            }
-            const T curl[3] = {dHz_y - dHy_z, dHx_z - dHz_x, dHy_x - dHx_y};
-            if (uniform) {
-                const T inv = slut[0].inv_eps;
-#pragma unroll
-                for (int c = 0; c < 3; ++c) bst(rW, wo, c * PB, ec[c] + inv * (cdt * curl[c]));
-            } else {
-                T inv[3];
-#pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                    if (NP == 0) {  // material ids were not decoded for the pole loads
-                        const int m = (mw >> (8 * c)) & 0xff;
-                        des[c] = m == kDesignMat;
-                        mm[c] = des[c] ? 0 : m;
-                    }
-                    inv[c] = slut[mm[c]].inv_eps;
-                }
-                if (a.emap) {  // per-cell eps_inf (smoothed maps)
-                    const Rsrc re = rsrc((const char*)a.emap + (long)pi * 3 * PB);
-#pragma unroll
-                    for (int c = 0; c < 3; ++c) inv[c] = bld<T>(re, wo, c * PB);
-                }
-                if (wave_any(des[0] || des[1] || des[2])) {
-                    const Rsrc rd = rsrc(a.dinv);
-                    const uint32_t dq = (uint32_t)(((pi - a.dlo[0]) * (a.dhi[1] - a.dlo[1]) + (j - a.dlo[1])) *
-                                                       (a.dhi[2] - a.dlo[2]) + (k - a.dlo[2])) * W;
-#pragma unroll
-                    for (int c = 0; c < 3; ++c) {
-                        const T v = bld<T>(rd, des[c] ? dq : kOOB, 0);
-                        inv[c] = des[c] ? v : inv[c];
-                    }
-                }
-                T sq[3] = {T(0), T(0), T(0)};
-#pragma unroll
-                for (int s = 0; s < NP; ++s) {
-                    if (!wave_any(s < npl[0] || s < npl[1] || s < npl[2])) continue;
-#pragma unroll
-                    for (int c = 0; c < 3; ++c) {
-                        const MatLut<T>& L = slut[mm[c]];
-                        const bool vq = s < npl[c];
-                        const bool vp = vq && ((L.lorentz_mask >> s) & 1);
-                        T qn;
-                        if constexpr (kPolePair<T>) {
-                            const T cur = podd ? Pv[c][s] : Qv[c][s];  // Lorentz: P^n
-                            const T old = podd ? Qv[c][s] : Pv[c][s];  // and P^{n-1}
-                            qn = vp ? L.alpha[s] * (cur - old) + L.beta[s] * cur + L.c3[s] * ec[c]
-                                    : L.alpha[s] * Qv[c][s] + L.c3[s] * ec[c];
-                            qn = vq ? qn : T(0);
-                            bst(rP, (vp && !podd) ? wo : kOOB, (s * 3 + c) * PB, cur + qn);
-                            bst(rQ, (vq && !(vp && !podd)) ? wo : kOOB, (s * 3 + c) * PB, vp ? cur + qn : qn);
-                        } else {
-                            // Pv is zero unless vp (out-of-range load), so beta * Pv adds nothing then
-                            qn = L.alpha[s] * Qv[c][s] + L.c3[s] * ec[c] + L.beta[s] * Pv[c][s];
-                            qn = vq ? qn : T(0);
-                            bst(rP, vp ? wo : kOOB, (s * 3 + c) * PB, Pv[c][s] + qn);
-                            bst(rQ, vq ? wo : kOOB, (s * 3 + c) * PB, qn);
-                        }
-                        sq[c] += qn;
-                    }
-                }
-#pragma unroll
-                for (int c = 0; c < 3; ++c) bst(rW, wo, c * PB, ec[c] + inv[c] * (cdt * curl[c] - sq[c]));
-            }
-        }
-
-        hp[0] = h[1];
-        hp[1] = h[2];
-        mw = mwn;
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
-            ec[c] = en[c];
-            en[c] = enn[c];
-            hc[c] = hn[c];
+            pin(h[c]);
+            bst<NTS>(rW, oo, (3 + c) * PB, h[c]);
+            e0[c] = reg_copy(ec[c]);
         }
-        te[0] = ten[0];
-        te[1] = ten[1];
-        ten[0] = tenn[0];
-        ten[1] = tenn[1];
+        sHxz[half + tid] = Pair{h[0], h[2]};
+        sHy[half + tid] = h[1];
+        sExz[other + tid] = Pair{en[0], en[2]};
+        sEy[other + tid] = en[1];
+        // ------------------------------- polarisation: sum of Q^{n+1} over the poles; 1/eps
+#pragma unroll
+        for (int c = 0; c < 3; ++c) inv[c] = iv, sq[c] = T(0);
+        if (cls & kSegSpecial) {
+            const MatLut<T>* L[3];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                L[c] = slut + ((mw >> (8 * c)) & 0xff);
+                inv[c] = L[c]->inv_eps;
+            }
+            const int npx = seg_poles(cls);
+            if (NP > 0 && npx > 0) {
+                const Rsrc rc = rsrc(Pcur + (long)pi * QPB), ro = rsrc(Pold + (long)pi * QPB);
+                int np[3];
+#pragma unroll
+                for (int c = 0; c < 3; ++c) np[c] = L[c]->np;
+#pragma unroll
+                for (int s = 0; s < NP; ++s) {
+                    if (s >= npx) break;
+                    PoleCoef<T> p[3];
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) p[c] = L[c]->pole[s];
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) {
+                        const uint32_t so = (s * 3 + c) * PB;
+                        const bool vq = s < np[c];
+                        const T cur = Qv[c][s], old = Pv[c][s];
+                        T qn;
+                        if constexpr (kPolePair<T>) {  // Lorentz: P^n, P^{n-1}; Drude (lor = beta = 0): Q^n
+                            qn = fma_(p[c].c3, e0[c], fma_(p[c].alpha, fma_(-p[c].lor, old, cur), p[c].beta * cur));
+                            bst<NTS>(ro, vq ? oo : kOOB, so, fma_(p[c].lor, cur, qn));
+                        } else {  // Q^n, P^n (zero for a Drude pole)
+                            qn = fma_(p[c].beta, old, fma_(p[c].c3, e0[c], p[c].alpha * cur));
+                            bst<NTS>(ro, vq && p[c].lor != T(0) ? oo : kOOB, so, old + qn);
+                            bst<NTS>(rc, vq ? oo : kOOB, so, qn);
+                        }
+                        sq[c] += vq ? qn : T(0);
+                    }
+                }
+            }
+            if (cls & kSegDesign) {
+                // design voxels: 1/eps from the design array [dx][dy][dz]
+                const Rsrc rd = rsrc(a.dinv);
+                const uint32_t dq = (uint32_t)(((pi - a.dlo[0]) * (a.dhi[1] - a.dlo[1]) + (j - a.dlo[1])) *
+                                                   (a.dhi[2] - a.dlo[2]) + (k - a.dlo[2])) * W;
+#pragma unroll
+                for (int c = 0; c < 3; ++c)
+                    dv[c] = bld<T>(rd, owned && (int)((mw >> (8 * c)) & 0xff) == a.nmat ? dq : kOOB, 0);
+                dw = mw;
+            }
+        }
+        // ------------------------------- loads for the planes ahead
+        uint32_t cn = 0u;
+        if (!uniform && next) {
+            cn = classify(mwn);
+            if (NP > 0 && seg_poles(cn) > 0) load_poles(pn, cn, mwn);
+        }
+        mw = reg_copy(mwn);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) ec[c] = reg_copy(en[c]);
+        if (tany) {
+            te[0] = reg_copy(ten[0]);
+            te[1] = reg_copy(ten[1]);
+        }
+        load_h(fN, next);
+        load_e(fNN, next && pnn < nx);
+        if (!uniform) mwn = bld<uint32_t>(rsrc((const char*)a.matw + (long)(i + 2 < x1 ? pnn : 0) * PW, i + 2 < x1), ow, 0);
+        if (next) load_psi_h(pn);
+        return cn;
+    };
+
+    auto e_phase = [&](const int i) __attribute__((always_inline)) {
+        const bool next = i + 1 < x1;
+        const bool xpml = in_x(pi);
+        const Rsrc rW = rsrc(fW + F01);
+        const int half = (i & 1) * B;
+        lds_barrier();
+        const Pair hd = sHxz[half + dn];
+        const T hxk = sHxz[half + kdn].x, hyk = sHy[half + kdn];
+        T dHz_y = h[2] - hd.y;
+        T dHx_y = h[0] - hd.x;
+        T dHy_z = h[1] - (km1 >= 0 ? hyk : T(0));
+        T dHx_z = h[0] - (km1 >= 0 ? hxk : T(0));
+        T dHz_x = h[2] - hp[1];
+        T dHy_x = h[1] - hp[0];
+        if (zany) {
+            const T q0 = aux_next(dHy_z, bEz, aEz, pEz.x), q1 = aux_next(dHx_z, bEz, aEz, pEz.y);
+            dHy_z += q0;
+            dHx_z += q1;
+            bst2<NTS>(rpz, ozw, pi * ZP, Pair{q0, q1});
+        }
+        if (yany) {
+            const T q0 = aux_next(dHz_y, bEy, aEy, pEy.x), q1 = aux_next(dHx_y, bEy, aEy, pEy.y);
+            dHz_y += q0;
+            dHx_y += q1;
+            bst2<NTS>(rpy, oyw, pi * YP, Pair{q0, q1});
+        }
+        if (__builtin_expect(xpml, 0)) {
+            const T b = cx[pi], c = cx[nx + pi];
+            const T q0 = aux_next(dHz_x, b, c, pEx.x), q1 = aux_next(dHy_x, b, c, pEx.y);
+            dHz_x += q0;
+            dHy_x += q1;
+            bst2<NTS>(rpx, two(oo), xslab(pi), Pair{q0, q1});
+        }
+        const T curl[3] = {dHz_y - dHy_z, dHx_z - dHz_x, dHy_x - dHx_y};
+        if (__builtin_expect(emap, 0)) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) inv[c] = em[c];
+        }
+        if (cls & kSegDesign) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) inv[c] = (int)((dw >> (8 * c)) & 0xff) == a.nmat ? dv[c] : inv[c];
+        }
+#pragma unroll
+        for (int c = 0; c < 3; ++c) bst<NTS>(rW, oo, c * PB, e_next(e0[c], inv[c], cdt, curl[c], sq[c]));
+        hp[0] = reg_copy(h[1]);
+        hp[1] = reg_copy(h[2]);
+        if (next) load_psi_e(pn);
+        // the next plane
+        fW = fN;
+        fN = fNN;
+        pi = pn;
+        pn = pnn;
+        ++pnn;
+        fNN += FPB;
+        if (__builtin_expect(pnn >= nx, 0)) {
+            if (a.px) pnn = 0;
+            fNN = F0;  // of plane 0, or not read
+        }
+    };
+
+    uint32_t cn = h_phase(x0);
+    for (int i = x0; i < x1; ++i) {
+        e_phase(i);
+        cls = cn;
+        cn = h_phase(i + 1);
     }
 }
+
 
 // XCD-aware tile order: hardware places workgroup w on XCD w % 8; map so that each XCD
 // receives a contiguous run of logical tiles (y-tile fastest, then x-chunk), then find the
@@ -1009,13 +1263,24 @@ __device__ __forceinline__ int tile_instance(const int* __restrict__ tile_first,
 }
 
 // Fused step over all instances of a launch set (rows-per-thread form).
-// Waves per SIMD the register allocator must leave room for: the FP32 one-row tile with up to
-// three pole slots fits 96 registers (5 waves; the z-pass variant keeps 12 bytes per lane in
-// scratch); the FP64 one-row tile is held to 168 registers (3 waves; with three pole slots it
-// spills about 30 bytes per lane and still runs 3% faster than at 2 waves on the 96^3 box);
-// other variants are unconstrained.
-template <typename T, int TY, int NP>
-constexpr int step_waves() { return (sizeof(T) == 4 && TY == 1 && NP <= 3) ? 5 : (sizeof(T) == 8 && TY == 1) ? 3 : 1; }
+// Waves per SIMD the register allocator must leave room for.  FP32 one-row tiles: 4 (109 registers
+// with three pole slots, no scratch; at 5 waves, 96 registers, 80-100 bytes of scratch per lane took
+// 2.3 times as long), 5 without poles (88 registers), 3 in z passes (161); FP64 one-row tiles: 2
+// (178-215 registers; at 3 waves 170-220 bytes of scratch took 1.4 times as long), 3 without poles
+// (162); two FP32 rows: 2 (178).
+template <typename T, int TY, int NP, bool ZP = false>
+constexpr int step_waves() {
+    if (TY > 2 || (TY == 2 && sizeof(T) == 8)) return 1;
+    if (sizeof(T) == 8) return NP == 0 && !ZP ? 3 : 2;
+    return TY == 2 ? 2 : ZP ? 3 : NP == 0 ? 5 : 4;
+}
+
+// The same of the row-of-threads tiles: FP32 81-117 registers, FP64 136 without poles, 155 with one,
+// 187-199 with more (no scratch up to 512 threads; FP64 at 1024 threads, 128 registers, spills).
+template <typename T, int NP>
+constexpr int rows_waves() {
+    return sizeof(T) == 4 ? 4 : NP <= 1 ? 3 : 2;
+}
 
 // NTS: stores with the non-temporal hint (launch sets that stream more than the caches hold).
 template <typename T, int TY, int NP, int MAXT, bool NTS = false>
@@ -1028,7 +1293,7 @@ k_step(const StepArgs<T>* __restrict__ args, const int* __restrict__ tile_first,
 
 // The same with the z line in passes of StepArgs::zseg cells (one row per thread)
 template <typename T, int NP, int MAXT, bool NTS = false>
-__global__ void __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(step_waves<T, 1, NP>())))
+__global__ void __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(step_waves<T, 1, NP, true>())))
 k_step_z(const StepArgs<T>* __restrict__ args, const int* __restrict__ tile_first, int ninst) {
     int t;
     const int b = tile_instance(tile_first, ninst, t);
@@ -1036,12 +1301,12 @@ k_step_z(const StepArgs<T>* __restrict__ args, const int* __restrict__ tile_firs
 }
 
 // Fused step over all instances of a launch set (row-of-threads form).
-template <typename T, int NP, int MAXT>
+template <typename T, int NP, int MAXT, bool NTS = false>
 __global__ void __launch_bounds__(MAXT) k_step_rows(const StepArgs<T>* __restrict__ args,
                                                     const int* __restrict__ tile_first, int ninst) {
     int t;
     const int b = tile_instance(tile_first, ninst, t);
-    step_rows<T, NP>(args[b], t);
+    step_rows<T, NP, NTS>(args[b], t);
 }
 
 // ---- per-step scalars live on the device --------------------------------------------------
@@ -1454,12 +1719,7 @@ __device__ __forceinline__ void adj_tile(const AdjArgs<T>& g, const int t) {
     T* se = reinterpret_cast<T*>(smem_raw);  // [2 parity][4][B]: z E-terms of rows -1 and 0
     T* sd = se + 8 * B;                      // [2 parity][2][B]: z H-terms of row 0
     MatLut<T>* slut = reinterpret_cast<MatLut<T>*>(sd + 4 * B);
-    {
-        GLOBAL const uint32_t* src = (GLOBAL const uint32_t*)a.lut;
-        uint32_t* dst = reinterpret_cast<uint32_t*>(slut);
-        const int words = (int)(sizeof(MatLut<T>) / 4) * a.nmat;
-        for (int q = threadIdx.x; q < words; q += B) dst[q] = src[q];
-    }
+    copy_lut(a, slut);
     const char* AR = (const char*)g.A[g.rd];
     const char* AW = (const char*)g.A[1 - g.rd];
     const char* matw = (const char*)a.matw;
@@ -1573,7 +1833,7 @@ __device__ __forceinline__ void adj_tile(const AdjArgs<T>& g, const int t) {
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
                 const int m = (wc1 >> (8 * c)) & 0xff;
-                des[c] = m == kDesignMat;
+                des[c] = m == a.nmat;
                 mm[c] = des[c] ? 0 : m;
                 npl[c] = des[c] ? 0 : slut[mm[c]].np;
             }
@@ -1798,9 +2058,9 @@ __device__ __forceinline__ void adj_tile(const AdjArgs<T>& g, const int t) {
                             const uint32_t so = (s * 3 + c) * PB;
                             const T pb = pv[s][c];
                             const T qb = vq ? qv[s][c] + pb - u0[c] : T(0);
-                            bst<NTS>(rQ, vq ? o : kOOB, so, L.alpha[s] * qb);
-                            bst<NTS>(rP, vp ? o : kOOB, so, pb + L.beta[s] * qb);
-                            out[c] += L.c3[s] * qb;
+                            bst<NTS>(rQ, vq ? o : kOOB, so, L.pole[s].alpha * qb);
+                            bst<NTS>(rP, vp ? o : kOOB, so, pb + L.pole[s].beta * qb);
+                            out[c] += L.pole[s].c3 * qb;
                         }
                     }
                 }
@@ -1854,14 +2114,9 @@ __device__ __forceinline__ void adj_rows(const AdjArgs<T>& g, const int t) {
     const int RT = a.rt, R = RT - 1;
     T* sE = reinterpret_cast<T*>(smem_raw);  // [4][B]: E-terms z (Ex->Hy), z (Ey->Hx), y (Ex->Hz), y (Ez->Hx)
     T* sEt = sE + 4 * B;                     // [2][nz]: y-terms of the row above the tile
-    T* sD = sEt + 2 * nz;                    // [4][B]: H-terms z (Hy->Ex), z (Hx->Ey), y (Hx->Ez), y (Hz->Ex)
+    T* sD = sEt + 2 * ((nz + 1) & ~1);       // [4][B]: H-terms z (Hy->Ex), z (Hx->Ey), y (Hx->Ez), y (Hz->Ex)
     MatLut<T>* slut = reinterpret_cast<MatLut<T>*>(sD + 4 * B);
-    {
-        GLOBAL const uint32_t* src = (GLOBAL const uint32_t*)a.lut;
-        uint32_t* dst = reinterpret_cast<uint32_t*>(slut);
-        const int words = (int)(sizeof(MatLut<T>) / 4) * a.nmat;
-        for (int q = threadIdx.x; q < words; q += B) dst[q] = src[q];
-    }
+    copy_lut(a, slut);
     const char* AR = (const char*)g.A[g.rd];
     const char* AW = (const char*)g.A[1 - g.rd];
     const char* matw = (const char*)a.matw;
@@ -1988,7 +2243,7 @@ __device__ __forceinline__ void adj_rows(const AdjArgs<T>& g, const int t) {
 #pragma unroll
             for (int c = 0; c < 3; ++c) {  // lanes of other rows: no poles, no design voxel
                 const int m = (wc >> (8 * c)) & 0xff;
-                des[c] = wr && m == kDesignMat;
+                des[c] = wr && m == a.nmat;
                 mm[c] = (wr && !des[c]) ? m : 0;
                 npl[c] = (wr && !des[c]) ? slut[mm[c]].np : 0;
             }
@@ -2152,9 +2407,9 @@ __device__ __forceinline__ void adj_rows(const AdjArgs<T>& g, const int t) {
                         const uint32_t so = (s * 3 + c) * PB;
                         const T pb = pv[s][c];
                         const T qb = vq ? qv[s][c] + pb - uc[c] : T(0);
-                        bst(rQ, vq ? o : kOOB, so, L.alpha[s] * qb);
-                        bst(rP, vp ? o : kOOB, so, pb + L.beta[s] * qb);
-                        out[c] += L.c3[s] * qb;
+                        bst(rQ, vq ? o : kOOB, so, L.pole[s].alpha * qb);
+                        bst(rP, vp ? o : kOOB, so, pb + L.pole[s].beta * qb);
+                        out[c] += L.pole[s].c3 * qb;
                     }
                 }
             }
