@@ -86,6 +86,8 @@ struct sjf_engine {
     uint32_t* matw = nullptr;
     uint32_t* seg = nullptr;  // material segment codes (k_segments)
     double pole_bytes = 0;    // pole state the step moves
+    void* stage = nullptr;    // pinned host memory of the read-outs (read_out)
+    size_t stage_bytes = 0;
     void* lut = nullptr;
     int nmat = 1;
     int maxp = 0;
@@ -1034,6 +1036,8 @@ int free_all(sjf_engine* e) {
     dev_free(e->coefbuf);
     for (int d = 0; d < 3; ++d) dev_free(e->psibuf[d]);
     dev_free(e->d_samples);
+    if (e->stage) (void)hipHostFree(e->stage);
+    e->stage = nullptr;
     for (auto& d : e->dft) {
         dev_free(d.acc);
         dev_free(d.cmp);
@@ -1063,33 +1067,65 @@ int write_component(sjf_engine* e, int comp, const double* src) {
     return SJF_OK;
 }
 
-template <typename T>
-int read_component(sjf_engine* e, int comp, double* dst) {
-    const size_t plane = sizeof(T) * (size_t)e->g.ny * e->g.nz;
-    std::vector<T> tmp(e->N);
-    const char* src = (const char*)field_set(e) + plane * comp;
-    HIPCHK(e, hipMemcpy2DAsync(tmp.data(), plane, src, 6 * plane, plane, e->g.nx, hipMemcpyDeviceToHost, e->stream));
-    HIPCHK(e, hipStreamSynchronize(e->stream));
-    for (long q = 0; q < e->N; ++q) dst[q] = (double)tmp[q];
+// Pinned host memory of an engine's read-outs, at least `bytes` (grown to the largest chunk read, at
+// most two chunks; freed with the engine).
+constexpr size_t kReadChunk = 4u << 20;
+int read_stage(sjf_engine* e, size_t bytes) {
+    if (bytes <= e->stage_bytes) return SJF_OK;
+    if (e->stage) (void)hipHostFree(e->stage);
+    e->stage = nullptr;
+    e->stage_bytes = 0;
+    const size_t want = std::max<size_t>(bytes, 4096);
+    if (hipHostMalloc(&e->stage, want, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        e->stage = nullptr;
+        return fail(e, SJF_E_NOMEM, "read-out buffer allocation failed");
+    }
+    e->stage_bytes = want;
     return SJF_OK;
 }
 
-// Copies the cell box [lo, hi) of one component: one strided 2-D copy (y rows of the box's z
-// span) per x plane of the box into a pinned-free host staging array, then converts to FP64.
+// n values of `size` bytes into dst: launch(first, count, p) has the device write values first ..
+// first + count - 1 to p.  More than one chunk: the device fills one half of the stage while the other
+// is copied out.
+template <typename L>
+int read_out(sjf_engine* e, void* dst, long n, size_t size, L launch) {
+    const long per = std::min<long>(n, (long)(kReadChunk / size));
+    const bool one = per >= n;
+    if (int rc = read_stage(e, (one ? 1 : 2) * (size_t)per * size)) return rc;
+    char* half[2] = {(char*)e->stage, (char*)e->stage + (one ? 0 : (size_t)per * size)};
+    long done = 0, have = 0;  // values copied out; values of the chunk the stage holds, not yet copied
+    for (long first = 0, c = 0; first < n || have > 0; ++c) {
+        const long count = std::min(per, n - first);
+        if (count > 0) {
+            launch(first, count, (void*)half[c & 1]);
+            HIPCHK(e, hipGetLastError());
+            first += count;
+        }
+        if (have > 0) std::memcpy((char*)dst + (size_t)done * size, half[(c & 1) ^ 1], (size_t)have * size);
+        done += have;
+        have = std::max(count, 0L);
+        HIPCHK(e, hipStreamSynchronize(e->stream));
+    }
+    return SJF_OK;
+}
+
+// The cell box [lo, hi) of one component of the current field set, z-fastest FP64.
 template <typename T>
 int read_component_box(sjf_engine* e, int comp, const int* lo, const int* hi, double* dst) {
-    const size_t plane = sizeof(T) * (size_t)e->g.ny * e->g.nz;
-    const size_t bx = (size_t)(hi[0] - lo[0]), by = (size_t)(hi[1] - lo[1]), bz = (size_t)(hi[2] - lo[2]);
-    std::vector<T> tmp(bx * by * bz);
-    const char* base = (const char*)field_set(e) + plane * comp;
-    for (size_t i = 0; i < bx; ++i) {
-        const char* src = base + 6 * plane * (size_t)(lo[0] + i) + sizeof(T) * ((size_t)lo[1] * e->g.nz + lo[2]);
-        HIPCHK(e, hipMemcpy2DAsync(tmp.data() + i * by * bz, sizeof(T) * bz, src, sizeof(T) * (size_t)e->g.nz,
-                                   sizeof(T) * bz, by, hipMemcpyDeviceToHost, e->stream));
-    }
-    HIPCHK(e, hipStreamSynchronize(e->stream));
-    for (size_t q = 0; q < tmp.size(); ++q) dst[q] = (double)tmp[q];
-    return SJF_OK;
+    const long plane = (long)e->g.ny * e->g.nz;
+    const int by = hi[1] - lo[1], bz = hi[2] - lo[2];
+    const T* base = (const T*)field_set(e) + (6L * lo[0] + comp) * plane + (long)lo[1] * e->g.nz + lo[2];
+    return read_out(e, dst, (long)(hi[0] - lo[0]) * by * bz, sizeof(double), [&](long first, long count, void* p) {
+        hipLaunchKernelGGL((sjf::k_read_box<T>), dim3((unsigned)std::min(1024L, (count + 255) / 256)), dim3(256), 0,
+                           e->stream, base, 6 * plane, e->g.nz, by, bz, first, count, (double*)p);
+    });
+}
+
+template <typename T>
+int read_component(sjf_engine* e, int comp, double* dst) {
+    const int lo[3] = {0, 0, 0}, hi[3] = {e->g.nx, e->g.ny, e->g.nz};
+    return read_component_box<T>(e, comp, lo, hi, dst);
 }
 
 template <typename T>
@@ -2512,22 +2548,21 @@ int sjf_get_field(sjf_engine* e, int comp, const double xyz[3], double out[2]) {
     long idx[8];
     double w[8];
     trilinear(e, comp, xyz, idx, w);
-    double v = 0;
+    sjf::GatherPoint g;
     for (int q = 0; q < 8; ++q) {
-        if (idx[q] < 0) continue;
-        const char* base = (const char*)field_set(e) + field_offset(e, comp, idx[q]);
-        if (e->prec == 4) {
-            float f;
-            int rc = d2h(e, &f, base, 4);
-            if (rc) return rc;
-            v += w[q] * f;
-        } else {
-            double f;
-            int rc = d2h(e, &f, base, 8);
-            if (rc) return rc;
-            v += w[q] * f;
-        }
+        g.idx[q] = idx[q] < 0 ? -1 : sjf::field_index(idx[q], comp, (long)e->g.ny * e->g.nz);
+        g.w[q] = w[q];
     }
+    double v = 0;
+    const int rc = read_out(e, &v, 1, sizeof(v), [&](long, long, void* p) {
+        if (e->prec == 4)
+            hipLaunchKernelGGL((sjf::k_read_point<float>), dim3(1), dim3(64), 0, e->stream, (const float*)field_set(e), g,
+                               (double*)p);
+        else
+            hipLaunchKernelGGL((sjf::k_read_point<double>), dim3(1), dim3(64), 0, e->stream, (const double*)field_set(e),
+                               g, (double*)p);
+    });
+    if (rc) return rc;
     out[0] = v;
     out[1] = 0.0;
     return SJF_OK;
@@ -2571,15 +2606,10 @@ int sjf_read_dft(sjf_engine* e, int id, double* out, size_t cap) {
     const long n = (long)d.ncomp * (long)d.freqs.size() * d.ncell;
     if ((size_t)(2 * n) > cap) return fail(e, SJF_E_ARG, "output buffer too small");
     if (int rc = sync_engine(e)) return rc;
-    std::vector<double2> a(n), c(n);
-    int rc = d2h(e, a.data(), d.acc, sizeof(double2) * n);
-    if (!rc) rc = d2h(e, c.data(), d.cmp, sizeof(double2) * n);
-    if (rc) return rc;
-    for (long q = 0; q < n; ++q) {
-        out[2 * q] = a[q].x + c[q].x;
-        out[2 * q + 1] = a[q].y + c[q].y;
-    }
-    return SJF_OK;
+    return read_out(e, out, n, sizeof(double2), [&](long first, long count, void* p) {
+        hipLaunchKernelGGL(sjf::k_read_dft, dim3((unsigned)std::min(1024L, (count + 255) / 256)), dim3(256), 0, e->stream,
+                           (const double2*)d.acc + first, (const double2*)d.cmp + first, count, (double2*)p);
+    });
 }
 
 int sjf_dft_flux(sjf_engine* e, int id, int axis, double* flux, size_t cap) {

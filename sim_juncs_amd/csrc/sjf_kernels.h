@@ -126,9 +126,12 @@ __device__ __forceinline__ bool in_pml(const StepArgs<T>& a, int d, int c, int n
 // compiler fuses.
 __device__ __forceinline__ float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 __device__ __forceinline__ double fma_(double a, double b, double c) { return __builtin_fma(a, b, c); }
-// the updated CPML auxiliary b psi + c d of a term d, which adds it
+// the updated CPML auxiliary b psi + c d of a term d, which adds it: along x and z, and along y (one
+// product is rounded, the other is not; which one is a choice that later sums must repeat)
 template <typename T>
-__device__ __forceinline__ T aux_next(T d, T b, T c, T psi) { return fma_(b, psi, c * d); }
+__device__ __forceinline__ T aux_next(T d, T b, T c, T psi) { return fma_(c, d, b * psi); }
+template <typename T>
+__device__ __forceinline__ T aux_next_y(T d, T b, T c, T psi) { return fma_(b, psi, c * d); }
 // H - cdt (x - y)
 template <typename T>
 __device__ __forceinline__ T h_next(T h, T cdt, T x, T y) { return fma_(-cdt, x - y, h); }
@@ -564,7 +567,7 @@ __device__ __forceinline__ void step_tile(const StepArgs<T>& a, const int t) {
                 T dEx_z = ekx[r] - eh[r][0];
                 T dEz_x = ec[r + 1][2] - eh[r][2];
                 T dEy_x = ec[r + 1][1] - eh[r][1];
-                if (in_y(r + 1)) dEx_y += aux_next(dEx_y, cy[2 * ny + gj[r + 1]], cy[3 * ny + gj[r + 1]], qy[r].y);
+                if (in_y(r + 1)) dEx_y += aux_next_y(dEx_y, cy[2 * ny + gj[r + 1]], cy[3 * ny + gj[r + 1]], qy[r].y);
                 if (zany) dEx_z += aux_next(dEx_z, bHz, aHz, qz[r].y);
                 if (xp) {
                     const T b = cx[2 * nx + p], c = cx[3 * nx + p];
@@ -624,7 +627,7 @@ __device__ __forceinline__ void step_tile(const StepArgs<T>& a, const int t) {
                 for (int r = 0; r < TY + 1; ++r) {
                     if (!in_y(r)) continue;
                     const T b = cy[2 * ny + gj[r]], c = cy[3 * ny + gj[r]];
-                    const T q0 = aux_next(d[r][0], b, c, pHy[r].x), q1 = aux_next(d[r][1], b, c, pHy[r].y);
+                    const T q0 = aux_next_y(d[r][0], b, c, pHy[r].x), q1 = aux_next_y(d[r][1], b, c, pHy[r].y);
                     d[r][0] += q0;
                     d[r][1] += q1;
                     if (r > 0 && own(r - 1) && live) bst2<NTS>(rpy, oK, hw * SP1 + yslab(pi, r), Pair{q0, q1});
@@ -703,7 +706,7 @@ __device__ __forceinline__ void step_tile(const StepArgs<T>& a, const int t) {
                                     qn = fma_(p[c].c3, e0[r][c], fma_(p[c].alpha, fma_(-p[c].lor, old, cur), p[c].beta * cur));
                                     bst<NTS>(ro, vq ? oR[r + 1] : kOOB, so, fma_(p[c].lor, cur, qn));
                                 } else {  // Q^n, P^n (zero for a Drude pole)
-                                    qn = fma_(p[c].beta, old, fma_(p[c].c3, e0[r][c], p[c].alpha * cur));
+                                    qn = fma_(p[c].beta, old, fma_(p[c].alpha, cur, p[c].c3 * e0[r][c]));
                                     bst<NTS>(ro, vq && p[c].lor != T(0) ? oR[r + 1] : kOOB, so, old + qn);
                                     bst<NTS>(rc, vq ? oR[r + 1] : kOOB, so, qn);
                                 }
@@ -768,7 +771,7 @@ __device__ __forceinline__ void step_tile(const StepArgs<T>& a, const int t) {
                 if (__builtin_expect(yany, 0)) {
                     if (in_y(r + 1)) {
                         const T b = cy[gj[r + 1]], c = cy[ny + gj[r + 1]];
-                        const T q0 = aux_next(dHz_y, b, c, pEy[r].x), q1 = aux_next(dHx_y, b, c, pEy[r].y);
+                        const T q0 = aux_next_y(dHz_y, b, c, pEy[r].x), q1 = aux_next_y(dHx_y, b, c, pEy[r].y);
                         dHz_y += q0;
                         dHx_y += q1;
                         bst2<NTS>(rpy, oK, yslab(pi, r + 1), Pair{q0, q1});
@@ -1034,7 +1037,7 @@ __device__ __forceinline__ void step_rows(const StepArgs<T>& a, const int t) {
         if (yany) qy = bld2<T>(rpy, oyw, hr * SP1 + p * YP);
         if (zany) qz = bld2<T>(rpz, ozw, hr * SP2 + p * ZP);
         T dEx_y = eu - eh[0], dEx_z = ekx - eh[0], dEz_x = ec[2] - eh[2], dEy_x = ec[1] - eh[1];
-        if (yany) dEx_y += aux_next(dEx_y, bHy, aHy, qy.y);
+        if (yany) dEx_y += aux_next_y(dEx_y, bHy, aHy, qy.y);
         if (zany) dEx_z += aux_next(dEx_z, bHz, aHz, qz.y);
         if (xp) {
             const T b = cx[2 * nx + p], c = cx[3 * nx + p];
@@ -1079,7 +1082,7 @@ __device__ __forceinline__ void step_rows(const StepArgs<T>& a, const int t) {
                 if (live) bst2<NTS>(rpz, ozw, hw * SP2 + pi * ZP, Pair{q0, q1});
             }
             if (yany) {
-                const T q0 = aux_next(dEz_y, bHy, aHy, pHy.x), q1 = aux_next(dEx_y, bHy, aHy, pHy.y);
+                const T q0 = aux_next_y(dEz_y, bHy, aHy, pHy.x), q1 = aux_next_y(dEx_y, bHy, aHy, pHy.y);
                 dEz_y += q0;
                 dEx_y += q1;
                 if (live) bst2<NTS>(rpy, oyw, hw * SP1 + pi * YP, Pair{q0, q1});
@@ -1138,7 +1141,7 @@ __device__ __forceinline__ void step_rows(const StepArgs<T>& a, const int t) {
                             qn = fma_(p[c].c3, e0[c], fma_(p[c].alpha, fma_(-p[c].lor, old, cur), p[c].beta * cur));
                             bst<NTS>(ro, vq ? oo : kOOB, so, fma_(p[c].lor, cur, qn));
                         } else {  // Q^n, P^n (zero for a Drude pole)
-                            qn = fma_(p[c].beta, old, fma_(p[c].c3, e0[c], p[c].alpha * cur));
+                            qn = fma_(p[c].beta, old, fma_(p[c].alpha, cur, p[c].c3 * e0[c]));
                             bst<NTS>(ro, vq && p[c].lor != T(0) ? oo : kOOB, so, old + qn);
                             bst<NTS>(rc, vq ? oo : kOOB, so, qn);
                         }
@@ -1198,7 +1201,7 @@ __device__ __forceinline__ void step_rows(const StepArgs<T>& a, const int t) {
             bst2<NTS>(rpz, ozw, pi * ZP, Pair{q0, q1});
         }
         if (yany) {
-            const T q0 = aux_next(dHz_y, bEy, aEy, pEy.x), q1 = aux_next(dHx_y, bEy, aEy, pEy.y);
+            const T q0 = aux_next_y(dHz_y, bEy, aEy, pEy.x), q1 = aux_next_y(dHx_y, bEy, aEy, pEy.y);
             dHz_y += q0;
             dHx_y += q1;
             bst2<NTS>(rpy, oyw, pi * YP, Pair{q0, q1});
@@ -1307,6 +1310,53 @@ __global__ void __launch_bounds__(MAXT) k_step_rows(const StepArgs<T>* __restric
     int t;
     const int b = tile_instance(tile_first, ninst, t);
     step_rows<T, NP, NTS>(args[b], t);
+}
+
+// ---- read-outs ---------------------------------------------------------------------------------
+// They write FP64 values into pinned host memory, in the order the caller receives them: one launch
+// and one wait per chunk, and the copy into the caller's array is a plain memcpy.  Bound by the
+// host link and by that memcpy, not by the kernels.
+
+// Cells first, first + 1, .. of the box at `base` (its first cell of the component) of by x bz cells
+// per x plane; planes are `plane` values apart, rows nz.
+template <typename T>
+__global__ void __launch_bounds__(256) k_read_box(const T* __restrict__ base, long plane, int nz, int by, int bz,
+                                                  long first, long count, double* __restrict__ out) {
+    const long stride = (long)gridDim.x * blockDim.x;
+    for (long q = (long)blockIdx.x * blockDim.x + threadIdx.x; q < count; q += stride) {
+        const long row = (first + q) / bz;
+        const int k = (int)(first + q - row * bz);
+        const long i = row / by;
+        out[q] = (double)base[i * plane + (row - i * by) * nz + k];
+    }
+}
+
+// DFT values: running sum and its compensation
+__global__ void __launch_bounds__(256) k_read_dft(const double2* __restrict__ acc, const double2* __restrict__ cmp,
+                                                  long count, double2* __restrict__ out) {
+    const long stride = (long)gridDim.x * blockDim.x;
+    for (long q = (long)blockIdx.x * blockDim.x + threadIdx.x; q < count; q += stride) {
+        const double2 a = acc[q], c = cmp[q];
+        out[q] = double2{a.x + c.x, a.y + c.y};
+    }
+}
+
+// A field value between cells: eight cells (element indices, -1: outside) and their weights, summed
+// in order with separate products and sums, as the host sums them
+struct GatherPoint {
+    long idx[8];
+    double w[8];
+};
+template <typename T>
+__global__ void k_read_point(const T* __restrict__ F, const GatherPoint g, double* __restrict__ out) {
+    T f[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) f[q] = g.idx[q] >= 0 ? F[g.idx[q]] : T(0);
+    double v = 0;
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+        if (g.idx[q] >= 0) v = __dadd_rn(v, __dmul_rn(g.w[q], (double)f[q]));
+    if (threadIdx.x == 0) out[0] = v;
 }
 
 // ---- per-step scalars live on the device --------------------------------------------------

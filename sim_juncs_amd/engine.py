@@ -213,9 +213,9 @@ class Engine:
     def read_dft(self, i: int) -> np.ndarray:
         """complex array [n_comp (ascending component order), n_freq, *box]"""
         ncomp, nf, ext = self._dft[i]
-        out = np.zeros((ncomp, nf) + ext + (2,))
-        self._chk(self.lib.sjf_read_dft(self.h, int(i), _dp(out), out.size), "sjf_read_dft")
-        return out[..., 0] + 1j * out[..., 1]
+        out = np.empty((ncomp, nf) + ext, dtype=np.complex128)
+        self._chk(self.lib.sjf_read_dft(self.h, int(i), _dp(out), 2 * out.size), "sjf_read_dft")
+        return out
 
     def dft_flux(self, i: int, axis: int) -> np.ndarray:
         """Flux along +axis through DFT plane i, one value per frequency (sjf_dft_flux)."""
@@ -255,12 +255,12 @@ class Engine:
     def read_field(self, comp, lo=None, hi=None) -> np.ndarray:
         """A whole component, or with lo/hi the cell box [lo, hi) of it (FP64, shape of the box)."""
         if lo is None and hi is None:
-            out = np.zeros(self.shape)
+            out = np.empty(self.shape)
             self._chk(self.lib.sjf_read_field(self.h, comp_index(comp), _dp(out)), "sjf_read_field")
             return out
         lo = np.ascontiguousarray(lo if lo is not None else (0, 0, 0), dtype=np.int32)
         hi = np.ascontiguousarray(hi if hi is not None else self.shape, dtype=np.int32)
-        out = np.zeros(tuple(max(int(h) - int(l), 0) for l, h in zip(lo, hi)))
+        out = np.empty(tuple(max(int(h) - int(l), 0) for l, h in zip(lo, hi)))
         self._chk(self.lib.sjf_read_field_box(self.h, comp_index(comp), _ip(lo), _ip(hi), _dp(out)),
                   "sjf_read_field_box")
         return out
