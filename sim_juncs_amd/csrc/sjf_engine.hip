@@ -75,17 +75,19 @@ struct sjf_engine {
     long* d_step = nullptr;
     long step = 0;
 
-    // materials: given_* as the caller set them; matw_h / lut_h / nmat / maxp are what the kernels
-    // run (the given map, with Lorentz poles folded out of the PML slabs when pml_fref > 0)
+    // materials: given* as the caller set them; matw / lut_h / nmat / maxp are what the kernels run
+    // (the given map, with Lorentz poles folded out of the PML slabs when pml_fref > 0: twin)
     bool have_mat = false;
-    std::vector<uint32_t> given_w;
+    uint32_t* given = nullptr;  // device, [x][y][z]
     std::vector<sjf_material> given_lut;
     double pml_fref = 0;
-    std::vector<uint32_t> matw_h;
+    std::vector<int> twin;  // per given material its id in the PML slabs, or -1
     std::vector<sjf_material> lut_h;
     uint32_t* matw = nullptr;
-    uint32_t* seg = nullptr;  // material segment codes (k_segments)
+    uint32_t* seg = nullptr;  // material segment codes (k_words)
     double pole_bytes = 0;    // pole state the step moves
+    double pole_values = 0;   // poles summed over cells and components
+    size_t pol_bytes = 0;     // size of Qbuf (and of Pbuf where there is one)
     void* stage = nullptr;    // pinned host memory of the read-outs (read_out)
     size_t stage_bytes = 0;
     void* lut = nullptr;
@@ -240,10 +242,11 @@ void axis_weights(int n, double dx, double off, int periodic, double lo, double 
     }
 }
 
-double inv_eps_at(const sjf_engine* e, long q, int c) {
+// 1/eps at component c of cell q, whose material word (as the kernels run it) is w
+double inv_eps_at(const sjf_engine* e, long q, int c, uint32_t w) {
     if (!e->have_mat) return 1.0;
-    const int m = (e->matw_h[q] >> (8 * c)) & 0xff;
-    if (m == sjf::kDesignMat) {
+    const int m = (w >> (8 * c)) & 0xff;
+    if (m == e->nmat) {
         const int k = (int)(q % e->g.nz);
         const long r = q / e->g.nz;
         const int j = (int)(r % e->g.ny), i = (int)(r / e->g.ny);
@@ -254,6 +257,43 @@ double inv_eps_at(const sjf_engine* e, long q, int c) {
     }
     if (!e->emap_eff.empty()) return 1.0 / e->emap_eff[(size_t)c * e->N + q];
     return 1.0 / e->lut_h[m].eps_inf;
+}
+
+// Pinned host memory of an engine's read-outs, at least `bytes` (grown to the largest chunk read, at
+// most two chunks; freed with the engine).
+constexpr size_t kReadChunk = 4u << 20;
+int read_stage(sjf_engine* e, size_t bytes) {
+    if (bytes <= e->stage_bytes) return SJF_OK;
+    if (e->stage) (void)hipHostFree(e->stage);
+    e->stage = nullptr;
+    e->stage_bytes = 0;
+    const size_t want = std::max<size_t>(bytes, 4096);
+    if (hipHostMalloc(&e->stage, want, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        e->stage = nullptr;
+        return fail(e, SJF_E_NOMEM, "read-out buffer allocation failed");
+    }
+    e->stage_bytes = want;
+    return SJF_OK;
+}
+
+// Material words of the listed cells, through the read-out stage
+int words_at(sjf_engine* e, const std::vector<long>& cells, std::vector<uint32_t>& w) {
+    const long n = (long)cells.size(), most = (long)(kReadChunk / 16);
+    w.assign(n, 0u);
+    if (!e->have_mat) return SJF_OK;
+    for (long q = 0; q < n; q += most) {
+        const long m = std::min(most, n - q);
+        if (int rc = read_stage(e, 16 * (size_t)m)) return rc;
+        long* in = (long*)e->stage;
+        uint32_t* out = (uint32_t*)(in + m);
+        std::memcpy(in, cells.data() + q, sizeof(long) * m);
+        hipLaunchKernelGGL(sjf::k_read_words, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, e->stream, e->matw, in, m, out);
+        HIPCHK(e, hipGetLastError());
+        HIPCHK(e, hipStreamSynchronize(e->stream));
+        std::memcpy(w.data() + q, out, sizeof(uint32_t) * m);
+    }
+    return SJF_OK;
 }
 
 // Row-of-threads form: (rows + 1) thread rows of nz threads per workgroup, 32-bit offsets.
@@ -541,9 +581,11 @@ int build_set_t(LaunchSet* s) {
                 const int sid = (int)srcs.size();
                 srcs.push_back(d);
                 const long base = (long)idx.size();
+                std::vector<uint32_t> word;
+                if (!mag && (rc = words_at(e, src.idx, word))) return rc;
                 for (size_t q = 0; q < src.idx.size(); ++q) {
                     idx.push_back(sjf::field_index(src.idx[q], src.comp, (long)e->g.ny * e->g.nz));
-                    coef.push_back(e->dt * src.wt[q] * (mag ? 1.0 : inv_eps_at(e, src.idx[q], src.comp)));
+                    coef.push_back(e->dt * src.wt[q] * (mag ? 1.0 : inv_eps_at(e, src.idx[q], src.comp, word[q])));
                 }
                 const long n = (long)src.idx.size();
                 for (long b = 0; b < n; b += 256) {
@@ -1026,6 +1068,7 @@ int free_all(sjf_engine* e) {
     e->own = nullptr;
     for (int b = 0; b < 2; ++b) dev_free(e->Fbuf[b]);
     dev_free(e->d_step);
+    dev_free(e->given);
     dev_free(e->matw);
     dev_free(e->seg);
     dev_free(e->lut);
@@ -1064,24 +1107,6 @@ int write_component(sjf_engine* e, int comp, const double* src) {
     char* dst = (char*)field_set(e) + plane * comp;
     HIPCHK(e, hipMemcpy2DAsync(dst, 6 * plane, tmp.data(), plane, plane, e->g.nx, hipMemcpyHostToDevice, e->stream));
     HIPCHK(e, hipStreamSynchronize(e->stream));
-    return SJF_OK;
-}
-
-// Pinned host memory of an engine's read-outs, at least `bytes` (grown to the largest chunk read, at
-// most two chunks; freed with the engine).
-constexpr size_t kReadChunk = 4u << 20;
-int read_stage(sjf_engine* e, size_t bytes) {
-    if (bytes <= e->stage_bytes) return SJF_OK;
-    if (e->stage) (void)hipHostFree(e->stage);
-    e->stage = nullptr;
-    e->stage_bytes = 0;
-    const size_t want = std::max<size_t>(bytes, 4096);
-    if (hipHostMalloc(&e->stage, want, hipHostMallocDefault) != hipSuccess) {
-        (void)hipGetLastError();
-        e->stage = nullptr;
-        return fail(e, SJF_E_NOMEM, "read-out buffer allocation failed");
-    }
-    e->stage_bytes = want;
     return SJF_OK;
 }
 
@@ -1160,25 +1185,36 @@ int upload_lut_t(sjf_engine* e) {
 
 int upload_lut(sjf_engine* e) { return e->prec == 4 ? upload_lut_t<float>(e) : upload_lut_t<double>(e); }
 
-// Segment codes of the material words and the LUT on the device (after a change of either), and the
-// bytes of pole state the step moves (whole segments).
-int update_segments(sjf_engine* e) {
-    const long rows = (long)e->g.nx * e->g.ny, n = rows * ((e->g.nz + 63) / 64);
-    if (int rc = dev_alloc(e, (void**)&e->seg, sizeof(uint32_t) * (n + 3))) return rc;
-    auto* slots = (unsigned long long*)(e->seg + n + (n & 1));
-    unsigned long long count = 0;
-    HIPCHK(e, hipMemcpyAsync(slots, &count, sizeof(count), hipMemcpyHostToDevice, e->stream));
-    const dim3 grid((unsigned)((n + 3) / 4)), block(256);
+// The words and segment codes the kernels run (k_words; after a change of the given words, the twins
+// or the LUT), and what the step moves of pole state: bytes of whole segments, and poles.
+int update_words(sjf_engine* e) {
+    const long n = (long)e->g.nx * e->g.ny * ((e->g.nz + 63) / 64);
+    int rc = dev_alloc(e, (void**)&e->matw, sizeof(uint32_t) * e->N);
+    if (!rc) rc = dev_alloc(e, (void**)&e->seg, sizeof(uint32_t) * (n + 5));
+    if (rc) return rc;
+    auto* sums = (unsigned long long*)(e->seg + n + (n & 1));
+    unsigned long long count[2] = {0, 0};
+    HIPCHK(e, hipMemcpyAsync(sums, count, sizeof(count), hipMemcpyHostToDevice, e->stream));
+    sjf::WordMap map;
+    const int dim[3] = {e->g.nx, e->g.ny, e->g.nz};
+    for (int d = 0; d < 3; ++d) {
+        map.lo[d] = e->pml_on[d] ? e->pml[2 * d] : 0;
+        map.hi[d] = dim[d] - (e->pml_on[d] ? e->pml[2 * d + 1] : 0);
+    }
+    for (int m = 0; m < 256; ++m)
+        map.twin[m] = (unsigned char)(m < (int)e->twin.size() && e->twin[m] >= 0 ? e->twin[m] : m);
+    const dim3 grid((unsigned)std::min(2048L, (n + 3) / 4)), block(256);
     if (e->prec == 4)
-        hipLaunchKernelGGL((sjf::k_segments<float>), grid, block, 0, e->stream, e->matw, (const sjf::MatLut<float>*)e->lut,
-                           e->seg, rows, e->g.nz, e->nmat, slots);
+        hipLaunchKernelGGL((sjf::k_words<float>), grid, block, 0, e->stream, e->given, e->matw, e->seg,
+                           (const sjf::MatLut<float>*)e->lut, dim[0], dim[1], dim[2], e->nmat, map, sums);
     else
-        hipLaunchKernelGGL((sjf::k_segments<double>), grid, block, 0, e->stream, e->matw,
-                           (const sjf::MatLut<double>*)e->lut, e->seg, rows, e->g.nz, e->nmat, slots);
+        hipLaunchKernelGGL((sjf::k_words<double>), grid, block, 0, e->stream, e->given, e->matw, e->seg,
+                           (const sjf::MatLut<double>*)e->lut, dim[0], dim[1], dim[2], e->nmat, map, sums);
     HIPCHK(e, hipGetLastError());
-    HIPCHK(e, hipMemcpyAsync(&count, slots, sizeof(count), hipMemcpyDeviceToHost, e->stream));
+    HIPCHK(e, hipMemcpyAsync(count, sums, sizeof(count), hipMemcpyDeviceToHost, e->stream));
     HIPCHK(e, hipStreamSynchronize(e->stream));
-    e->pole_bytes = 64.0 * 3 * (e->Pbuf ? 2 : 1) * e->prec * (double)count;
+    e->pole_bytes = 64.0 * 3 * (e->Pbuf ? 2 : 1) * e->prec * (double)count[0];
+    e->pole_values = (double)count[1];
     return SJF_OK;
 }
 
@@ -1221,8 +1257,7 @@ bool cell_in_pml(const sjf_engine* e, long q) {
 // Drude poles kept).  Uploads the words and the LUT and resets the polarisation state.
 int apply_materials(sjf_engine* e) {
     const int ng = (int)e->given_lut.size();
-    e->lut_h = e->given_lut;
-    e->matw_h = e->given_w;
+    std::vector<sjf_material> all = e->given_lut;  // and the twins
     bool any_pml = e->pml_on[0] || e->pml_on[1] || e->pml_on[2];
     std::vector<double> fold_add(ng, 0.0);  // sum of the folded Lorentz poles' Re chi per material
     std::vector<int> twin(ng, -1);
@@ -1250,34 +1285,30 @@ int apply_materials(sjf_engine* e) {
             fold_add[m] = eps - M.eps_inf;
             T.eps_inf = eps >= 1.0 ? eps : M.eps_inf;
             for (int s = T.npoles; s < SJF_MAX_POLES; ++s) T.f0[s] = T.gamma[s] = T.sigma[s] = 0, T.is_drude[s] = 0;
-            if ((int)e->lut_h.size() >= SJF_MAX_MATERIALS)
+            if ((int)all.size() >= SJF_MAX_MATERIALS)
                 return fail(e, SJF_E_UNSUPPORTED, "materials and their PML twins exceed 255");
-            twin[m] = (int)e->lut_h.size();
-            e->lut_h.push_back(T);
-        }
-        for (long q = 0; q < e->N; ++q) {
-            if (!cell_in_pml(e, q)) continue;
-            uint32_t w = e->matw_h[q];
-            for (int c = 0; c < 3; ++c) {
-                const int m = (w >> (8 * c)) & 0xff;
-                if (m < ng && twin[m] >= 0) w = (w & ~(0xffu << (8 * c))) | ((uint32_t)twin[m] << (8 * c));
-            }
-            e->matw_h[q] = w;
+            twin[m] = (int)all.size();
+            all.push_back(T);
         }
     }
+    e->lut_h = all;
+    e->twin = twin;
     // per-cell eps_inf map: the given values, with the same fold inside the PML slabs
     if (!e->emap_h.empty()) {
         e->emap_eff = e->emap_h;
-        if (fold)
+        if (fold) {
+            std::vector<uint32_t> given(e->N);
+            if (int rc = d2h(e, given.data(), e->given, sizeof(uint32_t) * e->N)) return rc;
             for (long q = 0; q < e->N; ++q) {
                 if (!cell_in_pml(e, q)) continue;
                 for (int c = 0; c < 3; ++c) {
-                    const int m = (e->given_w[q] >> (8 * c)) & 0xff;
+                    const int m = (given[q] >> (8 * c)) & 0xff;
                     if (m >= ng || twin[m] < 0) continue;
                     double& v = e->emap_eff[(size_t)c * e->N + q];
                     if (v + fold_add[m] >= 1.0) v += fold_add[m];
                 }
             }
+        }
         if (int rc = upload_emap(e)) return rc;
     }
     int maxp = 0;
@@ -1290,20 +1321,19 @@ int apply_materials(sjf_engine* e) {
     e->nmat = (int)e->lut_h.size();
     e->maxp = maxp;
     e->uniform = (e->nmat == 1 && maxp == 0 && e->deps_h.empty() && e->emap_h.empty());
-    int rc = dev_alloc(e, (void**)&e->matw, sizeof(uint32_t) * e->N);
-    if (!rc) rc = h2d(e, e->matw, e->matw_h.data(), sizeof(uint32_t) * e->N);
-    if (rc) return rc;
-    // polarisation state, zeroed
-    dev_free(e->Qbuf);
-    dev_free(e->Pbuf);
-    if (maxp > 0) {
-        rc = dev_alloc(e, &e->Qbuf, (size_t)e->prec * 3 * maxp * e->N);
-        // FP32 slots alternate between the two arrays, Drude ones included
-        if (!rc && (anylor || e->prec == 4)) rc = dev_alloc(e, &e->Pbuf, (size_t)e->prec * 3 * maxp * e->N);
-        if (rc) return rc;
+    // polarisation state, zeroed; FP32 slots alternate between the two arrays, Drude ones included
+    const size_t pol = maxp > 0 ? (size_t)e->prec * 3 * maxp * e->N : 0;
+    const bool pair = pol > 0 && (anylor || e->prec == 4);
+    if (pol != e->pol_bytes) dev_free(e->Qbuf), dev_free(e->Pbuf);
+    if (!pair) dev_free(e->Pbuf);
+    e->pol_bytes = pol;
+    for (void** b : {&e->Qbuf, &e->Pbuf}) {
+        if (pol == 0 || (b == &e->Pbuf && !pair)) continue;
+        if (*b) HIPCHK(e, hipMemsetAsync(*b, 0, pol, e->stream));
+        else if (int rc = dev_alloc(e, b, pol)) return rc;
     }
-    rc = upload_lut(e);
-    if (!rc) rc = update_segments(e);
+    int rc = upload_lut(e);
+    if (!rc) rc = update_words(e);
     if (rc) return rc;
     choose_tile(e);
     e->version++;
@@ -1343,15 +1373,7 @@ double engine_step_bytes(const sjf_engine* e) {
     double b = e->N * (12 * p + (e->uniform ? 0 : 4));
     // polarisation: per pole and dispersive component 3p, the compulsory state of the textbook
     // recurrence (read P^n and P^{n-1}, write P^{n+1})
-    if (e->have_mat && e->maxp > 0) {
-        long pc = 0;
-        for (long q = 0; q < e->N; ++q)
-            for (int c = 0; c < 3; ++c) {
-                const int m = (e->matw_h[q] >> (8 * c)) & 0xff;
-                if (m != sjf::kDesignMat) pc += e->lut_h[m].npoles;
-            }
-        b += 3 * p * (double)pc;
-    }
+    if (e->have_mat && e->maxp > 0) b += 3 * p * e->pole_values;
     if (!e->deps_h.empty()) b += p * (double)e->deps_h.size();
     if (!e->emap_h.empty()) b += 3 * p * (double)e->N;  // per-cell 1/eps_inf of the three E components
     // PML: per cell and PML axis, 2 E + 2 H auxiliaries, each read + written
@@ -1604,7 +1626,9 @@ int adjoint_run_t(sjf_engine* e, long nsteps, long K, long gap, double* J_out, d
         return bail(fail(e, SJF_E_UNSUPPORTED, "adjoint tile needs more than 64 KiB of LDS"));
     const int npv = np_variant_of(e->maxp, e->uniform);
     auto ebar = [&]() { return g.A[g.rd]; };
-    const double ie[3] = {inv_eps_at(e, gap, 0), inv_eps_at(e, gap, 1), inv_eps_at(e, gap, 2)};
+    std::vector<uint32_t> gw;
+    if ((rc = words_at(e, {gap}, gw))) return bail(rc);
+    const double ie[3] = {inv_eps_at(e, gap, 0, gw[0]), inv_eps_at(e, gap, 1, gw[0]), inv_eps_at(e, gap, 2, gw[0])};
     auto inject = [&](long sl) -> int {
         hipLaunchKernelGGL((sjf::k_adj_inject<T>), dim3(1), dim3(64), 0, e->stream, ebar(), nyz, ring, nd, sl, gap, dt,
                            ie[0], ie[1], ie[2]);
@@ -1814,10 +1838,12 @@ int batch_adjoint_run_t(LaunchSet* s, long nsteps, long K, const long* gaps, con
         d.nyz = (long)e->g.ny * e->g.nz;
         d.ny = e->g.ny;
         d.nz = e->g.nz;
+        std::vector<uint32_t> gw;
+        if ((rc = words_at(e, {gaps[i]}, gw))) return bail(rc);
         for (int q = 0; q < 3; ++q) {
             d.dlo[q] = e->dlo[q];
             d.de[q] = e->dhi[q] - e->dlo[q];
-            d.ie[q] = inv_eps_at(e, gaps[i], q);
+            d.ie[q] = inv_eps_at(e, gaps[i], q, gw[0]);
         }
         d.nd = nd;
         d.gap = gaps[i];
@@ -2269,16 +2295,30 @@ int sjf_set_materials(sjf_engine* e, const uint32_t* mat_word, const sjf_materia
             return fail(e, SJF_E_ARG, "npoles must be in [0, 4]");
         if (!(lut[m].eps_inf > 0)) return fail(e, SJF_E_ARG, "eps_inf must be positive");
     }
-    for (long q = 0; q < e->N; ++q)
-        for (int c = 0; c < 3; ++c) {
-            const int m = (mat_word[q] >> (8 * c)) & 0xff;
-            if (m >= n_mat && m != sjf::kDesignMat)
-                return fail(e, SJF_E_ARG, "material word references an id >= n_mat");
-            if (m == sjf::kDesignMat && e->deps_h.empty())
-                return fail(e, SJF_E_STATE, "design id 255 used before sjf_set_design_eps");
-        }
+    // the words go to a buffer of their own: a word that is refused leaves the materials as they were
+    uint32_t* words = nullptr;
+    unsigned long long *d_first = nullptr, first = ~0ull;
+    int rc = dev_alloc(e, (void**)&words, sizeof(uint32_t) * e->N);
+    if (!rc) rc = dev_alloc(e, (void**)&d_first, sizeof(first));
+    if (!rc) rc = h2d(e, words, mat_word, sizeof(uint32_t) * e->N);
+    if (!rc) rc = h2d(e, d_first, &first, sizeof(first));
+    if (!rc) {
+        hipLaunchKernelGGL(sjf::k_check_words, dim3((unsigned)std::min(2048L, (e->N + 255) / 256)), dim3(256), 0,
+                           e->stream, words, e->N, n_mat, !e->deps_h.empty(), d_first);
+        rc = hipGetLastError() == hipSuccess ? d2h(e, &first, d_first, sizeof(first))
+                                             : fail(e, SJF_E_HIP, "k_check_words launch failed");
+    }
+    dev_free(d_first);
+    if (!rc && first != ~0ull)
+        rc = first & 1 ? fail(e, SJF_E_STATE, "design id 255 used before sjf_set_design_eps")
+                       : fail(e, SJF_E_ARG, "material word references an id >= n_mat");
+    if (rc) {
+        dev_free(words);
+        return rc;
+    }
+    dev_free(e->given);
+    e->given = words;
     e->given_lut.assign(lut, lut + n_mat);
-    e->given_w.assign(mat_word, mat_word + e->N);
     e->have_mat = true;
     return apply_materials(e);
 }
@@ -2290,12 +2330,13 @@ int sjf_set_eps_maps(sjf_engine* e, const double* eps) {
         e->emap_h.clear();
         e->emap_eff.clear();
         dev_free(e->emap);
+        if (!e->have_mat) return SJF_OK;  // there was none
     } else {
         for (long q = 0; q < 3 * e->N; ++q)
             if (!(eps[q] > 0) || !std::isfinite(eps[q])) return fail(e, SJF_E_ARG, "map eps must be positive and finite");
         e->emap_h.assign(eps, eps + 3 * e->N);
         if (!e->have_mat) {
-            e->given_w.assign(e->N, 0u);
+            if (int rc = dev_alloc(e, (void**)&e->given, sizeof(uint32_t) * e->N)) return rc;
             e->given_lut = e->lut_h;
             e->have_mat = true;
         }
@@ -2341,21 +2382,15 @@ int sjf_set_design_eps(sjf_engine* e, const int lo[3], const int hi[3], const do
     if (rc) return rc;
     // mark design voxels in the material word (all three E components)
     if (!e->have_mat) {
-        e->matw_h.assign(e->N, 0u);
-        e->given_w.assign(e->N, 0u);
+        rc = dev_alloc(e, (void**)&e->given, sizeof(uint32_t) * e->N);
+        if (rc) return rc;
         e->given_lut = e->lut_h;
         e->have_mat = true;
-        rc = dev_alloc(e, (void**)&e->matw, sizeof(uint32_t) * e->N);
-        if (rc) return rc;
     }
-    for (int i = lo[0]; i < hi[0]; ++i)
-        for (int j = lo[1]; j < hi[1]; ++j)
-            for (int k = lo[2]; k < hi[2]; ++k) {
-                const long q = cell_index(e, i, j, k);
-                e->matw_h[q] = e->given_w[q] = 0x00ffffffu;
-            }
-    rc = h2d(e, e->matw, e->matw_h.data(), sizeof(uint32_t) * e->N);
-    if (!rc) rc = update_segments(e);
+    hipLaunchKernelGGL(sjf::k_mark_design, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, e->stream, e->given, n[1],
+                       n[2], lo[0], lo[1], lo[2], hi[1] - lo[1], hi[2] - lo[2], cnt);
+    HIPCHK(e, hipGetLastError());
+    rc = update_words(e);
     if (rc) return rc;
     e->uniform = false;
     choose_tile(e);

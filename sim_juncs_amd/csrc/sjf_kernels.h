@@ -80,7 +80,7 @@ struct StepArgs {
     int uniform;  // 1: single non-dispersive material, no material word read
     int nmat;     // materials; the id of design voxels in the words
     const uint32_t* matw;
-    const uint32_t* seg;  // one code per 64 cells of a z line (k_segments), [x][y][(nz + 63) / 64]
+    const uint32_t* seg;  // one code per 64 cells of a z line (k_words), [x][y][(nz + 63) / 64]
     const MatLut<T>* lut;
     T* Q;     // [x][slot * 3 + comp][y][z]
     T* P;     // [x][slot * 3 + comp][y][z] (Lorentz slots)
@@ -261,43 +261,96 @@ __device__ __forceinline__ int word_poles(uint32_t w) { return (int)((w >> 24) &
 __device__ __forceinline__ int seg_material(uint32_t code) { return (int)(code & 0xff); }
 __device__ __forceinline__ int seg_poles(uint32_t code) { return (int)((code >> 8) & 7); }
 
-// Segment codes of the material words, one wavefront per segment; in the words the design ids
-// (kDesignMat) become nmat, the index of the table's entry of zeros, and the marks above are set.
-// slots: pole slots of all segments.
+// ---- material words ------------------------------------------------------------------------------
+
+// Cells outside [lo, hi) of some axis lie in a PML slab and take material twin[m] for m.
+struct WordMap {
+    int lo[3], hi[3];
+    unsigned char twin[256];
+};
+
+// The words and segment codes the kernels run, from the given words: the PML twins, design ids
+// (kDesignMat) as nmat (the table's entry of zeros), the marks above.  One wavefront per segment;
+// count: pole slots of all segments, and poles over all cells and components.  Bound by memory: 256 x
+// 256 x 128 cells 0.03 ms (on the host, three loops over the cells and a second upload: 30 ms).
 template <typename T>
-__global__ void __launch_bounds__(256) k_segments(uint32_t* __restrict__ matw, const MatLut<T>* __restrict__ lut,
-                                                  uint32_t* __restrict__ seg, long rows, int nz, int nmat,
-                                                  unsigned long long* __restrict__ slots) {
+__global__ void __launch_bounds__(256) k_words(const uint32_t* __restrict__ given, uint32_t* __restrict__ matw,
+                                               uint32_t* __restrict__ seg, const MatLut<T>* __restrict__ lut, int nx,
+                                               int ny, int nz, int nmat, const WordMap map,
+                                               unsigned long long* __restrict__ count) {
     const int nseg = (nz + 63) >> 6, lane = threadIdx.x & 63;
-    const long q = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (q >= rows * nseg) return;
-    const long row = q / nseg;
-    const int k = (int)(q - row * nseg) * 64 + lane;
-    const bool in = k < nz;
-    uint32_t w = in ? matw[row * nz + k] : 0u;
-    bool des = false;
-    int np = 0;
-    uint32_t out = 0u;  // the three ids
-    for (int c = 0; c < 3; ++c) {
-        int m = (w >> (8 * c)) & 0xff;
-        const bool d = in && (m == kDesignMat || m == nmat);
-        m = d ? nmat : m;
-        des = des || d;
-        if (in) np = max(np, lut[m].np);
-        out |= (uint32_t)m << (8 * c);
+    const long n = (long)nx * ny * nseg;
+    unsigned long long slots = 0, poles = 0;
+    for (long q = (long)blockIdx.x * 4 + (threadIdx.x >> 6); q < n; q += (long)gridDim.x * 4) {
+        const long row = q / nseg;
+        const int k = (int)(q - row * nseg) * 64 + lane, i = (int)(row / ny), j = (int)(row - (long)i * ny);
+        const bool in = k < nz;
+        const bool slab = i < map.lo[0] || i >= map.hi[0] || j < map.lo[1] || j >= map.hi[1] || k < map.lo[2] ||
+                          k >= map.hi[2];
+        const uint32_t w = in ? given[row * nz + k] : 0u;
+        bool des = false;
+        int np = 0;
+        uint32_t out = 0u;  // the three ids
+        for (int c = 0; c < 3; ++c) {
+            int m = (w >> (8 * c)) & 0xff;
+            const bool d = in && m == kDesignMat;
+            if (slab) m = map.twin[m];
+            m = d ? nmat : min(m, nmat);
+            des = des || d;
+            const int p = in ? lut[m].np : 0;
+            np = max(np, p);
+            poles += p;
+            out |= (uint32_t)m << (8 * c);
+        }
+        if (in) matw[row * nz + k] = out | (uint32_t)np << 24 | (des ? kWordDesign : 0u);
+        const uint32_t first = (uint32_t)__builtin_amdgcn_readfirstlane((int)out);
+        const uint32_t id = first & 0xff;
+        const bool mixed = first != id * 0x010101u || wave_any(des) || wave_any(in && out != first);
+        uint32_t code = mixed ? kSegMixed | kSegSpecial | (wave_any(des) ? kSegDesign : 0u) : id;
+        for (int s = kMaxPoles; s > 0; --s)
+            if (wave_any(np >= s)) {
+                code |= kSegSpecial | (uint32_t)s << 8;
+                break;
+            }
+        if (lane == 0) seg[q] = code;
+        slots += seg_poles(code);
     }
-    if (in) matw[row * nz + k] = out | (uint32_t)np << 24 | (des ? kWordDesign : 0u);
-    const uint32_t first = (uint32_t)__builtin_amdgcn_readfirstlane((int)out);
-    const uint32_t id = first & 0xff;
-    const bool mixed = first != id * 0x010101u || wave_any(des) || wave_any(in && out != first);
-    uint32_t code = mixed ? kSegMixed | kSegSpecial | (wave_any(des) ? kSegDesign : 0u) : id;
-    for (int n = kMaxPoles; n > 0; --n)
-        if (wave_any(np >= n)) {
-            code |= kSegSpecial | (uint32_t)n << 8;
+    for (int o = 32; o > 0; o >>= 1) poles += __shfl_down(poles, o, 64);
+    if (lane == 0 && poles > 0) {
+        atomicAdd(count, slots);
+        atomicAdd(count + 1, poles);
+    }
+}
+
+// The first id that is neither below nmat nor an allowed design id, in the order of cells and
+// components: *first = 2 * (3 * cell + component), + 1 for a design id.
+__global__ void __launch_bounds__(256) k_check_words(const uint32_t* __restrict__ given, long n, int nmat, bool design,
+                                                     unsigned long long* __restrict__ first) {
+    for (long q = (long)blockIdx.x * blockDim.x + threadIdx.x; q < n; q += (long)gridDim.x * blockDim.x) {
+        const uint32_t w = given[q];
+        for (int c = 0; c < 3; ++c) {
+            const int m = (w >> (8 * c)) & 0xff;
+            if (m < nmat || (m == kDesignMat && design)) continue;
+            atomicMin(first, 2ull * (3 * q + c) + (m == kDesignMat ? 1 : 0));
             break;
         }
-    if (lane == 0) seg[q] = code;
-    if (lane == 0 && seg_poles(code) > 0) atomicAdd(slots, (unsigned long long)seg_poles(code));
+    }
+}
+
+// Design ids on the box [lo, lo + ext)
+__global__ void __launch_bounds__(256) k_mark_design(uint32_t* __restrict__ given, int ny, int nz, int lx, int ly, int lz,
+                                                     int ey, int ez, long n) {
+    const long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= n) return;
+    const long r = q / ez, i = r / ey;
+    given[((lx + i) * ny + ly + (r - i * ey)) * nz + lz + (q - r * ez)] = 0x00ffffffu;
+}
+
+// Words of listed cells
+__global__ void __launch_bounds__(256) k_read_words(const uint32_t* __restrict__ matw, const long* __restrict__ cell,
+                                                    long n, uint32_t* __restrict__ out) {
+    const long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (q < n) out[q] = matw[cell[q]];
 }
 
 // Fused H / polarisation / E update of one time step.  TY: y rows per thread; NP: pole slots
@@ -315,7 +368,7 @@ __global__ void __launch_bounds__(256) k_segments(uint32_t* __restrict__ matw, c
 //     wait counts need not assume the worse of two.  The loads and stores of a plane that is not
 //     needed (past the chunk, past a metallic edge) go through a descriptor of length zero: they
 //     return 0 or are dropped without a memory access.
-//   * One word per 64 cells of a z line (k_segments) says whether a wavefront's cells all run one
+//   * One word per 64 cells of a z line (k_words) says whether a wavefront's cells all run one
 //     material without poles; then its constant is a scalar and neither the per-cell words nor the
 //     material table are read.
 //   * A thread's byte offset within a component plane depends only on its row and z cell, so it is
@@ -832,7 +885,7 @@ __device__ __forceinline__ void step_tile(const StepArgs<T>& a, const int t) {
 // i + 1, which H^{n+1/2} of plane i needs anyway, goes to LDS together with that H (both in two
 // halves used in turn), so a plane's H phase starts from what the barrier before it published.
 // A wavefront can span rows, so row conditions are per lane and the wavefront's material is found
-// from its words (k_segments marks in them the cells with poles and the design voxels).
+// from its words (k_words marks in them the cells with poles and the design voxels).
 // Bound by the latency of a plane's serial part (exchange, barrier, pole recursion) at 4 waves per
 // SIMD on grids of up to about 3 M cells, by memory above.  Measured on MI355X, us per step before
 // (two barriers, loads waited for in the iteration that issued them) and now: 24 FP32 grids of 64^3
