@@ -200,10 +200,18 @@ __device__ __forceinline__ Pair2<T> bld2(Rsrc r, uint32_t v, uint32_t s) {
     if constexpr (sizeof(T) == 4) return __builtin_bit_cast(Pair2<T>, __builtin_amdgcn_raw_buffer_load_b64(r, (int)v, (int)s, 0));
     else return __builtin_bit_cast(Pair2<T>, __builtin_amdgcn_raw_buffer_load_b128(r, (int)v, (int)s, 0));
 }
+// (FP64: two stores.  One of 16 bytes with a scalar offset stored what the next instruction wrote to
+// its data registers: the compiler takes this form to need no wait state there, and on gfx950 pairs
+// of the x layers came out wrong under load.)
 template <bool NT = false, typename P>
 __device__ __forceinline__ void bst2(Rsrc r, uint32_t v, uint32_t s, P x) {
-    if constexpr (sizeof(P) == 8) __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, x), r, (int)v, (int)s, NT ? 2 : 0);
-    else __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x), r, (int)v, (int)s, NT ? 2 : 0);
+    if constexpr (sizeof(P) == 8) {
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, x), r, (int)v, (int)s, NT ? 2 : 0);
+    } else {
+        const u32x4 w = __builtin_bit_cast(u32x4, x);
+        __builtin_amdgcn_raw_buffer_store_b64(u32x2{w.x, w.y}, r, (int)v, (int)s, NT ? 2 : 0);
+        __builtin_amdgcn_raw_buffer_store_b64(u32x2{w.z, w.w}, r, (int)v, (int)s + 8, NT ? 2 : 0);
+    }
 }
 // the lane offset of a pair from that of a value (kOOB stays out of range)
 __device__ __forceinline__ uint32_t two(uint32_t o) { return o == kOOB ? kOOB : 2u * o; }
