@@ -278,10 +278,11 @@ int sjf_adjoint_run(sjf_engine* e, long nsteps, int checkpoint_every, const int 
  * per workgroup) or SJF_TILE_THREAD_ROWS (`rows` owned y rows of nz threads each plus one halo
  * row per workgroup, the y and z neighbours exchanged through LDS; needs (rows + 1) * nz <= 1024
  * and the exchange planes within 64 KiB of LDS), marching over `xchunk` x planes (0: enough
- * chunks for about 16384 workgroups).  The default is one row per workgroup.  The gradient is
- * the same to rounding either way (the same arithmetic per cell).  A batched adjoint run runs one row per workgroup unless its first engine's tile was set
- * to the row-of-threads form: then every engine runs that many rows (at most its ny) over the
- * first engine's x-chunk (6 planes where it gave none).  New (tuning). */
+ * chunks for about 16384 workgroups).  The default is as many thread rows as a workgroup holds where
+ * that is one owned row or more and the fields are 12 MB or more, else one row per workgroup.  The
+ * gradient has the same bits either way.  In a batched adjoint run a tile set on the first engine
+ * holds for every engine: rows of threads (at most its ny) over the first engine's x-chunk (6 planes
+ * where it gave none), or one row per workgroup.  New (tuning). */
 int sjf_set_adjoint_tile(sjf_engine* e, int form, int rows, int xchunk);
 /* The fused reverse-step kernel of the last sjf_adjoint_run: mean duration in ms (HIP events on
  * the engine's stream around the first min(nsteps, 64) reverse launches), threads per workgroup

@@ -359,6 +359,25 @@ int block_threads_for(const sjf_engine* e, int form, int ty, bool given) {
 
 int block_threads(const sjf_engine* e) { return block_threads_for(e, e->form, e->ty, e->tile_set); }
 
+// x-chunk of a tile with nty rows of tiles: a workgroup's time is its chunk and about `extra` planes
+// of start-up, and the chip runs `slots` workgroups at once; a launch that needs a little more than
+// a whole number of such rounds waits for a last one that is nearly empty (forward step of
+// 192x192x96 FP32, 9 thread rows, 256 slots: 242 workgroups of 18 planes 80.6 us, 264 of 16 planes
+// 112 us, 484 of 9 planes 83.9 us).  So: the rounds for which rounds * (chunk + extra) is least, with
+// chunks of at most 64 planes (a longer march drifts apart) and at most 16 rounds.
+int round_chunk(int nx, int nty, long slots, int extra) {
+    long best = LONG_MAX;
+    int xc = std::min(nx, 64);
+    for (int m = 1; m <= 16; ++m) {
+        const long nxc = std::min<long>(nx, m * slots / nty);
+        if (nxc < 1) continue;
+        const int c = (int)((nx + nxc - 1) / nxc);
+        if (c > 64) continue;
+        if (m * (long)(c + extra) <= best) best = m * (long)(c + extra), xc = c;
+    }
+    return xc;
+}
+
 int tiles_of(const sjf_engine* e, int ty, int xc) {
     const int nty = (e->g.ny + ty - 1) / ty;
     const int nxc = (e->g.nx + xc - 1) / xc;
@@ -1036,12 +1055,6 @@ int tile_waves(const sjf_engine* e) {
 // 192x192x96 80.4, 93.9; 151x133x117 54.4, 70.2; 256x256x128 191.7, 201.7; 150x150x200 90.0, 112.7;
 // 120x160x250 95.9, 120.6; 512x512x256 1061, 1039.
 //
-// x-chunk: a workgroup's time is its chunk and about two planes of start-up, and the chip runs
-// `slots` workgroups at once; a launch that needs a little more than a whole number of such rounds
-// waits for a last one that is nearly empty (192x192x96 FP32, 9 thread rows, 256 slots: 242
-// workgroups of 18 planes 80.6 us, 264 of 16 planes 112 us, 484 of 9 planes 83.9 us).  So: the
-// rounds for which rounds * (chunk + 2) is least, with chunks of at most 64 planes (a longer march
-// drifts apart) and at most 16 rounds.
 void choose_tile(sjf_engine* e) {
     if (e->tile_set) return;
     const int rows = default_thread_rows(e), full = e->prec == 8 ? 128 : 256;
@@ -1050,17 +1063,7 @@ void choose_tile(sjf_engine* e) {
     e->ty = thread_rows ? rows : 1;
     const int waves = e->prec == 4 ? tile_waves<float>(e) : tile_waves<double>(e);
     const long slots = 256L * std::max(1, 4 * waves / (block_threads(e) / 64));
-    const int nx = e->g.nx, nty = (e->g.ny + e->ty - 1) / e->ty;
-    long best = LONG_MAX;
-    int xc = std::min(nx, 64);
-    for (int m = 1; m <= 16; ++m) {
-        const long nxc = std::min<long>(nx, m * slots / nty);
-        if (nxc < 1) continue;
-        const int c = (int)((nx + nxc - 1) / nxc);
-        if (c > 64) continue;
-        if (m * (c + 2L) < best) best = m * (c + 2L), xc = c;
-    }
-    e->xc = xc;
+    e->xc = round_chunk(e->g.nx, (e->g.ny + e->ty - 1) / e->ty, slots, 2);
 }
 
 int free_all(sjf_engine* e) {
@@ -1455,20 +1458,28 @@ int adj_xchunk(const sjf_engine* e, long target = 16384, long rows = 0) {
 // workgroups the reverse launch of a batch aims at (x-chunks common to all engines)
 constexpr long kBatchAdjGroups = 32768;
 
-// Tile of the reverse step: the one sjf_set_adjoint_tile gave, else one row per workgroup (the
-// form a batch runs by default, so an engine alone and in a batch give the same bits).  Measured
-// on MI355X, one 192x192x96 FP32 engine: 0.139 ms per reverse step with row-of-threads tiles of
-// 9 rows and 6 planes, 0.155 ms one row per workgroup; sixteen such engines in one batch: 1.78 ms
-// per reverse launch with the 9-row tiles, 1.65 ms one row per workgroup; 256x256x128: 0.268 ms
-// for the best row-of-threads tile against 0.266 ms one row per workgroup.
+// Tile of the reverse step: the one sjf_set_adjoint_tile gave; else thread rows wherever one owned
+// row and the halo row fit a workgroup (FP64 512 threads), on grids, or batches, of at least
+// kAdjRowsBytes of fields; else one row per workgroup.  Both forms give the same bits.  Measured on
+// MI355X, us per reverse step, thread rows and one row: FP32 192x192x96 93, 138; 141x129x95 46, 73;
+// 256x256x128 226, 232; 120x120x256 80, 145; 120x100x320 91, 200; 100x100x500 150, 232; FP64
+// 72x64x56 22, 33; 100x100x128 80, 107; 100x100x200 140, 223; 52^3 19.1, 23.5.  Below the line a
+// launch fills no more than a part of the chip either way and one row per workgroup has the shorter
+// chain: FP32 52^3 17.8, 16.7; 32^3 13.9, 13.9.
+constexpr double kAdjRowsBytes = 12e6;
 struct AdjTile {
     bool rows;
-    int nrows, xc;  // xc 0: the default chunks
+    int nrows, xc;  // nrows 0: each engine's default; xc 0: the default chunks
 };
-AdjTile adj_tile_of(const sjf_engine* e) {
-    if (e->adj_set && e->adj_form == SJF_TILE_THREAD_ROWS)
-        return {true, e->adj_rows, e->adj_xc > 0 ? std::min(e->adj_xc, e->g.nx) : 0};
-    return {false, 1, e->adj_set && e->adj_xc > 0 ? std::min(e->adj_xc, e->g.nx) : 0};
+template <typename T>
+AdjTile adj_tile_of(const sjf_engine* e, double bytes, int nmat) {
+    if (e->adj_set)
+        return {e->adj_form == SJF_TILE_THREAD_ROWS, e->adj_form == SJF_TILE_THREAD_ROWS ? e->adj_rows : 1,
+                e->adj_xc > 0 ? std::min(e->adj_xc, e->g.nx) : 0};
+    const size_t block = sizeof(T) == 8 ? 512 : 1024;
+    const bool rows = bytes >= kAdjRowsBytes && (size_t)(default_thread_rows(e) + 1) * e->g.nz <= block &&
+                      lds_fits<T>(8 * block + 2 * (size_t)e->g.nz, nmat);
+    return {rows, rows ? 0 : 1, 0};
 }
 
 template <typename T, int NP, bool NTS>
@@ -1487,9 +1498,17 @@ void launch_adj_np(sjf_engine* e, const sjf::AdjArgs<T>& g, int block, unsigned 
 
 template <typename T, int NP>
 void launch_adj_rows_np(sjf_engine* e, const sjf::AdjArgs<T>& g, int block, unsigned tiles, size_t lds) {
-    if (block <= 256) hipLaunchKernelGGL((sjf::k_adj_rows<T, NP, 256>), dim3(tiles), dim3(block), lds, e->stream, g);
-    else if (block <= 512) hipLaunchKernelGGL((sjf::k_adj_rows<T, NP, 512>), dim3(tiles), dim3(block), lds, e->stream, g);
-    else hipLaunchKernelGGL((sjf::k_adj_rows<T, NP, 1024>), dim3(tiles), dim3(block), lds, e->stream, g);
+    const bool nts = step_set_bytes(e) > kStreamBytes;  // (192x192x96 FP32: 96.8 us without, 93.0 with the hint)
+#define SJF_LAUNCH(...) hipLaunchKernelGGL((__VA_ARGS__), dim3(tiles), dim3(block), lds, e->stream, g)
+    if (block <= 512) {
+        if (nts) SJF_LAUNCH(sjf::k_adj_rows<T, NP, 512, true>);
+        else SJF_LAUNCH(sjf::k_adj_rows<T, NP, 512>);
+    } else if (nts) {
+        SJF_LAUNCH(sjf::k_adj_rows<T, NP, 1024, true>);
+    } else {
+        SJF_LAUNCH(sjf::k_adj_rows<T, NP, 1024>);
+    }
+#undef SJF_LAUNCH
 }
 
 template <typename T>
@@ -1505,11 +1524,11 @@ int launch_adj_step(sjf_engine* e, const sjf::AdjArgs<T>& g, int npv, int block,
     return SJF_OK;
 }
 
-// LDS of the reverse step: E-term and H-term exchange planes and the material table
+// LDS of the reverse step: E-term and H-term exchange planes (row-of-threads form: twice) and the
+// material table
 template <typename T>
-size_t adj_lds_bytes(const sjf_engine* e, bool rows, int block) {
-    const size_t lut = sjf::lut_lds_bytes<T>(e->nmat);
-    return rows ? sizeof(T) * (8 * (size_t)block + 2 * (((size_t)e->g.nz + 1) & ~(size_t)1)) + lut : sizeof(T) * 12 * (size_t)block + lut;
+size_t adj_lds_bytes(bool rows, int block, int nmat) {
+    return sizeof(T) * (rows ? 16 : 12) * (size_t)block + sjf::lut_lds_bytes<T>(nmat);
 }
 
 template <typename T>
@@ -1603,14 +1622,18 @@ int adjoint_run_t(sjf_engine* e, long nsteps, long K, long gap, double* J_out, d
     sjf::AdjArgs<T> g;
     std::memset(&g, 0, sizeof(g));
     // register form: one y row per workgroup; row-of-threads form: arows owned rows
-    const AdjTile at = adj_tile_of(e);
+    const AdjTile at = adj_tile_of<T>(e, field_bytes(e), e->nmat);
     const bool rows = at.rows;
-    const int arows = at.nrows;
+    const int arows = at.nrows > 0 ? at.nrows : default_thread_rows(e);
+    const int npv = np_variant_of(e->maxp, e->uniform);
     int axc = at.xc > 0 ? at.xc : adj_xchunk(e);
-    if (rows && at.xc == 0) {  // about 16384 workgroups over the tile rows
+    if (rows && at.xc == 0 && at.nrows > 0) {  // about 16384 workgroups over the tile rows
         const long trows = (e->g.ny + arows - 1) / arows;
         const long nxc = std::min<long>(std::max(1L, (16384 + trows - 1) / trows), e->g.nx);
         axc = (int)((e->g.nx + nxc - 1) / nxc);
+    } else if (rows && at.xc == 0) {
+        const int waves = sizeof(T) == 4 ? 4 : npv == 0 ? 3 : 2, wg = ((arows + 1) * e->g.nz + 63) / 64;
+        axc = round_chunk(e->g.nx, (e->g.ny + arows - 1) / arows, 256L * std::max(1, 4 * waves / wg), 3);
     }
     g.f = step_args<T>(e, arows, axc);
     g.A[0] = A;
@@ -1621,10 +1644,9 @@ int adjoint_run_t(sjf_engine* e, long nsteps, long K, long gap, double* J_out, d
     for (int d = 0; d < 3; ++d) g.Apsi[d] = Apsi[d];
     const int block = (((rows ? arows + 1 : 1) * e->g.nz + 63) / 64) * 64;
     const unsigned tiles = (unsigned)((long)g.f.nty * ((e->g.nx + g.f.xc - 1) / g.f.xc));
-    const size_t lds = adj_lds_bytes<T>(e, rows, block);
+    const size_t lds = adj_lds_bytes<T>(rows, block, e->nmat);
     if (!lds_fits<T>(rows ? 8 * (size_t)block + 2 * (size_t)e->g.nz : 12 * (size_t)block, e->nmat))
         return bail(fail(e, SJF_E_UNSUPPORTED, "adjoint tile needs more than 64 KiB of LDS"));
-    const int npv = np_variant_of(e->maxp, e->uniform);
     auto ebar = [&]() { return g.A[g.rd]; };
     std::vector<uint32_t> gw;
     if ((rc = words_at(e, {gap}, gw))) return bail(rc);
@@ -1736,13 +1758,16 @@ template <typename T, int NP>
 void launch_adj_batch_np(LaunchSet* s, const sjf::AdjArgs<T>* args, const int* first, int n, int block,
                          unsigned tiles, size_t lds, bool rows) {
     if (rows) {
-        if (block <= 256)
-            hipLaunchKernelGGL((sjf::k_adj_rows_batch<T, NP, 256>), dim3(tiles), dim3(block), lds, s->stream, args, first, n);
-        else if (block <= 512)
-            hipLaunchKernelGGL((sjf::k_adj_rows_batch<T, NP, 512>), dim3(tiles), dim3(block), lds, s->stream, args, first, n);
-        else
-            hipLaunchKernelGGL((sjf::k_adj_rows_batch<T, NP, 1024>), dim3(tiles), dim3(block), lds, s->stream, args,
-                               first, n);
+#define SJF_LAUNCH(...) hipLaunchKernelGGL((__VA_ARGS__), dim3(tiles), dim3(block), lds, s->stream, args, first, n)
+        if (block <= 512) {
+            if (s->nts) SJF_LAUNCH(sjf::k_adj_rows_batch<T, NP, 512, true>);
+            else SJF_LAUNCH(sjf::k_adj_rows_batch<T, NP, 512>);
+        } else if (s->nts) {
+            SJF_LAUNCH(sjf::k_adj_rows_batch<T, NP, 1024, true>);
+        } else {
+            SJF_LAUNCH(sjf::k_adj_rows_batch<T, NP, 1024>);
+        }
+#undef SJF_LAUNCH
         return;
     }
     if (s->nts) launch_adj_batch_step<T, NP, true>(s, args, first, n, block, tiles, lds);
@@ -1802,11 +1827,20 @@ int batch_adjoint_run_t(LaunchSet* s, long nsteps, long K, const long* gaps, con
     long maxv = 0, rows = 0;
     // one row per workgroup with x-chunks common to all engines, or, when the first engine's tile
     // was set to the row-of-threads form, its rows (at most each engine's ny) and its x-chunk
-    const AdjTile bt = adj_tile_of(e0);
+    double bytes = 0;
+    for (const sjf_engine* e : s->eng) {
+        rows += e->g.ny;
+        bytes += field_bytes(e);
+        nmat = std::max(nmat, e->nmat);
+    }
+    AdjTile bt = adj_tile_of<T>(e0, bytes, nmat);
+    for (const sjf_engine* e : s->eng)
+        if (bt.nrows == 0 && (default_thread_rows(e) + 1) * e->g.nz > (sizeof(T) == 8 ? 512 : 1024)) bt = {false, 1, 0};
     const bool brows = bt.rows;
-    const int bxc = bt.xc > 0 ? bt.xc : 6;
+    // default chunks, six 192x192x96 FP32 engines: 4 planes 584 us per reverse launch, 6 549, 8 537, 12
+    // 526, 18 533, 24 540 (one row per workgroup: 657)
+    const int bxc = bt.xc > 0 ? bt.xc : bt.nrows > 0 ? 6 : 12;
     int bblock = 64;
-    for (const sjf_engine* e : s->eng) rows += e->g.ny;
     for (int i = 0; i < n; ++i) {
         sjf_engine* e = s->eng[i];
         const StateLayout L = state_layout(e);
@@ -1852,7 +1886,7 @@ int batch_adjoint_run_t(LaunchSet* s, long nsteps, long K, const long* gaps, con
         std::memset(&g, 0, sizeof(g));
         // the first engine's tile form for all (they share nz and the precision)
         if (brows) {
-            const int r = std::min(bt.nrows, e->g.ny);
+            const int r = bt.nrows > 0 ? std::min(bt.nrows, e->g.ny) : default_thread_rows(e);
             g.f = step_args<T>(e, r, std::min(bxc, e->g.nx));
             bblock = std::max(bblock, (((r + 1) * e->g.nz + 63) / 64) * 64);
         } else {
@@ -1866,7 +1900,6 @@ int batch_adjoint_run_t(LaunchSet* s, long nsteps, long K, const long* gaps, con
         for (int q = 0; q < 3; ++q) g.Apsi[q] = (T*)Apsi[q];
         first.push_back(t);
         t += (int)((long)g.f.nty * ((e->g.nx + g.f.xc - 1) / g.f.xc));
-        nmat = std::max(nmat, e->nmat);
         maxv = std::max(maxv, nd + 3);
     }
     first.push_back(t);
@@ -1894,8 +1927,7 @@ int batch_adjoint_run_t(LaunchSet* s, long nsteps, long K, const long* gaps, con
     const auto* tabp = (const sjf::AdjBatchDev<T>*)d_tab;
     const sjf::AdjArgs<T>* argd[2] = {(const sjf::AdjArgs<T>*)d_args0, (const sjf::AdjArgs<T>*)d_args1};
     const int block = brows ? bblock : ((e0->g.nz + 63) / 64) * 64;
-    const size_t lds = (brows ? sizeof(T) * (8 * (size_t)block + 2 * (((size_t)e0->g.nz + 1) & ~(size_t)1)) : sizeof(T) * 12 * (size_t)block) +
-                       sjf::lut_lds_bytes<T>(nmat);
+    const size_t lds = adj_lds_bytes<T>(brows, block, nmat);
     if (!lds_fits<T>(brows ? 8 * (size_t)block + 2 * (size_t)e0->g.nz : 12 * (size_t)block, nmat))
         return bail(fail(e0, SJF_E_UNSUPPORTED, "adjoint tile needs more than 64 KiB of LDS"));
     const int npv = np_variant_of(e0->maxp, e0->uniform);
@@ -2059,8 +2091,9 @@ extern "C" int sjf_set_adjoint_tile(sjf_engine* e, int form, int rows, int xchun
         // FP64 tiles stop at 512 threads: at 1024 the register budget of 128 per thread spills
         if (e->prec == 8 && block > 512)
             return fail(e, SJF_E_ARG, "FP64 row-of-threads reverse tile needs (rows + 1) * nz <= 512");
-        const size_t lds = e->prec == 4 ? adj_lds_bytes<float>(e, true, block) : adj_lds_bytes<double>(e, true, block);
-        if (lds > 65536) return fail(e, SJF_E_ARG, "adjoint row-of-threads tile needs more than 64 KiB of LDS");
+        const size_t values = 8 * (size_t)block + 2 * (size_t)e->g.nz;
+        if (!(e->prec == 4 ? lds_fits<float>(values, e->nmat) : lds_fits<double>(values, e->nmat)))
+            return fail(e, SJF_E_ARG, "adjoint row-of-threads tile needs more than 64 KiB of LDS");
     } else {
         return fail(e, SJF_E_ARG, "unknown tile form");
     }

@@ -883,6 +883,24 @@ __device__ __forceinline__ void step_tile(const StepArgs<T>& a, const int t) {
     }  // pass
 }
 
+// Material of a wavefront's cells from their words: kSegSpecial with the most pole slots of a lane
+// (bits 8-10), or the id of their one material without poles
+template <int NP>
+__device__ __forceinline__ uint32_t classify(uint32_t w) {
+    const uint32_t first = (uint32_t)__builtin_amdgcn_readfirstlane((int)w), id = first & 0xff;
+    if (first == id * 0x010101u && !wave_any(w != first)) return id;
+    uint32_t code = kSegSpecial;
+    if (wave_any((w & kWordDesign) != 0)) code |= kSegDesign;
+    const int np = word_poles(w);
+#pragma unroll
+    for (int s = NP; s > 0; --s)
+        if (wave_any(np >= s)) {
+            code |= (uint32_t)s << 8;
+            break;
+        }
+    return code;
+}
+
 // Fused step, row-of-threads form.  A workgroup holds a.rt rows of nz threads (one cell of a
 // y row per thread); thread row 0 recomputes H on the row below the tile (the y halo) and rows
 // 1..rt-1 own rows j0..j0+rt-2.  The y and z neighbours of E (for H) and of H (for E) are
@@ -1027,22 +1045,6 @@ __device__ __forceinline__ void step_rows(const StepArgs<T>& a, const int t) {
             for (int c = 0; c < 3; ++c) em[c] = bld<T>(re, oo, c * PB);
         }
     };
-    // kSegSpecial with the most pole slots of a lane (bits 8-10), or the id of the one material, without
-    // poles, of the wavefront's cells
-    auto classify = [&](uint32_t w) -> uint32_t {
-        const uint32_t first = (uint32_t)__builtin_amdgcn_readfirstlane((int)w), id = first & 0xff;
-        if (first == id * 0x010101u && !wave_any(w != first)) return id;
-        uint32_t code = kSegSpecial;
-        if (wave_any((w & kWordDesign) != 0)) code |= kSegDesign;
-        const int np = word_poles(w);
-#pragma unroll
-        for (int s = NP; s > 0; --s)
-            if (wave_any(np >= s)) {
-                code |= (uint32_t)s << 8;
-                break;
-            }
-        return code;
-    };
     auto load_poles = [&](int p, uint32_t code, uint32_t w) {
         const int npx = seg_poles(code);
         const Rsrc rc = rsrc(Pcur + (long)p * QPB), ro = rsrc(Pold + (long)p * QPB);
@@ -1115,7 +1117,7 @@ __device__ __forceinline__ void step_rows(const StepArgs<T>& a, const int t) {
     load_psi_h(pi);
     load_psi_e(pi);
     if (!uniform) {
-        cls = classify(mw);
+        cls = classify<NP>(mw);
         if (NP > 0 && seg_poles(cls) > 0) load_poles(pi, cls, mw);
     }
 
@@ -1224,7 +1226,7 @@ __device__ __forceinline__ void step_rows(const StepArgs<T>& a, const int t) {
         // ------------------------------- loads for the planes ahead
         uint32_t cn = 0u;
         if (!uniform && next) {
-            cn = classify(mwn);
+            cn = classify<NP>(mwn);
             if (NP > 0 && seg_poles(cn) > 0) load_poles(pn, cn, mwn);
         }
         mw = reg_copy(mwn);
@@ -1797,9 +1799,9 @@ __global__ void __launch_bounds__(64) k_dft_flux_sum(const double* __restrict__ 
 //   H-terms: (Hx, y, +, Ez, 0) (Hx, z, -, Ey, 0) (Hy, z, +, Ex, 1) (Hy, x, -, Ez, 0)
 //            (Hz, x, +, Ey, 1) (Hz, y, -, Ex, 1)
 // This has the dependency pattern of the forward step (phase 1 uses forward differences,
-// phase 2 backward ones), so the same tiling applies: a workgroup spans a z line, each thread
-// one y row plus a halo row below it where phase 1 is recomputed, z neighbours through LDS,
-// and the tile marches along x carrying u of the next planes.  Adjoint fields and E auxiliary
+// phase 2 backward ones), so the same tilings apply: rows of threads (adj_rows), or a workgroup that
+// spans a z line, each thread one y row plus a halo row below it where phase 1 is recomputed, z
+// neighbours through LDS (adj_tile); the tile marches along x carrying u of the next planes.  Adjoint fields and E auxiliary
 // bars are double-buffered (neighbouring workgroups read the old values of the halo row);
 // Qbar and Pbar are only touched by their owner and are updated in place.
 
@@ -1811,11 +1813,14 @@ struct AdjArgs {
     int rd;
     T* Aq;             // Qbar [x][slot * 3 + comp][y][z]
     T* Ap;             // Pbar, the same layout
-    T* Apsi[3];        // per axis [8][S]: E aux bar pair (0,1), H aux bar pairs (2,3) and (4,5),
-                       // E aux bar pair (6,7)
-    int er, ew;        // E aux bar pair read (0 or 6) / written (6 or 0)
-    int hr, hw;        // H aux bar pair read (2 or 4) / written (4 or 2)
+    T* Apsi[3];        // per axis four pairs of auxiliary bars [S][2]: E at 0 and 6 S, H at 2 S and 4 S
+    int er, ew;        // E pair read (0 or 6) / written (6 or 0)
+    int hr, hw;        // H pair read (2 or 4) / written (4 or 2)
 };
+
+// b dbar + (b - 1) psibar of a term and its auxiliary bar
+template <typename T>
+__device__ __forceinline__ T adj_term(T b, T t, T psi) { return fma_(b - T(1), psi, b * t); }
 
 // One tile of the fused reverse step: a z line of one y row (j0), marching along x.  Addressing
 // and predication as in step_tile: per-plane descriptors, lane offsets fixed for the march, the
@@ -1823,6 +1828,8 @@ struct AdjArgs {
 // pole slot or the design region; whole-wavefront conditions are uniform branches.
 template <typename T, int NP, bool NTS>
 __device__ __forceinline__ void adj_tile(const AdjArgs<T>& g, const int t) {
+#pragma clang fp contract(off)
+    typedef Pair2<T> Pair;
     constexpr uint32_t TS = sizeof(T);
     const StepArgs<T>& a = g.f;
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -1865,8 +1872,8 @@ __device__ __forceinline__ void adj_tile(const AdjArgs<T>& g, const int t) {
     }
     const bool zpml = kin && in_pml(a, 2, k, nz);
     const bool zany = wave_any(zpml);
-    const uint32_t oK = kin ? (uint32_t)k * TS : kOOB;
-    const uint32_t oZ = zpml ? (uint32_t)(k < a.plo[2] ? k : k - (nz - a.phi[2]) + a.plo[2]) * TS : kOOB;
+    const uint32_t oK = kin ? (uint32_t)k * 2u * TS : kOOB;  // in a y slab
+    const uint32_t oZ = zpml ? (uint32_t)(k < a.plo[2] ? k : k - (nz - a.phi[2]) + a.plo[2]) * 2u * TS : kOOB;
     GLOBAL const T* cy = coef + a.coff[1];
     GLOBAL const T* cz = coef + a.coff[2];
     GLOBAL const T* cx = coef + a.coff[0];
@@ -1902,8 +1909,8 @@ __device__ __forceinline__ void adj_tile(const AdjArgs<T>& g, const int t) {
         load_u(i + 1, un, wn1);
         const bool xpml = in_pml(a, 0, pi, nx);
         const bool xpmln = pn >= 0 && in_pml(a, 0, pn, nx);
-        const uint32_t sxo = xpml ? (uint32_t)(pi < a.plo[0] ? pi : pi - (nx - a.phi[0]) + a.plo[0]) * PB : 0u;
-        const uint32_t sxn = xpmln ? (uint32_t)(pn < a.plo[0] ? pn : pn - (nx - a.phi[0]) + a.plo[0]) * PB : 0u;
+        const uint32_t sxo = xpml ? (uint32_t)(pi < a.plo[0] ? pi : pi - (nx - a.phi[0]) + a.plo[0]) * 2u * PB : 0u;
+        const uint32_t sxn = xpmln ? (uint32_t)(pn < a.plo[0] ? pn : pn - (nx - a.phi[0]) + a.plo[0]) * 2u * PB : 0u;
         const T bEx = xpml ? cx[pi] : T(1), bHx = xpml ? cx[2 * nx + pi] : T(1);
         const T bExn = xpmln ? cx[pn] : T(1);
         const Rsrc rA = rsrc(AR + (long)pi * FPB);
@@ -1917,18 +1924,14 @@ __device__ __forceinline__ void adj_tile(const AdjArgs<T>& g, const int t) {
         for (int r = 0; r < 2; ++r)
 #pragma unroll
             for (int c = 0; c < 3; ++c) hb[r][c] = bld<T>(rA, oR[r], (3 + c) * PB);
-        T pzE[2][2] = {{T(0), T(0)}, {T(0), T(0)}}, phz[2] = {T(0), T(0)};
+        Pair pzE[2] = {Pair{T(0), T(0)}, Pair{T(0), T(0)}}, phz = Pair{T(0), T(0)};
         if (zany) {  // lanes outside the layers: b = 1 and a zero auxiliary
 #pragma unroll
             for (int r = 0; r < 2; ++r) {
                 if (!rv[r]) continue;
-                const uint32_t so = (uint32_t)((pi * ny + gj[r]) * Lz) * TS;
-                pzE[r][0] = bld<T>(rpz, oZ, er * SB2 + so);
-                pzE[r][1] = bld<T>(rpz, oZ, (er + 1) * SB2 + so);
-                if (r == 1) {
-                    phz[0] = bld<T>(rpz, oZ, hr * SB2 + so);
-                    phz[1] = bld<T>(rpz, oZ, (hr + 1) * SB2 + so);
-                }
+                const uint32_t so = (uint32_t)((pi * ny + gj[r]) * Lz) * 2u * TS;
+                pzE[r] = bld2<T>(rpz, oZ, er * SB2 + so);
+                if (r == 1) phz = bld2<T>(rpz, oZ, hr * SB2 + so);
             }
         }
         const bool wr = own_plane && rv[1];
@@ -1979,7 +1982,7 @@ __device__ __forceinline__ void adj_tile(const AdjArgs<T>& g, const int t) {
         // E-terms on rows r = 0, 1 (labels: y (Ex->Hz), z (Ex->Hy), z (Ey->Hx), x (Ey->Hz),
         // x (Ez->Hy), y (Ez->Hx)) and the y-terms of row 2
         T eb[3][6];
-        T pey[2] = {T(0), T(0)}, pex[2] = {T(0), T(0)};  // owned row's y and x E aux bars
+        Pair pey = Pair{T(0), T(0)}, pex = Pair{T(0), T(0)};  // owned row's y and x E aux bars
 #pragma unroll
         for (int r = 0; r < 3; ++r) {
             const bool ok = rv[r];
@@ -1989,28 +1992,22 @@ __device__ __forceinline__ void adj_tile(const AdjArgs<T>& g, const int t) {
               t_ez_y = -cdt * uz;
             if (ypml[r]) {
                 const T b = cy[j];
-                const uint32_t so = (uint32_t)((pi * Ly + sy[r]) * nz) * TS;
-                const T p0 = bld<T>(rpy, oK, er * SB1 + so), p1 = bld<T>(rpy, oK, (er + 1) * SB1 + so);
-                t_ex_y = b * t_ex_y + (b - T(1)) * p0;
-                t_ez_y = b * t_ez_y + (b - T(1)) * p1;
-                if (r == 1) {
-                    pey[0] = p0;
-                    pey[1] = p1;
-                }
+                const uint32_t so = (uint32_t)((pi * Ly + sy[r]) * nz) * 2u * TS;
+                const Pair q = bld2<T>(rpy, oK, er * SB1 + so);
+                t_ex_y = adj_term(b, t_ex_y, q.x);
+                t_ez_y = adj_term(b, t_ez_y, q.y);
+                if (r == 1) pey = q;
             }
             if (r < 2) {
                 if (ok && zany) {
-                    t_ex_z = bEz * t_ex_z + (bEz - T(1)) * pzE[r][0];
-                    t_ey_z = bEz * t_ey_z + (bEz - T(1)) * pzE[r][1];
+                    t_ex_z = adj_term(bEz, t_ex_z, pzE[r].x);
+                    t_ey_z = adj_term(bEz, t_ey_z, pzE[r].y);
                 }
                 if (ok && xpml) {
-                    const T p0 = bld<T>(rpx, oR[r], er * SB0 + sxo), p1 = bld<T>(rpx, oR[r], (er + 1) * SB0 + sxo);
-                    t_ey_x = bEx * t_ey_x + (bEx - T(1)) * p0;
-                    t_ez_x = bEx * t_ez_x + (bEx - T(1)) * p1;
-                    if (r == 1) {
-                        pex[0] = p0;
-                        pex[1] = p1;
-                    }
+                    const Pair q = bld2<T>(rpx, two(oR[r]), er * SB0 + sxo);
+                    t_ey_x = adj_term(bEx, t_ey_x, q.x);
+                    t_ez_x = adj_term(bEx, t_ez_x, q.y);
+                    if (r == 1) pex = q;
                 }
             }
             eb[r][0] = t_ex_y;
@@ -2026,8 +2023,9 @@ __device__ __forceinline__ void adj_tile(const AdjArgs<T>& g, const int t) {
         for (int r = 0; r < 2; ++r) {
             T a1 = -cdt * un[r][1], a2 = cdt * un[r][2];  // (Ey -> Hz), (Ez -> Hy)
             if (rv[r] && xpmln) {
-                a1 = bExn * a1 + (bExn - T(1)) * bld<T>(rpx, oR[r], er * SB0 + sxn);
-                a2 = bExn * a2 + (bExn - T(1)) * bld<T>(rpx, oR[r], (er + 1) * SB0 + sxn);
+                const Pair q = bld2<T>(rpx, two(oR[r]), er * SB0 + sxn);
+                a1 = adj_term(bExn, a1, q.x);
+                a2 = adj_term(bExn, a2, q.y);
             }
             ebn[r][0] = (rv[r] && pn >= 0) ? a1 : T(0);
             ebn[r][1] = (rv[r] && pn >= 0) ? a2 : T(0);
@@ -2052,16 +2050,12 @@ __device__ __forceinline__ void adj_tile(const AdjArgs<T>& g, const int t) {
             tot[r][2] = ok ? hb[r][2] + (eb[r][0] - eb[r + 1][0]) + (eb[r][3] - ebn[r][0]) : T(0);
         }
         // H auxiliary bars of the owned row (read by the update below and by phase 2)
-        T phy[2] = {T(0), T(0)}, phx[2] = {T(0), T(0)};
+        Pair phy = Pair{T(0), T(0)}, phx = Pair{T(0), T(0)};
         if (ypml[1]) {
-            const uint32_t so = (uint32_t)((pi * Ly + sy[1]) * nz) * TS;
-            phy[0] = bld<T>(rpy, oK, hr * SB1 + so);
-            phy[1] = bld<T>(rpy, oK, (hr + 1) * SB1 + so);
+            const uint32_t so = (uint32_t)((pi * Ly + sy[1]) * nz) * 2u * TS;
+            phy = bld2<T>(rpy, oK, hr * SB1 + so);
         }
-        if (rv[1] && xpml) {
-            phx[0] = bld<T>(rpx, oR[1], hr * SB0 + sxo);
-            phx[1] = bld<T>(rpx, oR[1], (hr + 1) * SB0 + sxo);
-        }
+        if (rv[1] && xpml) phx = bld2<T>(rpx, two(oR[1]), hr * SB0 + sxo);
         // own row: Hbar at the old time and the new H auxiliary bars
         if (wr) {
             const int j = gj[1];
@@ -2070,18 +2064,15 @@ __device__ __forceinline__ void adj_tile(const AdjArgs<T>& g, const int t) {
             bst<NTS>(rB, oR[1], 5 * PB, tot[1][2]);
             if (ypml[1]) {  // (Hx, y, +, slot 0), (Hz, y, -, slot 1)
                 const T b = cy[2 * ny + j];
-                const uint32_t so = (uint32_t)((pi * Ly + sy[1]) * nz) * TS;
-                bst<NTS>(rpy, oK, hw * SB1 + so, b * (-cdt * tot[1][0] + phy[0]));
-                bst<NTS>(rpy, oK, (hw + 1) * SB1 + so, b * (cdt * tot[1][2] + phy[1]));
+                const uint32_t so = (uint32_t)((pi * Ly + sy[1]) * nz) * 2u * TS;
+                bst2<NTS>(rpy, oK, hw * SB1 + so, Pair{b * (-cdt * tot[1][0] + phy.x), b * (cdt * tot[1][2] + phy.y)});
             }
             if (zany) {  // (Hx, z, -, slot 0), (Hy, z, +, slot 1)
-                const uint32_t so = (uint32_t)((pi * ny + j) * Lz) * TS;
-                bst<NTS>(rpz, oZ, hw * SB2 + so, bHz * (cdt * tot[1][0] + phz[0]));
-                bst<NTS>(rpz, oZ, (hw + 1) * SB2 + so, bHz * (-cdt * tot[1][1] + phz[1]));
+                const uint32_t so = (uint32_t)((pi * ny + j) * Lz) * 2u * TS;
+                bst2<NTS>(rpz, oZ, hw * SB2 + so, Pair{bHz * (cdt * tot[1][0] + phz.x), bHz * (-cdt * tot[1][1] + phz.y)});
             }
             if (xpml) {  // (Hy, x, -, slot 0), (Hz, x, +, slot 1)
-                bst<NTS>(rpx, oR[1], hw * SB0 + sxo, bHx * (cdt * tot[1][1] + phx[0]));
-                bst<NTS>(rpx, oR[1], (hw + 1) * SB0 + sxo, bHx * (-cdt * tot[1][2] + phx[1]));
+                bst2<NTS>(rpx, two(oR[1]), hw * SB0 + sxo, Pair{bHx * (cdt * tot[1][1] + phx.x), bHx * (-cdt * tot[1][2] + phx.y)});
             }
         }
 
@@ -2094,16 +2085,16 @@ __device__ __forceinline__ void adj_tile(const AdjArgs<T>& g, const int t) {
               d_hz_x = -cdt * tot[1][2], d_hz_y = cdt * tot[1][2];
             if (ypml[1]) {
                 const T b = cy[2 * ny + j];
-                d_hx_y = b * d_hx_y + (b - T(1)) * phy[0];
-                d_hz_y = b * d_hz_y + (b - T(1)) * phy[1];
+                d_hx_y = adj_term(b, d_hx_y, phy.x);
+                d_hz_y = adj_term(b, d_hz_y, phy.y);
             }
             if (rv[1] && zany) {
-                d_hx_z = bHz * d_hx_z + (bHz - T(1)) * phz[0];
-                d_hy_z = bHz * d_hy_z + (bHz - T(1)) * phz[1];
+                d_hx_z = adj_term(bHz, d_hx_z, phz.x);
+                d_hy_z = adj_term(bHz, d_hy_z, phz.y);
             }
             if (rv[1] && xpml) {
-                d_hy_x = bHx * d_hy_x + (bHx - T(1)) * phx[0];
-                d_hz_x = bHx * d_hz_x + (bHx - T(1)) * phx[1];
+                d_hy_x = adj_term(bHx, d_hy_x, phx.x);
+                d_hz_x = adj_term(bHx, d_hz_x, phx.y);
             }
             db[0] = d_hx_y;
             db[1] = d_hx_z;
@@ -2117,9 +2108,10 @@ __device__ __forceinline__ void adj_tile(const AdjArgs<T>& g, const int t) {
             T d_hx_y = -cdt * tot[0][0], d_hz_y = cdt * tot[0][2];
             if (ypml[0]) {
                 const T b = cy[2 * ny + j];
-                const uint32_t so = (uint32_t)((pi * Ly + sy[0]) * nz) * TS;
-                d_hx_y = b * d_hx_y + (b - T(1)) * bld<T>(rpy, oK, hr * SB1 + so);
-                d_hz_y = b * d_hz_y + (b - T(1)) * bld<T>(rpy, oK, (hr + 1) * SB1 + so);
+                const uint32_t so = (uint32_t)((pi * Ly + sy[0]) * nz) * 2u * TS;
+                const Pair q = bld2<T>(rpy, oK, hr * SB1 + so);
+                d_hx_y = adj_term(b, d_hx_y, q.x);
+                d_hz_y = adj_term(b, d_hz_y, q.y);
             }
             dbh[0] = rv[0] ? d_hx_y : T(0);
             dbh[1] = rv[0] ? d_hz_y : T(0);
@@ -2136,25 +2128,10 @@ __device__ __forceinline__ void adj_tile(const AdjArgs<T>& g, const int t) {
                 const T hxz_k = km1 >= 0 ? bufd[1 * B + km1] : T(0);
                 // Ex: (Hy, z) and (Hz, y); Ey: (Hx, z) and (Hz, x); Ez: (Hx, y) and (Hy, x)
                 const T u0[3] = {uc[1][0], uc[1][1], uc[1][2]};
-                // 1/eps and eps per component of the owned cell
-                T inv[3], epsc[3];
-#pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                    inv[c] = slut[mm[c]].inv_eps;
-                    epsc[c] = slut[mm[c]].eps_inf;
-                }
-                if (desany) {
-#pragma unroll
-                    for (int c = 0; c < 3; ++c) {
-                        inv[c] = des[c] ? dv[c] : inv[c];
-                        epsc[c] = des[c] ? T(1) / dv[c] : epsc[c];
-                    }
-                }
-                // Ebar' = eps Ubar' plus the differences
-                T out[3];
-                out[0] = epsc[0] * u0[0] + (hyz_k - db[2]) + (dbh[1] - db[5]);
-                out[1] = epsc[1] * u0[1] + (hxz_k - db[1]) + (dbx_prev[0] - db[4]);
-                out[2] = epsc[2] * u0[2] + (dbh[0] - db[0]) + (dbx_prev[1] - db[3]);
+                // the differences of each component; sum of the pole terms
+                const T x[3] = {(hyz_k - db[2]) + (dbh[1] - db[5]), (hxz_k - db[1]) + (dbx_prev[0] - db[4]),
+                                (dbh[0] - db[0]) + (dbx_prev[1] - db[3])};
+                T sq[3] = {T(0), T(0), T(0)};
                 if (NP > 0 && !uniform) {
                     const Rsrc rQ = rsrc((const char*)g.Aq + (long)pi * QPB);
                     const Rsrc rP = rsrc((const char*)g.Ap + (long)pi * QPB);
@@ -2170,31 +2147,31 @@ __device__ __forceinline__ void adj_tile(const AdjArgs<T>& g, const int t) {
                             const T pb = pv[s][c];
                             const T qb = vq ? qv[s][c] + pb - u0[c] : T(0);
                             bst<NTS>(rQ, vq ? o : kOOB, so, L.pole[s].alpha * qb);
-                            bst<NTS>(rP, vp ? o : kOOB, so, pb + L.pole[s].beta * qb);
-                            out[c] += L.pole[s].c3 * qb;
+                            bst<NTS>(rP, vp ? o : kOOB, so, fma_(L.pole[s].beta, qb, pb));
+                            sq[c] = fma_(L.pole[s].c3, qb, sq[c]);
                         }
                     }
                 }
                 // new E auxiliary bars: E-terms of row 0 with their signs
                 if (ypml[1]) {  // (Ex, y, +, slot 0), (Ez, y, -, slot 1)
                     const T b = cy[j];
-                    const uint32_t so = (uint32_t)((pi * Ly + sy[1]) * nz) * TS;
-                    bst<NTS>(rpy, oK, ew * SB1 + so, b * (cdt * u0[0] + pey[0]));
-                    bst<NTS>(rpy, oK, (ew + 1) * SB1 + so, b * (-cdt * u0[2] + pey[1]));
+                    const uint32_t so = (uint32_t)((pi * Ly + sy[1]) * nz) * 2u * TS;
+                    bst2<NTS>(rpy, oK, ew * SB1 + so, Pair{b * (cdt * u0[0] + pey.x), b * (-cdt * u0[2] + pey.y)});
                 }
                 if (zany) {  // (Ex, z, -, slot 0), (Ey, z, +, slot 1)
-                    const uint32_t so = (uint32_t)((pi * ny + j) * Lz) * TS;
-                    bst<NTS>(rpz, oZ, ew * SB2 + so, bEz * (-cdt * u0[0] + pzE[1][0]));
-                    bst<NTS>(rpz, oZ, (ew + 1) * SB2 + so, bEz * (cdt * u0[1] + pzE[1][1]));
+                    const uint32_t so = (uint32_t)((pi * ny + j) * Lz) * 2u * TS;
+                    bst2<NTS>(rpz, oZ, ew * SB2 + so, Pair{bEz * (-cdt * u0[0] + pzE[1].x), bEz * (cdt * u0[1] + pzE[1].y)});
                 }
                 if (xpml) {  // (Ey, x, -, slot 0), (Ez, x, +, slot 1)
-                    bst<NTS>(rpx, o, ew * SB0 + sxo, bEx * (-cdt * u0[1] + pex[0]));
-                    bst<NTS>(rpx, o, (ew + 1) * SB0 + sxo, bEx * (cdt * u0[2] + pex[1]));
+                    bst2<NTS>(rpx, two(o), ew * SB0 + sxo, Pair{bEx * (-cdt * u0[1] + pex.x), bEx * (cdt * u0[2] + pex.y)});
                 }
-                // the state is Ubar = Ebar / eps
-                bst<NTS>(rB, o, 0, inv[0] * out[0]);
-                bst<NTS>(rB, o, PB, inv[1] * out[1]);
-                bst<NTS>(rB, o, 2 * PB, inv[2] * out[2]);
+                // the state is Ubar = Ebar / eps: the differences and the pole terms add 1/eps of their sum
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    T inv = slut[mm[c]].inv_eps;
+                    if (desany) inv = des[c] ? dv[c] : inv;
+                    bst<NTS>(rB, o, c * PB, fma_(inv, x[c] + sq[c], u0[c]));
+                }
             }
         } else {
             lds_barrier();  // keep the barrier count uniform across iterations
@@ -2214,352 +2191,365 @@ __device__ __forceinline__ void adj_tile(const AdjArgs<T>& g, const int t) {
 // 1..rt-1 own rows j0..j0+rt-2, and the top thread row also forms the y-terms of the row above
 // the tile.  The y and z neighbours' E-terms (for Hbar) and H-terms (for Ebar) pass through LDS,
 // so each adjoint value is loaded once per tile and the y halo costs one row per rt-1 owned
-// rows.  The arithmetic of every cell is that of adj_tile.
-template <typename T, int NP>
+// rows.  The arithmetic of every cell is that of adj_tile, bit for bit.
+// Pipelined as step_rows is: every register is loaded for the plane that needs it next as soon as it
+// has been read, the loop starts with the Ebar phase, and one barrier per plane publishes both the
+// H-terms of plane i and the E-terms of plane i + 1 (which Hbar of plane i needs anyway), each in two
+// halves used in turn.  The plane before the chunk runs as an iteration whose stores are dropped.
+// Bound by latency and by the pole state's four accesses per slot; us per reverse step on MI355X
+// before (this form with the loads of a plane waited for in its iteration, and one row per workgroup)
+// and now: FP32 192x192x96 138 (one row), 93; 120x120x256 122, 80; FP64 72x64x56 33 (one row), 22.
+template <typename T, int NP, bool NTS>
 __device__ __forceinline__ void adj_rows(const AdjArgs<T>& g, const int t) {
-    constexpr uint32_t TS = sizeof(T);
+#pragma clang fp contract(off)
+    constexpr uint32_t W = sizeof(T);
+    constexpr int NS = NP > 0 ? NP : 1;
+    typedef Pair2<T> Pair;
     const StepArgs<T>& a = g.f;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const int B = blockDim.x;
+    Pair* sEz = reinterpret_cast<Pair*>(smem_raw);  // [2][B] E-terms (Ex->Hy, Ey->Hx) along z
+    Pair* sEy = sEz + 2 * B;                        // [2][B] E-terms (Ex->Hz, Ez->Hx) along y
+    Pair* sDz = sEy + 2 * B;                        // [2][B] H-terms (Hy->Ex, Hx->Ey) along z
+    Pair* sDy = sDz + 2 * B;                        // [2][B] H-terms (Hx->Ez, Hz->Ex) along y
+    MatLut<T>* slut = reinterpret_cast<MatLut<T>*>(sDy + 2 * B);
+    copy_lut(a, slut);
+
+    const char* A0 = (const char*)g.A[g.rd];
+    const long A01 = (const char*)g.A[1 - g.rd] - A0;  // from the set read to the set written
+    CONST const T* coef = (CONST const T*)a.coef;
+    CONST const MatLut<T>* clut = (CONST const MatLut<T>*)a.lut;
     const int nx = a.nx, ny = a.ny, nz = a.nz;
     const int RT = a.rt, R = RT - 1;
-    T* sE = reinterpret_cast<T*>(smem_raw);  // [4][B]: E-terms z (Ex->Hy), z (Ey->Hx), y (Ex->Hz), y (Ez->Hx)
-    T* sEt = sE + 4 * B;                     // [2][nz]: y-terms of the row above the tile
-    T* sD = sEt + 2 * ((nz + 1) & ~1);       // [4][B]: H-terms z (Hy->Ex), z (Hx->Ey), y (Hx->Ez), y (Hz->Ex)
-    MatLut<T>* slut = reinterpret_cast<MatLut<T>*>(sD + 4 * B);
-    copy_lut(a, slut);
-    const char* AR = (const char*)g.A[g.rd];
-    const char* AW = (const char*)g.A[1 - g.rd];
-    const char* matw = (const char*)a.matw;
-    GLOBAL const T* coef = (GLOBAL const T*)a.coef;
     const int tid = threadIdx.x;
     const bool act = tid < RT * nz;
     const int r = act ? tid / nz : 0;
     const int k = act ? tid - r * nz : 0;
-    const int tyi = t % a.nty, xci = t / a.nty;
-    const int x0 = xci * a.xc, x1 = min(x0 + a.xc, nx);
+    const int xci = t / a.nty, tyi = t - xci * a.nty;
     const int jr = tyi * R + r - 1;  // unwrapped global row of this thread row
     const int j = act ? wrap_or_ghost(jr, ny, a.py) : -1;
-    const bool rv = j >= 0;
-    const bool owned = act && r >= 1 && jr < ny;  // implies rv
+    const bool valid = j >= 0;
+    const bool owned = act && r >= 1 && jr < ny;  // implies valid
     const bool top = act && r == RT - 1;
-    const int jt = top ? wrap_or_ghost(jr + 1, ny, a.py) : -1;
-    const int kp1 = wrap_or_ghost(k + 1, nz, a.pz), km1 = wrap_or_ghost(k - 1, nz, a.pz);
+    const int ju = act ? wrap_or_ghost(jr + 1, ny, a.py) : -1;  // the row above
+    const int kp1 = k + 1 < nz ? k + 1 : a.pz ? 0 : -1;
+    const int km1 = k > 0 ? k - 1 : a.pz ? nz - 1 : -1;
     const T cdt = a.cdt;
     const bool uniform = a.uniform != 0;
-    const uint32_t er = g.er, ew = g.ew, hr = g.hr, hw = g.hw;
-    const uint32_t PB = (uint32_t)ny * (uint32_t)nz * TS;  // bytes of one component plane
+    const uint32_t PB = (uint32_t)ny * (uint32_t)nz * W;  // bytes of one component plane
     const long FPB = 6L * PB, QPB = (long)a.nqp * PB, PW = (long)ny * nz * 4;
     const int Ly = a.plo[1] + a.phi[1], Lz = a.plo[2] + a.phi[2];
-    const uint32_t SB0 = (uint32_t)(a.S[0] * TS), SB1 = (uint32_t)(a.S[1] * TS), SB2 = (uint32_t)(a.S[2] * TS);
-    const Rsrc rpx = rsrc(g.Apsi[0]), rpy = rsrc(g.Apsi[1]), rpz = rsrc(g.Apsi[2]);
-    const bool ypml = rv && in_pml(a, 1, j, ny);
-    const int sy = ypml ? (j < a.plo[1] ? j : j - (ny - a.phi[1]) + a.plo[1]) : 0;
-    const bool ypmlt = jt >= 0 && in_pml(a, 1, jt, ny);
-    const int syt = ypmlt ? (jt < a.plo[1] ? jt : jt - (ny - a.phi[1]) + a.plo[1]) : 0;
-    const uint32_t oR = rv ? (uint32_t)(j * nz + k) * TS : kOOB;
-    const uint32_t oW = owned ? (uint32_t)(j * nz + k) * 4u : kOOB;
-    const uint32_t oT = jt >= 0 ? (uint32_t)(jt * nz + k) * TS : kOOB;
-    const bool zpml = act && in_pml(a, 2, k, nz);
-    const bool zany = wave_any(zpml);
-    const uint32_t oK = act ? (uint32_t)k * TS : kOOB;
-    const uint32_t oZ = zpml ? (uint32_t)(k < a.plo[2] ? k : k - (nz - a.phi[2]) + a.plo[2]) * TS : kOOB;
-    GLOBAL const T* cy = coef + a.coff[1];
-    GLOBAL const T* cz = coef + a.coff[2];
-    GLOBAL const T* cx = coef + a.coff[0];
+    const uint32_t YP = (uint32_t)(Ly * nz) * 2u * W, ZP = (uint32_t)(ny * Lz) * 2u * W;  // bytes of a slab per plane
+    const uint32_t S0 = (uint32_t)(a.S[0] * W), S1 = (uint32_t)(a.S[1] * W), S2 = (uint32_t)(a.S[2] * W);
+    const uint32_t er0 = g.er * S0, er1 = g.er * S1, er2 = g.er * S2, ew0 = g.ew * S0, ew1 = g.ew * S1, ew2 = g.ew * S2;
+    const uint32_t hr0 = g.hr * S0, hr1 = g.hr * S1, hr2 = g.hr * S2, hw0 = g.hw * S0, hw1 = g.hw * S1, hw2 = g.hw * S2;
+    const int xlo = a.pml_on[0] ? a.plo[0] : 0;
+    const unsigned xin = a.pml_on[0] ? (unsigned)(nx - a.phi[0] - a.plo[0]) : 0xffffffffu;
+    auto in_x = [&](int p) { return p < nx && (unsigned)(p - xlo) >= xin; };
+    auto xslab = [&](int p) -> uint32_t { return (uint32_t)(p < a.plo[0] ? p : p - (nx - a.phi[0]) + a.plo[0]) * 2u * PB; };
+    CONST const T* cx = coef + a.coff[0];
+
+    // lane offsets; kOOB for lanes that neither read nor write
+    const uint32_t oc = valid ? ((uint32_t)j * nz + k) * W : kOOB;            // the cell
+    const uint32_t oo = owned ? oc : kOOB;                                    // owned cells
+    const uint32_t ot = top && ju >= 0 ? ((uint32_t)ju * nz + k) * W : kOOB;  // the row above the tile
+    const uint32_t ow = owned ? ((uint32_t)j * nz + k) * 4u : kOOB;           // material words
+    const bool ypml = valid && in_pml(a, 1, j, ny);
+    const bool tpml = top && ju >= 0 && in_pml(a, 1, ju, ny);
+    const bool zpml = valid && in_pml(a, 2, k, nz);
+    auto yrow = [&](int q) { return (uint32_t)((q < a.plo[1] ? q : q - (ny - a.phi[1]) + a.plo[1]) * nz + k) * 2u * W; };
+    const uint32_t oy = ypml ? yrow(j) : kOOB, oyt = tpml ? yrow(ju) : kOOB;
+    const uint32_t oz = zpml ? (uint32_t)(j * Lz + (k < a.plo[2] ? k : k - (nz - a.phi[2]) + a.plo[2])) * 2u * W : kOOB;
+    const uint32_t oyw = owned ? oy : kOOB, ozw = owned ? oz : kOOB;
+    // wavefront-uniform summaries of the per-lane conditions
+    const bool yany = wave_any(ypml), zany = wave_any(zpml), tany = wave_any(ot != kOOB), tyany = wave_any(tpml);
+    GLOBAL const T* cy = (GLOBAL const T*)a.coef + a.coff[1];
+    GLOBAL const T* cz = (GLOBAL const T*)a.coef + a.coff[2];
     const T bEz = zpml ? cz[k] : T(1), bHz = zpml ? cz[2 * nz + k] : T(1);
     const T bEy = ypml ? cy[j] : T(1), bHy = ypml ? cy[2 * ny + j] : T(1);
-    const T bEyt = ypmlt ? cy[jt] : T(1);
-    const Rsrc rd = rsrc(a.dinv);
-    const int dey = a.dhi[1] - a.dlo[1], dez = a.dhi[2] - a.dlo[2];
+    const T bEt = tpml ? cy[ju] : T(1);
+    // exchange slots of the row above (top row: tu), the row below and the z neighbours
+    const int up = (top || !act) ? tid : tid + nz, dn = owned ? tid - nz : tid;
+    const int kup = kp1 >= 0 ? r * nz + kp1 : tid, kdn = km1 >= 0 ? r * nz + km1 : tid;
 
-    const int istart = (x0 > 0 || a.px) ? x0 - 1 : x0;
-    // u = Ubar' of this thread's cell on planes i and i + 1, the top row's (Ubar'x, Ubar'z) of
-    // the row above, and the owned cell's material word
-    T uc[3], un[3], tc[2], tn[2];
-    uint32_t wc = 0u, wn = 0u;
-    auto load_u = [&](int p, T (&u)[3], T (&ut)[2], uint32_t& w) {
-        const int pp = wrap_or_ghost(p, nx, a.px);
-        const long pc = pp >= 0 ? pp : 0;
-        const Rsrc rf = rsrc(AR + pc * FPB);
-        const uint32_t o = pp >= 0 ? oR : kOOB;
+    const int x0 = xci * a.xc;
+    const int x1 = min(x0 + a.xc, nx);
+    const int istart = (x0 > 0 || a.px) ? x0 - 1 : x0;  // the plane before the chunk, where there is one
+
+    // the registers each plane loads anew
+    T un[3], ten[2] = {T(0), T(0)};      // u = Ubar' of plane i + 1; (x, z) of the row above the tile
+    T hb[3];                             // Hbar' of plane i
+    Pair pEx, pEy, pEz, pEt;             // E auxiliary bars of plane i + 1 (pEt: y, the row above the tile)
+    Pair pHx, pHy, pHz;                  // H auxiliary bars of plane i
+    T Qv[3][NS], Pv[3][NS];              // pole state
+    uint32_t mw = 0, mwn = 0;            // material words of planes i, i + 1
+    T uc[3];                             // u of plane i
+    T tc[6];                             // E-terms of plane i: Ex y, Ex z, Ey z, Ey x, Ez x, Ez y
+    T tu[2] = {T(0), T(0)};              // y-terms (Ex, Ez) of the row above the tile, plane i
+    T dx[2] = {T(0), T(0)};              // x H-terms (Hz, Hy) of plane i - 1
+    T u0[3], inv[3], sq[3], d[6], dv[3];
+    uint32_t dw = 0, cls = 0;            // cls: material of the wavefront on plane i (classify)
+
+    auto load_u = [&](const char* f, bool need) {
+        const Rsrc rn = rsrc(f, need);
 #pragma unroll
-        for (int c = 0; c < 3; ++c) u[c] = bld<T>(rf, o, c * PB);
-        ut[0] = ut[1] = T(0);
-        if (top) {
-            const uint32_t ot = pp >= 0 ? oT : kOOB;
-            ut[0] = bld<T>(rf, ot, 0);
-            ut[1] = bld<T>(rf, ot, 2 * PB);
+        for (int c = 0; c < 3; ++c) un[c] = bld<T>(rn, oc, c * PB);
+        if (tany) {
+            ten[0] = bld<T>(rn, ot, 0);
+            ten[1] = bld<T>(rn, ot, 2 * PB);
         }
-        w = uniform ? 0u : bld<uint32_t>(rsrc(matw + pc * PW), pp >= 0 ? oW : kOOB, 0);
     };
-    lds_barrier();  // LUT in LDS
-    load_u(istart, uc, tc, wc);
-    T dbx_prev[2] = {T(0), T(0)};  // x H-terms of this row on plane i - 1: (Hz -> Ey), (Hy -> Ez)
-
-    for (int i = istart; i < x1; ++i) {
-        const bool own_plane = i >= x0;
-        const int pi = wrap_or_ghost(i, nx, a.px);
-        const int pn = wrap_or_ghost(i + 1, nx, a.px);
-        load_u(i + 1, un, tn, wn);
-        const bool xpml = in_pml(a, 0, pi, nx);
-        const bool xpmln = pn >= 0 && in_pml(a, 0, pn, nx);
-        const uint32_t sxo = xpml ? (uint32_t)(pi < a.plo[0] ? pi : pi - (nx - a.phi[0]) + a.plo[0]) * PB : 0u;
-        const uint32_t sxn = xpmln ? (uint32_t)(pn < a.plo[0] ? pn : pn - (nx - a.phi[0]) + a.plo[0]) * PB : 0u;
-        const T bEx = xpml ? cx[pi] : T(1), bHx = xpml ? cx[2 * nx + pi] : T(1);
-        const T bExn = xpmln ? cx[pn] : T(1);
-        const Rsrc rA = rsrc(AR + (long)pi * FPB);
-        const Rsrc rB = rsrc(AW + (long)pi * FPB);
-
-        // ---- the global loads of plane i: Hbar', the E and H auxiliary bars of this row, the
-        // owned cell's design 1/eps and pole state
-        T hb[3];
+    auto load_aux_e = [&](int p, bool yz) {
+        if (yz) {
+            if (zany) pEz = bld2<T>(rsrc(g.Apsi[2]), oz, er2 + p * ZP);
+            if (yany) pEy = bld2<T>(rsrc(g.Apsi[1]), oy, er1 + p * YP);
+            if (tyany) pEt = bld2<T>(rsrc(g.Apsi[1]), oyt, er1 + p * YP);
+        }
+        if (__builtin_expect(in_x(p), 0)) pEx = bld2<T>(rsrc(g.Apsi[0]), two(oc), er0 + xslab(p));
+    };
+    auto load_h = [&](const char* f, int p, bool need) {
+        const Rsrc rn = rsrc(f, need);
 #pragma unroll
-        for (int c = 0; c < 3; ++c) hb[c] = bld<T>(rA, oR, (3 + c) * PB);
-        T pzE[2] = {T(0), T(0)}, phz[2] = {T(0), T(0)};
-        if (zany && rv) {  // lanes outside the layers: b = 1 and a zero auxiliary
-            const uint32_t so = (uint32_t)((pi * ny + j) * Lz) * TS;
-            pzE[0] = bld<T>(rpz, oZ, er * SB2 + so);
-            pzE[1] = bld<T>(rpz, oZ, (er + 1) * SB2 + so);
-            if (owned) {
-                phz[0] = bld<T>(rpz, oZ, hr * SB2 + so);
-                phz[1] = bld<T>(rpz, oZ, (hr + 1) * SB2 + so);
-            }
+        for (int c = 0; c < 3; ++c) hb[c] = bld<T>(rn, oc, (3 + c) * PB);
+        if (need) {
+            if (zany) pHz = bld2<T>(rsrc(g.Apsi[2]), ozw, hr2 + p * ZP);
+            if (yany) pHy = bld2<T>(rsrc(g.Apsi[1]), oy, hr1 + p * YP);
+            if (__builtin_expect(in_x(p), 0)) pHx = bld2<T>(rsrc(g.Apsi[0]), two(oo), hr0 + xslab(p));
         }
-        T pey[2] = {T(0), T(0)}, phy[2] = {T(0), T(0)};
-        if (ypml) {
-            const uint32_t so = (uint32_t)((pi * Ly + sy) * nz) * TS;
-            pey[0] = bld<T>(rpy, oK, er * SB1 + so);
-            pey[1] = bld<T>(rpy, oK, (er + 1) * SB1 + so);
-            phy[0] = bld<T>(rpy, oK, hr * SB1 + so);
-            phy[1] = bld<T>(rpy, oK, (hr + 1) * SB1 + so);
-        }
-        T pex[2] = {T(0), T(0)}, phx[2] = {T(0), T(0)};
-        if (rv && xpml) {
-            pex[0] = bld<T>(rpx, oR, er * SB0 + sxo);
-            pex[1] = bld<T>(rpx, oR, (er + 1) * SB0 + sxo);
-            if (owned) {
-                phx[0] = bld<T>(rpx, oR, hr * SB0 + sxo);
-                phx[1] = bld<T>(rpx, oR, (hr + 1) * SB0 + sxo);
-            }
-        }
-        const bool wr = own_plane && owned;
-        int mm[3] = {0, 0, 0}, npl[3] = {0, 0, 0};
-        bool des[3] = {false, false, false};
-        T dv[3];
-        bool desany = false;
-        uint32_t sact = 0u;  // pole slots some lane of the wavefront uses (uniform)
-        T qv[NP > 0 ? NP : 1][3], pv[NP > 0 ? NP : 1][3];
-        if (wave_any(wr) && !uniform) {
+    };
+    auto load_poles = [&](int p, uint32_t code, uint32_t w) {
+        const int npx = seg_poles(code);
+        const Rsrc rq = rsrc((const char*)g.Aq + (long)p * QPB), rp = rsrc((const char*)g.Ap + (long)p * QPB);
+        int np[3], lm[3];
 #pragma unroll
-            for (int c = 0; c < 3; ++c) {  // lanes of other rows: no poles, no design voxel
-                const int m = (wc >> (8 * c)) & 0xff;
-                des[c] = wr && m == a.nmat;
-                mm[c] = (wr && !des[c]) ? m : 0;
-                npl[c] = (wr && !des[c]) ? slut[mm[c]].np : 0;
-            }
-            desany = wave_any(des[0] || des[1] || des[2]);
-            if (desany) {
-                const uint32_t dq = (uint32_t)(((pi - a.dlo[0]) * dey + (j - a.dlo[1])) * dez + (k - a.dlo[2])) * TS;
+        for (int c = 0; c < 3; ++c) {
+            const MatLut<T>& L = slut[(w >> (8 * c)) & 0xff];
+            np[c] = L.np;
+            lm[c] = L.lorentz_mask;
+        }
 #pragma unroll
-                for (int c = 0; c < 3; ++c) dv[c] = bld<T>(rd, des[c] ? dq : kOOB, 0);
-            }
-            if (NP > 0) {
-                const Rsrc rQ = rsrc((const char*)g.Aq + (long)pi * QPB);
-                const Rsrc rP = rsrc((const char*)g.Ap + (long)pi * QPB);
-#pragma unroll
-                for (int s = 0; s < NP; ++s) {
-                    if (!wave_any(s < npl[0] || s < npl[1] || s < npl[2])) continue;
-                    sact |= 1u << s;
-#pragma unroll
-                    for (int c = 0; c < 3; ++c) {
-                        const bool vq = s < npl[c];
-                        const bool vp = vq && ((slut[mm[c]].lorentz_mask >> s) & 1);
-                        const uint32_t so = (s * 3 + c) * PB;
-                        pv[s][c] = bld<T>(rP, vp ? oR : kOOB, so);
-                        qv[s][c] = bld<T>(rQ, vq ? oR : kOOB, so);
-                    }
-                }
-            }
-        }
-
-        // ---- phase 1: E-terms of this row, Hbar_total ---------------------------------------
-        T t_ex_y = cdt * uc[0], t_ex_z = -cdt * uc[0], t_ey_z = cdt * uc[1], t_ey_x = -cdt * uc[1],
-          t_ez_x = cdt * uc[2], t_ez_y = -cdt * uc[2];
-        if (ypml) {
-            t_ex_y = bEy * t_ex_y + (bEy - T(1)) * pey[0];
-            t_ez_y = bEy * t_ez_y + (bEy - T(1)) * pey[1];
-        }
-        if (rv && zany) {
-            t_ex_z = bEz * t_ex_z + (bEz - T(1)) * pzE[0];
-            t_ey_z = bEz * t_ey_z + (bEz - T(1)) * pzE[1];
-        }
-        if (rv && xpml) {
-            t_ey_x = bEx * t_ey_x + (bEx - T(1)) * pex[0];
-            t_ez_x = bEx * t_ez_x + (bEx - T(1)) * pex[1];
-        }
-        // x-terms of plane i + 1: (Ey -> Hz), (Ez -> Hy)
-        T xn0 = -cdt * un[1], xn1 = cdt * un[2];
-        if (rv && xpmln) {
-            xn0 = bExn * xn0 + (bExn - T(1)) * bld<T>(rpx, oR, er * SB0 + sxn);
-            xn1 = bExn * xn1 + (bExn - T(1)) * bld<T>(rpx, oR, (er + 1) * SB0 + sxn);
-        }
-        xn0 = (rv && pn >= 0) ? xn0 : T(0);
-        xn1 = (rv && pn >= 0) ? xn1 : T(0);
-        if (act) {
-            sE[0 * B + tid] = t_ex_z;
-            sE[1 * B + tid] = t_ey_z;
-            sE[2 * B + tid] = t_ex_y;
-            sE[3 * B + tid] = t_ez_y;
-        }
-        if (top) {  // y-terms of the row above the tile
-            T ay = cdt * tc[0], az = -cdt * tc[1];
-            if (ypmlt) {
-                const uint32_t so = (uint32_t)((pi * Ly + syt) * nz) * TS;
-                ay = bEyt * ay + (bEyt - T(1)) * bld<T>(rpy, oK, er * SB1 + so);
-                az = bEyt * az + (bEyt - T(1)) * bld<T>(rpy, oK, (er + 1) * SB1 + so);
-            }
-            sEt[k] = ay;
-            sEt[nz + k] = az;
-        }
-        lds_barrier();
-        T tot[3];
-        {
-            const T exz_k = kp1 >= 0 ? sE[0 * B + r * nz + kp1] : T(0);
-            const T eyz_k = kp1 >= 0 ? sE[1 * B + r * nz + kp1] : T(0);
-            const T exy_up = !act ? T(0) : r + 1 < RT ? sE[2 * B + tid + nz] : sEt[k];
-            const T ezy_up = !act ? T(0) : r + 1 < RT ? sE[3 * B + tid + nz] : sEt[nz + k];
-            // Hx: (Ey, z) and (Ez, y); Hy: (Ex, z) and (Ez, x); Hz: (Ex, y) and (Ey, x)
-            tot[0] = rv ? hb[0] + (t_ey_z - eyz_k) + (t_ez_y - ezy_up) : T(0);
-            tot[1] = rv ? hb[1] + (t_ex_z - exz_k) + (t_ez_x - xn1) : T(0);
-            tot[2] = rv ? hb[2] + (t_ex_y - exy_up) + (t_ey_x - xn0) : T(0);
-        }
-        // owned row: Hbar at the old time and the new H auxiliary bars
-        if (wr) {
-            bst(rB, oR, 3 * PB, tot[0]);
-            bst(rB, oR, 4 * PB, tot[1]);
-            bst(rB, oR, 5 * PB, tot[2]);
-            if (ypml) {  // (Hx, y, +, slot 0), (Hz, y, -, slot 1)
-                const uint32_t so = (uint32_t)((pi * Ly + sy) * nz) * TS;
-                bst(rpy, oK, hw * SB1 + so, bHy * (-cdt * tot[0] + phy[0]));
-                bst(rpy, oK, (hw + 1) * SB1 + so, bHy * (cdt * tot[2] + phy[1]));
-            }
-            if (zany) {  // (Hx, z, -, slot 0), (Hy, z, +, slot 1)
-                const uint32_t so = (uint32_t)((pi * ny + j) * Lz) * TS;
-                bst(rpz, oZ, hw * SB2 + so, bHz * (cdt * tot[0] + phz[0]));
-                bst(rpz, oZ, (hw + 1) * SB2 + so, bHz * (-cdt * tot[1] + phz[1]));
-            }
-            if (xpml) {  // (Hy, x, -, slot 0), (Hz, x, +, slot 1)
-                bst(rpx, oR, hw * SB0 + sxo, bHx * (cdt * tot[1] + phx[0]));
-                bst(rpx, oR, (hw + 1) * SB0 + sxo, bHx * (-cdt * tot[2] + phx[1]));
-            }
-        }
-
-        // ---- phase 2: H-terms of this row, Ebar of the owned rows --------------------------
-        T d_hx_y = -cdt * tot[0], d_hx_z = cdt * tot[0], d_hy_z = -cdt * tot[1], d_hy_x = cdt * tot[1],
-          d_hz_x = -cdt * tot[2], d_hz_y = cdt * tot[2];
-        if (ypml) {
-            d_hx_y = bHy * d_hx_y + (bHy - T(1)) * phy[0];
-            d_hz_y = bHy * d_hz_y + (bHy - T(1)) * phy[1];
-        }
-        if (owned && zany) {
-            d_hx_z = bHz * d_hx_z + (bHz - T(1)) * phz[0];
-            d_hy_z = bHz * d_hy_z + (bHz - T(1)) * phz[1];
-        }
-        if (owned && xpml) {
-            d_hy_x = bHx * d_hy_x + (bHx - T(1)) * phx[0];
-            d_hz_x = bHx * d_hz_x + (bHx - T(1)) * phx[1];
-        }
-        d_hx_y = rv ? d_hx_y : T(0);
-        d_hz_y = rv ? d_hz_y : T(0);
-        if (act) {
-            sD[0 * B + tid] = d_hy_z;
-            sD[1 * B + tid] = d_hx_z;
-            sD[2 * B + tid] = d_hx_y;
-            sD[3 * B + tid] = d_hz_y;
-        }
-        lds_barrier();
-        if (wr) {
-            const uint32_t o = oR;
-            const T hyz_k = km1 >= 0 ? sD[0 * B + r * nz + km1] : T(0);
-            const T hxz_k = km1 >= 0 ? sD[1 * B + r * nz + km1] : T(0);
-            const T hxy_dn = sD[2 * B + tid - nz];  // y-terms of the row below (r >= 1)
-            const T hzy_dn = sD[3 * B + tid - nz];
-            T inv[3], epsc[3];
+        for (int s = 0; s < NP; ++s) {
+            if (s >= npx) break;
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
-                inv[c] = slut[mm[c]].inv_eps;
-                epsc[c] = slut[mm[c]].eps_inf;
+                Qv[c][s] = bld<T>(rq, s < np[c] ? oo : kOOB, (s * 3 + c) * PB);
+                Pv[c][s] = bld<T>(rp, (lm[c] >> s) & 1 ? oo : kOOB, (s * 3 + c) * PB);
             }
-            if (desany) {
+        }
+    };
+    // E-terms te and tt (row above the tile) of plane p from un, ten and the E auxiliary bars, and the new
+    // bars (`own`: of a plane of this chunk)
+    auto e_terms = [&](int p, bool own, T (&te)[6], T (&tt)[2]) {
+        te[0] = cdt * un[0], te[1] = -cdt * un[0], te[2] = cdt * un[1];
+        te[3] = -cdt * un[1], te[4] = cdt * un[2], te[5] = -cdt * un[2];
+        tt[0] = cdt * ten[0], tt[1] = -cdt * ten[1];
+        if (zany) {  // (Ex, z, -, slot 0), (Ey, z, +, slot 1); lanes outside the layers: b = 1
+            bst2<NTS>(rsrc(g.Apsi[2], own), ozw, ew2 + p * ZP, Pair{bEz * (te[1] + pEz.x), bEz * (te[2] + pEz.y)});
+            te[1] = adj_term(bEz, te[1], pEz.x);
+            te[2] = adj_term(bEz, te[2], pEz.y);
+        }
+        if (yany) {  // (Ex, y, +, slot 0), (Ez, y, -, slot 1)
+            bst2<NTS>(rsrc(g.Apsi[1], own), oyw, ew1 + p * YP, Pair{bEy * (te[0] + pEy.x), bEy * (te[5] + pEy.y)});
+            te[0] = adj_term(bEy, te[0], pEy.x);
+            te[5] = adj_term(bEy, te[5], pEy.y);
+        }
+        if (tyany) {
+            tt[0] = adj_term(bEt, tt[0], pEt.x);
+            tt[1] = adj_term(bEt, tt[1], pEt.y);
+        }
+        if (__builtin_expect(in_x(p), 0)) {  // (Ey, x, -, slot 0), (Ez, x, +, slot 1)
+            const T b = cx[p];
+            bst2<NTS>(rsrc(g.Apsi[0], own), two(oo), ew0 + xslab(p), Pair{b * (te[3] + pEx.x), b * (te[4] + pEx.y)});
+            te[3] = adj_term(b, te[3], pEx.x);
+            te[4] = adj_term(b, te[4], pEx.y);
+        }
+    };
+
+    // ---- the first plane's E-terms
+    int pi = istart < 0 ? nx - 1 : istart, pn = wrap_up(pi + 1, nx, a.px), pnn = wrap_up(pn + 1, nx, a.px);
+    const char* fW = A0 + (long)pi * FPB;  // plane i, then i + 1 and i + 2, of the set read
+    const char* fN = A0 + (long)min(pn, nx - 1) * FPB;
+    const char* fNN = A0 + (long)min(pnn, nx - 1) * FPB;
+    load_u(fW, true);
+    load_aux_e(pi, true);
+    load_h(fW, pi, true);
+    if (!uniform) {
+        mw = bld<uint32_t>(rsrc((const char*)a.matw + (long)pi * PW, istart == x0), ow, 0);
+        mwn = bld<uint32_t>(rsrc((const char*)a.matw + (long)min(pn, nx - 1) * PW, istart + 1 < x1), ow, 0);
+    }
+    e_terms(pi, istart == x0, tc, tu);
 #pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                    inv[c] = des[c] ? dv[c] : inv[c];
-                    epsc[c] = des[c] ? T(1) / dv[c] : epsc[c];
-                }
+    for (int c = 0; c < 3; ++c) uc[c] = un[c];
+    sEz[(istart & 1) * B + tid] = Pair{tc[1], tc[2]};
+    sEy[(istart & 1) * B + tid] = Pair{tc[0], tc[5]};
+    lds_barrier();  // also the material table
+    load_u(fN, pn < nx);
+    load_aux_e(pn, istart + 1 < x1);
+    if (!uniform && istart == x0) {
+        cls = classify<NP>(mw);
+        if (NP > 0 && seg_poles(cls) > 0) load_poles(pi, cls, mw);
+    }
+
+    auto h_phase = [&](const int i) __attribute__((always_inline)) {
+        const bool own = i >= x0 && i < x1, next = i + 1 < x1;
+        const bool xpml = in_x(pi) && i < x1;
+        const int half = (i & 1) * B, other = B - half;
+        // ------------------------------- E-terms of plane i + 1
+        T tn[6], tun[2];
+        e_terms(pn, next, tn, tun);
+        // ------------------------------- Hbar and the H auxiliary bars of plane i
+        {
+            const Pair ez = sEz[half + kup], ey = sEy[half + up];
+            const T exz = kp1 >= 0 ? ez.x : T(0), eyz = kp1 >= 0 ? ez.y : T(0);
+            const T exy = top ? tu[0] : ey.x, ezy = top ? tu[1] : ey.y;
+            T tot[3];
+            // Hx: (Ey, z) and (Ez, y); Hy: (Ex, z) and (Ez, x); Hz: (Ex, y) and (Ey, x)
+            tot[0] = valid ? hb[0] + (tc[2] - eyz) + (tc[5] - ezy) : T(0);
+            tot[1] = valid ? hb[1] + (tc[1] - exz) + (tc[4] - tn[4]) : T(0);
+            tot[2] = valid ? hb[2] + (tc[0] - exy) + (tc[3] - tn[3]) : T(0);
+            const Rsrc rW = rsrc(fW + A01, own);
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                pin(tot[c]);
+                bst<NTS>(rW, oo, (3 + c) * PB, tot[c]);
             }
-            // Ebar' = eps Ubar' plus the differences
-            // Ex: (Hy, z) and (Hz, y); Ey: (Hx, z) and (Hz, x); Ez: (Hx, y) and (Hy, x)
-            T out[3];
-            out[0] = epsc[0] * uc[0] + (hyz_k - d_hy_z) + (hzy_dn - d_hz_y);
-            out[1] = epsc[1] * uc[1] + (hxz_k - d_hx_z) + (dbx_prev[0] - d_hz_x);
-            out[2] = epsc[2] * uc[2] + (hxy_dn - d_hx_y) + (dbx_prev[1] - d_hy_x);
-            if (NP > 0 && !uniform) {
-                const Rsrc rQ = rsrc((const char*)g.Aq + (long)pi * QPB);
-                const Rsrc rP = rsrc((const char*)g.Ap + (long)pi * QPB);
+            // H-terms: Hx y, Hx z, Hy z, Hy x, Hz x, Hz y
+            d[0] = -cdt * tot[0], d[1] = cdt * tot[0], d[2] = -cdt * tot[1];
+            d[3] = cdt * tot[1], d[4] = -cdt * tot[2], d[5] = cdt * tot[2];
+            if (yany) {  // (Hx, y, +, slot 0), (Hz, y, -, slot 1)
+                bst2<NTS>(rsrc(g.Apsi[1], own), oyw, hw1 + pi * YP, Pair{bHy * (d[0] + pHy.x), bHy * (d[5] + pHy.y)});
+                d[0] = adj_term(bHy, d[0], pHy.x);
+                d[5] = adj_term(bHy, d[5], pHy.y);
+            }
+            if (zany) {  // (Hx, z, -, slot 0), (Hy, z, +, slot 1)
+                bst2<NTS>(rsrc(g.Apsi[2], own), ozw, hw2 + pi * ZP, Pair{bHz * (d[1] + pHz.x), bHz * (d[2] + pHz.y)});
+                d[1] = adj_term(bHz, d[1], pHz.x);
+                d[2] = adj_term(bHz, d[2], pHz.y);
+            }
+            if (__builtin_expect(xpml, 0)) {  // (Hy, x, -, slot 0), (Hz, x, +, slot 1)
+                const T b = cx[2 * nx + pi];
+                bst2<NTS>(rsrc(g.Apsi[0], own), two(oo), hw0 + xslab(pi), Pair{b * (d[3] + pHx.x), b * (d[4] + pHx.y)});
+                d[3] = adj_term(b, d[3], pHx.x);
+                d[4] = adj_term(b, d[4], pHx.y);
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < 6; ++c) pin(d[c]);
+        sDz[half + tid] = Pair{d[2], d[1]};
+        sDy[half + tid] = Pair{d[0], d[5]};
+        sEz[other + tid] = Pair{tn[1], tn[2]};
+        sEy[other + tid] = Pair{tn[0], tn[5]};
+#pragma unroll
+        for (int c = 0; c < 6; ++c) tc[c] = reg_copy(tn[c]);
+        tu[0] = reg_copy(tun[0]);
+        tu[1] = reg_copy(tun[1]);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) u0[c] = reg_copy(uc[c]);
+        // ------------------------------- pole recursions of plane i; 1/eps
+        const T iv = clut[cls & 0xff].inv_eps;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) inv[c] = iv, sq[c] = T(0);
+        if (cls & kSegSpecial) {
+            const MatLut<T>* L[3];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                L[c] = slut + ((mw >> (8 * c)) & 0xff);
+                inv[c] = L[c]->inv_eps;
+            }
+            const int npx = seg_poles(cls);
+            if (NP > 0 && npx > 0) {
+                const Rsrc rq = rsrc((const char*)g.Aq + (long)pi * QPB), rp = rsrc((const char*)g.Ap + (long)pi * QPB);
+                int np[3];
+#pragma unroll
+                for (int c = 0; c < 3; ++c) np[c] = L[c]->np;
 #pragma unroll
                 for (int s = 0; s < NP; ++s) {
-                    if (!((sact >> s) & 1u)) continue;
+                    if (s >= npx) break;
+                    PoleCoef<T> p[3];
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) p[c] = L[c]->pole[s];
 #pragma unroll
                     for (int c = 0; c < 3; ++c) {
-                        const MatLut<T>& L = slut[mm[c]];
-                        const bool vq = s < npl[c];
-                        const bool vp = vq && ((L.lorentz_mask >> s) & 1);
                         const uint32_t so = (s * 3 + c) * PB;
-                        const T pb = pv[s][c];
-                        const T qb = vq ? qv[s][c] + pb - uc[c] : T(0);
-                        bst(rQ, vq ? o : kOOB, so, L.pole[s].alpha * qb);
-                        bst(rP, vp ? o : kOOB, so, pb + L.pole[s].beta * qb);
-                        out[c] += L.pole[s].c3 * qb;
+                        const bool vq = s < np[c];
+                        const T pb = Pv[c][s];
+                        const T qb = vq ? Qv[c][s] + pb - u0[c] : T(0);
+                        bst<NTS>(rq, vq ? oo : kOOB, so, p[c].alpha * qb);
+                        bst<NTS>(rp, vq && p[c].lor != T(0) ? oo : kOOB, so, fma_(p[c].beta, qb, pb));
+                        sq[c] = fma_(p[c].c3, qb, sq[c]);
                     }
                 }
             }
-            // new E auxiliary bars: E-terms of this row with their signs
-            if (ypml) {  // (Ex, y, +, slot 0), (Ez, y, -, slot 1)
-                const uint32_t so = (uint32_t)((pi * Ly + sy) * nz) * TS;
-                bst(rpy, oK, ew * SB1 + so, bEy * (cdt * uc[0] + pey[0]));
-                bst(rpy, oK, (ew + 1) * SB1 + so, bEy * (-cdt * uc[2] + pey[1]));
-            }
-            if (zany) {  // (Ex, z, -, slot 0), (Ey, z, +, slot 1)
-                const uint32_t so = (uint32_t)((pi * ny + j) * Lz) * TS;
-                bst(rpz, oZ, ew * SB2 + so, bEz * (-cdt * uc[0] + pzE[0]));
-                bst(rpz, oZ, (ew + 1) * SB2 + so, bEz * (cdt * uc[1] + pzE[1]));
-            }
-            if (xpml) {  // (Ey, x, -, slot 0), (Ez, x, +, slot 1)
-                bst(rpx, o, ew * SB0 + sxo, bEx * (-cdt * uc[1] + pex[0]));
-                bst(rpx, o, (ew + 1) * SB0 + sxo, bEx * (cdt * uc[2] + pex[1]));
-            }
-            // the state is Ubar = Ebar / eps
-            bst(rB, o, 0, inv[0] * out[0]);
-            bst(rB, o, PB, inv[1] * out[1]);
-            bst(rB, o, 2 * PB, inv[2] * out[2]);
-        }
-        dbx_prev[0] = owned ? d_hz_x : T(0);
-        dbx_prev[1] = owned ? d_hy_x : T(0);
+            if (cls & kSegDesign) {
+                // design voxels: 1/eps from the design array [dx][dy][dz]
+                const Rsrc rd = rsrc(a.dinv);
+                const uint32_t dq = (uint32_t)(((pi - a.dlo[0]) * (a.dhi[1] - a.dlo[1]) + (j - a.dlo[1])) *
+                                                   (a.dhi[2] - a.dlo[2]) + (k - a.dlo[2])) * W;
 #pragma unroll
-        for (int c = 0; c < 3; ++c) uc[c] = un[c];
-        tc[0] = tn[0];
-        tc[1] = tn[1];
-        wc = wn;
+                for (int c = 0; c < 3; ++c)
+                    dv[c] = bld<T>(rd, owned && (int)((mw >> (8 * c)) & 0xff) == a.nmat ? dq : kOOB, 0);
+                dw = mw;
+            }
+        }
+        // ------------------------------- loads for the planes ahead
+        uint32_t cn = 0u;
+        if (!uniform && next) {
+            cn = classify<NP>(mwn);
+            if (NP > 0 && seg_poles(cn) > 0) load_poles(pn, cn, mwn);
+        }
+        mw = reg_copy(mwn);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) uc[c] = reg_copy(un[c]);
+        load_u(fNN, next && pnn < nx);
+        if (next) load_aux_e(pnn, i + 2 < x1);
+        load_h(fN, pn, next);
+        if (!uniform) mwn = bld<uint32_t>(rsrc((const char*)a.matw + (long)(i + 2 < x1 ? pnn : 0) * PW, i + 2 < x1), ow, 0);
+        return cn;
+    };
+
+    auto e_phase = [&](const int i) __attribute__((always_inline)) {
+        const Rsrc rW = rsrc(fW + A01, i >= x0);
+        const int half = (i & 1) * B;
+        lds_barrier();
+        const Pair dz = sDz[half + kdn], dy = sDy[half + dn];
+        const T hyz = km1 >= 0 ? dz.x : T(0), hxz = km1 >= 0 ? dz.y : T(0);
+        if (cls & kSegDesign) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) inv[c] = (int)((dw >> (8 * c)) & 0xff) == a.nmat ? dv[c] : inv[c];
+        }
+        // Ex: (Hy, z) and (Hz, y); Ey: (Hx, z) and (Hz, x); Ez: (Hx, y) and (Hy, x)
+        bst<NTS>(rW, oo, 0, fma_(inv[0], ((hyz - d[2]) + (dy.y - d[5])) + sq[0], u0[0]));
+        bst<NTS>(rW, oo, PB, fma_(inv[1], ((hxz - d[1]) + (dx[0] - d[4])) + sq[1], u0[1]));
+        bst<NTS>(rW, oo, 2 * PB, fma_(inv[2], ((dy.x - d[0]) + (dx[1] - d[3])) + sq[2], u0[2]));
+        dx[0] = reg_copy(d[4]);
+        dx[1] = reg_copy(d[3]);
+        // the next plane
+        fW = fN;
+        fN = fNN;
+        pi = pn;
+        pn = pnn;
+        ++pnn;
+        fNN += FPB;
+        if (__builtin_expect(pnn >= nx, 0)) {
+            if (a.px) pnn = 0;
+            fNN = A0;  // of plane 0, or not read
+        }
+    };
+
+    uint32_t cn = h_phase(istart);
+    for (int i = istart; i < x1; ++i) {
+        e_phase(i);
+        cls = cn;
+        cn = h_phase(i + 1);
     }
 }
 
 // Fused reverse step over one engine, row-of-threads form (tile t after the XCD-aware remap).
-template <typename T, int NP, int MAXT>
+template <typename T, int NP, int MAXT, bool NTS = false>
 __global__ void __launch_bounds__(MAXT) k_adj_rows(const AdjArgs<T> g) {
     const int w = blockIdx.x, nw = gridDim.x;
     const int t = (nw % 8 == 0) ? ((w & 7) * (nw >> 3) + (w >> 3)) : w;
-    adj_rows<T, NP>(g, t);
+    adj_rows<T, NP, NTS>(g, t);
 }
 
 // Fused reverse step over one engine: workgroup w handles tile w after the XCD-aware remap.
@@ -2745,12 +2735,12 @@ k_adj_step_batch(const AdjArgs<T>* __restrict__ args, const int* __restrict__ ti
 }
 
 // The same, row-of-threads form
-template <typename T, int NP, int MAXT>
+template <typename T, int NP, int MAXT, bool NTS = false>
 __global__ void __launch_bounds__(MAXT) k_adj_rows_batch(const AdjArgs<T>* __restrict__ args,
                                                          const int* __restrict__ tile_first, int ninst) {
     int t;
     const int b = tile_instance(tile_first, ninst, t);
-    adj_rows<T, NP>(args[b], t);
+    adj_rows<T, NP, NTS>(args[b], t);
 }
 
 // ---- plain streaming copy (achievable-bandwidth probe and counter calibration) -----------
