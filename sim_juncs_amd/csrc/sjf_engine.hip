@@ -72,7 +72,7 @@ struct sjf_engine {
     long version = 0;  // bumped by every change that invalidates compiled launch tables
 
     void* Fbuf[2] = {};  // field sets [x][Ex Ey Ez Hx Hy Hz][y][z]; step n reads set n&1
-    long* d_step = nullptr;
+    long* d_step = nullptr;  // step counter and its shadow (sjf_kernels.h)
     long step = 0;
 
     // materials: given* as the caller set them; matw / lut_h / nmat / maxp are what the kernels run
@@ -480,9 +480,8 @@ struct LaunchSet {
     long dft_total = 0;
     int dft_maxnf = 0;  // most frequencies of any region (the launch's second dimension)
     bool src_dft_one_launch = false;  // no DFT region holds a source cell: one launch for both
-    // step counters, and the sign-off word of the last kernel of a step that advances them
+    // step counters, which the last kernel of a step advances
     long** d_counters = nullptr;
-    unsigned* d_done = nullptr;
     // graph
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec = nullptr;
@@ -508,7 +507,6 @@ void set_free_tables(LaunchSet* s) {
     dev_free(s->d_mon);
     dev_free(s->d_dft);
     dev_free(s->d_counters);
-    dev_free(s->d_done);
     if (s->gexec) (void)hipGraphExecDestroy(s->gexec);
     if (s->graph) (void)hipGraphDestroy(s->graph);
     s->gexec = nullptr;
@@ -714,7 +712,6 @@ int build_set_t(LaunchSet* s) {
     for (sjf_engine* e : s->eng) ctr.push_back(e->d_step);
     rc = upload_vec(e0, s->stream, (void**)&s->d_counters, ctr);
     if (rc) return rc;
-    rc = upload_vec(e0, s->stream, (void**)&s->d_done, std::vector<unsigned>(sjf::kDoneWords, 0u));  // armed at zero
     if (rc) return rc;
 
     s->versions.clear();
@@ -815,23 +812,23 @@ int launch_one_step_t(LaunchSet* s, bool sample, hipEvent_t ev_a, hipEvent_t ev_
     const bool dft = s->ndft && !bare;
     const sjf::SrcTables<T> st{(const sjf::SrcDev<T>*)s->d_src, s->d_blk_src, s->d_blk_first, s->d_blk_end,
                                s->d_src_idx, s->d_src_coef};
-    const sjf::Tick tick{s->d_counters, n, s->d_done};
+    const sjf::Tick tick{s->d_counters, n};
     const int dftx = (int)((s->dft_total + 255) / 256);
+    const unsigned ndb = (unsigned)(dftx * s->dft_maxnf);
     if (dft && s->src_dft_one_launch) {
-        hipLaunchKernelGGL((sjf::k_source_dft<T>), dim3((unsigned)(s->nsrcblk + dftx * s->dft_maxnf)), dim3(256), 0,
-                           s->stream, st, s->nsrcblk, (const sjf::DftDev<T>*)s->d_dft, s->ndft, s->dft_total, dftx,
-                           tick);
+        hipLaunchKernelGGL((sjf::k_source_dft<T>), dim3(s->nsrcblk + ndb), dim3(256), 0, s->stream, st, s->nsrcblk,
+                           (const sjf::DftDev<T>*)s->d_dft, s->ndft, s->dft_total, dftx, tick);
         SETCHK(s, hipGetLastError());
         return SJF_OK;
     }
     if (s->nsrcblk) {
-        const sjf::Tick src_tick{s->d_counters, n, dft ? nullptr : s->d_done};
+        const sjf::Tick src_tick{s->d_counters, dft ? 0 : n};
         hipLaunchKernelGGL((sjf::k_source<T>), dim3(s->nsrcblk), dim3(256), 0, s->stream, st, src_tick);
         SETCHK(s, hipGetLastError());
     }
     if (dft) {
-        hipLaunchKernelGGL((sjf::k_dft<T>), dim3((unsigned)dftx, (unsigned)s->dft_maxnf), dim3(256), 0, s->stream,
-                           (const sjf::DftDev<T>*)s->d_dft, s->ndft, s->dft_total, tick);
+        hipLaunchKernelGGL((sjf::k_dft<T>), dim3(ndb), dim3(256), 0, s->stream, (const sjf::DftDev<T>*)s->d_dft, s->ndft,
+                           s->dft_total, dftx, tick);
         SETCHK(s, hipGetLastError());
     } else if (!s->nsrcblk) {
         hipLaunchKernelGGL(sjf::k_tick, dim3((n + 63) / 64), dim3(64), 0, s->stream, s->d_counters, n);
@@ -1206,7 +1203,7 @@ int update_words(sjf_engine* e) {
     }
     for (int m = 0; m < 256; ++m)
         map.twin[m] = (unsigned char)(m < (int)e->twin.size() && e->twin[m] >= 0 ? e->twin[m] : m);
-    const dim3 grid((unsigned)std::min(2048L, (n + 3) / 4)), block(256);
+    const dim3 grid((unsigned)std::min(512L, (n + 3) / 4)), block(256);
     if (e->prec == 4)
         hipLaunchKernelGGL((sjf::k_words<float>), grid, block, 0, e->stream, e->given, e->matw, e->seg,
                            (const sjf::MatLut<float>*)e->lut, dim[0], dim[1], dim[2], e->nmat, map, sums);
@@ -1594,10 +1591,10 @@ int adjoint_run_t(sjf_engine* e, long nsteps, long K, long gap, double* J_out, d
     const unsigned gdes = (unsigned)((nd + 3 + 255) / 256);
     const int de0 = e->dhi[0] - e->dlo[0], de1 = e->dhi[1] - e->dlo[1], de2 = e->dhi[2] - e->dlo[2];
     const long nyz = (long)e->g.ny * e->g.nz;
-    auto record = [&](long sl) -> int {
+    auto record = [&](long sl, bool objective = false) -> int {
         const T* E = (const T*)e->Fbuf[e->step & 1];
         hipLaunchKernelGGL((sjf::k_adj_record<T>), dim3(gdes), dim3(256), 0, e->stream, E, nyz, e->g.ny, e->g.nz,
-                           e->dlo[0], e->dlo[1], e->dlo[2], de0, de1, de2, gap, ring, sl);
+                           e->dlo[0], e->dlo[1], e->dlo[2], de0, de1, de2, gap, ring, sl, dt, objective ? dJ : nullptr);
         HIPCHK(e, hipGetLastError());
         return SJF_OK;
     };
@@ -1609,10 +1606,13 @@ int adjoint_run_t(sjf_engine* e, long nsteps, long K, long gap, double* J_out, d
         }
         if ((rc = launch_one_step(s, samples_at(s, e->step)))) return bail(rc);
         advance_hosts(s, 1);
+        if (rec_all) {
+            if ((rc = record(n + 1, true))) return bail(rc);
+            continue;
+        }
         const T* E = (const T*)e->Fbuf[e->step & 1];
         hipLaunchKernelGGL((sjf::k_adj_objective<T>), dim3(1), dim3(64), 0, e->stream, E, nyz, gap, dt, dJ);
         HIPCHK(e, hipGetLastError());
-        if (rec_all && (rc = record(n + 1))) return bail(rc);
     }
     if (!rec_all && (rc = copy_state(e, cks + L.total * nck, L, true))) return bail(rc);
     HIPCHK(e, hipStreamSynchronize(e->stream));
@@ -2276,7 +2276,7 @@ int sjf_create(const sjf_grid* g, sjf_engine** out) {
         int rc = dev_alloc(e, &e->Fbuf[b], (size_t)e->prec * 6 * e->N);
         if (rc) return bail(rc);
     }
-    if (int rc = dev_alloc(e, (void**)&e->d_step, sizeof(long))) return bail(rc);
+    if (int rc = dev_alloc(e, (void**)&e->d_step, 2 * sizeof(long))) return bail(rc);
     // PML tables for all axes (b = 1, a = 0 until sjf_set_pml fills an axis)
     {
         const int n3[3] = {g->nx, g->ny, g->nz};

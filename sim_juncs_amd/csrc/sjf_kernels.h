@@ -76,7 +76,7 @@ struct StepArgs {
     long N;       // cells
     T cdt;        // dt / dx
     T* F[2];              // field sets [x][Ex Ey Ez Hx Hy Hz][y][z]; step n reads F[n&1], writes F[~n&1]
-    const long* d_step;   // the engine's step counter
+    long* d_step;         // the engine's step counter and its shadow
     int uniform;  // 1: single non-dispersive material, no material word read
     int nmat;     // materials; the id of design voxels in the words
     const uint32_t* matw;
@@ -324,9 +324,13 @@ __global__ void __launch_bounds__(256) k_words(const uint32_t* __restrict__ give
         slots += seg_poles(code);
     }
     for (int o = 32; o > 0; o >>= 1) poles += __shfl_down(poles, o, 64);
-    if (lane == 0 && poles > 0) {
-        atomicAdd(count, slots);
-        atomicAdd(count + 1, poles);
+    __shared__ unsigned long long sums[4][2];
+    if (lane == 0) sums[threadIdx.x >> 6][0] = slots, sums[threadIdx.x >> 6][1] = poles;
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        unsigned long long t = 0;
+        for (int w = 0; w < 4; ++w) t += sums[w][threadIdx.x];
+        if (t) atomicAdd(count + threadIdx.x, t);
     }
 }
 
@@ -403,6 +407,7 @@ __device__ __forceinline__ void step_tile(const StepArgs<T>& a, const int t) {
     if (threadIdx.x < 2 * TY) sh[threadIdx.x * (B + 1) + B] = Pair{T(0), T(0)};
 
     const long step = *(CONST const long*)a.d_step;
+    if (t == 0 && threadIdx.x == 0) a.d_step[1] = step;  // for the kernels after this one
     const bool odd = (step & 1) != 0;
     const char* F0 = (const char*)a.F[odd ? 1 : 0];
     const long F01 = (const char*)a.F[odd ? 0 : 1] - F0;  // from the set read to the set written
@@ -932,6 +937,7 @@ __device__ __forceinline__ void step_rows(const StepArgs<T>& a, const int t) {
     copy_lut(a, slut);
 
     const long step = *(CONST const long*)a.d_step;
+    if (t == 0 && threadIdx.x == 0) a.d_step[1] = step;  // for the kernels after this one
     const bool odd = (step & 1) != 0;
     const char* F0 = (const char*)a.F[odd ? 1 : 0];
     const long F01 = (const char*)a.F[odd ? 0 : 1] - F0;  // from the set read to the set written
@@ -1423,55 +1429,27 @@ __global__ void k_read_point(const T* __restrict__ F, const GatherPoint g, doubl
 }
 
 // ---- per-step scalars live on the device --------------------------------------------------
-// Every engine owns a device step counter.  Kernels read the step from it (which also fixes
-// the read/write field buffer by its parity) and the last kernel of a step increments it, so a
-// sequence of steps can be captured once in a hipGraph and replayed at any step.
+// Every engine owns a device step counter and its shadow (d_step[0], d_step[1]), so a sequence of steps
+// can be captured once in a hipGraph and replayed at any step.  The kernels up to the fused update
+// read the counter, which also fixes the read/write field buffer by its parity; the fused update's
+// first tile copies it to the shadow, which the source and DFT kernels after it read, and the
+// first workgroup of a step's last kernel sets the counter to shadow + 1: no kernel writes a word
+// that one of its workgroups reads, and no workgroup has to know that the others are done, or signs off
+// on a shared word.
 
 __global__ void k_tick(long* const* counters, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) counters[i][0] += 1;
 }
 
-// The same, folded into the DFT kernel when a step has one (one launch fewer): each workgroup
-// signs off after all of its threads have finished (and so have read the counters); the last
-// one to sign off advances every counter.  Sign-offs go to eight group words (workgroup index
-// mod 8) and the last of each group signs off on a top word, so no word takes more than an
-// eighth of the atomics; the words re-arm themselves for the next step.  Each word has a
-// 256-byte slot of its own: atomics on one cache line are served one after another, and with
-// the eight words in one line a launch of 1300 workgroups spent ~10 us signing off.  No fence
-// is needed: no workgroup reads what another writes within the kernel (the counters were read
-// before signing off, and the kernel boundary publishes the increment).
-// `done` == nullptr: the step ends with k_tick instead.
-constexpr int kDoneStride = 64;  // unsigned words per sign-off slot (256 bytes)
-constexpr int kDoneWords = 9 * kDoneStride;
-
+// The same, in the first workgroup of the step's last kernel (n = 0: not the last)
 struct Tick {
     long* const* counters;
     int n;
-    unsigned* done;  // kDoneWords: top word at [0], group g at [(1 + g) * kDoneStride]
 };
-
-__device__ __forceinline__ void tick_tail(const Tick& tk) {
-    if (!tk.done) return;
-    __shared__ int last;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const unsigned nblk = gridDim.x * gridDim.y * gridDim.z;
-        const unsigned b = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
-        const unsigned G = nblk < 8u ? nblk : 8u;
-        const unsigned g = b % G;
-        const unsigned members = (nblk - g + G - 1) / G;  // workgroups of group g
-        bool fin = atomicAdd(tk.done + (1 + g) * kDoneStride, 1u) == members - 1;
-        if (fin) {
-            atomicExch(tk.done + (1 + g) * kDoneStride, 0u);
-            fin = atomicAdd(tk.done, 1u) == G - 1;
-            if (fin) atomicExch(tk.done, 0u);
-        }
-        last = fin ? 1 : 0;
-    }
-    __syncthreads();
-    if (last)
-        for (int i = threadIdx.x; i < tk.n; i += blockDim.x) tk.counters[i][0] += 1;
+__device__ __forceinline__ void advance(const Tick& tk) {
+    if (blockIdx.x == 0)
+        for (int i = threadIdx.x; i < tk.n; i += blockDim.x) tk.counters[i][0] = tk.counters[i][1] + 1;
 }
 
 // ---- source time functions (FP64) ---------------------------------------------------------
@@ -1545,7 +1523,7 @@ template <typename T>
 struct SrcDev {
     PulseDev p;
     T* F[2];             // field set 0 / 1 (entries hold layout indices of the source component)
-    const long* d_step;  // the owning engine's step counter
+    const long* d_step;  // the owning engine's step counter and its shadow
 };
 
 // the tables of the source launch: per workgroup its source and range of entries; per entry
@@ -1566,7 +1544,7 @@ __device__ __forceinline__ void source_block(const SrcTables<T>& t, const int bl
     __shared__ double J;
     const int sid = t.blk_src[blk];
     const SrcDev<T>& S = t.src[sid];
-    const long step = *S.d_step;
+    const long step = S.d_step[1];
     if (threadIdx.x == 0) J = source_current(S.p, step);
     __syncthreads();
     const long e = t.blk_first[blk] + threadIdx.x;
@@ -1600,7 +1578,7 @@ __global__ void __launch_bounds__(256) k_source_h(const SrcTables<T> t) {
 template <typename T>
 __global__ void __launch_bounds__(256) k_source(const SrcTables<T> t, const Tick tk) {
     source_block(t, blockIdx.x);
-    tick_tail(tk);
+    advance(tk);
 }
 
 // ---- point monitors: trilinear gather, FP64 result --------------------------------------
@@ -1642,7 +1620,7 @@ __device__ __forceinline__ void neumaier(double& s, double& c, double x) {
 template <typename T>
 struct DftDev {
     const T* F[2];       // field set 0 / 1 base, [x][6][y][z]
-    const long* d_step;  // owning engine's counter
+    const long* d_step;  // owning engine's counter and its shadow
     long N, nyz, nz;
     int lo[3], ext[3];
     long ncell;
@@ -1656,81 +1634,83 @@ struct DftDev {
     double2* cmp;        // compensation terms, same layout
 };
 
-// accumulation of one (component, cell, frequency) of region ri
+// One thread per (component, cell, frequency): workgroup b takes frequency b / dftx and 256 (component,
+// cell) pairs.  Bound by the latency of a thread's chain on small regions and by memory (an accumulator
+// and its compensation, 32 bytes read and written) on large ones: the loads are issued before the
+// phase is formed, the phase is one FP64 sincos (of the component's own time level), and indices
+// are split with 32-bit divisions where the launch's pairs allow it.  Several accumulators per thread
+// shared the sincos but left too few loads in flight (102 us in the case below).  Measured on MI355X,
+// two planes of 150 x 150 cells, 4 components, 20 frequencies (3.6 M accumulators, 230 MB): with two
+// sincos each, 64-bit divisions and a sign-off per workgroup 85 us, now 75; 96 x 96 cells, 5 frequencies
+// in FP64 7.9, 7.0.
+template <typename T, typename I>
+__device__ __forceinline__ void dft_cell(const DftDev<T>& a, const long g, const int f) {
+    if (f >= a.nf) return;
+    const I local = (I)(g - a.first), ncell = (I)a.ncell;
+    const int s = (int)(local / ncell);  // component slot
+    const I cell = local - (I)s * ncell;
+    const I rest = cell / (I)a.ext[2];
+    const int kk = (int)(cell - rest * (I)a.ext[2]);
+    const int ii = (int)(rest / (I)a.ext[1]);
+    const int jj = (int)(rest - (I)ii * (I)a.ext[1]);
+    const int c = a.comps[s];
+    const long step = a.d_step[1];
+    const long o = ((long)s * a.nf + f) * a.ncell + (long)cell;
+    double2 sm = a.acc[o], cp = a.cmp[o];
+    // component c of cell (lo + (ii, jj, kk)) in the layout [x][6][y][z]
+    const double v = (double)a.F[(step + 1) & 1][(6L * (a.lo[0] + ii) + c) * a.nyz + (long)(a.lo[1] + jj) * a.nz +
+                                                 (a.lo[2] + kk)] * a.dt;
+    // phase at the time level of E, t = (n+1) dt, or of H, (n+1/2) dt
+    double co, si;
+    sincos(2 * M_PI * a.freq[f] * (c < 3 ? (step + 1) * a.dt : (step + 0.5) * a.dt), &si, &co);
+    neumaier(sm.x, cp.x, v * co);
+    neumaier(sm.y, cp.y, v * si);
+    a.acc[o] = sm;
+    a.cmp[o] = cp;
+}
+// the region of pair g
 template <typename T>
-__device__ __forceinline__ void dft_cell(const DftDev<T>* __restrict__ regs, int ri, int f, long g);
-
-// One thread per (component, cell, frequency): blockIdx.y is the frequency index, and the
-// threads of a region run over its components' cells one component after another.  The phase
-// factors depend only on the step and the frequency; each thread evaluates them itself (two
-// FP64 sincos), which measured faster than one thread per block sharing them through LDS
-// behind a barrier.
+__device__ __forceinline__ int dft_region(const DftDev<T>* __restrict__ regs, const int nreg, const long g) {
+    int ri = 0;
+    for (int hi = nreg - 1; ri < hi;) {  // region with first <= g
+        const int mid = (ri + hi + 1) / 2;
+        if (regs[mid].first <= g) ri = mid;
+        else hi = mid - 1;
+    }
+    return ri;
+}
 template <typename T>
 __device__ __forceinline__ void dft_block(const DftDev<T>* __restrict__ regs, const int nreg, const long total,
-                                          const int bx, const int f) {
-    const long g = (long)bx * blockDim.x + threadIdx.x;
-    auto region_of = [&](long x) {
-        int lo = 0, hi = nreg - 1;
-        while (lo < hi) {  // region with first <= x
-            const int mid = (lo + hi + 1) / 2;
-            if (regs[mid].first <= x) lo = mid;
-            else hi = mid - 1;
-        }
-        return lo;
-    };
-    if (g < total) dft_cell(regs, region_of(g), f, g);
+                                          const int dftx, const int b) {
+    const int f = b / dftx;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const long g0 = (long)(b - f * dftx) * 256 + wave * 64, g = g0 + (threadIdx.x & 63);
+    if (g0 >= total) return;
+    // a wavefront within one region reads its description as scalars
+    const int ri = dft_region(regs, nreg, g0);
+    if (g0 + 63 < (ri + 1 < nreg ? regs[ri + 1].first : total)) {
+        if (total < 0x7fffffff) dft_cell<T, uint32_t>(regs[ri], g, f);
+        else dft_cell<T, long>(regs[ri], g, f);
+    } else if (g < total) {
+        dft_cell<T, long>(regs[dft_region(regs, nreg, g)], g, f);
+    }
 }
 
 template <typename T>
-__global__ void __launch_bounds__(256) k_dft(const DftDev<T>* __restrict__ regs, int nreg, long total, const Tick tk) {
-    dft_block(regs, nreg, total, blockIdx.x, blockIdx.y);
-    tick_tail(tk);
+__global__ void __launch_bounds__(256) k_dft(const DftDev<T>* __restrict__ regs, int nreg, long total, int dftx, const Tick tk) {
+    dft_block(regs, nreg, total, dftx, blockIdx.x);
+    advance(tk);
 }
 
 // Source injection and DFT in one launch, for steps whose DFT regions hold no source cell (so
-// neither part reads what the other writes): workgroups [0, nsrc) inject, the rest accumulate
-// (dftx workgroups per frequency); the last workgroup advances the step counters.
+// neither part reads what the other writes): workgroups [0, nsrc) inject, the rest accumulate.
 template <typename T>
 __global__ void __launch_bounds__(256) k_source_dft(const SrcTables<T> t, int nsrc, const DftDev<T>* __restrict__ regs,
                                                     int nreg, long total, int dftx, const Tick tk) {
     const int b = blockIdx.x;
-    if (b < nsrc) {
-        source_block(t, b);
-    } else {
-        const int d = b - nsrc;
-        dft_block(regs, nreg, total, d % dftx, d / dftx);
-    }
-    tick_tail(tk);
-}
-
-template <typename T>
-__device__ __forceinline__ void dft_cell(const DftDev<T>* __restrict__ regs, const int ri, const int f, const long g) {
-    const DftDev<T>& a = regs[ri];
-    if (f >= a.nf) return;
-    const long local = g - a.first;
-    const int s = (int)(local / a.ncell);  // component slot
-    const long cell = local - (long)s * a.ncell;
-    const long step = *a.d_step;
-    const T* F = a.F[(step + 1) & 1];
-    const int kk = (int)(cell % a.ext[2]);
-    const long rest = cell / a.ext[2];
-    const int jj = (int)(rest % a.ext[1]);
-    const int ii = (int)(rest / a.ext[1]);
-    const long q = (long)(a.lo[0] + ii) * a.nyz + (long)(a.lo[1] + jj) * a.nz + (a.lo[2] + kk);
-    // phases of this thread's frequency at the E and H time levels, t = (n+1) dt and (n+1/2) dt
-    // (each thread forms its own: no serial set-up ahead of the loads)
-    double cE, sE, cH, sH;
-    const double w = 2 * M_PI * a.freq[f];
-    sincos(w * ((step + 1) * a.dt), &sE, &cE);
-    sincos(w * ((step + 0.5) * a.dt), &sH, &cH);
-    const int c = a.comps[s];
-    const double v = (double)F[field_index(q, c, a.nyz)] * a.dt;
-    const long o = ((long)s * a.nf + f) * a.ncell + cell;
-    double2 sm = a.acc[o], cp = a.cmp[o];
-    neumaier(sm.x, cp.x, v * (c < 3 ? cE : cH));
-    neumaier(sm.y, cp.y, v * (c < 3 ? sE : sH));
-    a.acc[o] = sm;
-    a.cmp[o] = cp;
+    if (b < nsrc) source_block(t, b);
+    else dft_block(regs, nreg, total, dftx, b - nsrc);
+    advance(tk);
 }
 
 // ---- flux through a DFT plane ------------------------------------------------------------
@@ -1801,9 +1781,9 @@ __global__ void __launch_bounds__(64) k_dft_flux_sum(const double* __restrict__ 
 // This has the dependency pattern of the forward step (phase 1 uses forward differences,
 // phase 2 backward ones), so the same tilings apply: rows of threads (adj_rows), or a workgroup that
 // spans a z line, each thread one y row plus a halo row below it where phase 1 is recomputed, z
-// neighbours through LDS (adj_tile); the tile marches along x carrying u of the next planes.  Adjoint fields and E auxiliary
-// bars are double-buffered (neighbouring workgroups read the old values of the halo row);
-// Qbar and Pbar are only touched by their owner and are updated in place.
+// neighbours through LDS (adj_tile); the tile marches along x carrying u of the next planes.  Adjoint
+// fields and E auxiliary bars are double-buffered (neighbouring workgroups read the old values of the
+// halo row); Qbar and Pbar are only touched by their owner and are updated in place.
 
 template <typename T>
 struct AdjArgs {
@@ -1982,7 +1962,7 @@ __device__ __forceinline__ void adj_tile(const AdjArgs<T>& g, const int t) {
         // E-terms on rows r = 0, 1 (labels: y (Ex->Hz), z (Ex->Hy), z (Ey->Hx), x (Ey->Hz),
         // x (Ez->Hy), y (Ez->Hx)) and the y-terms of row 2
         T eb[3][6];
-        Pair pey = Pair{T(0), T(0)}, pex = Pair{T(0), T(0)};  // owned row's y and x E aux bars
+        // (the new E auxiliary bars of the owned row are stored as soon as its terms are formed)
 #pragma unroll
         for (int r = 0; r < 3; ++r) {
             const bool ok = rv[r];
@@ -1996,10 +1976,14 @@ __device__ __forceinline__ void adj_tile(const AdjArgs<T>& g, const int t) {
                 const Pair q = bld2<T>(rpy, oK, er * SB1 + so);
                 t_ex_y = adj_term(b, t_ex_y, q.x);
                 t_ez_y = adj_term(b, t_ez_y, q.y);
-                if (r == 1) pey = q;
+                if (r == 1 && wr)  // (Ex, y, +, slot 0), (Ez, y, -, slot 1)
+                    bst2<NTS>(rpy, oK, ew * SB1 + so, Pair{b * (cdt * ux + q.x), b * (-cdt * uz + q.y)});
             }
             if (r < 2) {
                 if (ok && zany) {
+                    if (r == 1 && wr)  // (Ex, z, -, slot 0), (Ey, z, +, slot 1)
+                        bst2<NTS>(rpz, oZ, ew * SB2 + (uint32_t)((pi * ny + j) * Lz) * 2u * TS,
+                                  Pair{bEz * (-cdt * ux + pzE[1].x), bEz * (cdt * uy + pzE[1].y)});
                     t_ex_z = adj_term(bEz, t_ex_z, pzE[r].x);
                     t_ey_z = adj_term(bEz, t_ey_z, pzE[r].y);
                 }
@@ -2007,7 +1991,8 @@ __device__ __forceinline__ void adj_tile(const AdjArgs<T>& g, const int t) {
                     const Pair q = bld2<T>(rpx, two(oR[r]), er * SB0 + sxo);
                     t_ey_x = adj_term(bEx, t_ey_x, q.x);
                     t_ez_x = adj_term(bEx, t_ez_x, q.y);
-                    if (r == 1) pex = q;
+                    if (r == 1 && wr)  // (Ey, x, -, slot 0), (Ez, x, +, slot 1)
+                        bst2<NTS>(rpx, two(oR[1]), ew * SB0 + sxo, Pair{bEx * (-cdt * uy + q.x), bEx * (cdt * uz + q.y)});
                 }
             }
             eb[r][0] = t_ex_y;
@@ -2151,19 +2136,6 @@ __device__ __forceinline__ void adj_tile(const AdjArgs<T>& g, const int t) {
                             sq[c] = fma_(L.pole[s].c3, qb, sq[c]);
                         }
                     }
-                }
-                // new E auxiliary bars: E-terms of row 0 with their signs
-                if (ypml[1]) {  // (Ex, y, +, slot 0), (Ez, y, -, slot 1)
-                    const T b = cy[j];
-                    const uint32_t so = (uint32_t)((pi * Ly + sy[1]) * nz) * 2u * TS;
-                    bst2<NTS>(rpy, oK, ew * SB1 + so, Pair{b * (cdt * u0[0] + pey.x), b * (-cdt * u0[2] + pey.y)});
-                }
-                if (zany) {  // (Ex, z, -, slot 0), (Ey, z, +, slot 1)
-                    const uint32_t so = (uint32_t)((pi * ny + j) * Lz) * 2u * TS;
-                    bst2<NTS>(rpz, oZ, ew * SB2 + so, Pair{bEz * (-cdt * u0[0] + pzE[1].x), bEz * (cdt * u0[1] + pzE[1].y)});
-                }
-                if (xpml) {  // (Ey, x, -, slot 0), (Ez, x, +, slot 1)
-                    bst2<NTS>(rpx, two(o), ew * SB0 + sxo, Pair{bEx * (-cdt * u0[1] + pex.x), bEx * (cdt * u0[2] + pex.y)});
                 }
                 // the state is Ubar = Ebar / eps: the differences and the pole terms add 1/eps of their sum
 #pragma unroll
@@ -2566,11 +2538,23 @@ k_adj_step(const AdjArgs<T> g) {
     adj_tile<T, NP, NTS>(g, t);
 }
 
-// record E of the design box and of the objective cell into slot `slot` of a ring buffer
+// objective J += dt * sum_c E_c(gap)^2 for the state after a step (FP64)
+template <typename T>
+__device__ __forceinline__ void add_objective(const T* E, long nyz, long gap, double dt, double* J) {
+    double s = 0;
+    for (int c = 0; c < 3; ++c) {
+        const double v = (double)E[field_index(gap, c, nyz)];
+        s += v * v;
+    }
+    *J += s * dt;
+}
+
+// record E of the design box and of the objective cell into slot `slot` of a ring buffer; with J, the
+// thread of the objective cell's first component adds the objective
 template <typename T>
 __global__ void __launch_bounds__(256) k_adj_record(const T* E, long nyz, int ny, int nz, int dlo0, int dlo1,
                                                     int dlo2, int de0, int de1, int de2, long gap,
-                                                    T* ring, long slot) {
+                                                    T* ring, long slot, double dt, double* J) {
     const long nd = (long)de0 * de1 * de2;
     const long v = (long)blockIdx.x * blockDim.x + threadIdx.x;
     T* out = ring + slot * (3 * nd + 3);
@@ -2584,20 +2568,13 @@ __global__ void __launch_bounds__(256) k_adj_record(const T* E, long nyz, int ny
     } else if (v < nd + 3) {
         const int c = (int)(v - nd);
         out[3 * nd + c] = E[field_index(gap, c, nyz)];
+        if (J && c == 0) add_objective(E, nyz, gap, dt, J);
     }
 }
 
-// objective J += dt * sum_c E_c(gap)^2 for the state after a step (FP64)
 template <typename T>
 __global__ void k_adj_objective(const T* E, long nyz, long gap, double dt, double* J) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        double s = 0;
-        for (int c = 0; c < 3; ++c) {
-            const double v = (double)E[field_index(gap, c, nyz)];
-            s += v * v;
-        }
-        *J += s * dt;
-    }
+    if (threadIdx.x == 0 && blockIdx.x == 0) add_objective(E, nyz, gap, dt, J);
 }
 
 // gradient term of step n:
@@ -2679,14 +2656,7 @@ __global__ void __launch_bounds__(256) k_adj_record_batch(const AdjBatchDev<T>* 
     } else {
         const int c = (int)(v - nd);
         out[3 * nd + c] = E[field_index(a.gap, c, a.nyz)];
-        if (objective && c == 0) {
-            double sum = 0;
-            for (int k = 0; k < 3; ++k) {
-                const double x = (double)E[field_index(a.gap, k, a.nyz)];
-                sum += x * x;
-            }
-            *a.J += sum * a.dt;
-        }
+        if (objective && c == 0) add_objective(E, a.nyz, a.gap, a.dt, a.J);
     }
 }
 
