@@ -24,8 +24,8 @@ XCHUNKS = (4, 6, 8, 10, 12, 16, 20, 24, 32, 48, 64)
 
 
 def candidates(shape, xchunks=XCHUNKS):
-    """(form, rows, xchunk, zseg) tuples worth timing for a grid shape; zseg 0 is the engine's
-    default z passes, other values a z pass length of one-row register tiles (lines of 512 cells
+    """(form, rows, xchunk, zseg) tuples worth timing for a grid shape; zseg 0 is the
+    default z passes of a set tile, other values a z pass length of one-row register tiles (lines of 512 cells
     or more: 128- and 256-cell passes and one pass over the line)."""
     nx, ny, nz = shape
     out = []

@@ -1825,8 +1825,9 @@ int batch_adjoint_run_t(LaunchSet* s, long nsteps, long K, const long* gaps, con
     std::vector<int> first;
     int t = 0, nmat = 1;
     long maxv = 0, rows = 0;
-    // one row per workgroup with x-chunks common to all engines, or, when the first engine's tile
-    // was set to the row-of-threads form, its rows (at most each engine's ny) and its x-chunk
+    // rows of threads where the batch takes them (adj_tile_of), each engine its default rows; else one
+    // row per workgroup with x-chunks common to all engines; a tile set on the first engine holds for
+    // all (its rows at most each engine's ny, its x-chunk)
     double bytes = 0;
     for (const sjf_engine* e : s->eng) {
         rows += e->g.ny;
