@@ -281,7 +281,7 @@ int read_stage(sjf_engine* e, size_t bytes) {
 int words_at(sjf_engine* e, const std::vector<long>& cells, std::vector<uint32_t>& w) {
     const long n = (long)cells.size(), most = (long)(kReadChunk / 16);
     w.assign(n, 0u);
-    if (!e->have_mat) return SJF_OK;
+    if (!e->matw) return SJF_OK;  // no materials yet, or refused ones
     for (long q = 0; q < n; q += most) {
         const long m = std::min(most, n - q);
         if (int rc = read_stage(e, 16 * (size_t)m)) return rc;
@@ -540,6 +540,8 @@ int build_set_t(LaunchSet* s) {
     int t = 0;
     size_t zh = 0;  // register form with z passes: values of the pass halo in LDS
     for (sjf_engine* e : s->eng) {
+        if (e->maxp > 0 && (!e->Qbuf || (e->prec == 4 && !e->Pbuf)))  // its allocation failed earlier
+            return fail(e0, SJF_E_NOMEM, "polarisation state is not allocated");
         // the engine's own set runs its tuned rows; a batch picks rows per engine for its form
         const int rows = (s == e->own) ? e->ty
                                        : (s->form == SJF_TILE_THREAD_ROWS ? default_thread_rows(e) : s->ty);
