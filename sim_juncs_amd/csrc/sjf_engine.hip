@@ -478,7 +478,8 @@ struct LaunchSet {
     void* d_dft = nullptr;
     int ndft = 0;
     long dft_total = 0;
-    int dft_maxnf = 0;  // most frequencies of any region (the launch's second dimension)
+    int dft_blocks = 0;  // workgroups of one frequency
+    int dft_maxnf = 0;   // most frequencies of any region (the launch's second dimension)
     bool src_dft_one_launch = false;  // no DFT region holds a source cell: one launch for both
     // step counters, which the last kernel of a step advances
     long** d_counters = nullptr;
@@ -705,6 +706,12 @@ int build_set_t(LaunchSet* s) {
     }
     s->dft_maxnf = 0;
     for (const auto& r : regs) s->dft_maxnf = std::max(s->dft_maxnf, r.nf);
+    // a grid dimension holds less than 2^32 threads
+    constexpr long most = (1L << 24) - 1;  // workgroups of 256 threads
+    const long per_freq = (tot + 255) / 256;
+    if (per_freq > most) return fail(e0, SJF_E_UNSUPPORTED, "DFT regions exceed 2^32 values per frequency");
+    s->dft_blocks = (int)per_freq;
+    if (s->nsrcblk + per_freq * s->dft_maxnf > most) s->src_dft_one_launch = false;
     if (s->ndft) {
         rc = upload_vec(e0, s->stream, &s->d_dft, regs);
         if (rc) return rc;
@@ -815,11 +822,10 @@ int launch_one_step_t(LaunchSet* s, bool sample, hipEvent_t ev_a, hipEvent_t ev_
     const sjf::SrcTables<T> st{(const sjf::SrcDev<T>*)s->d_src, s->d_blk_src, s->d_blk_first, s->d_blk_end,
                                s->d_src_idx, s->d_src_coef};
     const sjf::Tick tick{s->d_counters, n};
-    const int dftx = (int)((s->dft_total + 255) / 256);
-    const unsigned ndb = (unsigned)(dftx * s->dft_maxnf);
     if (dft && s->src_dft_one_launch) {
-        hipLaunchKernelGGL((sjf::k_source_dft<T>), dim3(s->nsrcblk + ndb), dim3(256), 0, s->stream, st, s->nsrcblk,
-                           (const sjf::DftDev<T>*)s->d_dft, s->ndft, s->dft_total, dftx, tick);
+        hipLaunchKernelGGL((sjf::k_source_dft<T>), dim3((unsigned)(s->nsrcblk + s->dft_blocks * s->dft_maxnf)), dim3(256), 0,
+                           s->stream, st, s->nsrcblk, (const sjf::DftDev<T>*)s->d_dft, s->ndft, s->dft_total,
+                           s->dft_blocks, tick);
         SETCHK(s, hipGetLastError());
         return SJF_OK;
     }
@@ -829,8 +835,8 @@ int launch_one_step_t(LaunchSet* s, bool sample, hipEvent_t ev_a, hipEvent_t ev_
         SETCHK(s, hipGetLastError());
     }
     if (dft) {
-        hipLaunchKernelGGL((sjf::k_dft<T>), dim3(ndb), dim3(256), 0, s->stream, (const sjf::DftDev<T>*)s->d_dft, s->ndft,
-                           s->dft_total, dftx, tick);
+        hipLaunchKernelGGL((sjf::k_dft<T>), dim3((unsigned)s->dft_blocks, (unsigned)s->dft_maxnf), dim3(256), 0, s->stream,
+                           (const sjf::DftDev<T>*)s->d_dft, s->ndft, s->dft_total, tick);
         SETCHK(s, hipGetLastError());
     } else if (!s->nsrcblk) {
         hipLaunchKernelGGL(sjf::k_tick, dim3((n + 63) / 64), dim3(64), 0, s->stream, s->d_counters, n);

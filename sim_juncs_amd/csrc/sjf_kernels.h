@@ -1448,7 +1448,7 @@ struct Tick {
     int n;
 };
 __device__ __forceinline__ void advance(const Tick& tk) {
-    if (blockIdx.x == 0)
+    if (blockIdx.x == 0 && blockIdx.y == 0)
         for (int i = threadIdx.x; i < tk.n; i += blockDim.x) tk.counters[i][0] = tk.counters[i][1] + 1;
 }
 
@@ -1634,7 +1634,7 @@ struct DftDev {
     double2* cmp;        // compensation terms, same layout
 };
 
-// One thread per (component, cell, frequency): workgroup b takes frequency b / dftx and 256 (component,
+// One thread per (component, cell, frequency): a workgroup takes one frequency and 256 (component,
 // cell) pairs.  Bound by the latency of a thread's chain on small regions and by memory (an accumulator
 // and its compensation, 32 bytes read and written) on large ones: the loads are issued before the
 // phase is formed, the phase is one FP64 sincos (of the component's own time level), and indices
@@ -1681,10 +1681,9 @@ __device__ __forceinline__ int dft_region(const DftDev<T>* __restrict__ regs, co
 }
 template <typename T>
 __device__ __forceinline__ void dft_block(const DftDev<T>* __restrict__ regs, const int nreg, const long total,
-                                          const int dftx, const int b) {
-    const int f = b / dftx;
+                                          const int bx, const int f) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const long g0 = (long)(b - f * dftx) * 256 + wave * 64, g = g0 + (threadIdx.x & 63);
+    const long g0 = (long)bx * 256 + wave * 64, g = g0 + (threadIdx.x & 63);
     if (g0 >= total) return;
     // a wavefront within one region reads its description as scalars
     const int ri = dft_region(regs, nreg, g0);
@@ -1696,20 +1695,27 @@ __device__ __forceinline__ void dft_block(const DftDev<T>* __restrict__ regs, co
     }
 }
 
+// (the frequency is the grid's y: regions of many pairs beside one of many frequencies have more threads
+// than HIP takes along one dimension)
 template <typename T>
-__global__ void __launch_bounds__(256) k_dft(const DftDev<T>* __restrict__ regs, int nreg, long total, int dftx, const Tick tk) {
-    dft_block(regs, nreg, total, dftx, blockIdx.x);
+__global__ void __launch_bounds__(256) k_dft(const DftDev<T>* __restrict__ regs, int nreg, long total, const Tick tk) {
+    dft_block(regs, nreg, total, blockIdx.x, blockIdx.y);
     advance(tk);
 }
 
 // Source injection and DFT in one launch, for steps whose DFT regions hold no source cell (so
-// neither part reads what the other writes): workgroups [0, nsrc) inject, the rest accumulate.
+// neither part reads what the other writes): workgroups [0, nsrc) inject, the rest accumulate (dftx per
+// frequency; a launch too large for one grid dimension goes out as two).
 template <typename T>
 __global__ void __launch_bounds__(256) k_source_dft(const SrcTables<T> t, int nsrc, const DftDev<T>* __restrict__ regs,
                                                     int nreg, long total, int dftx, const Tick tk) {
     const int b = blockIdx.x;
-    if (b < nsrc) source_block(t, b);
-    else dft_block(regs, nreg, total, dftx, b - nsrc);
+    if (b < nsrc) {
+        source_block(t, b);
+    } else {
+        const int f = (b - nsrc) / dftx;
+        dft_block(regs, nreg, total, b - nsrc - f * dftx, f);
+    }
     advance(tk);
 }
 

@@ -1,0 +1,84 @@
+"""What the engine's host code allocates and launches, on the CPU: libsjf runs against
+tests/host/fake_hip.cpp, a stand-in for the HIP runtime that records launches (no kernel runs),
+knows which memory is live and can fail a chosen allocation.  Each case runs in a process of its
+own, since the stand-in has to be loaded before libsjf.
+"""
+import ctypes as C
+import os
+import shutil
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+
+@pytest.fixture(scope="module")
+def fake_path(tmp_path_factory):
+    if shutil.which("g++") is None:
+        pytest.skip("no host compiler")
+    out = str(tmp_path_factory.mktemp("fake_hip") / "fake_hip.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", os.path.join(HERE, "host", "fake_hip.cpp"), "-o", out],
+                   check=True, capture_output=True, text=True)
+    return out
+
+
+def run_case(fake, name, *args):
+    r = subprocess.run([sys.executable, os.path.abspath(__file__), fake, name, *map(str, args)], cwd=ROOT,
+                       capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stdout[-3000:] + r.stderr[-3000:]
+
+
+class Fake:
+    def __init__(self, path):
+        self.lib = C.CDLL(path, mode=C.RTLD_GLOBAL)
+        for f, res in (("fake_log", C.c_char_p), ("fake_last_kernel", C.c_char_p), ("fake_live_bytes", C.c_double),
+                       ("fake_steps", C.c_long), ("fake_refused", C.c_long), ("fake_allocations", C.c_long),
+                       ("fake_last_table", C.c_size_t)):
+            getattr(self.lib, f).restype = res
+        self.lib.fake_fail_at.argtypes = [C.c_long]
+        self.lib.fake_last_table.argtypes = [C.c_char_p, C.c_size_t]
+
+    def __getattr__(self, name):
+        return getattr(self.lib, "fake_" + name)
+
+    def table(self):
+        """The argument table of the last fused step."""
+        buf = C.create_string_buffer(self.lib.fake_last_table(None, 0))
+        self.lib.fake_last_table(buf, len(buf))
+        return buf.raw
+
+
+# ---- DFT launches -------------------------------------------------------------------------------
+
+def case_dft_launch(fake, source):
+    """Many (component, cell) pairs at one frequency beside one cell at 64: more threads than one grid
+    dimension takes, whether or not the source could share the launch."""
+    from sim_juncs_amd.engine import Engine
+
+    n = 236
+    e = Engine((n, n, n), 0.01)
+    at = 0.01 * (n // 2 if source == "inside" else 1)
+    e.add_source("Ex", [at - 0.005, at, at] * 2, freq=1.0, width=1.0, t_end=10.0)
+    e.add_dft((8, 8, 8), (n, n, n), ("Ex", "Ey", "Ez", "Hx", "Hy", "Hz"), [1.0])
+    e.add_dft((6, 6, 6), (7, 7, 7), ("Ex",), np.linspace(0.5, 1.5, 64))
+    pairs = 6 * (n - 8) ** 3 + 1
+    assert pairs * 64 >= 2 ** 32
+    e.step(2)
+    assert fake.refused() == 0 and fake.steps() == 2
+    log = [line for line in fake.log().decode().split("\n") if "k_dft<" in line or "k_source_dft<" in line]
+    assert len(log) == 2 and all("k_dft<" in line for line in log), log
+    assert all(f" {-(-pairs // 256)} 64 1 x 256" in line for line in log), log
+
+
+@pytest.mark.parametrize("source", ["inside", "outside"])
+def test_dft_of_many_values_and_many_frequencies_is_launched(fake_path, source):
+    run_case(fake_path, "dft_launch", source)
+
+
+if __name__ == "__main__":
+    sys.path.insert(0, ROOT)
+    globals()["case_" + sys.argv[2]](Fake(sys.argv[1]), *sys.argv[3:])
