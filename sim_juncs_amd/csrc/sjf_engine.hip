@@ -152,9 +152,17 @@ int fail(sjf_engine* e, int code, const std::string& m) {
     return code;
 }
 
+// A failed allocation is reported by its own call alone: the error it leaves behind would otherwise be
+// taken for that of the next launch, and a step that has run be reported as failed.
+hipError_t device_malloc(void** p, size_t bytes) {
+    const hipError_t st = hipMalloc(p, bytes);
+    if (st != hipSuccess) (void)hipGetLastError();
+    return st;
+}
+
 int dev_alloc(sjf_engine* e, void** p, size_t bytes) {
     if (*p) return SJF_OK;
-    hipError_t st = hipMalloc(p, bytes ? bytes : 16);
+    hipError_t st = device_malloc(p, bytes ? bytes : 16);
     if (st != hipSuccess) {
         *p = nullptr;
         e->err = std::string("hipMalloc(") + std::to_string(bytes) + "): " + hipGetErrorString(st);
@@ -519,7 +527,7 @@ void set_free_tables(LaunchSet* s) {
 template <typename V>
 int upload_vec(sjf_engine* e, hipStream_t st, void** dst, const std::vector<V>& v) {
     const size_t bytes = sizeof(V) * std::max<size_t>(v.size(), 1);
-    hipError_t rc = hipMalloc(dst, bytes);
+    hipError_t rc = device_malloc(dst, bytes);
     if (rc != hipSuccess) return fail(e, SJF_E_NOMEM, "launch table allocation failed");
     if (!v.empty()) {
         rc = hipMemcpyAsync(*dst, v.data(), sizeof(V) * v.size(), hipMemcpyHostToDevice, st);
@@ -870,7 +878,7 @@ int ensure_sample_capacity(sjf_engine* e, long need) {
     if (int rc = sync_engine(e)) return rc;
     const long cap = std::max(need, 2 * e->samp_cap);
     double* p = nullptr;
-    if (hipMalloc((void**)&p, sizeof(double) * cap * npt) != hipSuccess)
+    if (device_malloc((void**)&p, sizeof(double) * cap * npt) != hipSuccess)
         return fail(e, SJF_E_NOMEM, "sample buffer allocation failed");
     if (e->d_samples && e->nsamp > 0)
         HIPCHK(e, hipMemcpyAsync(p, e->d_samples, sizeof(double) * e->nsamp * npt, hipMemcpyDeviceToDevice,
@@ -1558,7 +1566,7 @@ int adjoint_run_t(sjf_engine* e, long nsteps, long K, long gap, double* J_out, d
     const long nck = rec_all ? 0 : (nsteps + K - 1) / K;
     const long nslots = rec_all ? nsteps + 1 : K + 1;
     char* cks = nullptr;
-    if (!rec_all && hipMalloc((void**)&cks, L.total * (nck + 1)) != hipSuccess)
+    if (!rec_all && device_malloc((void**)&cks, L.total * (nck + 1)) != hipSuccess)
         return fail(e, SJF_E_NOMEM, "checkpoint storage allocation failed (" +
                                         std::to_string((double)L.total * (nck + 1) / 1e9) + " GB)");
     double* dJ = nullptr;
@@ -3044,8 +3052,8 @@ int sjf_copy_probe(int device, size_t bytes, int iters, double* gbs) {
     if (hipSetDevice(device) != hipSuccess) return SJF_E_HIP;
     const long n = (long)(bytes / 16);
     float4 *a = nullptr, *b = nullptr;
-    if (hipMalloc((void**)&a, n * 16) != hipSuccess) return SJF_E_NOMEM;
-    if (hipMalloc((void**)&b, n * 16) != hipSuccess) {
+    if (device_malloc((void**)&a, n * 16) != hipSuccess) return SJF_E_NOMEM;
+    if (device_malloc((void**)&b, n * 16) != hipSuccess) {
         (void)hipFree(a);
         return SJF_E_NOMEM;
     }

@@ -79,6 +79,50 @@ def test_dft_of_many_values_and_many_frequencies_is_launched(fake_path, source):
     run_case(fake_path, "dft_launch", source)
 
 
+# ---- allocations that fail ----------------------------------------------------------------------
+
+SHAPE = (10, 9, 12)
+
+
+def case_failed_allocation(fake):
+    """A call that runs out of memory before it has changed anything fails alone: the next step runs
+    and is not reported as failed (its launches ask for the last error)."""
+    from sim_juncs_amd import materials as M
+    from sim_juncs_amd._lib import EngineError
+    from sim_juncs_amd.engine import Engine
+
+    words = np.zeros(SHAPE, np.uint32)
+    calls = {
+        "materials": lambda e: e.set_materials(words, [M.AU.scaled(1.0)]),
+        "dft": lambda e: e.add_dft((1, 1, 1), (3, 3, 3), ("Ex",), [1.0]),
+        "flux": lambda e: e.dft_flux(0, 2),
+        "monitors": lambda e: e.reserve_steps(100),
+        "adjoint": lambda e: e.adjoint_run(4, 2, (5, 4, 6), 8),
+    }
+    for name, call in calls.items():
+        with Engine(SHAPE, 0.02) as e:
+            if name == "flux":
+                e.add_dft((0, 0, 6), SHAPE[:2] + (7,), ("Ex", "Ey", "Hx", "Hy"), [1.0])
+            if name == "monitors":
+                e.add_monitors("Ex", [[0.1, 0.1, 0.1]])
+            if name == "adjoint":
+                e.set_design_eps((2, 2, 2), (4, 4, 4), np.full((2, 2, 2), 3.0))
+                e.reserve_steps(1)
+            else:
+                e.step(1)
+            fake.fail_at(0)
+            with pytest.raises(EngineError):
+                call(e)
+            fake.fail_at(-1)
+            before = fake.steps()
+            e.step(1)
+            assert fake.steps() == before + 1, name
+
+
+def test_a_failed_allocation_is_not_reported_by_the_next_step(fake_path):
+    run_case(fake_path, "failed_allocation")
+
+
 if __name__ == "__main__":
     sys.path.insert(0, ROOT)
     globals()["case_" + sys.argv[2]](Fake(sys.argv[1]), *sys.argv[3:])
