@@ -78,6 +78,7 @@ struct sjf_engine {
     // materials: given* as the caller set them; matw / lut_h / nmat / maxp are what the kernels run
     // (the given map, with Lorentz poles folded out of the PML slabs when pml_fref > 0: twin)
     bool have_mat = false;
+    bool mat_ready = true;  // false from the first change a call makes until it has made all of them
     uint32_t* given = nullptr;  // device, [x][y][z]
     std::vector<sjf_material> given_lut;
     double pml_fref = 0;
@@ -549,8 +550,7 @@ int build_set_t(LaunchSet* s) {
     int t = 0;
     size_t zh = 0;  // register form with z passes: values of the pass halo in LDS
     for (sjf_engine* e : s->eng) {
-        if (e->maxp > 0 && (!e->Qbuf || (e->prec == 4 && !e->Pbuf)))  // its allocation failed earlier
-            return fail(e0, SJF_E_NOMEM, "polarisation state is not allocated");
+        if (!e->mat_ready) return fail(e0, SJF_E_STATE, "the materials are incomplete: the call that last set them failed");
         // the engine's own set runs its tuned rows; a batch picks rows per engine for its form
         const int rows = (s == e->own) ? e->ty
                                        : (s->form == SJF_TILE_THREAD_ROWS ? default_thread_rows(e) : s->ty);
@@ -1267,47 +1267,81 @@ bool cell_in_pml(const sjf_engine* e, long q) {
     return false;
 }
 
-// The material map the kernels run: the given map, except that with pml_fref > 0 every cell inside
-// a PML slab whose material has Lorentz poles takes a twin of that material with them folded out
-// (their real susceptibility at pml_fref added to eps_inf when the sum stays >= 1, else eps_inf kept;
-// Drude poles kept).  Uploads the words and the LUT and resets the polarisation state.
-int apply_materials(sjf_engine* e) {
-    const int ng = (int)e->given_lut.size();
-    std::vector<sjf_material> all = e->given_lut;  // and the twins
-    bool any_pml = e->pml_on[0] || e->pml_on[1] || e->pml_on[2];
-    std::vector<double> fold_add(ng, 0.0);  // sum of the folded Lorentz poles' Re chi per material
-    std::vector<int> twin(ng, -1);
-    const bool fold = e->pml_fref > 0 && any_pml;
-    if (fold) {
-        for (int m = 0; m < ng; ++m) {
-            const sjf_material& M = e->given_lut[m];
-            sjf_material T = M;
-            T.npoles = 0;
-            double eps = M.eps_inf;
-            bool has_lor = false;
-            for (int s = 0; s < M.npoles; ++s) {
-                if (M.is_drude[s]) {
-                    const int t = T.npoles++;
-                    T.f0[t] = M.f0[s];
-                    T.gamma[t] = M.gamma[s];
-                    T.sigma[t] = M.sigma[s];
-                    T.is_drude[t] = 1;
-                } else {
-                    has_lor = true;
-                    eps += lorentz_re_chi(M, s, e->pml_fref);
-                }
+// What the kernels run for a LUT: with pml_fref > 0 every cell inside a PML slab whose material has
+// Lorentz poles takes a twin of that material with them folded out (their real susceptibility at
+// pml_fref added to eps_inf when the sum stays >= 1, else eps_inf kept; Drude poles kept).
+struct MatPlan {
+    std::vector<sjf_material> lut;  // the given materials and the twins
+    std::vector<int> twin;          // per given material its twin, or -1
+    std::vector<double> fold_add;   // sum of the folded Lorentz poles' Re chi
+};
+
+// The plan for `given`; refuses without changing the engine.
+int plan_materials(sjf_engine* e, const std::vector<sjf_material>& given, double fref, bool any_pml, MatPlan* p) {
+    const int ng = (int)given.size();
+    p->lut = given;
+    p->twin.assign(ng, -1);
+    p->fold_add.assign(ng, 0.0);
+    if (!(fref > 0 && any_pml)) return SJF_OK;
+    for (int m = 0; m < ng; ++m) {
+        const sjf_material& M = given[m];
+        sjf_material T = M;
+        T.npoles = 0;
+        double eps = M.eps_inf;
+        bool has_lor = false;
+        for (int s = 0; s < M.npoles; ++s) {
+            if (M.is_drude[s]) {
+                const int t = T.npoles++;
+                T.f0[t] = M.f0[s];
+                T.gamma[t] = M.gamma[s];
+                T.sigma[t] = M.sigma[s];
+                T.is_drude[t] = 1;
+            } else {
+                has_lor = true;
+                eps += lorentz_re_chi(M, s, fref);
             }
-            if (!has_lor) continue;
-            fold_add[m] = eps - M.eps_inf;
-            T.eps_inf = eps >= 1.0 ? eps : M.eps_inf;
-            for (int s = T.npoles; s < SJF_MAX_POLES; ++s) T.f0[s] = T.gamma[s] = T.sigma[s] = 0, T.is_drude[s] = 0;
-            if ((int)all.size() >= SJF_MAX_MATERIALS)
-                return fail(e, SJF_E_UNSUPPORTED, "materials and their PML twins exceed 255");
-            twin[m] = (int)all.size();
-            all.push_back(T);
         }
+        if (!has_lor) continue;
+        p->fold_add[m] = eps - M.eps_inf;
+        T.eps_inf = eps >= 1.0 ? eps : M.eps_inf;
+        for (int s = T.npoles; s < SJF_MAX_POLES; ++s) T.f0[s] = T.gamma[s] = T.sigma[s] = 0, T.is_drude[s] = 0;
+        if ((int)p->lut.size() >= SJF_MAX_MATERIALS)
+            return fail(e, SJF_E_UNSUPPORTED, "materials and their PML twins exceed 255");
+        p->twin[m] = (int)p->lut.size();
+        p->lut.push_back(T);
     }
-    e->lut_h = all;
+    return SJF_OK;
+}
+
+bool any_pml(const sjf_engine* e) { return e->pml_on[0] || e->pml_on[1] || e->pml_on[2]; }
+
+int plan_materials(sjf_engine* e, MatPlan* p) { return plan_materials(e, e->given_lut, e->pml_fref, any_pml(e), p); }
+
+// A call that changes what the kernels read begins: launch tables built before are void, and steps are
+// refused until `ready` is set again.  A call that fails half-way so leaves an engine that says so
+// instead of one that reads freed memory.
+void begin_change(sjf_engine* e, bool& ready) {
+    ready = false;
+    e->version++;
+}
+
+// The default medium as given words and LUT, where a map or a design box comes before any materials.
+int default_words(sjf_engine* e) {
+    if (e->have_mat) return SJF_OK;
+    if (int rc = dev_alloc(e, (void**)&e->given, sizeof(uint32_t) * e->N)) return rc;
+    e->given_lut = e->lut_h;
+    e->have_mat = true;
+    return SJF_OK;
+}
+
+// The material map of the plan: uploads the words, the LUT and the eps maps and resets the
+// polarisation state.
+int apply_materials(sjf_engine* e, const MatPlan& plan) {
+    begin_change(e, e->mat_ready);
+    const int ng = (int)e->given_lut.size();
+    const std::vector<int>& twin = plan.twin;
+    const bool fold = plan.lut.size() > (size_t)ng;
+    e->lut_h = plan.lut;
     e->twin = twin;
     // per-cell eps_inf map: the given values, with the same fold inside the PML slabs
     if (!e->emap_h.empty()) {
@@ -1321,7 +1355,7 @@ int apply_materials(sjf_engine* e) {
                     const int m = (given[q] >> (8 * c)) & 0xff;
                     if (m >= ng || twin[m] < 0) continue;
                     double& v = e->emap_eff[(size_t)c * e->N + q];
-                    if (v + fold_add[m] >= 1.0) v += fold_add[m];
+                    if (v + plan.fold_add[m] >= 1.0) v += plan.fold_add[m];
                 }
             }
         }
@@ -1352,7 +1386,7 @@ int apply_materials(sjf_engine* e) {
     if (!rc) rc = update_words(e);
     if (rc) return rc;
     choose_tile(e);
-    e->version++;
+    e->mat_ready = true;
     return SJF_OK;
 }
 
@@ -2362,6 +2396,8 @@ int sjf_set_materials(sjf_engine* e, const uint32_t* mat_word, const sjf_materia
     if (!rc && first != ~0ull)
         rc = first & 1 ? fail(e, SJF_E_STATE, "design id 255 used before sjf_set_design_eps")
                        : fail(e, SJF_E_ARG, "material word references an id >= n_mat");
+    MatPlan plan;
+    if (!rc) rc = plan_materials(e, std::vector<sjf_material>(lut, lut + n_mat), e->pml_fref, any_pml(e), &plan);
     if (rc) {
         dev_free(words);
         return rc;
@@ -2370,28 +2406,30 @@ int sjf_set_materials(sjf_engine* e, const uint32_t* mat_word, const sjf_materia
     e->given = words;
     e->given_lut.assign(lut, lut + n_mat);
     e->have_mat = true;
-    return apply_materials(e);
+    return apply_materials(e, plan);
 }
 
 int sjf_set_eps_maps(sjf_engine* e, const double* eps) {
     if (!e) return SJF_E_ARG;
     if (int rc = sync_engine(e)) return rc;
     if (!eps) {
-        e->emap_h.clear();
-        e->emap_eff.clear();
-        dev_free(e->emap);
-        if (!e->have_mat) return SJF_OK;  // there was none
+        if (!e->have_mat) return SJF_OK;  // there is none
     } else {
         for (long q = 0; q < 3 * e->N; ++q)
             if (!(eps[q] > 0) || !std::isfinite(eps[q])) return fail(e, SJF_E_ARG, "map eps must be positive and finite");
-        e->emap_h.assign(eps, eps + 3 * e->N);
-        if (!e->have_mat) {
-            if (int rc = dev_alloc(e, (void**)&e->given, sizeof(uint32_t) * e->N)) return rc;
-            e->given_lut = e->lut_h;
-            e->have_mat = true;
-        }
+        if (int rc = default_words(e)) return rc;
     }
-    return apply_materials(e);
+    MatPlan plan;
+    if (int rc = plan_materials(e, &plan)) return rc;
+    begin_change(e, e->mat_ready);
+    if (eps) {
+        e->emap_h.assign(eps, eps + 3 * e->N);
+    } else {
+        e->emap_h.clear();
+        e->emap_eff.clear();
+        dev_free(e->emap);
+    }
+    return apply_materials(e, plan);
 }
 
 int sjf_set_pml_dispersion(sjf_engine* e, double f_ref) {
@@ -2399,8 +2437,11 @@ int sjf_set_pml_dispersion(sjf_engine* e, double f_ref) {
     if (!(f_ref >= 0) || !std::isfinite(f_ref)) return fail(e, SJF_E_ARG, "f_ref must be >= 0");
     if (e->step != 0) return fail(e, SJF_E_STATE, "the PML media must be set before the first step");
     if (int rc = sync_engine(e)) return rc;
+    MatPlan plan;
+    if (e->have_mat)
+        if (int rc = plan_materials(e, e->given_lut, f_ref, any_pml(e), &plan)) return rc;
     e->pml_fref = f_ref;
-    return e->have_mat ? apply_materials(e) : SJF_OK;
+    return e->have_mat ? apply_materials(e, plan) : SJF_OK;
 }
 
 int sjf_set_design_eps(sjf_engine* e, const int lo[3], const int hi[3], const double* eps) {
@@ -2418,6 +2459,17 @@ int sjf_set_design_eps(sjf_engine* e, const int lo[3], const int hi[3], const do
     for (long q = 0; q < cnt; ++q)
         if (!(eps[q] > 0)) return fail(e, SJF_E_ARG, "design eps must be positive");
     if (int rc = sync_engine(e)) return rc;
+    const bool first = !e->dinv, whole = !e->mat_ready;  // whole: an earlier call left the materials incomplete
+    MatPlan plan;
+    if (whole)
+        if (int rc = plan_materials(e, &plan)) return rc;
+    int rc = dev_alloc(e, &e->dinv, (size_t)e->prec * cnt);
+    if (!rc) rc = default_words(e);
+    if (rc) {
+        if (first) dev_free(e->dinv);
+        return rc;
+    }
+    begin_change(e, e->mat_ready);
     for (int d = 0; d < 3; ++d) {
         e->dlo[d] = lo[d];
         e->dhi[d] = hi[d];
@@ -2425,26 +2477,19 @@ int sjf_set_design_eps(sjf_engine* e, const int lo[3], const int hi[3], const do
     e->deps_h.assign(eps, eps + cnt);
     std::vector<double> inv(cnt);
     for (long q = 0; q < cnt; ++q) inv[q] = 1.0 / eps[q];
-    int rc = dev_alloc(e, &e->dinv, (size_t)e->prec * cnt);
-    if (rc) return rc;
     rc = e->prec == 4 ? convert_to_device<float>(e, e->dinv, inv.data(), cnt)
                       : convert_to_device<double>(e, e->dinv, inv.data(), cnt);
     if (rc) return rc;
     // mark design voxels in the material word (all three E components)
-    if (!e->have_mat) {
-        rc = dev_alloc(e, (void**)&e->given, sizeof(uint32_t) * e->N);
-        if (rc) return rc;
-        e->given_lut = e->lut_h;
-        e->have_mat = true;
-    }
     hipLaunchKernelGGL(sjf::k_mark_design, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, e->stream, e->given, n[1],
                        n[2], lo[0], lo[1], lo[2], hi[1] - lo[1], hi[2] - lo[2], cnt);
     HIPCHK(e, hipGetLastError());
+    if (whole) return apply_materials(e, plan);
     rc = update_words(e);
     if (rc) return rc;
     e->uniform = false;
     choose_tile(e);
-    e->version++;
+    e->mat_ready = true;
     return SJF_OK;
 }
 
@@ -2503,7 +2548,11 @@ int sjf_set_pml(sjf_engine* e, const int cells[6], double R, double power) {
     int rc = e->prec == 4 ? convert_to_device<float>(e, e->coefbuf, tab.data(), off)
                           : convert_to_device<double>(e, e->coefbuf, tab.data(), off);
     if (rc) return rc;
-    if (e->have_mat && e->pml_fref > 0) return apply_materials(e);  // the slabs moved
+    if (e->have_mat && e->pml_fref > 0) {  // the slabs moved
+        MatPlan plan;
+        if ((rc = plan_materials(e, &plan))) return rc;
+        return apply_materials(e, plan);
+    }
     e->version++;
     return SJF_OK;
 }

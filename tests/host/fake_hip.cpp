@@ -37,10 +37,10 @@ struct State {
     std::map<const void*, std::pair<void*, size_t>> vars;
     long countdown = -1;  // allocations until one fails; -1: none does
     long allocations = 0;
-    int bad_copies = 0;
+    int bad_copies = 0;  // copies from, to, or word passes over memory that is not live
     Launch last_step;
     long steps = 0, launches = 0, refused = 0;
-    std::string log;
+    std::string log, words;
     dim3 grid, block;
     size_t shmem = 0;
     void* stream = nullptr;
@@ -118,6 +118,11 @@ size_t fake_last_table(char* out, size_t cap) {            // the argument table
 }
 long fake_refused() { return st().refused; }
 int fake_bad_copies() { return st().bad_copies; }
+int fake_first_word() {                                    // first given material word of the last k_words launch
+    int w = -1;
+    if (st().words.size() >= 4) memcpy(&w, st().words.data(), 4);
+    return w;
+}
 const char* fake_log() { return st().log.c_str(); }        // one line per launch since the last clear
 void fake_clear_log() { st().log.clear(); }
 
@@ -210,6 +215,12 @@ int hipLaunchKernel(const void* f, dim3 grid, dim3 block, void** args, size_t sh
     if (l.refused) {
         s.refused++;
         return result(kInvalidConfiguration);
+    }
+    if (l.kernel.find("::k_words<") != std::string::npos) {  // given, matw, seg, lut: all have to be there
+        for (int q = 0; q < 4; ++q)
+            if (!is_live(*(uintptr_t*)args[q], 1)) s.bad_copies++;
+        const auto it = s.live.find(*(uintptr_t*)args[0]);
+        if (it != s.live.end()) s.words.assign((const char*)it->first, it->second);
     }
     if (l.kernel.find("k_step") != std::string::npos) {
         s.steps++;

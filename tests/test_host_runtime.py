@@ -123,6 +123,123 @@ def test_a_failed_allocation_is_not_reported_by_the_next_step(fake_path):
     run_case(fake_path, "failed_allocation")
 
 
+# ---- material changes that fail -----------------------------------------------------------------
+
+def _blocks(ids):
+    w = np.zeros(SHAPE, np.uint32)
+    for q, m in enumerate(ids):
+        w[q::len(ids)] = m * 0x010101
+    return w
+
+
+def _changes():
+    """name -> (calls that come first, the call that is made to fail)"""
+    from sim_juncs_amd import materials as M
+
+    vac, sio2, au, drude = M.VACUUM, M.SIO2.scaled(1.0), M.AU.scaled(1.0), M.AU_REFERENCE_AS_RUN.scaled(1.0)
+
+    def mats(*lut):
+        return lambda e: e.set_materials(_blocks(range(len(lut))), list(lut))
+
+    def pml(e):
+        e.set_pml([2] * 6)
+        e.set_pml_dispersion(1.25)
+
+    maps = lambda e: e.set_eps_maps(np.full((3,) + SHAPE, 2.0))  # noqa: E731
+    design = lambda e: e.set_design_eps((2, 2, 2), (5, 6, 7), np.full((3, 4, 5), 3.0))  # noqa: E731
+    return {
+        "first": ([], mats(vac, au)),
+        "more poles": ([mats(vac, drude)], mats(vac, sio2, au)),
+        "more materials": ([mats(vac, au)], mats(vac, sio2, au, drude, sio2)),
+        "folded": ([pml, mats(vac, sio2)], mats(vac, sio2, au)),
+        "fold": ([lambda e: e.set_pml([2] * 6), mats(vac, au)], lambda e: e.set_pml_dispersion(1.25)),
+        "first maps": ([], maps),
+        "maps": ([mats(vac, au)], maps),
+        "no maps": ([mats(vac, au), maps], lambda e: e.set_eps_maps(None)),
+        "first design": ([], design),
+        "design": ([mats(vac, au)], design),
+        "design of maps": ([maps], design),
+    }
+
+
+def _pointers(table):
+    """Which words of an argument table are pointers (the stand-in's range is far above any size)."""
+    w = np.frombuffer(table[:len(table) // 8 * 8], np.uint64)
+    return [i for i, v in enumerate(w) if 1 << 40 < v < 1 << 47]
+
+
+def case_failed_change(fake, precision):
+    from sim_juncs_amd._lib import EngineError
+    from sim_juncs_amd.engine import Engine
+
+    for name, (before, change) in _changes().items():
+        def engine():
+            e = Engine(SHAPE, 0.02, precision=precision)
+            for f in before:
+                f(e)
+            if name == "fold":  # set before the first step: tables that are built, no step
+                e.reserve_steps(1)
+            else:
+                e.step(1)
+            return e
+
+        with engine() as e:  # how it ends when nothing fails
+            start = fake.allocations()
+            change(e)
+            count = fake.allocations() - start
+            e.step(1)
+            want = _pointers(fake.table())
+        assert count > 0 or name == "no maps"
+        for k in range(count):
+            with engine() as e:
+                old, steps = fake.table(), fake.steps()
+                fake.fail_at(k)
+                with pytest.raises(EngineError):
+                    change(e)
+                fake.fail_at(-1)
+                try:
+                    e.step(1)
+                except EngineError:
+                    assert fake.steps() == steps, (name, k)  # refused: nothing ran
+                else:  # the state before the call
+                    assert fake.last_stale() == 0 and (fake.table() == old or name == "fold"), (name, k)
+                    if name == "fold":
+                        continue
+                change(e)  # memory is there again
+                e.step(1)
+                assert fake.last_stale() == 0 and _pointers(fake.table()) == want, (name, k)
+    assert fake.bad_copies() == 0
+
+
+@pytest.mark.parametrize("precision", ["fp32", "fp64"])
+def test_material_changes_that_run_out_of_memory_leave_no_stale_tables(fake_path, precision):
+    run_case(fake_path, "failed_change", precision)
+
+
+def case_refused_twins(fake):
+    """More than 255 materials with their PML twins: refused, and the earlier map stays whole."""
+    from sim_juncs_amd import materials as M
+    from sim_juncs_amd._lib import EngineError
+    from sim_juncs_amd.engine import Engine
+
+    e = Engine(SHAPE, 0.02)
+    e.set_materials(_blocks([1, 0]), [M.VACUUM, M.AU.scaled(1.0)])
+    e.set_pml([2] * 6)
+    e.set_pml_dispersion(1.25)
+    e.step(1)
+    old, live = fake.table(), fake.live_bytes()
+    with pytest.raises(EngineError, match="twins"):
+        e.set_materials(_blocks([7, 8]), [M.SIO2.scaled(1.0)] * 200)
+    e.step(1)
+    assert fake.table() == old and fake.live_bytes() == live
+    e.set_design_eps((2, 2, 2), (5, 6, 7), np.full((3, 4, 5), 3.0))
+    assert fake.first_word() == 0x010101  # the words that belong to the LUT in use
+
+
+def test_refused_materials_leave_the_earlier_ones(fake_path):
+    run_case(fake_path, "refused_twins")
+
+
 if __name__ == "__main__":
     sys.path.insert(0, ROOT)
     globals()["case_" + sys.argv[2]](Fake(sys.argv[1]), *sys.argv[3:])
