@@ -109,8 +109,8 @@ const char* sjf_last_error(const sjf_engine* e);
 /* ---- structure ----------------------------------------------------------------------- */
 
 /* A call of this section that refuses its arguments leaves the engine as it was.  One that runs out of
- * memory leaves it as it was, or with incomplete materials: steps and adjoint runs are then refused
- * (SJF_E_STATE) until a call that sets the materials succeeds. */
+ * memory leaves it as it was, or with incomplete materials (an incomplete PML): steps and adjoint runs
+ * are then refused (SJF_E_STATE) until a call that sets the materials (the PML) succeeds. */
 
 /* Replaces the structure's chi1p1 sampling and add_susceptibility calls
  * (src/disp.cpp:515-548, in_bound at src/disp.cpp:264-283).  mat_word holds one uint32 per

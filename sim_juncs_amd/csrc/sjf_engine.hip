@@ -107,10 +107,11 @@ struct sjf_engine {
     // PML
     int pml[6] = {0, 0, 0, 0, 0, 0};
     bool pml_on[3] = {false, false, false};
+    bool pml_ready = true;    // as mat_ready
     void* coefbuf = nullptr;  // per axis: bE[n], aE[n], bH[n], aH[n]
     int coff[3] = {0, 0, 0};
     long slab[3] = {0, 0, 0};
-    void* psibuf[3] = {};  // per axis [6][slab]: E aux x2, H aux pair A x2, pair B x2
+    void* psibuf[3] = {};  // per axis [3][slab][2]: E pair, H pairs A and B
 
     std::vector<Source> src;
     std::vector<Monitor> mon;
@@ -551,6 +552,7 @@ int build_set_t(LaunchSet* s) {
     size_t zh = 0;  // register form with z passes: values of the pass halo in LDS
     for (sjf_engine* e : s->eng) {
         if (!e->mat_ready) return fail(e0, SJF_E_STATE, "the materials are incomplete: the call that last set them failed");
+        if (!e->pml_ready) return fail(e0, SJF_E_STATE, "the PML is incomplete: the call that last set it failed");
         // the engine's own set runs its tuned rows; a batch picks rows per engine for its form
         const int rows = (s == e->own) ? e->ty
                                        : (s->form == SJF_TILE_THREAD_ROWS ? default_thread_rows(e) : s->ty);
@@ -2497,13 +2499,23 @@ int sjf_set_pml(sjf_engine* e, const int cells[6], double R, double power) {
     if (!e || !cells) return SJF_E_ARG;
     if (!(R > 0 && R < 1) || !(power >= 0)) return fail(e, SJF_E_ARG, "R must be in (0,1), power >= 0");
     if (e->step != 0) return fail(e, SJF_E_STATE, "PML must be set before the first step");
+    bool some = false;
     for (int d = 0; d < 3; ++d) {
         const int n = axis_n(e, d);
         const int lo = cells[2 * d], hi = cells[2 * d + 1];
         if (lo < 0 || hi < 0 || lo + hi > n) return fail(e, SJF_E_ARG, "PML thicker than the grid");
         if ((lo > 0 || hi > 0) && e->g.periodic[d]) return fail(e, SJF_E_ARG, "PML on a periodic axis");
+        // the step kernels address the six auxiliary slots of a slab within one 2 GiB buffer range
+        if ((double)e->prec * 6 * (lo + hi) * (e->N / n) >= 2147483648.0)
+            return fail(e, SJF_E_UNSUPPORTED, "PML slab auxiliaries exceed 2 GiB on one axis");
+        some = some || lo > 0 || hi > 0;
     }
+    MatPlan plan;
+    const bool fold = e->have_mat && e->pml_fref > 0;
+    if (fold)
+        if (int rc = plan_materials(e, e->given_lut, e->pml_fref, some, &plan)) return rc;
     if (int rc = sync_engine(e)) return rc;
+    begin_change(e, e->pml_ready);
     int off = 0;
     for (int d = 0; d < 3; ++d) off += 4 * axis_n(e, d);
     std::vector<double> tab(off, 0.0);
@@ -2539,22 +2551,14 @@ int sjf_set_pml(sjf_engine* e, const int cells[6], double R, double power) {
         }
         if (!e->pml_on[d]) continue;
         e->slab[d] = (long)(lo + hi) * (e->N / n);
-        // the step kernels address the six auxiliary slots of a slab within one 2 GiB buffer range
-        if ((double)e->prec * 6 * e->slab[d] >= 2147483648.0)
-            return fail(e, SJF_E_UNSUPPORTED, "PML slab auxiliaries exceed 2 GiB on one axis");
         int rc = dev_alloc(e, &e->psibuf[d], (size_t)e->prec * 6 * e->slab[d]);
         if (rc) return rc;
     }
     int rc = e->prec == 4 ? convert_to_device<float>(e, e->coefbuf, tab.data(), off)
                           : convert_to_device<double>(e, e->coefbuf, tab.data(), off);
     if (rc) return rc;
-    if (e->have_mat && e->pml_fref > 0) {  // the slabs moved
-        MatPlan plan;
-        if ((rc = plan_materials(e, &plan))) return rc;
-        return apply_materials(e, plan);
-    }
-    e->version++;
-    return SJF_OK;
+    e->pml_ready = true;
+    return fold ? apply_materials(e, plan) : SJF_OK;  // the slabs moved
 }
 
 int sjf_add_source(sjf_engine* e, int comp, const double box[6], const sjf_pulse* p, double amp_re,

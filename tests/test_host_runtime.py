@@ -240,6 +240,65 @@ def test_refused_materials_leave_the_earlier_ones(fake_path):
     run_case(fake_path, "refused_twins")
 
 
+def case_failed_pml(fake, precision):
+    """The same for sjf_set_pml, on engines whose tables are built, with and without an earlier PML."""
+    from sim_juncs_amd import materials as M
+    from sim_juncs_amd._lib import EngineError
+    from sim_juncs_amd.engine import Engine
+
+    def thin(e):
+        e.set_pml([1, 0, 2, 2, 0, 1])
+
+    def folded(e):
+        e.set_materials(_blocks([0, 1]), [M.VACUUM, M.AU.scaled(1.0)])
+        e.set_pml_dispersion(1.25)
+
+    for before in ([], [thin], [folded], [thin, folded]):
+        def engine():
+            e = Engine(SHAPE, 0.02, precision=precision)
+            for f in before:
+                f(e)
+            e.reserve_steps(1)
+            return e
+
+        with engine() as e:
+            start = fake.allocations()
+            e.set_pml([2, 1, 2, 2, 3, 1])
+            count = fake.allocations() - start
+            e.step(1)
+            want = _pointers(fake.table())
+        assert count >= 3
+        for k in range(count):
+            with engine() as e:
+                steps = fake.steps()
+                fake.fail_at(k)
+                with pytest.raises(EngineError):
+                    e.set_pml([2, 1, 2, 2, 3, 1])
+                fake.fail_at(-1)
+                with pytest.raises(EngineError, match="incomplete"):
+                    e.step(1)
+                assert fake.steps() == steps
+                e.set_pml([2, 1, 2, 2, 3, 1])
+                e.step(1)
+                assert fake.last_stale() == 0 and _pointers(fake.table()) == want, k
+    # layers too large for one buffer range are refused before anything changes
+    with Engine((700, 700, 230), 0.02, precision="fp64") as e:
+        e.set_pml([0, 0, 0, 0, 2, 2])
+        e.step(0)
+        live = fake.live_bytes()
+        with pytest.raises(EngineError, match="2 GiB"):
+            e.set_pml([0, 0, 0, 0, 60, 60])
+        assert fake.live_bytes() == live
+        e.step(1)
+        assert fake.last_stale() == 0
+    assert fake.bad_copies() == 0
+
+
+@pytest.mark.parametrize("precision", ["fp32", "fp64"])
+def test_a_pml_that_runs_out_of_memory_leaves_no_stale_tables(fake_path, precision):
+    run_case(fake_path, "failed_pml", precision)
+
+
 if __name__ == "__main__":
     sys.path.insert(0, ROOT)
     globals()["case_" + sys.argv[2]](Fake(sys.argv[1]), *sys.argv[3:])
