@@ -428,7 +428,8 @@ sjf::StepArgs<T> step_args(const sjf_engine* e, int ty, int xc, bool given = fal
     a.seg = e->seg;
     a.lut = (const sjf::MatLut<T>*)e->lut;
     a.Q = (T*)e->Qbuf;
-    a.P = (T*)e->Pbuf;
+    // FP32 slots alternate between two arrays; Drude slots alone are updated in place
+    a.P = (T*)(e->Pbuf || !sjf::kPolePair<T> ? e->Pbuf : e->Qbuf);
     a.nqp = e->Qbuf ? 3 * e->maxp : 0;
     for (int d = 0; d < 3; ++d) {
         a.pml_on[d] = e->pml_on[d] ? 1 : 0;
@@ -1373,9 +1374,9 @@ int apply_materials(sjf_engine* e, const MatPlan& plan) {
     e->nmat = (int)e->lut_h.size();
     e->maxp = maxp;
     e->uniform = (e->nmat == 1 && maxp == 0 && e->deps_h.empty() && e->emap_h.empty());
-    // polarisation state, zeroed; FP32 slots alternate between the two arrays, Drude ones included
+    // polarisation state, zeroed (the second array where a slot holds a Lorentz pole)
     const size_t pol = maxp > 0 ? (size_t)e->prec * 3 * maxp * e->N : 0;
-    const bool pair = pol > 0 && (anylor || e->prec == 4);
+    const bool pair = pol > 0 && anylor;
     if (pol != e->pol_bytes) dev_free(e->Qbuf), dev_free(e->Pbuf);
     if (!pair) dev_free(e->Pbuf);
     e->pol_bytes = pol;

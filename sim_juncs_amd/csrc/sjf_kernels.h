@@ -415,7 +415,8 @@ __device__ __forceinline__ void step_tile(const StepArgs<T>& a, const int t) {
     const int hw = odd ? 1 : 2;  // and written
     // FP32 pole slots alternate between two arrays: step n reads P^n (Lorentz) or Q^n (Drude) from
     // Q when n is even, from P when it is odd, and writes the new value to the other, where a
-    // Lorentz pole has read P^{n-1}.  FP64 slots hold Q^n and P^n.
+    // Lorentz pole has read P^{n-1}.  Without a Lorentz pole both are one array: each slot is read and
+    // written by one lane, the read before the write.  FP64 slots hold Q^n and P^n.
     const char* Pcur = (const char*)(kPolePair<T> && odd ? a.P : a.Q);
     const char* Pold = (const char*)(kPolePair<T> && odd ? a.Q : a.P);
     CONST const uint32_t* seg = (CONST const uint32_t*)a.seg;

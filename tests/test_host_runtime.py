@@ -299,6 +299,30 @@ def test_a_pml_that_runs_out_of_memory_leaves_no_stale_tables(fake_path, precisi
     run_case(fake_path, "failed_pml", precision)
 
 
+# ---- pole state ---------------------------------------------------------------------------------
+
+def case_pole_memory(fake, precision):
+    """A second array of pole state is there for Lorentz poles alone."""
+    from sim_juncs_amd import materials as M
+    from sim_juncs_amd.engine import Engine
+
+    one = (4 if precision == "fp32" else 8) * 3 * np.prod(SHAPE)  # one slot of one array
+    used = {}
+    for name, metal in (("drude", M.AU_REFERENCE_AS_RUN), ("lorentz", M.SIO2)):
+        with Engine(SHAPE, 0.02, precision=precision) as e:
+            e.set_materials(_blocks([0, 1]), [M.VACUUM, metal.scaled(1.0)])
+            used[name] = fake.live_bytes()
+            e.step(2)
+            e.step(1)
+            assert fake.last_stale() == 0
+    assert used["lorentz"] - used["drude"] == one
+
+
+@pytest.mark.parametrize("precision", ["fp32", "fp64"])
+def test_drude_media_hold_one_array_of_pole_state(fake_path, precision):
+    run_case(fake_path, "pole_memory", precision)
+
+
 if __name__ == "__main__":
     sys.path.insert(0, ROOT)
     globals()["case_" + sys.argv[2]](Fake(sys.argv[1]), *sys.argv[3:])
