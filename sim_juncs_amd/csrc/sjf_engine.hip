@@ -785,10 +785,14 @@ int launch_step_np(LaunchSet* s) {
         else if (s->nts) SJF_LAUNCH(sjf::k_step<T, 1, NP, M, true>);
         else SJF_LAUNCH(sjf::k_step<T, 1, NP, M>);
     } else if (s->ty == 2) {
-        if (s->block <= 512) SJF_LAUNCH(sjf::k_step<T, 2, NP, 512>);
+        constexpr int M = sizeof(T) == 4 ? 512 : 256;  // FP64: 512 registers per lane up to 256 threads, none spilled
+        if (s->block <= M) SJF_LAUNCH(sjf::k_step<T, 2, NP, M>);
+        else if (s->block <= 512) SJF_LAUNCH(sjf::k_step<T, 2, NP, 512>);
         else SJF_LAUNCH(sjf::k_step<T, 2, NP, 1024>);
     } else if (s->ty == 4) {
-        if (s->block <= 512) SJF_LAUNCH(sjf::k_step<T, 4, NP, 512>);
+        constexpr int M = sizeof(T) == 4 ? 512 : 256;
+        if (s->block <= M) SJF_LAUNCH(sjf::k_step<T, 4, NP, M>);
+        else if (s->block <= 512) SJF_LAUNCH(sjf::k_step<T, 4, NP, 512>);
         else SJF_LAUNCH(sjf::k_step<T, 4, NP, 1024>);
     } else {
         return fail(s->eng[0], SJF_E_ARG, "tile rows must be 1, 2 or 4");

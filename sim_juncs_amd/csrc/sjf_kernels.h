@@ -397,6 +397,11 @@ template <typename T, int TY, int NP, bool ZP, bool NTS>
 __device__ __forceinline__ void step_tile(const StepArgs<T>& a, const int t) {
     constexpr uint32_t TS = sizeof(T);
     constexpr int NS = NP > 0 ? NP : 1;
+    // FP64 rows of two or four with poles have no registers for the loads of a plane ahead: they load H, the
+    // auxiliaries and the pole state where they use them.  us per step, all of it ahead and with 256 registers
+    // per lane, and as now (512 registers up to 256 threads): 100x100x96 two rows 163, 119, four rows 637, 193;
+    // 120x120x250 four rows 968, 283; without poles (ahead, 512 registers) four rows 252, 137 and 447, 184
+    constexpr bool kAhead = sizeof(T) == 4 || TY == 1 || NP == 0;
     typedef T Pair __attribute__((ext_vector_type(2)));
     typedef T Erows[TY + 2][3];  // E of rows -1..TY (Ey of row TY unused)
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -646,17 +651,19 @@ __device__ __forceinline__ void step_tile(const StepArgs<T>& a, const int t) {
             }
         }
         load_e(fN, pn < nx, en);
-        load_h(fW, true);
-        load_psi_h(pi);
+        if (kAhead) {
+            load_h(fW, true);
+            load_psi_h(pi);
+        }
 #pragma unroll
         for (int r = 0; r < TY; ++r) {
             if (!own(r)) continue;
-            load_psi_e(pi, r);
+            if (kAhead) load_psi_e(pi, r);
             load_word(pi, r, cc[r], mw[r]);
             load_word(pn, r, cn[r], mwn[r]);
             if (cc[r] & kSegSpecial) {
                 mw[r] = words(cc[r], mw[r]);
-                if (NP > 0 && seg_poles(cc[r]) > 0) load_poles(pi, r, cc[r], mw[r]);
+                if (kAhead && NP > 0 && seg_poles(cc[r]) > 0) load_poles(pi, r, cc[r], mw[r]);
             }
         }
 
@@ -668,6 +675,10 @@ __device__ __forceinline__ void step_tile(const StepArgs<T>& a, const int t) {
             for (int r = 0; r < TY; ++r) {
                 cnn[r] = uniform || !own(r) || i + 2 >= x1 ? 0u : code_of(pnn, r);
                 iv[r] = clut[seg_material(cc[r])].inv_eps;
+            }
+            if (!kAhead) {
+                load_h(fW, live);
+                if (live) load_psi_h(pi);
             }
             T d[TY + 1][6];  // dEz_y, dEx_y, dEy_z, dEx_z, dEz_x, dEy_x
 #pragma unroll
@@ -753,6 +764,7 @@ __device__ __forceinline__ void step_tile(const StepArgs<T>& a, const int t) {
                     }
                     const int npx = seg_poles(code);
                     if (NP > 0 && npx > 0) {
+                        if (!kAhead) load_poles(pi, r, code, mw[r]);
                         const Rsrc rc = rsrc(Pcur + (long)pi * QPB), ro = rsrc(Pold + (long)pi * QPB);
                         int np[3];
 #pragma unroll
@@ -793,7 +805,7 @@ __device__ __forceinline__ void step_tile(const StepArgs<T>& a, const int t) {
                 }
                 if (cn[r] & kSegSpecial) {
                     const uint32_t w = words(cn[r], mwn[r]);
-                    if (NP > 0 && seg_poles(cn[r]) > 0) load_poles(pn, r, cn[r], w);
+                    if (kAhead && NP > 0 && seg_poles(cn[r]) > 0) load_poles(pn, r, cn[r], w);
                     mw[r] = reg_copy(w);
                 }
                 load_word(pnn, r, cnn[r], mwn[r]);
@@ -804,9 +816,9 @@ __device__ __forceinline__ void step_tile(const StepArgs<T>& a, const int t) {
 #pragma unroll
                 for (int c = 0; c < 3; ++c)
                     if (c != 1 || r < TY + 1) ec[r][c] = reg_copy(en[r][c]);
-            load_h(fN, next);
+            if (kAhead) load_h(fN, next);
             load_e(fNN, next && pnn < nx, en);
-            if (next) load_psi_h(pn);
+            if (kAhead && next) load_psi_h(pn);
         };
 
         auto e_phase = [&](const int i) __attribute__((always_inline)) {
@@ -819,6 +831,7 @@ __device__ __forceinline__ void step_tile(const StepArgs<T>& a, const int t) {
 #pragma unroll
             for (int r = 0; r < TY; ++r) {
                 if (!own(r)) continue;
+                if (!kAhead) load_psi_e(pi, r);
                 const uint32_t o = oR[r + 1];
                 const Pair* below = buf + r * (B + 1) + kb;
                 if (ZP && pass > 0 && kl == 0) below = zh + (((pass - 1) & 1) * a.xc + (i - x0)) * TY + r;
@@ -864,7 +877,7 @@ __device__ __forceinline__ void step_tile(const StepArgs<T>& a, const int t) {
                 for (int c = 0; c < 3; ++c) bst<NTS>(rW, o, c * PB, e_next(e0[r][c], inv[r][c], cdt, curl[c], sq[r][c]));
                 hp[r][0] = reg_copy(h[r + 1][1]);
                 hp[r][1] = reg_copy(h[r + 1][2]);
-                if (next) load_psi_e(pn, r);
+                if (kAhead && next) load_psi_e(pn, r);
                 cc[r] = cn[r];
                 cn[r] = cnn[r];
             }
