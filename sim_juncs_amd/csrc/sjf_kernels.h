@@ -651,19 +651,20 @@ __device__ __forceinline__ void step_tile(const StepArgs<T>& a, const int t) {
             }
         }
         load_e(fN, pn < nx, en);
-        if (kAhead) {
+        if constexpr (kAhead) {
             load_h(fW, true);
             load_psi_h(pi);
         }
 #pragma unroll
         for (int r = 0; r < TY; ++r) {
             if (!own(r)) continue;
-            if (kAhead) load_psi_e(pi, r);
+            if constexpr (kAhead) load_psi_e(pi, r);
             load_word(pi, r, cc[r], mw[r]);
             load_word(pn, r, cn[r], mwn[r]);
             if (cc[r] & kSegSpecial) {
                 mw[r] = words(cc[r], mw[r]);
-                if (kAhead && NP > 0 && seg_poles(cc[r]) > 0) load_poles(pi, r, cc[r], mw[r]);
+                if constexpr (kAhead)
+                    if (NP > 0 && seg_poles(cc[r]) > 0) load_poles(pi, r, cc[r], mw[r]);
             }
         }
 
@@ -676,7 +677,7 @@ __device__ __forceinline__ void step_tile(const StepArgs<T>& a, const int t) {
                 cnn[r] = uniform || !own(r) || i + 2 >= x1 ? 0u : code_of(pnn, r);
                 iv[r] = clut[seg_material(cc[r])].inv_eps;
             }
-            if (!kAhead) {
+            if constexpr (!kAhead) {
                 load_h(fW, live);
                 if (live) load_psi_h(pi);
             }
@@ -764,7 +765,7 @@ __device__ __forceinline__ void step_tile(const StepArgs<T>& a, const int t) {
                     }
                     const int npx = seg_poles(code);
                     if (NP > 0 && npx > 0) {
-                        if (!kAhead) load_poles(pi, r, code, mw[r]);
+                        if constexpr (!kAhead) load_poles(pi, r, code, mw[r]);
                         const Rsrc rc = rsrc(Pcur + (long)pi * QPB), ro = rsrc(Pold + (long)pi * QPB);
                         int np[3];
 #pragma unroll
@@ -805,7 +806,8 @@ __device__ __forceinline__ void step_tile(const StepArgs<T>& a, const int t) {
                 }
                 if (cn[r] & kSegSpecial) {
                     const uint32_t w = words(cn[r], mwn[r]);
-                    if (kAhead && NP > 0 && seg_poles(cn[r]) > 0) load_poles(pn, r, cn[r], w);
+                    if constexpr (kAhead)
+                        if (NP > 0 && seg_poles(cn[r]) > 0) load_poles(pn, r, cn[r], w);
                     mw[r] = reg_copy(w);
                 }
                 load_word(pnn, r, cnn[r], mwn[r]);
@@ -816,9 +818,10 @@ __device__ __forceinline__ void step_tile(const StepArgs<T>& a, const int t) {
 #pragma unroll
                 for (int c = 0; c < 3; ++c)
                     if (c != 1 || r < TY + 1) ec[r][c] = reg_copy(en[r][c]);
-            if (kAhead) load_h(fN, next);
+            if constexpr (kAhead) load_h(fN, next);
             load_e(fNN, next && pnn < nx, en);
-            if (kAhead && next) load_psi_h(pn);
+            if constexpr (kAhead)
+                if (next) load_psi_h(pn);
         };
 
         auto e_phase = [&](const int i) __attribute__((always_inline)) {
@@ -831,7 +834,7 @@ __device__ __forceinline__ void step_tile(const StepArgs<T>& a, const int t) {
 #pragma unroll
             for (int r = 0; r < TY; ++r) {
                 if (!own(r)) continue;
-                if (!kAhead) load_psi_e(pi, r);
+                if constexpr (!kAhead) load_psi_e(pi, r);
                 const uint32_t o = oR[r + 1];
                 const Pair* below = buf + r * (B + 1) + kb;
                 if (ZP && pass > 0 && kl == 0) below = zh + (((pass - 1) & 1) * a.xc + (i - x0)) * TY + r;
@@ -877,7 +880,8 @@ __device__ __forceinline__ void step_tile(const StepArgs<T>& a, const int t) {
                 for (int c = 0; c < 3; ++c) bst<NTS>(rW, o, c * PB, e_next(e0[r][c], inv[r][c], cdt, curl[c], sq[r][c]));
                 hp[r][0] = reg_copy(h[r + 1][1]);
                 hp[r][1] = reg_copy(h[r + 1][2]);
-                if (kAhead && next) load_psi_e(pn, r);
+                if constexpr (kAhead)
+                    if (next) load_psi_e(pn, r);
                 cc[r] = cn[r];
                 cn[r] = cnn[r];
             }
