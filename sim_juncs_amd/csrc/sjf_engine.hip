@@ -1086,6 +1086,43 @@ void choose_tile(sjf_engine* e) {
     e->xc = round_chunk(e->g.nx, (e->g.ny + e->ty - 1) / e->ty, slots, 2);
 }
 
+// Default form of a batch: thread rows where some instance would take them alone (choose_tile) and all
+// fit.  Measured on MI355X, us per step, thread rows and one register row: 24 grids of 64^3 to
+// 192x192x128 (FP32) 915, 1074; six of 192x192x96 467, 487; two 170, 191; FP32 lines of 100 and 500
+// cells (1.5 M cells each) 95, 137; of 100 and three of 400 cells 224, 233; FP64 lines of 100 and 200
+// cells 187, 216.  The chunk matters little with many rounds of workgroups (24 grids: 4 planes 919, 6
+// 915, 8 918, 12 941, 18 955; four grids: 4 planes 139, 6 132, 8 132, 12 130, 18 159).
+//
+// FP64 workgroups of more than 512 threads spill and cost about 1.6 times as much a thread: there
+// thread rows are taken where they leave so many fewer lanes idle (or run half of the threads of a long
+// line on its halo row) that this is made up for, or where all of them run at once.  FP64, 1.5 M cells
+// each: lines of 60, 60, 60, 300 cells 688, 999; 64, 500 346, 464; 100, 100, 100, 500 730, 749; 100, 500
+// 383, 311; 100, 300 393, 287; 120, 300, 400, 500 741, 463; 100, 300 of 0.3 M cells (245 workgroups) 83, 95.
+constexpr int kBatchRowsChunk = 8;
+int batch_form(sjf_engine* const* engines, int n) {
+    bool any = false;
+    int rows_block = 64, line_block = 64;
+    long groups = 0;
+    for (int i = 0; i < n; ++i) {
+        const sjf_engine* e = engines[i];
+        const int rows = default_thread_rows(e);
+        if (!thread_rows_fit(e, rows)) return SJF_TILE_REGISTER_ROWS;
+        any = any || e->g.nz < (e->prec == 8 ? 128 : 256);
+        rows_block = std::max(rows_block, ((rows + 1) * e->g.nz + 63) / 64 * 64);
+        line_block = std::max(line_block, (e->g.nz + 63) / 64 * 64);
+        groups += tiles_of(e, rows, std::min(kBatchRowsChunk, e->g.nx));
+    }
+    if (!any) return SJF_TILE_REGISTER_ROWS;
+    if (engines[0]->prec == 4 || rows_block <= 512 || groups <= 256) return SJF_TILE_THREAD_ROWS;
+    double by_rows = 0, by_lines = 0;  // threads times planes
+    for (int i = 0; i < n; ++i) {
+        const sjf_engine* e = engines[i];
+        by_rows += (double)e->N * rows_block / (default_thread_rows(e) * e->g.nz);
+        by_lines += (double)e->N * line_block / e->g.nz;
+    }
+    return 1.6 * by_rows < by_lines ? SJF_TILE_THREAD_ROWS : SJF_TILE_REGISTER_ROWS;
+}
+
 int free_all(sjf_engine* e) {
     destroy_set(e->own);
     e->own = nullptr;
@@ -2933,17 +2970,8 @@ int sjf_batch_create(sjf_engine* const* engines, int n, sjf_batch** out) {
     s->own_stream = true;
     s->prec = e0->prec;
     s->ty = 1;
-    // Thread rows where some instance would take them alone (choose_tile) and all fit.  Measured on
-    // MI355X, us per step, thread rows and one register row: 24 grids of 64^3 to 192x192x128 (FP32)
-    // 915, 1074; six of 192x192x96 467, 487; two 170, 191.  The chunk matters little with many rounds
-    // of workgroups (24 grids: 4 planes 919, 6 915, 8 918, 12 941, 18 955; four grids: 4 planes 139,
-    // 6 132, 8 132, 12 130, 18 159).
-    s->form = SJF_TILE_REGISTER_ROWS;
-    for (int i = 0; i < n; ++i)
-        if (engines[i]->g.nz < (engines[i]->prec == 8 ? 128 : 256)) s->form = SJF_TILE_THREAD_ROWS;
-    for (int i = 0; i < n; ++i)
-        if (!thread_rows_fit(engines[i], default_thread_rows(engines[i]))) s->form = SJF_TILE_REGISTER_ROWS;
-    s->xc = s->form == SJF_TILE_THREAD_ROWS ? 8 : 16;
+    s->form = batch_form(engines, n);
+    s->xc = s->form == SJF_TILE_THREAD_ROWS ? kBatchRowsChunk : 16;
     for (int i = 0; i < n; ++i) {
         s->eng.push_back(engines[i]);
         engines[i]->batch = b;

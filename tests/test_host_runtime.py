@@ -323,6 +323,34 @@ def test_drude_media_hold_one_array_of_pole_state(fake_path, precision):
     run_case(fake_path, "pole_memory", precision)
 
 
+# ---- batches ------------------------------------------------------------------------------------
+
+def case_batch_form(fake, precision, lines, cells, form, threads):
+    from sim_juncs_amd.engine import Batch, Engine
+
+    engines = []
+    for nz in map(int, lines.split(",")):
+        n = round((float(cells) / nz) ** 0.5)
+        engines.append(Engine((n, n, nz), 0.02, precision=precision))
+    b = Batch(engines)
+    b.step(1)
+    kernel = {"rows": "k_step_rows<", "lines": "k_step<", "passes": "k_step_z<"}[form]
+    assert kernel in fake.last_kernel().decode()
+    assert b.launch_info()[0] == int(threads)
+
+
+@pytest.mark.parametrize("precision,lines,cells,form,threads", [
+    ("fp32", "100,500", 1.5e6, "rows", 1024), ("fp32", "256,300", 1.5e6, "lines", 320),
+    ("fp64", "100,200", 1.5e6, "rows", 512), ("fp64", "128,200", 1.5e6, "lines", 256),
+    ("fp64", "100,300", 1.5e6, "lines", 320), ("fp64", "100,300", 2e5, "rows", 640),
+    ("fp64", "120,255,257", 1.5e6, "lines", 320), ("fp64", "60,60,60,300", 1.5e6, "rows", 640),
+    ("fp64", "64,513", 2e5, "passes", 256),
+])
+def test_default_form_of_a_batch(fake_path, precision, lines, cells, form, threads):
+    """Thread rows where they were measured to be faster: FP64 workgroups above 512 threads spill."""
+    run_case(fake_path, "batch_form", precision, lines, cells, form, threads)
+
+
 if __name__ == "__main__":
     sys.path.insert(0, ROOT)
     globals()["case_" + sys.argv[2]](Fake(sys.argv[1]), *sys.argv[3:])
