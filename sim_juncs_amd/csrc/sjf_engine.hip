@@ -1573,6 +1573,38 @@ AdjTile adj_tile_of(const sjf_engine* e, double bytes, int nmat) {
     return {rows, rows ? 0 : 1, 0};
 }
 
+// Waves per SIMD of the row-of-threads reverse kernel (its registers)
+template <typename T>
+int adj_rows_waves(int npv) {
+    return sizeof(T) == 4 ? 4 : npv == 0 ? 3 : 2;
+}
+
+// Default x-chunk of a batched reverse launch in rows of threads: 12 planes (six 192x192x96 FP32 engines, us
+// per reverse launch: 4 planes 584, 6 549, 8 537, 12 526, 18 533, 24 540), or the shorter one for which
+// the rounds of resident workgroups times chunk and start-up (round_chunk) are fewer, where the launch does
+// not fill the chip twice.  Gold, us per launch at 12 planes, so, and one row per workgroup: FP32 four of
+// 48^3 52, 22.5, 30.7; two of 64^3 57, 24, 29; two of 96^3 54, 44, 79; FP64 two of 64^3 55, 34, 38.
+template <typename T>
+int adj_batch_chunk(const LaunchSet* s) {
+    int block = 64, npv = 0;
+    for (const sjf_engine* e : s->eng) {
+        block = std::max(block, ((default_thread_rows(e) + 1) * e->g.nz + 63) / 64 * 64);
+        npv = std::max(npv, np_variant_of(e->maxp, e->uniform));
+    }
+    const long slots = 256L * std::max(1, 4 * adj_rows_waves<T>(npv) / (block / 64));
+    auto groups = [&](int c) {
+        long g = 0;
+        for (const sjf_engine* e : s->eng) g += tiles_of(e, default_thread_rows(e), std::min(c, e->g.nx));
+        return g;
+    };
+    int best = 12;
+    if (groups(best) >= 2 * slots) return best;
+    auto cost = [&](int c) { return (groups(c) + slots - 1) / slots * (c + 3); };
+    for (int c = 11; c > 0; --c)
+        if (cost(c) < cost(best)) best = c;
+    return best;
+}
+
 template <typename T, int NP, bool NTS>
 void launch_adj_one_row(sjf_engine* e, const sjf::AdjArgs<T>& g, int block, unsigned tiles, size_t lds) {
     if (block <= 256) hipLaunchKernelGGL((sjf::k_adj_step<T, NP, 256, NTS>), dim3(tiles), dim3(block), lds, e->stream, g);
@@ -1726,8 +1758,8 @@ int adjoint_run_t(sjf_engine* e, long nsteps, long K, long gap, double* J_out, d
         const long nxc = std::min<long>(std::max(1L, (16384 + trows - 1) / trows), e->g.nx);
         axc = (int)((e->g.nx + nxc - 1) / nxc);
     } else if (rows && at.xc == 0) {
-        const int waves = sizeof(T) == 4 ? 4 : npv == 0 ? 3 : 2, wg = ((arows + 1) * e->g.nz + 63) / 64;
-        axc = round_chunk(e->g.nx, (e->g.ny + arows - 1) / arows, 256L * std::max(1, 4 * waves / wg), 3);
+        const int wg = ((arows + 1) * e->g.nz + 63) / 64;
+        axc = round_chunk(e->g.nx, (e->g.ny + arows - 1) / arows, 256L * std::max(1, 4 * adj_rows_waves<T>(npv) / wg), 3);
     }
     g.f = step_args<T>(e, arows, axc);
     g.A[0] = A;
@@ -1932,9 +1964,7 @@ int batch_adjoint_run_t(LaunchSet* s, long nsteps, long K, const long* gaps, con
     for (const sjf_engine* e : s->eng)
         if (bt.nrows == 0 && (default_thread_rows(e) + 1) * e->g.nz > (sizeof(T) == 8 ? 512 : 1024)) bt = {false, 1, 0};
     const bool brows = bt.rows;
-    // default chunks, six 192x192x96 FP32 engines: 4 planes 584 us per reverse launch, 6 549, 8 537, 12
-    // 526, 18 533, 24 540 (one row per workgroup: 657)
-    const int bxc = bt.xc > 0 ? bt.xc : bt.nrows > 0 ? 6 : 12;
+    const int bxc = bt.xc > 0 ? bt.xc : bt.nrows > 0 ? 6 : brows ? adj_batch_chunk<T>(s) : 12;
     int bblock = 64;
     for (int i = 0; i < n; ++i) {
         sjf_engine* e = s->eng[i];

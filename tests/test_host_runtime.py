@@ -351,6 +351,34 @@ def test_default_form_of_a_batch(fake_path, precision, lines, cells, form, threa
     run_case(fake_path, "batch_form", precision, lines, cells, form, threads)
 
 
+def case_reverse_chunk(fake, precision, count, shape, groups):
+    from sim_juncs_amd.engine import Batch, Engine
+
+    shape = tuple(map(int, shape.split(",")))
+    engines = []
+    for _ in range(int(count)):
+        e = Engine(shape, 0.02, precision=precision)
+        lo = tuple(n // 2 for n in shape)
+        e.set_design_eps(lo, tuple(n + 2 for n in lo), np.full((2, 2, 2), 3.0))
+        engines.append(e)
+    b = Batch(engines)
+    b.adjoint_run(3, [(1, 1, 1)] * len(engines), [8] * len(engines))
+    assert b.adjoint_kernel_info()[2] == int(groups)
+
+
+@pytest.mark.parametrize("precision,count,shape,groups", [
+    # 3 tiles of 16 rows each: one round of 3-plane chunks on 256 places (12 planes: 48 workgroups)
+    ("fp32", 4, "48,48,48", 4 * 3 * 16),
+    # 15 tiles of 9 rows: 12 planes fill the chip more than twice
+    ("fp32", 4, "128,128,96", 4 * 15 * 11),
+    # 10 tiles of 7 rows in workgroups of 8 waves, 12 waves to a CU without poles
+    ("fp64", 2, "64,64,64", 2 * 10 * 11),
+])
+def test_default_chunk_of_a_batched_reverse_launch(fake_path, precision, count, shape, groups):
+    """Small batches take chunks short enough to fill the chip once."""
+    run_case(fake_path, "reverse_chunk", precision, count, shape, groups)
+
+
 if __name__ == "__main__":
     sys.path.insert(0, ROOT)
     globals()["case_" + sys.argv[2]](Fake(sys.argv[1]), *sys.argv[3:])
