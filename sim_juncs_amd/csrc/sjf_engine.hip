@@ -89,8 +89,6 @@ struct sjf_engine {
     double pole_bytes = 0;    // pole state the step moves
     double pole_values = 0;   // poles summed over cells and components
     size_t pol_bytes = 0;     // size of Qbuf (and of Pbuf where there is one)
-    void* stage = nullptr;    // pinned host memory of the read-outs (read_out)
-    size_t stage_bytes = 0;
     void* lut = nullptr;
     int nmat = 1;
     int maxp = 0;
@@ -269,33 +267,93 @@ double inv_eps_at(const sjf_engine* e, long q, int c, uint32_t w) {
     return 1.0 / e->lut_h[m].eps_inf;
 }
 
-// Pinned host memory of an engine's read-outs, at least `bytes` (grown to the largest chunk read, at
-// most two chunks; freed with the engine).
+// Pinned host memory of the read-outs.  A read-out takes a buffer for its duration and gives it back; at
+// most kStageKept bytes are kept for later ones (two large read-outs at a time), whatever the number of
+// engines, and none once the last engine is gone.  Allocating one costs as much as a small read-out.
 constexpr size_t kReadChunk = 4u << 20;
-int read_stage(sjf_engine* e, size_t bytes) {
-    if (bytes <= e->stage_bytes) return SJF_OK;
-    if (e->stage) (void)hipHostFree(e->stage);
-    e->stage = nullptr;
-    e->stage_bytes = 0;
-    const size_t want = std::max<size_t>(bytes, 4096);
-    if (hipHostMalloc(&e->stage, want, hipHostMallocDefault) != hipSuccess) {
-        (void)hipGetLastError();
-        e->stage = nullptr;
-        return fail(e, SJF_E_NOMEM, "read-out buffer allocation failed");
+constexpr size_t kStageKept = 4 * kReadChunk;
+struct Stage {
+    void* p;
+    size_t bytes;
+    int device;
+};
+std::mutex g_stage_mu;
+std::vector<Stage> g_stages;  // given back
+size_t g_stage_bytes = 0;     // of these
+long g_engines = 0;
+
+void stage_engines(int change) {
+    std::vector<Stage> last;
+    {
+        std::lock_guard<std::mutex> lk(g_stage_mu);
+        g_engines += change;
+        if (g_engines > 0) return;
+        last.swap(g_stages);
+        g_stage_bytes = 0;
     }
-    e->stage_bytes = want;
-    return SJF_OK;
+    for (const Stage& s : last) (void)hipHostFree(s.p);
 }
+
+// At least `bytes` of pinned memory while it lives.  done(): the device no longer writes to it.
+class StageLease {
+public:
+    StageLease(sjf_engine* e, size_t bytes) : e_(e) {
+        {
+            std::lock_guard<std::mutex> lk(g_stage_mu);
+            int best = -1;  // the smallest that holds it
+            for (int q = 0; q < (int)g_stages.size(); ++q)
+                if (g_stages[q].device == e->g.device && g_stages[q].bytes >= bytes &&
+                    (best < 0 || g_stages[q].bytes < g_stages[best].bytes))
+                    best = q;
+            if (best >= 0) {
+                s_ = g_stages[best];
+                g_stages.erase(g_stages.begin() + best);
+                g_stage_bytes -= s_.bytes;
+                return;
+            }
+        }
+        s_ = {nullptr, std::max<size_t>(bytes, 4096), e->g.device};
+        if (hipHostMalloc(&s_.p, s_.bytes, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            s_.p = nullptr;
+            e->err = "read-out buffer allocation failed";
+        }
+    }
+    StageLease(const StageLease&) = delete;
+    ~StageLease() {
+        if (!s_.p) return;
+        if (done_) {
+            std::lock_guard<std::mutex> lk(g_stage_mu);
+            if (g_stage_bytes + s_.bytes <= kStageKept) {
+                g_stages.push_back(s_);
+                g_stage_bytes += s_.bytes;
+                return;
+            }
+        } else {
+            (void)hipStreamSynchronize(e_->stream);  // a call in between failed
+        }
+        (void)hipHostFree(s_.p);
+    }
+    void* get() const { return s_.p; }
+    void done() { done_ = true; }
+
+private:
+    sjf_engine* e_;
+    Stage s_{};
+    bool done_ = false;
+};
 
 // Material words of the listed cells, through the read-out stage
 int words_at(sjf_engine* e, const std::vector<long>& cells, std::vector<uint32_t>& w) {
     const long n = (long)cells.size(), most = (long)(kReadChunk / 16);
     w.assign(n, 0u);
     if (!e->matw) return SJF_OK;  // no materials yet, or refused ones
+    if (n == 0) return SJF_OK;
+    StageLease stage(e, 16 * (size_t)std::min(n, most));
+    if (!stage.get()) return SJF_E_NOMEM;
     for (long q = 0; q < n; q += most) {
         const long m = std::min(most, n - q);
-        if (int rc = read_stage(e, 16 * (size_t)m)) return rc;
-        long* in = (long*)e->stage;
+        long* in = (long*)stage.get();
         uint32_t* out = (uint32_t*)(in + m);
         std::memcpy(in, cells.data() + q, sizeof(long) * m);
         hipLaunchKernelGGL(sjf::k_read_words, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, e->stream, e->matw, in, m, out);
@@ -303,6 +361,7 @@ int words_at(sjf_engine* e, const std::vector<long>& cells, std::vector<uint32_t
         HIPCHK(e, hipStreamSynchronize(e->stream));
         std::memcpy(w.data() + q, out, sizeof(uint32_t) * m);
     }
+    stage.done();
     return SJF_OK;
 }
 
@@ -1139,8 +1198,6 @@ int free_all(sjf_engine* e) {
     dev_free(e->coefbuf);
     for (int d = 0; d < 3; ++d) dev_free(e->psibuf[d]);
     dev_free(e->d_samples);
-    if (e->stage) (void)hipHostFree(e->stage);
-    e->stage = nullptr;
     for (auto& d : e->dft) {
         dev_free(d.acc);
         dev_free(d.cmp);
@@ -1177,8 +1234,9 @@ template <typename L>
 int read_out(sjf_engine* e, void* dst, long n, size_t size, L launch) {
     const long per = std::min<long>(n, (long)(kReadChunk / size));
     const bool one = per >= n;
-    if (int rc = read_stage(e, (one ? 1 : 2) * (size_t)per * size)) return rc;
-    char* half[2] = {(char*)e->stage, (char*)e->stage + (one ? 0 : (size_t)per * size)};
+    StageLease stage(e, (one ? 1 : 2) * (size_t)per * size);
+    if (!stage.get()) return SJF_E_NOMEM;
+    char* half[2] = {(char*)stage.get(), (char*)stage.get() + (one ? 0 : (size_t)per * size)};
     long done = 0, have = 0;  // values copied out; values of the chunk the stage holds, not yet copied
     for (long first = 0, c = 0; first < n || have > 0; ++c) {
         const long count = std::min(per, n - first);
@@ -1192,6 +1250,7 @@ int read_out(sjf_engine* e, void* dst, long n, size_t size, L launch) {
         have = std::max(count, 0L);
         HIPCHK(e, hipStreamSynchronize(e->stream));
     }
+    stage.done();
     return SJF_OK;
 }
 
@@ -2379,6 +2438,7 @@ int sjf_create(const sjf_grid* g, sjf_engine** out) {
         return SJF_E_HIP;
     }
     if (int rc = scratch_setup(g->device)) return rc;
+    stage_engines(1);
     sjf_engine* e = new sjf_engine();
     e->g = *g;
     e->prec = g->precision;
@@ -2388,6 +2448,7 @@ int sjf_create(const sjf_grid* g, sjf_engine** out) {
     if (st != hipSuccess) {
         g_create_error = std::string("hipStreamCreate: ") + hipGetErrorString(st);
         delete e;
+        stage_engines(-1);
         return SJF_E_HIP;
     }
     auto bail = [&](int rc) {
@@ -2395,6 +2456,7 @@ int sjf_create(const sjf_grid* g, sjf_engine** out) {
         free_all(e);
         (void)hipStreamDestroy(e->stream);
         delete e;
+        stage_engines(-1);
         return rc;
     };
     for (int b = 0; b < 2; ++b) {
@@ -2439,6 +2501,7 @@ int sjf_destroy(sjf_engine* e) {
     free_all(e);
     (void)hipStreamDestroy(e->stream);
     delete e;
+    stage_engines(-1);
     return SJF_OK;
 }
 

@@ -33,6 +33,8 @@ struct State {
     char* base = nullptr;
     size_t used = 0, live_bytes = 0;
     std::map<uintptr_t, size_t> live;
+    std::map<void*, size_t> host;  // pinned
+    size_t host_bytes = 0;
     std::map<const void*, std::string> kernels;
     std::map<const void*, std::pair<void*, size_t>> vars;
     long countdown = -1;  // allocations until one fails; -1: none does
@@ -106,6 +108,7 @@ extern "C" {
 void fake_fail_at(long n) { st().countdown = n; }          // the n-th allocation from now (0: the next)
 long fake_allocations() { return st().allocations; }
 double fake_live_bytes() { return (double)st().live_bytes; }
+double fake_host_bytes() { return (double)st().host_bytes; }  // pinned host memory
 long fake_steps() { return st().steps; }                   // fused steps launched
 int fake_last_stale() { return st().last_step.stale; }
 const char* fake_last_kernel() { return st().last_step.kernel.c_str(); }
@@ -148,9 +151,16 @@ int hipFree(void* p) {
 }
 int hipHostMalloc(void** p, size_t n, unsigned) {
     *p = malloc(n);
-    return *p ? kOk : kOutOfMemory;
+    if (!*p) return result(kOutOfMemory);
+    st().host[*p] = n;
+    st().host_bytes += n;
+    return kOk;
 }
 int hipHostFree(void* p) {
+    const auto it = st().host.find(p);
+    if (it == st().host.end()) return result(kInvalidValue);
+    st().host_bytes -= it->second;
+    st().host.erase(it);
     free(p);
     return kOk;
 }

@@ -36,6 +36,7 @@ class Fake:
     def __init__(self, path):
         self.lib = C.CDLL(path, mode=C.RTLD_GLOBAL)
         for f, res in (("fake_log", C.c_char_p), ("fake_last_kernel", C.c_char_p), ("fake_live_bytes", C.c_double),
+                       ("fake_host_bytes", C.c_double),
                        ("fake_steps", C.c_long), ("fake_refused", C.c_long), ("fake_allocations", C.c_long),
                        ("fake_last_table", C.c_size_t)):
             getattr(self.lib, f).restype = res
@@ -377,6 +378,30 @@ def case_reverse_chunk(fake, precision, count, shape, groups):
 def test_default_chunk_of_a_batched_reverse_launch(fake_path, precision, count, shape, groups):
     """Small batches take chunks short enough to fill the chip once."""
     run_case(fake_path, "reverse_chunk", precision, count, shape, groups)
+
+
+# ---- read-outs ----------------------------------------------------------------------------------
+
+def case_pinned_memory(fake):
+    """Read-outs keep at most 16 MiB of pinned memory however many engines read, and none without one."""
+    from sim_juncs_amd.engine import Engine
+
+    most, kept = 16 << 20, []
+    for _ in range(2):
+        engines = [Engine((128, 128, 80), 0.02) for _ in range(6)]  # 10 MB of FP64 values per component
+        for e in engines:
+            e.step(1)
+            e.read_field("Ex")
+            e.get_field("Ey", (0.1, 0.1, 0.1))
+            e.read_field("Hz", (3, 3, 3), (100, 90, 20))
+            kept.append(fake.host_bytes())
+        for e in engines:
+            e.close()
+        assert 0 < max(kept) <= most and fake.host_bytes() == 0
+
+
+def test_read_outs_share_their_pinned_memory(fake_path):
+    run_case(fake_path, "pinned_memory")
 
 
 if __name__ == "__main__":
