@@ -382,9 +382,10 @@ constexpr double kAdjStreamBytes = 128e6;
 // 70.4; FP64 128x128x100 (350 MB) 87.5, 78.4; FP32 192x192x96 (386 MB) 80.0, 74.6; FP32 200x200x125
 // (592 MB) 125.2, 113.9.
 constexpr double kStreamBytes = 300e6;
-// What one step touches: two field sets, pole state, PML auxiliaries, material words
+// What one fused step touches: two field sets, pole state, PML auxiliaries, material words, eps maps
 double step_set_bytes(const sjf_engine* e) {
     double b = field_bytes(e) + e->pole_bytes + (e->uniform ? 0.0 : 4.0 * (double)e->N);
+    if (e->emap) b += 3.0 * e->prec * (double)e->N;
     for (int d = 0; d < 3; ++d) b += 6.0 * e->prec * (double)e->slab[d];
     return b;
 }

@@ -380,6 +380,29 @@ def test_default_chunk_of_a_batched_reverse_launch(fake_path, precision, count, 
     run_case(fake_path, "reverse_chunk", precision, count, shape, groups)
 
 
+def case_store_hint(fake, precision, shape, maps, hint):
+    """Sides of the line (300 MB) from which stores take the non-temporal hint."""
+    from sim_juncs_amd.engine import Engine
+
+    shape = tuple(map(int, shape.split(",")))
+    e = Engine(shape, 0.02, precision=precision)
+    if maps == "maps":
+        e.set_eps_maps(np.full((3,) + shape, 2.0))
+    e.step(1)
+    assert fake.last_kernel().decode().split(">")[0].endswith(hint.lower())
+
+
+@pytest.mark.parametrize("precision,shape,maps,hint", [
+    # cells x (96 fields, 4 words, 24 maps) bytes in FP64, x (48, 4, 12) in FP32
+    ("fp64", "136,136,136", "maps", True), ("fp64", "136,136,136", "no", False),  # 312 MB, 241 MB
+    ("fp64", "132,132,136", "maps", False),                                       # 294 MB
+    ("fp32", "170,170,166", "maps", True), ("fp32", "170,170,166", "no", False),  # 307 MB, 230 MB
+    ("fp32", "166,166,168", "maps", False),                                       # 296 MB
+])
+def test_eps_maps_count_in_what_a_step_touches(fake_path, precision, shape, maps, hint):
+    run_case(fake_path, "store_hint", precision, shape, maps, hint)
+
+
 # ---- read-outs ----------------------------------------------------------------------------------
 
 def case_pinned_memory(fake):
