@@ -370,10 +370,6 @@ bool thread_rows_fit(const sjf_engine* e, int rows) { return rows >= 1 && (long)
 
 double field_bytes(const sjf_engine* e) { return 12.0 * e->prec * (double)e->N; }
 
-// Field bytes above which the one-row reverse step stores with the non-temporal hint (measured on
-// MI355X: 256x256x128 FP32 0.282 -> 0.267 ms).
-constexpr double kAdjStreamBytes = 128e6;
-
 // Bytes one step touches above which its stores take the non-temporal hint: below, the 256 MB Infinity
 // Cache holds what a step wrote until the next one reads it.  Pole state counts in whole 64-cell
 // segments, so the line lies above that size.  Measured on MI355X, us per step without and with the
@@ -1674,8 +1670,9 @@ void launch_adj_one_row(sjf_engine* e, const sjf::AdjArgs<T>& g, int block, unsi
 
 template <typename T, int NP>
 void launch_adj_np(sjf_engine* e, const sjf::AdjArgs<T>& g, int block, unsigned tiles, size_t lds) {
-    // the reverse step streams the adjoint fields as the forward step streams E and H
-    if (field_bytes(e) > kAdjStreamBytes) launch_adj_one_row<T, NP, true>(e, g, block, tiles, lds);
+    // the reverse step streams the adjoint fields as the forward step streams E and H: the same line, alone
+    // and in a batch (FP64 70x70x300, 141 MB of fields: 106 us without the hint, 117 with it)
+    if (step_set_bytes(e) > kStreamBytes) launch_adj_one_row<T, NP, true>(e, g, block, tiles, lds);
     else launch_adj_one_row<T, NP, false>(e, g, block, tiles, lds);
 }
 

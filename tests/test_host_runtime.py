@@ -403,6 +403,30 @@ def test_eps_maps_count_in_what_a_step_touches(fake_path, precision, shape, maps
     run_case(fake_path, "store_hint", precision, shape, maps, hint)
 
 
+def case_reverse_hint(fake, shape, hint):
+    from sim_juncs_amd.engine import Batch, Engine
+
+    shape = tuple(map(int, shape.split(",")))
+    for batch in (False, True):
+        e = Engine(shape, 0.02, precision="fp64")
+        e.set_design_eps((2, 2, 2), (4, 4, 4), np.full((2, 2, 2), 3.0))
+        fake.clear_log()
+        if batch:
+            b = Batch([e])
+            b.adjoint_run(2, [(1, 1, 1)], [8])
+            b.close()
+        else:
+            e.adjoint_run(2, 0, (1, 1, 1), 8)
+        e.close()
+        names = {x.split(">")[0] for x in fake.log().decode().split("\n") if "k_adj_step" in x}
+        assert len(names) == 1 and names.pop().endswith(hint.lower()), batch
+
+
+@pytest.mark.parametrize("shape,hint", [("70,70,300", False), ("110,110,300", True)])  # 147 and 363 MB
+def test_reverse_stores_follow_the_forward_line_alone_and_in_a_batch(fake_path, shape, hint):
+    run_case(fake_path, "reverse_hint", shape, hint)
+
+
 # ---- read-outs ----------------------------------------------------------------------------------
 
 def case_pinned_memory(fake):
