@@ -403,6 +403,34 @@ def test_eps_maps_count_in_what_a_step_touches(fake_path, precision, shape, maps
     run_case(fake_path, "store_hint", precision, shape, maps, hint)
 
 
+def case_store_scenes(fake, index):
+    import test_gpu_store_hint as g
+
+    from sim_juncs_amd.engine import Batch
+
+    precision, shape, count, tile, kernel = g.CASES[int(index)]
+    grouped = g.engines(precision, shape, count)
+    (single,) = g.engines(precision, shape, 1)
+    g.alone(single, tile)
+    single.step(1)
+    threads = fake.last_block()
+    off = fake.last_kernel().decode()
+    b = Batch(grouped)
+    if tile:
+        b.set_tile(*tile)
+    b.step(1)
+    on = fake.last_kernel().decode()
+    assert kernel in off and off.split(">")[0].endswith("false"), off
+    assert kernel in on and on.split(">")[0].endswith("true"), on
+    assert off.replace("false", "true") == on and fake.last_block() == threads
+
+
+@pytest.mark.parametrize("index", range(6))
+def test_scenes_lie_on_either_side_of_the_store_line(fake_path, index):
+    """The scenes of test_gpu_store_hint.py run the kernels that it means to compare."""
+    run_case(fake_path, "store_scenes", index)
+
+
 def case_reverse_hint(fake, shape, hint):
     from sim_juncs_amd.engine import Batch, Engine
 
@@ -452,5 +480,5 @@ def test_read_outs_share_their_pinned_memory(fake_path):
 
 
 if __name__ == "__main__":
-    sys.path.insert(0, ROOT)
+    sys.path[:0] = [ROOT, HERE]
     globals()["case_" + sys.argv[2]](Fake(sys.argv[1]), *sys.argv[3:])
