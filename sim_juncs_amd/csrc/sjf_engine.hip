@@ -444,6 +444,33 @@ int round_chunk(int nx, int nty, long slots, int extra) {
     return xc;
 }
 
+// Workgroups of w wavefronts that a CU holds at once where the registers leave `waves` per SIMD.  Beyond
+// four wavefronts a workgroup is placed only where every SIMD has room for the most that it puts on one: of
+// five wavefronts 3, 2 and 1 fit at 5, 4 and 3 per SIMD, not 4, 3 and 2 (43x46x320 FP32 with gold, 4 per
+// SIMD: 690 workgroups of 3 planes 30.3 us, 506 of 4 planes 24.9; without poles, 5 per SIMD: 1012 of 2
+// planes 26.2, 690 of 3 22.5; 32x35x300 FP64 without poles, 3 per SIMD: 385 of 3 planes 30.6, 245 of 5
+// 25.7), of six 2 and 1 at 5 and 3 (40x43x384 FP32: 602 of 3 planes 27.0, 430 of 4 23.4).
+int resident(int w, int waves) {
+    const int most = (w + 3) / 4;
+    if (w <= 4) return std::max(1, 4 * waves / w);
+    int n = std::max(1, waves / most);
+    if (w % 4 == 1)  // the odd wavefront goes to another SIMD each time
+        for (n = 1; (n * w + 3) / 4 + most <= waves;) ++n;
+    return n;
+}
+
+// x-chunk of a tile whose workgroups have w wavefronts: round_chunk on the places that the registers leave,
+// or, where fewer workgroups are resident and that would make a second round, the shortest chunk that runs
+// in one if it saves 15 % of the planes (less was as often lost as gained).
+int resident_chunk(int nx, int nty, int w, int waves) {
+    const long all = 256L * std::max(1, 4 * waves / w), held = 256L * resident(w, waves);
+    const int xc = round_chunk(nx, nty, all, 2);
+    if (held >= all || nty > held) return xc;
+    const int nxc = (int)std::min<long>(nx, held / nty), one = (nx + nxc - 1) / nxc;
+    const long rounds = ((long)nty * ((nx + xc - 1) / xc) + held - 1) / held;
+    return one <= 64 && 1.15 * (one + 2) < (double)rounds * (xc + 2) ? one : xc;
+}
+
 int tiles_of(const sjf_engine* e, int ty, int xc) {
     const int nty = (e->g.ny + ty - 1) / ty;
     const int nxc = (e->g.nx + xc - 1) / xc;
@@ -1138,8 +1165,7 @@ void choose_tile(sjf_engine* e) {
     e->form = thread_rows ? SJF_TILE_THREAD_ROWS : SJF_TILE_REGISTER_ROWS;
     e->ty = thread_rows ? rows : 1;
     const int waves = e->prec == 4 ? tile_waves<float>(e) : tile_waves<double>(e);
-    const long slots = 256L * std::max(1, 4 * waves / (block_threads(e) / 64));
-    e->xc = round_chunk(e->g.nx, (e->g.ny + e->ty - 1) / e->ty, slots, 2);
+    e->xc = resident_chunk(e->g.nx, (e->g.ny + e->ty - 1) / e->ty, block_threads(e) / 64, waves);
 }
 
 // Default form of a batch: thread rows where some instance would take them alone (choose_tile) and all

@@ -380,6 +380,29 @@ def test_default_chunk_of_a_batched_reverse_launch(fake_path, precision, count, 
     run_case(fake_path, "reverse_chunk", precision, count, shape, groups)
 
 
+def case_chunk(fake, precision, shape, xchunk):
+    from sim_juncs_amd.engine import Engine
+
+    e = Engine(tuple(map(int, shape.split(","))), 0.02, precision=precision)
+    assert e.launch_info()["xchunk"] == int(xchunk)
+    e.step(1)
+    assert fake.last_grid() == e.launch_info()["groups"]
+
+
+@pytest.mark.parametrize("precision,shape,xchunk", [
+    ("fp32", "43,46,320", 3),    # five wavefronts: three workgroups to a CU, 768 places
+    ("fp32", "40,43,384", 4),    # six: two
+    ("fp32", "44,46,512", 4),    # eight: two, as the registers alone say
+    ("fp64", "32,35,300", 5),    # five at three per SIMD: one
+    ("fp64", "45,48,180", 3),    # three wavefronts pack as the registers say
+    ("fp64", "125,128,320", 32),  # one round would save too little
+    ("fp32", "6,2000,300", 6),   # more rows than places: whole lines
+])
+def test_default_chunk_of_one_row_tiles(fake_path, precision, shape, xchunk):
+    """Chunks that run in one round of the workgroups a CU really holds."""
+    run_case(fake_path, "chunk", precision, shape, xchunk)
+
+
 def case_store_hint(fake, precision, shape, maps, hint):
     """Sides of the line (300 MB) from which stores take the non-temporal hint."""
     from sim_juncs_amd.engine import Engine
