@@ -38,6 +38,7 @@ struct Source {
     sjf::PulseDev dev;
     std::vector<long> idx;
     std::vector<double> wt;
+    std::vector<int> ids[3];  // its cells: the product of these, each ascending
 };
 
 struct Monitor {
@@ -230,6 +231,10 @@ void axis_weights(int n, double dx, double off, int periodic, double lo, double 
             if (ww == 0.0) continue;
             if (periodic) i = ((i % n) + n) % n;
             else if (i < 0 || i >= n) continue;
+            if (!ids.empty() && ids.back() == i) {  // a periodic axis of one cell: both images are it
+                w.back() += ww;
+                continue;
+            }
             ids.push_back(i);
             w.push_back(ww);
         }
@@ -556,7 +561,7 @@ struct LaunchSet {
     long* d_blk_end = nullptr;
     long* d_src_idx = nullptr;
     double* d_src_coef = nullptr;
-    int nsrcblk = 0;
+    std::vector<int> src_at;  // first workgroup of each layer (source_layers) and their number
     // magnetic sources (injected into H before the fused update), same table layout
     void* d_hsrc = nullptr;
     int* d_hblk_src = nullptr;
@@ -564,7 +569,7 @@ struct LaunchSet {
     long* d_hblk_end = nullptr;
     long* d_hsrc_idx = nullptr;
     double* d_hsrc_coef = nullptr;
-    int nhsrcblk = 0;
+    std::vector<int> hsrc_at;
     // monitors
     void* d_mon = nullptr;
     int nmon = 0;
@@ -598,7 +603,8 @@ void set_free_tables(LaunchSet* s) {
     dev_free(s->d_hblk_end);
     dev_free(s->d_hsrc_idx);
     dev_free(s->d_hsrc_coef);
-    s->nsrcblk = s->nhsrcblk = 0;
+    s->src_at.clear();
+    s->hsrc_at.clear();
     dev_free(s->d_mon);
     dev_free(s->d_dft);
     dev_free(s->d_counters);
@@ -621,6 +627,28 @@ int upload_vec(sjf_engine* e, hipStream_t st, void** dst, const std::vector<V>& 
         if (rc != hipSuccess) return fail(e, SJF_E_HIP, hipGetErrorString(rc));
     }
     return SJF_OK;
+}
+
+// Whether two sources inject into a common value
+bool sources_meet(const Source& a, const Source& b) {
+    if (a.comp != b.comp) return false;
+    for (int d = 0; d < 3; ++d) {
+        size_t i = 0, j = 0;
+        const std::vector<int>&p = a.ids[d], &q = b.ids[d];
+        while (i < p.size() && j < q.size() && p[i] != q[j]) ++(p[i] < q[j] ? i : j);
+        if (i == p.size() || j == q.size()) return false;
+    }
+    return true;
+}
+
+// Layer of each source of an engine: sources of a layer share no value, so that one launch adds them
+// without a race; sources that meet are added in the order in which they were given.
+std::vector<int> source_layers(const std::vector<Source>& src) {
+    std::vector<int> layer(src.size(), 0);
+    for (size_t b = 1; b < src.size(); ++b)
+        for (size_t a = 0; a < b; ++a)
+            if (layer[a] >= layer[b] && sources_meet(src[a], src[b])) layer[b] = layer[a] + 1;
+    return layer;
 }
 
 template <typename T>
@@ -674,40 +702,51 @@ int build_set_t(LaunchSet* s) {
     if (!rc) rc = upload_vec(e0, s->stream, (void**)&s->d_tile_first, first);
     if (rc) return rc;
 
-    // sources: entries of every source of every engine, in blocks of 256 of one source; electric
-    // sources (coefficient dt * weight / eps) and magnetic ones (dt * weight, mu = 1) in separate
-    // tables
+    // sources: entries of every source of every engine, in blocks of 256 of one source, layer by layer;
+    // electric sources (coefficient dt * weight / eps) and magnetic ones (dt * weight, mu = 1) in
+    // separate tables
+    std::vector<std::vector<int>> layers;
+    int nlayer = 0;
+    for (sjf_engine* e : s->eng) {
+        layers.push_back(source_layers(e->src));
+        for (const int l : layers.back()) nlayer = std::max(nlayer, l + 1);
+    }
     for (int mag = 0; mag < 2; ++mag) {
         std::vector<sjf::SrcDev<T>> srcs;
-        std::vector<int> blk_src;
+        std::vector<int> blk_src, at(1, 0);
         std::vector<long> blk_first, blk_end, idx;
         std::vector<double> coef;
-        for (sjf_engine* e : s->eng) {
-            for (const Source& src : e->src) {
-                if (src.idx.empty() || (src.comp >= 3) != (mag == 1)) continue;
-                sjf::SrcDev<T> d;
-                std::memset(&d, 0, sizeof(d));
-                d.p = src.dev;
-                d.p.part = e->g.part;
-                d.p.dt = e->dt;
-                for (int b = 0; b < 2; ++b) d.F[b] = (T*)e->Fbuf[b];
-                d.d_step = e->d_step;
-                const int sid = (int)srcs.size();
-                srcs.push_back(d);
-                const long base = (long)idx.size();
-                std::vector<uint32_t> word;
-                if (!mag && (rc = words_at(e, src.idx, word))) return rc;
-                for (size_t q = 0; q < src.idx.size(); ++q) {
-                    idx.push_back(sjf::field_index(src.idx[q], src.comp, (long)e->g.ny * e->g.nz));
-                    coef.push_back(e->dt * src.wt[q] * (mag ? 1.0 : inv_eps_at(e, src.idx[q], src.comp, word[q])));
-                }
-                const long n = (long)src.idx.size();
-                for (long b = 0; b < n; b += 256) {
-                    blk_src.push_back(sid);
-                    blk_first.push_back(base + b);
-                    blk_end.push_back(base + std::min(n, b + 256));
+        for (int layer = 0; layer < nlayer; ++layer) {
+            for (size_t i = 0; i < s->eng.size(); ++i) {
+                sjf_engine* e = s->eng[i];
+                for (size_t k = 0; k < e->src.size(); ++k) {
+                    const Source& src = e->src[k];
+                    if (layers[i][k] != layer || src.idx.empty() || (src.comp >= 3) != (mag == 1)) continue;
+                    sjf::SrcDev<T> d;
+                    std::memset(&d, 0, sizeof(d));
+                    d.p = src.dev;
+                    d.p.part = e->g.part;
+                    d.p.dt = e->dt;
+                    for (int b = 0; b < 2; ++b) d.F[b] = (T*)e->Fbuf[b];
+                    d.d_step = e->d_step;
+                    const int sid = (int)srcs.size();
+                    srcs.push_back(d);
+                    const long base = (long)idx.size();
+                    std::vector<uint32_t> word;
+                    if (!mag && (rc = words_at(e, src.idx, word))) return rc;
+                    for (size_t q = 0; q < src.idx.size(); ++q) {
+                        idx.push_back(sjf::field_index(src.idx[q], src.comp, (long)e->g.ny * e->g.nz));
+                        coef.push_back(e->dt * src.wt[q] * (mag ? 1.0 : inv_eps_at(e, src.idx[q], src.comp, word[q])));
+                    }
+                    const long n = (long)src.idx.size();
+                    for (long b = 0; b < n; b += 256) {
+                        blk_src.push_back(sid);
+                        blk_first.push_back(base + b);
+                        blk_end.push_back(base + std::min(n, b + 256));
+                    }
                 }
             }
+            if ((int)blk_src.size() > at.back()) at.push_back((int)blk_src.size());
         }
         const int nblk = (int)blk_src.size();
         if (!nblk) continue;
@@ -717,7 +756,7 @@ int build_set_t(LaunchSet* s) {
         long** tbe = mag ? &s->d_hblk_end : &s->d_blk_end;
         long** tidx = mag ? &s->d_hsrc_idx : &s->d_src_idx;
         double** tcoef = mag ? &s->d_hsrc_coef : &s->d_src_coef;
-        (mag ? s->nhsrcblk : s->nsrcblk) = nblk;
+        (mag ? s->hsrc_at : s->src_at) = at;
         rc = upload_vec(e0, s->stream, tsrc, srcs);
         if (!rc) rc = upload_vec(e0, s->stream, (void**)tbs, blk_src);
         if (!rc) rc = upload_vec(e0, s->stream, (void**)tbf, blk_first);
@@ -787,7 +826,7 @@ int build_set_t(LaunchSet* s) {
     s->dft_total = tot;
     // sources and DFT can share a launch when no DFT region of an engine holds one of its
     // source cells
-    s->src_dft_one_launch = s->nsrcblk > 0 && s->ndft > 0;
+    s->src_dft_one_launch = !s->src_at.empty() && s->ndft > 0;
     for (sjf_engine* e : s->eng) {
         const long nyz = (long)e->g.ny * e->g.nz;
         for (const Source& src : e->src)
@@ -805,7 +844,7 @@ int build_set_t(LaunchSet* s) {
     const long per_freq = (tot + 255) / 256;
     if (per_freq > most) return fail(e0, SJF_E_UNSUPPORTED, "DFT regions exceed 2^32 values per frequency");
     s->dft_blocks = (int)per_freq;
-    if (s->nsrcblk + per_freq * s->dft_maxnf > most) s->src_dft_one_launch = false;
+    if (s->src_dft_one_launch && s->src_at.back() + per_freq * s->dft_maxnf > most) s->src_dft_one_launch = false;
     if (s->ndft) {
         rc = upload_vec(e0, s->stream, &s->d_dft, regs);
         if (rc) return rc;
@@ -903,10 +942,11 @@ int launch_one_step_t(LaunchSet* s, bool sample, hipEvent_t ev_a, hipEvent_t ev_
                            (const sjf::MonDev<T>*)s->d_mon, s->nmon);
         SETCHK(s, hipGetLastError());
     }
-    if (s->nhsrcblk) {
-        const sjf::SrcTables<T> ht{(const sjf::SrcDev<T>*)s->d_hsrc, s->d_hblk_src, s->d_hblk_first,
-                                   s->d_hblk_end, s->d_hsrc_idx, s->d_hsrc_coef};
-        hipLaunchKernelGGL((sjf::k_source_h<T>), dim3(s->nhsrcblk), dim3(256), 0, s->stream, ht);
+    for (size_t l = 0; l + 1 < s->hsrc_at.size(); ++l) {
+        const int first = s->hsrc_at[l], blocks = s->hsrc_at[l + 1] - first;
+        const sjf::SrcTables<T> ht{(const sjf::SrcDev<T>*)s->d_hsrc, s->d_hblk_src + first, s->d_hblk_first + first,
+                                   s->d_hblk_end + first, s->d_hsrc_idx, s->d_hsrc_coef};
+        hipLaunchKernelGGL((sjf::k_source_h<T>), dim3(blocks), dim3(256), 0, s->stream, ht);
         SETCHK(s, hipGetLastError());
     }
     if (ev_a) SETCHK(s, hipEventRecord(ev_a, s->stream));
@@ -917,26 +957,28 @@ int launch_one_step_t(LaunchSet* s, bool sample, hipEvent_t ev_a, hipEvent_t ev_
     // one, else the source kernel, else k_tick
     const int n = (int)s->eng.size();
     const bool dft = s->ndft && !bare;
-    const sjf::SrcTables<T> st{(const sjf::SrcDev<T>*)s->d_src, s->d_blk_src, s->d_blk_first, s->d_blk_end,
-                               s->d_src_idx, s->d_src_coef};
-    const sjf::Tick tick{s->d_counters, n};
-    if (dft && s->src_dft_one_launch) {
-        hipLaunchKernelGGL((sjf::k_source_dft<T>), dim3((unsigned)(s->nsrcblk + s->dft_blocks * s->dft_maxnf)), dim3(256), 0,
-                           s->stream, st, s->nsrcblk, (const sjf::DftDev<T>*)s->d_dft, s->ndft, s->dft_total,
-                           s->dft_blocks, tick);
-        SETCHK(s, hipGetLastError());
-        return SJF_OK;
-    }
-    if (s->nsrcblk) {
-        const sjf::Tick src_tick{s->d_counters, dft ? 0 : n};
-        hipLaunchKernelGGL((sjf::k_source<T>), dim3(s->nsrcblk), dim3(256), 0, s->stream, st, src_tick);
+    const sjf::Tick tick{s->d_counters, n}, none{s->d_counters, 0};
+    const size_t nlayer = s->src_at.empty() ? 0 : s->src_at.size() - 1;
+    for (size_t l = 0; l < nlayer; ++l) {
+        const int first = s->src_at[l], blocks = s->src_at[l + 1] - first;
+        const bool last = l + 1 == nlayer;
+        const sjf::SrcTables<T> st{(const sjf::SrcDev<T>*)s->d_src, s->d_blk_src + first, s->d_blk_first + first,
+                                   s->d_blk_end + first, s->d_src_idx, s->d_src_coef};
+        if (last && dft && s->src_dft_one_launch) {
+            hipLaunchKernelGGL((sjf::k_source_dft<T>), dim3((unsigned)(blocks + s->dft_blocks * s->dft_maxnf)), dim3(256), 0,
+                               s->stream, st, blocks, (const sjf::DftDev<T>*)s->d_dft, s->ndft, s->dft_total,
+                               s->dft_blocks, tick);
+            SETCHK(s, hipGetLastError());
+            return SJF_OK;
+        }
+        hipLaunchKernelGGL((sjf::k_source<T>), dim3(blocks), dim3(256), 0, s->stream, st, last && !dft ? tick : none);
         SETCHK(s, hipGetLastError());
     }
     if (dft) {
         hipLaunchKernelGGL((sjf::k_dft<T>), dim3((unsigned)s->dft_blocks, (unsigned)s->dft_maxnf), dim3(256), 0, s->stream,
                            (const sjf::DftDev<T>*)s->d_dft, s->ndft, s->dft_total, tick);
         SETCHK(s, hipGetLastError());
-    } else if (!s->nsrcblk) {
+    } else if (nlayer == 0) {
         hipLaunchKernelGGL(sjf::k_tick, dim3((n + 63) / 64), dim3(64), 0, s->stream, s->d_counters, n);
         SETCHK(s, hipGetLastError());
     }
@@ -2760,6 +2802,10 @@ int sjf_add_source(sjf_engine* e, int comp, const double box[6], const sjf_pulse
                 s.idx.push_back(cell_index(e, ids[0][a], ids[1][b], ids[2][c]));
                 s.wt.push_back(ws[0][a] * ws[1][b] * ws[2][c]);
             }
+    for (int d = 0; d < 3; ++d) {
+        s.ids[d] = ids[d];
+        std::sort(s.ids[d].begin(), s.ids[d].end());
+    }
     e->src.push_back(std::move(s));
     e->version++;
     return SJF_OK;

@@ -41,7 +41,7 @@ struct State {
     long allocations = 0;
     int bad_copies = 0;  // copies from, to, or word passes over memory that is not live
     Launch last_step;
-    long steps = 0, launches = 0, refused = 0;
+    long steps = 0, launches = 0, refused = 0, entries = 0, shared = 0;
     std::string log, words;
     dim3 grid, block;
     size_t shmem = 0;
@@ -119,6 +119,8 @@ size_t fake_last_table(char* out, size_t cap) {            // the argument table
     memcpy(out, t.data(), t.size() < cap ? t.size() : cap);
     return t.size();
 }
+long fake_source_entries() { return st().entries; }  // entries of all source launches (of one engine each)
+long fake_source_shared() { return st().shared; }    // of these, on a value that another entry of the launch writes
 long fake_refused() { return st().refused; }
 int fake_bad_copies() { return st().bad_copies; }
 int fake_first_word() {                                    // first given material word of the last k_words launch
@@ -225,6 +227,18 @@ int hipLaunchKernel(const void* f, dim3 grid, dim3 block, void** args, size_t sh
     if (l.refused) {
         s.refused++;
         return result(kInvalidConfiguration);
+    }
+    if (l.kernel.find("::k_source") != std::string::npos) {
+        // SrcTables: sources, and per workgroup its source and entries first .. end - 1; per entry a value's index
+        const void* const* t = (const void* const*)args[0];
+        const long *first = (const long*)t[2], *end = (const long*)t[3], *idx = (const long*)t[4];
+        const int blocks = l.kernel.find("k_source_dft") != std::string::npos ? *(const int*)args[1] : (int)grid.x;
+        std::map<long, int> seen;
+        for (int b = 0; b < blocks; ++b)
+            for (long q = first[b]; q < end[b]; ++q) {
+                s.entries++;
+                if (seen[idx[q]]++) s.shared++;
+            }
     }
     if (l.kernel.find("::k_words<") != std::string::npos) {  // given, matw, seg, lut: all have to be there
         for (int q = 0; q < 4; ++q)

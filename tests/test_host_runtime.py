@@ -37,7 +37,7 @@ class Fake:
         self.lib = C.CDLL(path, mode=C.RTLD_GLOBAL)
         for f, res in (("fake_log", C.c_char_p), ("fake_last_kernel", C.c_char_p), ("fake_live_bytes", C.c_double),
                        ("fake_host_bytes", C.c_double),
-                       ("fake_steps", C.c_long), ("fake_refused", C.c_long), ("fake_allocations", C.c_long),
+                       ("fake_steps", C.c_long), ("fake_refused", C.c_long), ("fake_source_entries", C.c_long), ("fake_source_shared", C.c_long), ("fake_allocations", C.c_long),
                        ("fake_last_table", C.c_size_t)):
             getattr(self.lib, f).restype = res
         self.lib.fake_fail_at.argtypes = [C.c_long]
@@ -78,6 +78,40 @@ def case_dft_launch(fake, source):
 @pytest.mark.parametrize("source", ["inside", "outside"])
 def test_dft_of_many_values_and_many_frequencies_is_launched(fake_path, source):
     run_case(fake_path, "dft_launch", source)
+
+
+# ---- sources ------------------------------------------------------------------------------------
+
+def case_shared_cells(fake, which):
+    """No launch has two threads add to one value: sources that share cells go out one after another."""
+    from sim_juncs_amd.engine import Engine
+
+    shape, periodic = (12, 11, 14), (0, 0, 0)
+    if which == "thin":
+        shape, periodic = (1, 1, 14), (1, 1, 0)
+    e = Engine(shape, 0.1, periodic=periodic)
+    pulse = dict(freq=1.0, width=0.3, t_start=-1.0, t_end=2.0)
+    sheet = [0.0, 0.0, 0.6, 0.1 * shape[0], 0.1 * shape[1], 0.6]
+    expect = 1
+    if which == "thin":
+        e.add_source("Ex", [0.03, 0.07, 0.63] * 2, **pulse)
+    else:
+        comps = {"electric": ("Ex",) * 3, "magnetic": ("Hy",) * 3, "mixed": ("Ex", "Ey", "Ex", "Hx", "Hx")}[which]
+        for c in comps:
+            e.add_source(c, sheet, **pulse)
+        e.add_source(comps[0], [0.55, 0.55, 0.6] * 2, **pulse)
+        e.add_source(comps[0], [0.5, 0.5, 1.1] * 2, **pulse)  # apart from the sheets
+        expect = 4 if which != "mixed" else 3 + 2
+    e.add_dft((0, 0, 13), shape, ("Ex",), [1.0])
+    e.step(2)
+    launches = [x for x in fake.log().decode().split("\n") if "k_source" in x]
+    assert fake.source_shared() == 0 and fake.source_entries() > 0
+    assert len(launches) == 2 * expect, launches
+
+
+@pytest.mark.parametrize("which", ["electric", "magnetic", "mixed", "thin"])
+def test_sources_that_share_cells_do_not_share_a_launch(fake_path, which):
+    run_case(fake_path, "shared_cells", which)
 
 
 # ---- allocations that fail ----------------------------------------------------------------------
