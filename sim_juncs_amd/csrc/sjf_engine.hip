@@ -2936,7 +2936,12 @@ int sjf_add_dft(sjf_engine* e, const int lo[3], const int hi[3], int comp_mask, 
     if (!rc) rc = dev_alloc(e, (void**)&d.cmp, bytes);
     if (!rc) rc = dev_alloc(e, (void**)&d.d_freq, sizeof(double) * nf);
     if (!rc) rc = h2d(e, d.d_freq, d.freqs.data(), sizeof(double) * nf);
-    if (rc) return rc;
+    if (rc) {
+        dev_free(d.acc);
+        dev_free(d.cmp);
+        dev_free(d.d_freq);
+        return rc;
+    }
     e->dft.push_back(d);
     *id = (int)e->dft.size() - 1;
     e->version++;

@@ -158,6 +158,51 @@ def test_a_failed_allocation_is_not_reported_by_the_next_step(fake_path):
     run_case(fake_path, "failed_allocation")
 
 
+def case_no_leak(fake):
+    """Each allocation of each of these calls fails in turn: the call can be made again, and nothing is
+    left once the engine is closed."""
+    from sim_juncs_amd import materials as M
+    from sim_juncs_amd._lib import EngineError
+    from sim_juncs_amd.engine import Engine
+
+    def engine():
+        e = Engine(SHAPE, 0.02, precision="fp64")
+        e.set_materials(_blocks([0, 1]), [M.VACUUM, M.AU.scaled(1.0)])
+        e.set_pml([2] * 6)
+        e.set_design_eps((2, 2, 2), (4, 4, 4), np.full((2, 2, 2), 3.0))
+        for c in ("Ex", "Hy"):
+            e.add_source(c, [0.1, 0.1, 0.1] * 2, freq=1.0, width=1.0, t_end=10.0)
+        e.add_monitors("Ex", [[0.1, 0.1, 0.1]])
+        return e
+
+    calls = {
+        "dft": lambda e: e.add_dft((1, 1, 1), (3, 3, 3), ("Ex",), [1.0]),
+        "step": lambda e: e.step(2),
+        "record": lambda e: e.adjoint_run(4, 0, (5, 4, 6), 8),
+        "checkpoints": lambda e: e.adjoint_run(4, 2, (5, 4, 6), 8),
+    }
+    engine().close()
+    none = fake.live_bytes()
+    for name, call in calls.items():
+        with engine() as e:
+            start = fake.allocations()
+            call(e)
+            count = fake.allocations() - start
+        assert count >= 3
+        for k in range(count):
+            with engine() as e:
+                fake.fail_at(k)
+                with pytest.raises(EngineError):
+                    call(e)
+                fake.fail_at(-1)
+                call(e)
+            assert fake.live_bytes() == none, (name, k)
+
+
+def test_calls_that_run_out_of_memory_leave_nothing_behind(fake_path):
+    run_case(fake_path, "no_leak")
+
+
 # ---- material changes that fail -----------------------------------------------------------------
 
 def _blocks(ids):
