@@ -854,7 +854,6 @@ int build_set_t(LaunchSet* s) {
     for (sjf_engine* e : s->eng) ctr.push_back(e->d_step);
     rc = upload_vec(e0, s->stream, (void**)&s->d_counters, ctr);
     if (rc) return rc;
-    if (rc) return rc;
 
     s->versions.clear();
     for (sjf_engine* e : s->eng) s->versions.push_back(e->version);
@@ -1199,7 +1198,6 @@ int tile_waves(const sjf_engine* e) {
 // 13.0, 15.3; 72x64x56 20.4, 21.0; 96^3 36.1, 42.0; 101^3 39.7, 54.0; 128^3 105.7, 105.3; FP32
 // 192x192x96 80.4, 93.9; 151x133x117 54.4, 70.2; 256x256x128 191.7, 201.7; 150x150x200 90.0, 112.7;
 // 120x160x250 95.9, 120.6; 512x512x256 1061, 1039.
-//
 void choose_tile(sjf_engine* e) {
     if (e->tile_set) return;
     const int rows = default_thread_rows(e), full = e->prec == 8 ? 128 : 256;
@@ -1346,7 +1344,6 @@ int upload_lut_t(sjf_engine* e) {
         const sjf_material& M = e->lut_h[m];
         sjf::MatLut<T>& L = l[m];
         L.inv_eps = (T)(1.0 / M.eps_inf);
-        L.eps_inf = (T)M.eps_inf;
         L.np = M.npoles;
         for (int s = 0; s < M.npoles; ++s) {
             // coefficients formed in FP64 (sigma * w0^2 spans ~1e21 * 1e-22 for Au Drude)

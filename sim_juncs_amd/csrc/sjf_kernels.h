@@ -51,10 +51,9 @@ struct __align__(16) PoleCoef {
 // One entry per material and, last, one of zeros that design voxels index.
 template <typename T>
 struct __align__(16) MatLut {
-    T inv_eps;
-    T eps_inf;
     int np;
     int lorentz_mask;
+    T inv_eps;
     PoleCoef<T> pole[kMaxPoles];
 };
 
@@ -87,7 +86,7 @@ struct StepArgs {
     int nqp;  // polarisation planes per x plane (3 * slots)
     int pml_on[3], plo[3], phi[3];
     long S[3];      // PML slab sizes (cells) per axis
-    T* psi[3];      // per axis [6][S]: E aux (2 comps), H aux pair A (2), H aux pair B (2);
+    T* psi[3];      // per axis [3][S][2]: E auxiliary pair, H pairs A and B (two components each);
                     // step n reads pair A and writes pair B when n is even, the reverse when odd
     const T* coef;  // PML tables: for axis d at coff[d]: bE[n], aE[n], bH[n], aH[n]
     int coff[3];
@@ -2549,8 +2548,8 @@ __global__ void __launch_bounds__(MAXT) k_adj_rows(const AdjArgs<T> g) {
 }
 
 // Fused reverse step over one engine: workgroup w handles tile w after the XCD-aware remap.
-// With the loads of a plane issued together, the FP32 reverse step needs 95 registers with three
-// pole slots (5 wavefronts per SIMD) and 102 with four (4 wavefronts), without spilling.
+// With the loads of a plane issued together, the FP32 reverse step needs 92 registers with three
+// pole slots (5 wavefronts per SIMD) and 98 with four (4 wavefronts).
 template <typename T>
 constexpr int adj_waves() { return sizeof(T) == 4 ? 4 : 1; }
 
