@@ -127,6 +127,12 @@ def step_kernel(info, nz=None):
     return "k_step_z" if nz is not None and info["threads"] < nz else "k_step"
 
 
+def reverse_kernel(threads, nz, batch=""):
+    """Name of the fused reverse kernel of that workgroup size: one y row is one z line of threads,
+    anything larger is rows of threads."""
+    return ("k_adj_step" if threads == -(-nz // 64) * 64 else "k_adj_rows") + batch
+
+
 def set_tile(a, eng):
     """--tile form,rows,xchunk, else the tuned tile of the shape when cached."""
     from sim_juncs_amd import autotune
@@ -189,7 +195,7 @@ def sweep(a):
     wall = time.perf_counter() - t
     _, ms_kernel = b.timed_steps(a.kernel_steps)
     threads, groups = b.launch_info()
-    # the batch default for z lines under 96 cells is the row-of-threads form
+    # the batch default for z lines under 256 cells (FP32) is the row-of-threads form
     kernel = "k_step" if a.batch_tile and a.batch_tile.startswith("register_rows") else "k_step_rows"
     b.close()
     for e in engs:
@@ -233,7 +239,7 @@ def adjoint_batched(a):
         e.close()
     s0 = scns[0]
     workload = f"variants_{len(scns)}_batched"
-    rl = roofline(bytes_rev, ms, "k_adj_step_batch", threads, groups, workload)
+    rl = roofline(bytes_rev, ms, reverse_kernel(threads, s0.shape[2], "_batch"), threads, groups, workload)
     cpu = None if a.no_cpu else cpu_baseline([s0], a.cpu_steps or cpu_budget_steps(s0.cells), s0.steps)
     if cpu:
         cpu["value"] /= 2.0
@@ -275,8 +281,7 @@ def adjoint(a, variants=False):
         eng.close()
     s0 = scns[0]
     workload = ("variants_" if variants else "") + s0.name
-    rkernel = "k_adj_rows" if a.adjoint_tile and a.adjoint_tile.startswith("thread_rows") else "k_adj_step"
-    rl = roofline(rev[0], rev[1], rkernel, rev[2], rev[3], workload)
+    rl = roofline(rev[0], rev[1], reverse_kernel(rev[2], s0.shape[2]), rev[2], rev[3], workload)
     cpu = None if a.no_cpu else cpu_baseline([s0], a.cpu_steps or cpu_budget_steps(s0.cells), s0.steps)
     if cpu:
         # the adjoint costs a forward and a reverse sweep per step (the design fields of every
